@@ -173,8 +173,8 @@ __global__ __launch_bounds__(kStreamThreads) void pack_stream_kernel(StreamArgs 
       }
       continue;
     }
-    // Edge: per-lane predicates, padding, and a byte-wise tail for the chunk
-    // that straddles the right edge (never reading past it).
+    // Edge: per-lane predicates, padding, and the chunk that straddles the
+    // right edge (never reading past it).
     u32x4 pad_vec;
     {
       uint64_t p = a.padding;
@@ -190,16 +190,8 @@ __global__ __launch_bounds__(kStreamThreads) void pack_stream_kernel(StreamArgs 
       if (r >= a.padded_rows) continue;
       u32x4 v = pad_vec;
       if (r < a.m_size0 && c < a.m_size1) {
-        const char* src = a.mat + (r * a.m_stride0 + c) * ES;
-        if (c + CE <= a.m_size1) {
-          v = *(const src_vec_t*)src;
-        } else {
-          union { u32x4 vec; uint8_t b[16]; } tmp;
-          tmp.vec = pad_vec;
-          const int valid = (int)(a.m_size1 - c) * ES;
-          for (int i = 0; i < valid; ++i) tmp.b[i] = ((const uint8_t*)src)[i];
-          v = tmp.vec;
-        }
+        const int valid = c + CE <= a.m_size1 ? 16 : (int)(a.m_size1 - c) * ES;
+        v = load_edge_chunk<ES>(a.mat + (r * a.m_stride0 + c) * ES, valid, a.m_size1 * ES, pad_vec);
       }
       *(u32x4*)(a.tiled + tiled_chunk_offset<kPow2>(a, r, j)) = v;
     }
@@ -240,15 +232,8 @@ __global__ __launch_bounds__(kStreamThreads) void unpack_stream_kernel(StreamArg
       const int64_t r = r0 + u * kBlockRows + (lane >> 3);
       if (r >= a.m_size0) continue;
       const u32x4 v = *(const u32x4*)(a.tiled + tiled_chunk_offset<kPow2>(a, r, j));
-      char* dst = (char*)a.mat + (r * a.m_stride0 + c) * ES;
-      if (c + CE <= a.m_size1) {
-        *(dst_vec_t*)dst = v;
-      } else {
-        union { u32x4 vec; uint8_t b[16]; } tmp;
-        tmp.vec = v;
-        const int valid = (int)(a.m_size1 - c) * ES;
-        for (int i = 0; i < valid; ++i) ((uint8_t*)dst)[i] = tmp.b[i];
-      }
+      store_edge_chunk<ES>((char*)a.mat + (r * a.m_stride0 + c) * ES, v,
+                           c + CE <= a.m_size1 ? 16 : (int)(a.m_size1 - c) * ES);
     }
   }
 }

@@ -17,6 +17,68 @@ template <> struct Chunk<1> { typedef u32x4 aligned_t __attribute__((aligned(1))
 template <> struct Chunk<2> { typedef u32x4 aligned_t __attribute__((aligned(2))); typedef uint16_t elem_t; };
 template <> struct Chunk<4> { typedef u32x4 aligned_t __attribute__((aligned(4))); typedef uint32_t elem_t; };
 
+// Chunks that straddle the right edge of the matrix. Everything stays in named
+// registers: an array indexed at run time is promoted to LDS, and the kernel
+// then reads its workgroup size from the dispatch packet in HOST memory in
+// every edge wave, and loads the elements one after the other. (bf16, 2000 x
+// 3001 into 32x8 tiles 15.5 -> 6.8 us, the same back 16.0 -> 7.1; 2000 x 3008,
+// which has no such chunk, takes 6.9 and 5.9.)
+
+// v shifted right (towards lower addresses) by 0 <= bytes < 16.
+__device__ __forceinline__ u32x4 shift_chunk_right(u32x4 v, uint32_t bytes) {
+  const bool by8 = (bytes & 8) != 0, by4 = (bytes & 4) != 0;
+  const uint32_t a0 = by8 ? v.z : v.x, a1 = by8 ? v.w : v.y, a2 = by8 ? 0u : v.z, a3 = by8 ? 0u : v.w;
+  const uint32_t b0 = by4 ? a1 : a0, b1 = by4 ? a2 : a1, b2 = by4 ? a3 : a2, b3 = by4 ? 0u : a3;
+  return u32x4{__builtin_amdgcn_alignbyte(b1, b0, bytes & 3), __builtin_amdgcn_alignbyte(b2, b1, bytes & 3),
+               __builtin_amdgcn_alignbyte(b3, b2, bytes & 3), __builtin_amdgcn_alignbyte(0u, b3, bytes & 3)};
+}
+
+// The first `valid` bytes (0..16) of v, the rest from `pad`.
+__device__ __forceinline__ u32x4 pad_chunk(u32x4 v, u32x4 pad, int valid) {
+  u32x4 out;
+#pragma unroll
+  for (int d = 0; d < 4; ++d) {
+    const int n = valid - 4 * d;
+    const uint32_t keep = n >= 4 ? ~0u : n <= 0 ? 0u : (1u << (8 * n)) - 1u;
+    out[d] = (v[d] & keep) | (pad[d] & ~keep);
+  }
+  return out;
+}
+
+// The chunk at `src` of which `valid` bytes (0..16) lie inside its row of
+// row_bytes bytes; the rest is padding. A row of 16 bytes and more is read with
+// one 16-byte load that ends at the row's end, shorter ones by elements.
+template <int ES>
+__device__ __forceinline__ u32x4 load_edge_chunk(const char* src, int valid, int64_t row_bytes, u32x4 pad) {
+  typedef typename Chunk<ES>::aligned_t mat_vec_t;
+  typedef typename Chunk<ES>::elem_t elem_t;
+  if (valid <= 0) return pad;
+  u32x4 v = {0u, 0u, 0u, 0u};
+  if (row_bytes >= 16) {
+    v = *(const mat_vec_t*)(src - (16 - valid));
+    v = shift_chunk_right(v, 16 - valid);
+  } else {
+#pragma unroll
+    for (int e = 0; e < 16 / ES; ++e)
+      if (e * ES < valid) v[e * ES / 4] |= (uint32_t)((const elem_t*)src)[e] << (8 * (e * ES % 4));
+  }
+  return pad_chunk(v, pad, valid);
+}
+
+// The first `valid` bytes (whole elements) of v to `dst`.
+template <int ES>
+__device__ __forceinline__ void store_edge_chunk(char* dst, u32x4 v, int valid) {
+  typedef typename Chunk<ES>::aligned_t mat_vec_t;
+  typedef typename Chunk<ES>::elem_t elem_t;
+  if (valid >= 16) {
+    *(mat_vec_t*)dst = v;
+    return;
+  }
+#pragma unroll
+  for (int e = 0; e < 16 / ES; ++e)
+    if (e * ES < valid) ((elem_t*)dst)[e] = (elem_t)(v[e * ES / 4] >> (8 * (e * ES % 4)));
+}
+
 constexpr int kStreamThreads = 256;
 constexpr int kStreamUnroll = 2;
 
@@ -145,8 +207,8 @@ __device__ __forceinline__ void stream_pow2_body(const Pow2Args a) {
     }
     return;
   }
-  // Edge blocks: per-lane predicates, padding (pack), byte-wise handling of the
-  // chunk that straddles the right edge.
+  // Edge blocks: per-lane predicates, padding (pack), the chunk that straddles
+  // the right edge.
   if (j0 + jl >= col_limit) return;
   const int64_t c = (int64_t)(j0 + jl) * CE;
   u32x4 pad_vec;
@@ -163,16 +225,11 @@ __device__ __forceinline__ void stream_pow2_body(const Pow2Args a) {
     if (r >= row_limit) continue;
     const bool in_matrix = r < a.m_size0 && c < a.m_size1;
     const int valid = in_matrix ? (c + CE <= a.m_size1 ? 16 : (int)(a.m_size1 - c) * ES) : 0;
-    union { u32x4 vec; uint8_t b[16]; } tmp;
     if (kPack) {
-      tmp.vec = pad_vec;
-      if (valid == 16) tmp.vec = *(const mat_vec_t*)(mat_base + mat_off[u]);
-      else for (int i = 0; i < valid; ++i) tmp.b[i] = ((const uint8_t*)(mat_base + mat_off[u]))[i];
-      *(u32x4*)(tiled_base + tiled_off[u]) = tmp.vec;
+      *(u32x4*)(tiled_base + tiled_off[u]) =
+          load_edge_chunk<ES>(mat_base + mat_off[u], valid, a.m_size1 * ES, pad_vec);
     } else {
-      tmp.vec = *(const u32x4*)(tiled_base + tiled_off[u]);
-      if (valid == 16) *(mat_vec_t*)((char*)mat_base + mat_off[u]) = tmp.vec;
-      else for (int i = 0; i < valid; ++i) ((uint8_t*)mat_base + mat_off[u])[i] = tmp.b[i];
+      store_edge_chunk<ES>((char*)mat_base + mat_off[u], *(const u32x4*)(tiled_base + tiled_off[u]), valid);
     }
   }
 }

@@ -476,14 +476,7 @@ __device__ __forceinline__ void unpack_transpose_block_body(const TransArgs& a) 
     for (int i = 0; i < CE; ++i) {
       const int64_t r = g * CE + i;
       if (r >= a.m_size0) continue;
-      union { u32x4 vec; elem_t e[CE]; } row;
-      row.vec = block_row(v[0], i);
-      char* p = dst + r * a.m_pitch_bytes;
-      if (n_cols == CE) {
-        *(mat_vec_t*)p = row.vec;
-      } else {
-        for (int j = 0; j < n_cols; ++j) ((elem_t*)p)[j] = row.e[j];
-      }
+      store_edge_chunk<ES>(dst + r * a.m_pitch_bytes, block_row(v[0], i), n_cols * ES);
     }
   }
 }

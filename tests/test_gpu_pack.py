@@ -75,6 +75,25 @@ def test_streaming_shapes_with_ragged_edges(uk, cuda, type_flag, t0, t1, rows, c
             assert np.array_equal(gpucase.run_unpack(ucase), ucase.run_oracle()), (to,)
 
 
+@pytest.mark.parametrize("type_flag,t0,t1", [
+    (F.PACK_TYPE_I8I8, 32, 16), (F.PACK_TYPE_F16F16, 32, 8), (F.PACK_TYPE_F32F32, 8, 4),
+    (F.PACK_TYPE_BF16BF16, 32, 32), (F.PACK_TYPE_I32I32, 24, 12),
+])
+def test_every_width_of_the_last_chunk(uk, cuda, type_flag, t0, t1):
+    """Rows shorter than one 16-byte chunk, and every number of elements that a
+    row's last chunk can hold, with a padding value (exact)."""
+    rng = np.random.default_rng(7 * t0 + t1)
+    ce = 16 // F.PACK_ELEM_BYTES[type_flag]
+    for cols in [*range(1, 2 * ce + 2), *range(8 * ce + 1, 9 * ce + 1)]:
+        for ti in (0, 1):
+            o0, o1 = -(-37 // t0), -(-cols // t1)
+            case = ukref.PackCase(rng, type_flag, o0, o1, t0, t1, transpose_inner=ti, pad=3, in_size=(37, cols))
+            assert np.array_equal(gpucase.run_pack(case), case.run_oracle()), (cols, ti)
+            if type_flag != F.PACK_TYPE_I8I8:
+                ucase = ukref.UnpackCase(rng, type_flag, o0, o1, t0, t1, transpose_inner=ti, out_size=(37, cols))
+                assert np.array_equal(gpucase.run_unpack(ucase), ucase.run_oracle()), (cols, ti)
+
+
 @pytest.mark.parametrize("type_flag,tr,tc,rows,cols", [
     (F.PACK_TYPE_F16F16, 8, 32, 1001, 333),    # f16 right-hand side: K0 = 8 rows x N0 = 32 columns
     (F.PACK_TYPE_F16F16, 16, 32, 200, 95),     # two 16-byte row groups per tile
