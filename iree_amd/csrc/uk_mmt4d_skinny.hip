@@ -500,6 +500,8 @@ int launch_cfg(SkinnyArgs a, int chunks, hipStream_t s) {
   // halves: N = 4096, K = 4096 f16 as 256 workgroups of 16 columns 8.4 us, as
   // 128 of 32 with K split over two rows and the launch that adds them 10.85;
   // K = 1024: 4.8 against 7.4).
+  // (a batch whose K is split as well: the planes share that many with their rows)
+  if (a.batch > 1 && chunks > 1) per_plane = (2 * cus + a.batch * chunks - 1) / (a.batch * chunks);
   int blocks = a.N < per_plane ? a.N : per_plane;
   if (a.batch <= 1) blocks = a.N * 2 < per_plane ? a.N * 2 : per_plane;
   // K split over workgroup rows: the rows share the compute units, one round in
@@ -587,9 +589,36 @@ iree_amd_uk_mmt4d_params_t exchanged(const iree_amd_uk_mmt4d_params_t& p) {
 }
 }  // namespace
 
-// `batch` problems of one narrow shape as the planes of one launch; only what a
-// single launch row takes (K short enough to stay in registers), at most 65535
-// entries and batch strides of whole 16 bytes.
+namespace {
+// Adds the `chunks` partial sums of a K split (dense arrays of `elems` elements
+// each) in order into the result at `out`, after the old result when accumulating.
+int reduce_chunks(const iree_amd_uk_mmt4d_params_t& p, const void* partials, int64_t chunks, int64_t elems,
+                  void* out, hipStream_t s) {
+  KSplitReduceArgs r;
+  r.partials = partials;
+  r.slices = (int)chunks;
+  r.M = 1; r.N = 1;
+  r.flat_elems = elems;
+  r.out = out;
+  r.out_stride_bytes = 0;
+  r.accumulate = (p.flags & IREE_AMD_UK_FLAG_MMT4D_ACCUMULATE) != 0;
+  r.row_major_out = 0; r.out_rows = r.out_cols = 0;
+  r.out_scale = 1.0f;
+  const uint32_t type = p.flags & IREE_AMD_UK_FLAG_MMT4D_TYPE_MASK;
+  r.acc_is_float = type != IREE_AMD_UK_FLAG_MMT4D_TYPE_S8S8S32;
+  r.out_kind = type == IREE_AMD_UK_FLAG_MMT4D_TYPE_F16F16F16 ? 1
+               : type == IREE_AMD_UK_FLAG_MMT4D_TYPE_BF16BF16BF16 ? 2 : 0;
+  return launch_ksplit_reduce(r, s);
+}
+}  // namespace
+
+// `batch` problems of one narrow shape as the planes of one launch, at most
+// 65535 entries and batch strides of whole 16 bytes. A K that one launch row
+// cannot hold in registers, or that leaves half of the compute units idle, is
+// split over workgroup rows as for a single problem (launch_mmt4d_skinny); the
+// partial sums of all entries are then added by one second launch. (The values
+// of a decode step of attention, 32 heads x 1x128x32768 f16, 268 MB: 340 us as
+// 32 single calls of two launches each, 57 as one.)
 int launch_batch_mmt4d_skinny(const iree_amd_uk_mmt4d_params_t& p0, int64_t batch, int64_t lhs_batch_stride,
                               int64_t rhs_batch_stride, int64_t out_batch_stride, hipStream_t s) {
   if (!mmt4d_skinny_supported(p0.flags, p0.M0, p0.N0, p0.K0)) return IREE_AMD_UK_STATUS_NOT_FOUND;
@@ -606,8 +635,37 @@ int launch_batch_mmt4d_skinny(const iree_amd_uk_mmt4d_params_t& p0, int64_t batc
   if (p.M != 1 || p.K == 0 || p.N > 0x3FFFFFF || batch > 65535)
     return IREE_AMD_UK_STATUS_NOT_FOUND;
   const int64_t steps = (k_elems + mk - 1) / mk;   // (the last one may be partial)
-  if (steps > max_steps_per_launch(mk)) return IREE_AMD_UK_STATUS_NOT_FOUND;
+  const int max_steps = max_steps_per_launch(mk);
+  const int cus = device_cu_count();
+  int64_t chunks = (steps + max_steps - 1) / max_steps;
+  const int64_t col_blocks = p.N < cus ? p.N : cus;
+  if (col_blocks * batch * chunks * 2 <= cus && steps >= 64) {
+    int64_t more = cus / (col_blocks * batch);
+    if (more > steps / 32) more = steps / 32;
+    if (more > 8) more = 8;
+    if (more > chunks) chunks = more;
+  }
+  const int64_t elems = p.N * p.M0 * 32;
+  const bool transposed = (p.flags & kTransposedOut) != 0;
+  const bool dense_out = out_batch_stride == elems &&
+                         (!transposed || p.N == 1 || p.out_stride0 == (int64_t)p.M0 * 32);
   const BatchStrides bs = {batch, lhs_batch_stride, rhs_batch_stride, out_batch_stride};
+  if (chunks > 1 && chunks <= 65535 && dense_out) {
+    const int64_t chunk_steps = (steps + chunks - 1) / chunks;
+    chunks = (steps + chunk_steps - 1) / chunk_steps;
+    const size_t bytes = (size_t)(chunks * batch * elems * 4);
+    ScratchLease lease(s, bytes);
+    if (lease.overflowed()) return scratch_overflow_status("batch_mmt4d: the K split of narrow tiles", bytes);
+    if (lease.ptr() && chunks > 1) {
+      const int st = launch_chunk(p, (int)chunks, (int)chunk_steps, lease.ptr(), s, &bs);
+      if (st) return st;
+      Mmt4dTypeInfo ti;
+      mmt4d_type_info(p.flags, &ti);
+      return reduce_chunks(p, lease.ptr(), chunks, batch * elems,
+                           (char*)p.out_buffer + p.out_offset * ti.out_bytes, s);
+    }
+  }
+  if (steps > max_steps) return IREE_AMD_UK_STATUS_NOT_FOUND;
   return launch_chunk(p, 1, (int)steps, nullptr, s, &bs);
 }
 
@@ -655,21 +713,7 @@ int launch_mmt4d_skinny(const iree_amd_uk_mmt4d_params_t& p0, hipStream_t s) {
     if (scratch && chunks > 1) {
       int st = launch_chunk(p, (int)chunks, (int)chunk_steps, scratch, s);
       if (st) return st;
-      KSplitReduceArgs r;
-      r.partials = scratch;
-      r.slices = (int)chunks;
-      r.M = 1; r.N = 1;
-      r.flat_elems = elems;
-      r.out = (char*)p.out_buffer + p.out_offset * ti.out_bytes;
-      r.out_stride_bytes = 0;
-      r.accumulate = (p.flags & IREE_AMD_UK_FLAG_MMT4D_ACCUMULATE) != 0;
-      r.row_major_out = 0; r.out_rows = r.out_cols = 0;
-      r.out_scale = 1.0f;
-      r.acc_is_float = (p.flags & IREE_AMD_UK_FLAG_MMT4D_TYPE_MASK) != IREE_AMD_UK_FLAG_MMT4D_TYPE_S8S8S32;
-      const uint32_t type = p.flags & IREE_AMD_UK_FLAG_MMT4D_TYPE_MASK;
-      r.out_kind = type == IREE_AMD_UK_FLAG_MMT4D_TYPE_F16F16F16 ? 1
-                   : type == IREE_AMD_UK_FLAG_MMT4D_TYPE_BF16BF16BF16 ? 2 : 0;
-      return launch_ksplit_reduce(r, s);
+      return reduce_chunks(p, scratch, chunks, elems, (char*)p.out_buffer + p.out_offset * ti.out_bytes, s);
     }
   }
   if (steps <= max_steps) return launch_chunk(p, 1, (int)steps, nullptr, s);
@@ -744,7 +788,9 @@ int launch_chunk(const iree_amd_uk_mmt4d_params_t& p, int chunks, int chunk_step
   if (chunks > 1) {
     a.out = (char*)scratch;
     a.accumulate = 0;
-    a.chunk_out_elems = (int64_t)p.N * p.M0 * 32;
+    const int64_t elems = (int64_t)p.N * p.M0 * 32;
+    a.chunk_out_elems = elems * a.batch;
+    a.out_batch_bytes = elems * 4;
     a.out_stride_elems = (int64_t)p.M0 * 32;     // (partial sums are dense)
   }
   switch (p.flags & IREE_AMD_UK_FLAG_MMT4D_TYPE_MASK) {
@@ -848,21 +894,7 @@ int launch_matmul_rows_skinny(const iree_amd_uk_mmt4d_params_t& p, int64_t M, in
     default: return IREE_AMD_UK_STATUS_NOT_FOUND;
   }
   if (st || chunks == 1) return st;
-  KSplitReduceArgs r;
-  r.partials = lease->ptr();
-  r.slices = (int)chunks;
-  r.M = 1; r.N = 1;
-  r.flat_elems = M * out_cols;
-  r.out = (char*)p.out_buffer + p.out_offset * ti.out_bytes;
-  r.out_stride_bytes = 0;
-  r.accumulate = (p.flags & IREE_AMD_UK_FLAG_MMT4D_ACCUMULATE) != 0;
-  r.row_major_out = 0; r.out_rows = r.out_cols = 0;
-  r.out_scale = 1.0f;
-  r.acc_is_float = (p.flags & IREE_AMD_UK_FLAG_MMT4D_TYPE_MASK) != IREE_AMD_UK_FLAG_MMT4D_TYPE_S8S8S32;
-  const uint32_t type = p.flags & IREE_AMD_UK_FLAG_MMT4D_TYPE_MASK;
-  r.out_kind = type == IREE_AMD_UK_FLAG_MMT4D_TYPE_F16F16F16 ? 1
-               : type == IREE_AMD_UK_FLAG_MMT4D_TYPE_BF16BF16BF16 ? 2 : 0;
-  return launch_ksplit_reduce(r, s);
+  return reduce_chunks(p, lease->ptr(), chunks, M * out_cols, (char*)p.out_buffer + p.out_offset * ti.out_bytes, s);
 }
 
 }  // namespace uk

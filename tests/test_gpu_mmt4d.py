@@ -1032,6 +1032,29 @@ def test_batch_mmt4d_bit_exact(uk, cuda, type_flag, tile, batch, shape, gap, acc
     assert np.array_equal(got.view(np.uint8), want.view(np.uint8))
 
 
+@pytest.mark.parametrize("type_flag,tile,batch,shape,gap", [
+    # more K than one launch row keeps in registers (256 steps; fp8 128): split
+    # over workgroup rows, the last row shorter, a partial last step
+    (F.MMT4D_TYPE_F16F16F32, (1, 32, 8), 5, (1, 3, 2 * 700), (0, 0, 0)),
+    (F.MMT4D_TYPE_BF16BF16BF16, (8, 32, 8), 3, (1, 4, 2 * 300 + 1), (8, 0, 0)),
+    (F.MMT4D_TYPE_S8S8S32, (4, 32, 16), 2, (1, 2, 2 * 515), (0, 64, 0)),
+    (F.MMT4D_TYPE_F8E4M3F8E4M3F32, (2, 32, 16), 3, (1, 2, 4 * 130), (0, 0, 0)),
+    (F.MMT4D_TYPE_F16F16F32, (32, 4, 8), 3, (2, 1, 2 * 300), (0, 0, 0)),     # narrow N: tiles stored transposed
+    # a K that fits, but compute units to spare
+    (F.MMT4D_TYPE_F16F16F32, (2, 32, 8), 2, (1, 1, 2 * 64), (0, 0, 0)),
+    # results with gaps between the entries: entry by entry
+    (F.MMT4D_TYPE_F16F16F32, (1, 32, 8), 2, (1, 2, 2 * 300), (0, 0, 32)),
+])
+@pytest.mark.parametrize("acc", [False, True])
+def test_batch_of_narrow_tiles_with_a_long_k(uk, cuda, type_flag, tile, batch, shape, gap, acc):
+    """Small integers, whose sums are exact in any order."""
+    rng = np.random.default_rng(77 + batch + shape[2])
+    case = ukref.BatchMmt4dCase(rng, type_flag, batch, *shape, *tile, accumulate=acc, gap=gap)
+    if type_flag == F.MMT4D_TYPE_BF16BF16BF16:
+        case.flags |= F.MMT4D_SKIP_INTERMEDIATE_ROUNDINGS
+    assert np.array_equal(gpucase.run_batch_mmt4d(case), case.run_oracle())
+
+
 def test_batch_mmt4d_degenerate_and_large_batch(uk, cuda):
     rng = np.random.default_rng(8200)
     # batch == 0: nothing is touched
