@@ -154,6 +154,11 @@ __device__ __forceinline__ void load_bits(const void* p, uint32_t* dst) {
 // Rows [m_base, m_base + m_eff), m_eff <= 16, through the per-wave-column kernel
 // (uk_quant_gemv.hip); IREE_AMD_UK_STATUS_NOT_FOUND for shapes it does not take.
 int launch_dequant_gemv_i4(const i4::I4Args& p, int m_base, int m_eff, hipStream_t s);
+// Many rows of activations (uk_quant_gemm.hip): tiled weights, packed uint4 zero
+// points, power-of-two groups of 32 and more, K in whole 128s, 16-byte aligned
+// operands (the caller has checked); NOT_FOUND for sizes that 32-bit offsets
+// cannot address.
+int launch_dequant_gemm_i4(const i4::I4Args& p, hipStream_t s);
 
 }  // namespace uk
 

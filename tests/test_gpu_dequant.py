@@ -301,3 +301,23 @@ def test_reassociated_on_the_per_thread_default_stream(uk, cuda, M, N, K, gs, ti
 ])
 def test_reassociated_other_shapes(uk, cuda, M, N, K, gs, zp_u4, tiled):
     run_reassoc_case(uk, M, N, K, gs, zp_u4, tiled, seed=M + N)
+
+
+@pytest.mark.parametrize("M,N,K,gs", [
+    (65, 32, 128, 128),       # one span, one group, half of a 64-column tile
+    (66, 96, 384, 32),        # groups of 32: a refill of scales per span; three spans
+    (127, 288, 896, 128),     # 7 groups: columns whose scales start 2 and zero points 1 byte past a boundary
+    (128, 352, 1280, 64),     # 20 groups, the last column block of a wave past N
+    (129, 64, 2304, 256),     # groups of two spans, nine spans
+    (193, 160, 640, 128),     # 5 groups, rows past M in the last tile
+    (100, 64, 14336, 128),    # few tiles: K split over workgroup rows
+    (257, 576, 1024, 1024),   # one group for all of K
+    (300, 4128, 256, 64),     # many tiles, two spans
+])
+def test_many_rows(uk, cuda, M, N, K, gs):
+    """The tiled kernel for prompts: edges of row and column tiles, the shortest
+    K, group counts that leave the groups of a column unaligned. Every product
+    is exact and the sums are f32, so the result is within one f16 unit of the
+    oracle's."""
+    err, mag = run_case(uk, M, N, K, gs, True, True, seed=M + N + K, want_path="dequant_i4:gemm", repeats=1)
+    assert err <= float(np.spacing(np.float16(max(1.0, mag))))
