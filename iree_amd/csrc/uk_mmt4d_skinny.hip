@@ -614,8 +614,8 @@ int reduce_chunks(const iree_amd_uk_mmt4d_params_t& p, const void* partials, int
 
 // `batch` problems of one narrow shape as the planes of one launch, at most
 // 65535 entries and batch strides of whole 16 bytes. A K that one launch row
-// cannot hold in registers, or that leaves half of the compute units idle, is
-// split over workgroup rows as for a single problem (launch_mmt4d_skinny); the
+// cannot hold in registers is split over workgroup rows as for a single problem
+// (launch_mmt4d_skinny), into more of them where compute units would idle; the
 // partial sums of all entries are then added by one second launch. (The values
 // of a decode step of attention, 32 heads x 1x128x32768 f16, 268 MB: 340 us as
 // 32 single calls of two launches each, 57 as one.)
@@ -639,7 +639,10 @@ int launch_batch_mmt4d_skinny(const iree_amd_uk_mmt4d_params_t& p0, int64_t batc
   const int cus = device_cu_count();
   int64_t chunks = (steps + max_steps - 1) / max_steps;
   const int64_t col_blocks = p.N < cus ? p.N : cus;
-  if (col_blocks * batch * chunks * 2 <= cus && steps >= 64) {
+  // (a K that fits stays whole even where compute units idle: the second launch
+  // costs more than it gives; 8 heads x 1x128x1216 f16 as part of a decode step
+  // 10.8 us whole, 14.4 as two slices)
+  if (chunks > 1 && col_blocks * batch * chunks * 2 <= cus) {
     int64_t more = cus / (col_blocks * batch);
     if (more > steps / 32) more = steps / 32;
     if (more > 8) more = 8;
