@@ -150,10 +150,16 @@ int launch_variant(const MfmaArgs& a0, hipStream_t s) {
     return IREE_AMD_UK_STATUS_NOT_FOUND;
 }
 
-// The four macro tiles (in outer tiles of 32 rows: 8x8, 8x4, 4x8, 4x4) with
-// their LDS rings: 8 K-steps and a barrier every 2 for the single-occupancy
-// tiles (fp8 and the 16-row shapes, whose K-step is twice as large: 5 and every
-// step), 6 (wide: 3) for the double-occupancy ones.
+// Configurations that also have the macro tiles with a side of 192: their block
+// of 16 rows deals the operand rows of such a tile evenly to the four waves.
+template <typename Cfg, bool kSiluMul>
+constexpr bool kHasMediumTiles = Cfg::kRows == 16 && !kSiluMul;
+
+// The macro tiles (in outer tiles of 32 rows: 8x8, 8x4, 4x8, 4x4, and 8x6, 6x8,
+// 6x6) with their LDS rings: 8 K-steps and a barrier every 2 for the
+// single-occupancy tiles (fp8 and the 16-row shapes, whose K-step is twice as
+// large: 5 and every step; 6x6: 6), 6 (wide: 3) for the double-occupancy ones.
+constexpr int kTilesWithMedium = 7;
 template <typename Cfg, bool kSiluMul>
 int launch_by_index(int v, const MfmaArgs& b, hipStream_t s) {
   constexpr int S = 32 / Cfg::kRows;
@@ -162,6 +168,15 @@ int launch_by_index(int v, const MfmaArgs& b, hipStream_t s) {
     case 0: return launch_variant<Cfg, 4 * S, 4 * S, kWide ? 5 : 8, kWide ? 1 : 2, 1, kSiluMul>(b, s);
     case 1: return launch_variant<Cfg, 4 * S, 2 * S, kWide ? 3 : 6, kWide ? 1 : 2, 2, kSiluMul>(b, s);
     case 2: return launch_variant<Cfg, 2 * S, 4 * S, kWide ? 3 : 6, kWide ? 1 : 2, 2, kSiluMul>(b, s);
+    case 4:
+      if constexpr (kHasMediumTiles<Cfg, kSiluMul>) return launch_variant<Cfg, 4 * S, 3 * S, 5, 1, 1>(b, s);
+      return IREE_AMD_UK_STATUS_NOT_FOUND;
+    case 5:
+      if constexpr (kHasMediumTiles<Cfg, kSiluMul>) return launch_variant<Cfg, 3 * S, 4 * S, 5, 1, 1>(b, s);
+      return IREE_AMD_UK_STATUS_NOT_FOUND;
+    case 6:
+      if constexpr (kHasMediumTiles<Cfg, kSiluMul>) return launch_variant<Cfg, 3 * S, 3 * S, 6, 1, 1>(b, s);
+      return IREE_AMD_UK_STATUS_NOT_FOUND;
     default: return launch_variant<Cfg, 2 * S, 2 * S, S == 2 ? 4 : 8, S == 2 ? 1 : 2, 1, kSiluMul>(b, s);
   }
 }
@@ -215,134 +230,57 @@ int launch_k_split(const MfmaArgs& a, int v, int slices, hipStream_t s) {
   return st;
 }
 
-template <typename Cfg, bool kSiluMul = false>
-int launch_cfg(const MfmaArgs& a, hipStream_t s) {
-  // Pick the macro tile. 256x256 (one workgroup per compute unit, all of its
-  // registers) has the best operand reuse: 1 KiB of operand per two MFMAs.
-  // 256x128 / 128x256 run two workgroups per compute unit, so one workgroup's
-  // output stores overlap the other's MFMAs, and they spread a problem over
-  // more compute units; 128x128 spreads small problems further still.
-  // Estimated cost of a variant, in units of one 32x32 block row of MFMAs:
-  // rounds of resident workgroups x work per workgroup / relative efficiency
-  // (measured on MI355X against the 256x256 tile's rate).
-  // LDS rings: 8 K-steps with a barrier every 2 for the single-occupancy
-  // tiles (fp8, whose K-step is twice as large: 5 with a barrier every step),
-  // 6 (fp8: 3) for the double-occupancy ones.
+// Estimated time in microseconds of the 16-row shapes on macro tile v with K in
+// `slices`, for M x N outer tiles. A step is 64 bytes of K. A workgroup's step
+// takes longer the more of the compute units are busy (power, the L2s), from
+// idle to idle + busy; two workgroups on one compute unit take
+// shared times as long as one; a row-major left-hand side with the weights it
+// meets, which come from memory, row_major times. The constants are a fit to
+// the measured times of every tile and slice count on 457 problems (f16, bf16,
+// i8; 34 to 4096 rows, 64 to 14336 columns, K 256 to 14336, under sustained
+// load): what the estimate picks is 0.9 % slower than the best of them on
+// average and at most 25 %, 1.2 % on 420 other problems, where the rule before
+// it, on the first four tiles, was at 4.1 %. A bf16 1984 x 4128 x 3008 mmt4d takes
+// 45 us on 192x192 tiles (242 workgroups) and 58 on the best of the first four.
+struct MediumTile { int wm, wn, occ; float idle, busy, shared, row_major; };
+constexpr MediumTile kMediumTiles[kTilesWithMedium] = {
+    {4, 4, 1, 0.386f, 0.321f, 1.0f, 1.152f},   {4, 2, 2, 0.291f, 0.148f, 1.819f, 1.143f},
+    {2, 4, 2, 0.255f, 0.177f, 1.856f, 1.126f}, {2, 2, 2, 0.133f, 0.128f, 1.890f, 1.060f},
+    {4, 3, 1, 0.354f, 0.275f, 1.0f, 1.112f},   {3, 4, 1, 0.354f, 0.275f, 1.0f, 1.101f},
+    {3, 3, 1, 0.258f, 0.245f, 1.0f, 1.083f}};
+inline double estimate_us(const MfmaArgs& a, int out_bytes, int v, int64_t M, int64_t N, int slices) {
+  const MediumTile& t = kMediumTiles[v];
   const int cus = device_cu_count();
-  // (fp8 runs the two-per-compute-unit tiles on a ring of only 3 K-steps:
-  // 2048 x 28672 x 4096 measured 238 us with the large tile, 267 with 256x128.
-  // With the SiLU epilogue, whose arithmetic the second workgroup hides and
-  // whose output is an eighth of the bytes, it is the other way round: 218
-  // against 198 us.)
-  // S: blocks per 32 rows. The 16-row shapes and fp8 have K-steps of twice the
-  // bytes ("wide"), hence the shorter rings.
-  constexpr int S = 32 / Cfg::kRows;
-  constexpr bool kWide = Cfg::kSub == 2 || S == 2;
-  constexpr bool kShallow = Cfg::kSub == 2 && !kSiluMul;
-  struct Variant { int wm, wn, occ; double eff_alone, eff_full; };
-  // (16-row shapes: 256x128 measured 115 us against 104 for 256x256 at 4096^3)
-  constexpr double kEffAlone = kSiluMul ? 1.0 : kShallow ? 0.85 : S == 2 ? 0.86 : 0.9;
-  constexpr double kEffFull = kSiluMul ? 1.05 : kShallow ? 0.82 : S == 2 ? 0.9 : 0.94;
-  static const Variant variants[4] = {{4, 4, 1, 1.0, 1.0},
-                                      {4, 2, 2, kEffAlone, kEffFull},
-                                      {2, 4, 2, kEffAlone, kEffFull},
-                                      {2, 2, 2, 0.7, 0.75}};
-  // cost of variant v on an M x N (outer tiles) problem
-  auto cost_of = [&](int v, int64_t M, int64_t N, int64_t k_slices = 1) -> double {
-    const Variant& t = variants[v];
-    const int64_t tiles = ceil_div(M, (int64_t)2 * t.wm) * ceil_div(N, (int64_t)2 * t.wn) * k_slices *
-                          (a.batch > 1 ? a.batch : 1);
-    const int64_t slots = (int64_t)t.occ * cus;
-    const double work = t.wm * t.wn;
-    double cost = (double)(tiles / slots) * t.occ * work / t.eff_full;
-    const int64_t rest = tiles % slots;
-    if (rest > 0) {
-      const int resident = (int)ceil_div(rest, (int64_t)cus);   // workgroups sharing a compute unit
-      cost += resident * work / (resident == t.occ ? t.eff_full : t.eff_alone);
-    }
-    // Of the two half-size tiles the one with more columns than rows is the
-    // faster one for the SiLU form (the gate/up matmul of the fp8 MLP block
-    // alone, sustained: 187.7 -> 180.0 us; inside the block 292 -> 289). For
-    // row-major results on the 32-row instructions the two measure either way:
-    // 128x256 ahead by 3-7 % when the call is repeated on operands that stay
-    // in the last-level cache (fp8 2048 x 4096 x 14336 100.6 -> 97.4 us),
-    // 256x128 ahead by 2 % inside the MLP block, where the weights come from
-    // memory every time (block 289 -> 283 us): the latter is what a model does,
-    // so those keep the first of the two.
-    if (kSiluMul && Cfg::kRows == 32 && v == 1) cost *= 1.03;
-    // A row-major left-hand side is the dearer operand to fetch (half or
-    // quarter cache lines per row and K-step, each line asked for again on the
-    // next step): tiles with more rows than columns pay most. Measured at
-    // 2048 x 4096 x 4096 against the packed operand, K-steps of 64 bytes of a
-    // row (f16, i8 on the 16-row instruction; fp8 alike): 256x256 1.01,
-    // 256x128 1.09-1.14, 128x256 1.02-1.03, 128x128 1.13; K-steps of 32 bytes
-    // (i8 otherwise): 1.16, 1.37, 1.06, 1.28.
-    if (a.lhs_row_major) {
-      constexpr bool kHalfLines = Cfg::kRows == 16 || Cfg::kSub == 2;
-      static const double penalty[2][4] = {{1.16, 1.37, 1.06, 1.28}, {1.02, 1.13, 1.03, 1.13}};
-      cost *= penalty[kHalfLines][v];
-    }
-    return cost;
-  };
-  auto pick = [&](int64_t M, int64_t N, double* out_cost) -> int {
-    int best = 0;
-    double best_cost = 0;
-    for (int v = 0; v < 4; ++v) {
-      const double cost = cost_of(v, M, N);
-      if (v == 0 || cost < best_cost * 0.999) { best = v; best_cost = cost; }
-    }
-    *out_cost = best_cost;
-    return best;
-  };
-  auto launch = [&](int v, const MfmaArgs& b) -> int { return launch_by_index<Cfg, kSiluMul>(v, b, s); };
-  double best_cost = 0;
-  const int best = pick(a.M, a.N, &best_cost);
-  // Few macro tiles and a long K (a few hundred rows against a wide K, as in the
-  // down projection of an MLP at small batch) leave most compute units idle:
-  // K is then split over workgroup rows. Estimated times in microseconds: cost
-  // units (block rows of MFMAs per K-step) x K-steps x the measured time of a
-  // unit, plus, for a split, the second launch and the traffic of the partial
-  // sums (written once, read once, at about 3 TB/s).
-  if constexpr (!kSiluMul) {
-    const Variant& bv = variants[best];
-    const int64_t best_tiles = ceil_div((int64_t)a.M, (int64_t)2 * bv.wm) * ceil_div((int64_t)a.N, (int64_t)2 * bv.wn);
-    if (a.k_slices == 0 && a.batch <= 1 && a.ksteps >= 64 && best_tiles * 2 <= (int64_t)bv.occ * cus) {
-      const double unit_us = Cfg::kStepUs / 16.0;
-      const double out_mb = (double)a.M * a.N * 4096.0 / 1e6;
-      // A split must win by 5 % (with 10 %, 512 x 4096 x 4096 f16 stayed unsplit
-      // at 31.2 us where two slices of 128x128 tiles take 26.5; over 21 shapes
-      // of few tiles in f16 and i8 the lower bar gained up to 15 % and cost at
-      // most 4 %).
-      double best_us = best_cost * a.ksteps * unit_us * 0.95;
-      int split_v = -1, split_n = 0;
-      for (int v = 0; v < 4; ++v) {
-        // (up to 64 rows: with the tile and slice count forced, 128x128 tiles
-        // won on every such shape measured, by up to 10 % over what this
-        // estimate picked among the larger tiles, whose rows are as idle and
-        // whose workgroups are half as many)
-        if (a.M <= 2 && v != 3) continue;
-        for (int n = 2; n <= 8; ++n) {
-          if (a.ksteps / n < 24) break;
-          const int64_t tiles = ceil_div((int64_t)a.M, (int64_t)2 * variants[v].wm) *
-                                ceil_div((int64_t)a.N, (int64_t)2 * variants[v].wn) * n;
-          if (tiles > (int64_t)variants[v].occ * cus) break;     // at most one round
-          const double us = cost_of(v, a.M, a.N, n) * ceil_div((int64_t)a.ksteps, (int64_t)n) * unit_us + 6.0 +
-                            (n + 1 + (a.accumulate ? 1 : 0)) * out_mb / 3.0;
-          if (us < best_us) { best_us = us; split_v = v; split_n = n; }
-        }
-      }
-      if (split_n > 1) {
-        const int st = launch_k_split<Cfg>(a, split_v, split_n, s);
-        if (st != IREE_AMD_UK_STATUS_NOT_FOUND) return st;
-      }
-    }
+  const int64_t tiles = ceil_div(M, (int64_t)2 * t.wm) * ceil_div(N, (int64_t)2 * t.wn) * slices *
+                        (a.batch > 1 ? a.batch : 1);
+  const int64_t slots = (int64_t)t.occ * cus, rounds = tiles / slots, rest = tiles % slots;
+  const double steps = (double)ceil_div((int64_t)a.ksteps, (int64_t)slices) *
+                       (a.lhs_row_major ? t.row_major : 1.0);
+  const double fixed = 1.93 + 0.596 * t.wm * t.wn / 16;      // ring fill and result of a workgroup
+  double us = 2.4 + rounds * (steps * (t.idle + t.busy) * t.shared + fixed);
+  if (rest > 0) {
+    const double busy = rest < cus ? (double)rest / cus : 1.0;
+    us += steps * (rest > cus ? (t.idle + t.busy) * t.shared : t.idle + t.busy * busy) + fixed;
   }
-  // A last round that fills only part of the device costs a whole round. When
-  // the large tile leaves such a round, the longer outer dimension is split:
-  // whole rounds of 256x256 tiles first, the remaining rows or columns as a
-  // second launch with whatever suits them (usually tiles of half the size, one
-  // per compute unit). Taken when the model predicts at least 5 % (a launch costs a few
-  // microseconds, so only for long K).
+  const double elems = (double)M * N * 1024e-6 * (a.batch > 1 ? a.batch : 1);
+  if (slices == 1) return us + elems * out_bytes / 13.2;
+  // the partial sums, written and read, and the launch that adds them
+  const double mb = slices * elems * 4;
+  return us + 2.28 + mb / 7.7 + (mb > 10.0 ? (mb - 10.0) * 0.075 : 0.0) + 0.314 * (slices - 1) +
+         (a.accumulate ? elems * out_bytes / 13.2 : 0.0);
+}
+
+// A last round that fills only part of the device costs a whole round. When
+// the large tile leaves such a round, the longer outer dimension is split:
+// whole rounds of 256x256 tiles first, the remaining rows or columns as a
+// second launch with whatever suits them (usually tiles of half the size, one
+// per compute unit). Taken when `cost` (of a tile, M and N; any unit) predicts
+// at least 5 % against best_cost (a launch costs a few microseconds, so only for
+// long K). NOT_FOUND when it is not taken.
+template <typename Cfg, bool kSiluMul, typename Cost, typename Pick>
+int launch_whole_rounds(const MfmaArgs& a, double best_cost, Cost cost_of, Pick pick, hipStream_t s) {
+  const int cus = device_cu_count();
+  auto launch = [&](int v, const MfmaArgs& b) -> int { return launch_by_index<Cfg, kSiluMul>(v, b, s); };
   const int64_t rows0 = ceil_div((int64_t)a.M, (int64_t)8);   // macro-tile rows of the large tile
   const int64_t cols0 = ceil_div((int64_t)a.N, (int64_t)8);
   const int64_t rounds0 = rows0 * cols0 / cus;
@@ -390,6 +328,166 @@ int launch_cfg(const MfmaArgs& a, hipStream_t s) {
         return launch(rest_v, rest);
       }
     }
+  }
+  return IREE_AMD_UK_STATUS_NOT_FOUND;
+}
+
+// The 16-row shapes: whatever tile and number of K slices the estimate says.
+template <typename Cfg>
+int launch_estimated(const MfmaArgs& a, hipStream_t s) {
+  constexpr int kOutBytes = (int)sizeof(typename Cfg::out_t);
+  const int cus = device_cu_count();
+  auto us_of = [&](int v, int64_t M, int64_t N) -> double { return estimate_us(a, kOutBytes, v, M, N, 1); };
+  auto pick = [&](int64_t M, int64_t N, double* out_us) -> int {
+    int best = 0;
+    for (int v = 0; v < kTilesWithMedium; ++v) {
+      const double us = us_of(v, M, N);
+      if (v == 0 || us < *out_us) { best = v; *out_us = us; }
+    }
+    return best;
+  };
+  double best_us = 0;
+  const int best = pick(a.M, a.N, &best_us);
+  // K over workgroup rows: at most one round, slices of 768 elements and more
+  // of K; it has to win by 3 %.
+  if (a.k_slices == 0 && a.batch <= 1) {
+    double split_us = best_us * 0.97;
+    int split_v = 0, split_n = 0;
+    for (int n = 2; n <= 8 && (int64_t)a.ksteps * Cfg::kMfmaK / n >= 768; ++n)
+      for (int v = 0; v < kTilesWithMedium; ++v) {
+        const MediumTile& t = kMediumTiles[v];
+        const int64_t tiles = ceil_div((int64_t)a.M, (int64_t)2 * t.wm) * ceil_div((int64_t)a.N, (int64_t)2 * t.wn) * n;
+        if (tiles > (int64_t)t.occ * cus) continue;
+        const double us = estimate_us(a, kOutBytes, v, a.M, a.N, n);
+        if (us < split_us) { split_us = us; split_v = v; split_n = n; }
+      }
+    if (split_n > 1) {
+      const int st = launch_k_split<Cfg>(a, split_v, split_n, s);
+      if (st != IREE_AMD_UK_STATUS_NOT_FOUND) return st;
+    }
+  }
+  const int st = launch_whole_rounds<Cfg, false>(a, best_us, us_of, pick, s);
+  if (st != IREE_AMD_UK_STATUS_NOT_FOUND) return st;
+  return launch_by_index<Cfg, false>(best, a, s);
+}
+
+template <typename Cfg, bool kSiluMul = false>
+int launch_cfg(const MfmaArgs& a, hipStream_t s) {
+  if constexpr (kHasMediumTiles<Cfg, kSiluMul>) return launch_estimated<Cfg>(a, s);
+  // The 32-row shapes (f32, fp8, the SiLU forms, i8 with K in whole 32s only).
+  // Pick the macro tile. 256x256 (one workgroup per compute unit, all of its
+  // registers) has the best operand reuse: 1 KiB of operand per two MFMAs.
+  // 256x128 / 128x256 run two workgroups per compute unit, so one workgroup's
+  // output stores overlap the other's MFMAs, and they spread a problem over
+  // more compute units; 128x128 spreads small problems further still.
+  // Estimated cost of a variant, in units of one 32x32 block row of MFMAs:
+  // rounds of resident workgroups x work per workgroup / relative efficiency
+  // (measured on MI355X against the 256x256 tile's rate).
+  const int cus = device_cu_count();
+  // (fp8 runs the two-per-compute-unit tiles on a ring of only 3 K-steps:
+  // 2048 x 28672 x 4096 measured 238 us with the large tile, 267 with 256x128.
+  // With the SiLU epilogue, whose arithmetic the second workgroup hides and
+  // whose output is an eighth of the bytes, it is the other way round: 218
+  // against 198 us.)
+  constexpr bool kShallow = Cfg::kSub == 2 && !kSiluMul;
+  struct Variant { int wm, wn, occ; double eff_alone, eff_full; };
+  constexpr double kEffAlone = kSiluMul ? 1.0 : kShallow ? 0.85 : 0.9;
+  constexpr double kEffFull = kSiluMul ? 1.05 : kShallow ? 0.82 : 0.94;
+  static const Variant variants[4] = {{4, 4, 1, 1.0, 1.0},
+                                      {4, 2, 2, kEffAlone, kEffFull},
+                                      {2, 4, 2, kEffAlone, kEffFull},
+                                      {2, 2, 2, 0.7, 0.75}};
+  // cost of variant v on an M x N (outer tiles) problem
+  auto cost_of = [&](int v, int64_t M, int64_t N, int64_t k_slices = 1) -> double {
+    const Variant& t = variants[v];
+    const int64_t tiles = ceil_div(M, (int64_t)2 * t.wm) * ceil_div(N, (int64_t)2 * t.wn) * k_slices *
+                          (a.batch > 1 ? a.batch : 1);
+    const int64_t slots = (int64_t)t.occ * cus;
+    const double work = t.wm * t.wn;
+    double cost = (double)(tiles / slots) * t.occ * work / t.eff_full;
+    const int64_t rest = tiles % slots;
+    if (rest > 0) {
+      const int resident = (int)ceil_div(rest, (int64_t)cus);   // workgroups sharing a compute unit
+      cost += resident * work / (resident == t.occ ? t.eff_full : t.eff_alone);
+    }
+    // Of the two half-size tiles the one with more columns than rows is the
+    // faster one for the SiLU form (the gate/up matmul of the fp8 MLP block
+    // alone, sustained: 187.7 -> 180.0 us; inside the block 292 -> 289). For
+    // row-major results on the 32-row instructions the two measure either way:
+    // 128x256 ahead by 3-7 % when the call is repeated on operands that stay
+    // in the last-level cache (fp8 2048 x 4096 x 14336 100.6 -> 97.4 us),
+    // 256x128 ahead by 2 % inside the MLP block, where the weights come from
+    // memory every time (block 289 -> 283 us): the latter is what a model does,
+    // so those keep the first of the two.
+    if (kSiluMul && Cfg::kRows == 32 && v == 1) cost *= 1.03;
+    // A row-major left-hand side is the dearer operand to fetch (half or
+    // quarter cache lines per row and K-step, each line asked for again on the
+    // next step): tiles with more rows than columns pay most. Measured at
+    // 2048 x 4096 x 4096 against the packed operand, K-steps of 64 bytes of a
+    // row (fp8): 256x256 1.01, 256x128 1.09-1.14, 128x256 1.02-1.03, 128x128
+    // 1.13; K-steps of 32 bytes (i8 on the 32-row instruction): 1.16, 1.37,
+    // 1.06, 1.28.
+    if (a.lhs_row_major) {
+      constexpr bool kHalfLines = Cfg::kSub == 2;
+      static const double penalty[2][4] = {{1.16, 1.37, 1.06, 1.28}, {1.02, 1.13, 1.03, 1.13}};
+      cost *= penalty[kHalfLines][v];
+    }
+    return cost;
+  };
+  auto pick = [&](int64_t M, int64_t N, double* out_cost) -> int {
+    int best = 0;
+    double best_cost = 0;
+    for (int v = 0; v < 4; ++v) {
+      const double cost = cost_of(v, M, N);
+      if (v == 0 || cost < best_cost * 0.999) { best = v; best_cost = cost; }
+    }
+    *out_cost = best_cost;
+    return best;
+  };
+  auto launch = [&](int v, const MfmaArgs& b) -> int { return launch_by_index<Cfg, kSiluMul>(v, b, s); };
+  double best_cost = 0;
+  const int best = pick(a.M, a.N, &best_cost);
+  // Few macro tiles and a long K (a few hundred rows against a wide K, as in the
+  // down projection of an MLP at small batch) leave most compute units idle:
+  // K is then split over workgroup rows. Estimated times in microseconds: cost
+  // units (block rows of MFMAs per K-step) x K-steps x the measured time of a
+  // unit, plus, for a split, the second launch and the traffic of the partial
+  // sums (written once, read once, at about 3 TB/s).
+  if constexpr (!kSiluMul) {
+    const Variant& bv = variants[best];
+    const int64_t best_tiles = ceil_div((int64_t)a.M, (int64_t)2 * bv.wm) * ceil_div((int64_t)a.N, (int64_t)2 * bv.wn);
+    if (a.k_slices == 0 && a.batch <= 1 && a.ksteps >= 64 && best_tiles * 2 <= (int64_t)bv.occ * cus) {
+      const double unit_us = Cfg::kStepUs / 16.0;
+      const double out_mb = (double)a.M * a.N * 4096.0 / 1e6;
+      // A split must win by 5 %.
+      double best_us = best_cost * a.ksteps * unit_us * 0.95;
+      int split_v = -1, split_n = 0;
+      for (int v = 0; v < 4; ++v) {
+        // (up to 64 rows: with the tile and slice count forced, 128x128 tiles
+        // won on every such shape measured, by up to 10 % over what this
+        // estimate picked among the larger tiles, whose rows are as idle and
+        // whose workgroups are half as many)
+        if (a.M <= 2 && v != 3) continue;
+        for (int n = 2; n <= 8; ++n) {
+          if (a.ksteps / n < 24) break;
+          const int64_t tiles = ceil_div((int64_t)a.M, (int64_t)2 * variants[v].wm) *
+                                ceil_div((int64_t)a.N, (int64_t)2 * variants[v].wn) * n;
+          if (tiles > (int64_t)variants[v].occ * cus) break;     // at most one round
+          const double us = cost_of(v, a.M, a.N, n) * ceil_div((int64_t)a.ksteps, (int64_t)n) * unit_us + 6.0 +
+                            (n + 1 + (a.accumulate ? 1 : 0)) * out_mb / 3.0;
+          if (us < best_us) { best_us = us; split_v = v; split_n = n; }
+        }
+      }
+      if (split_n > 1) {
+        const int st = launch_k_split<Cfg>(a, split_v, split_n, s);
+        if (st != IREE_AMD_UK_STATUS_NOT_FOUND) return st;
+      }
+    }
+  }
+  {
+    const int st = launch_whole_rounds<Cfg, kSiluMul>(a, best_cost, [&](int v, int64_t M, int64_t N) { return cost_of(v, M, N); },
+                                                      pick, s);
+    if (st != IREE_AMD_UK_STATUS_NOT_FOUND) return st;
   }
   return launch(best, a);
 }

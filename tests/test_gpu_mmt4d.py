@@ -1165,3 +1165,28 @@ def test_batch_forms_of_the_fused_entry_points_match_single_calls(uk, cuda, type
     with pytest.raises(uk.UkError):
         uk.batch_mmt4d_unpack(lhs_t, rhs_t, out, 2, 33, 65, 2, 3, K1, K0, flags,
                               lhs_batch_stride=2 * K1 * 32 * K0 + 3, rhs_batch_stride=0)
+
+
+@pytest.mark.parametrize("M,N", [(1981, 4101), (2164, 4101), (2347, 3713)])
+@pytest.mark.parametrize("type_flag,dt,out_dt", [
+    (F.MMT4D_TYPE_F16F16F32, "float16", "float32"), (F.MMT4D_TYPE_BF16BF16BF16, "bfloat16", "bfloat16"),
+    (F.MMT4D_TYPE_S8S8S32, "int8", "int32"),
+])
+def test_medium_macro_tiles(uk, cuda, type_flag, dt, out_dt, M, N):
+    """Sizes for which, on 256 compute units, the launcher takes 192x192, 256x192
+    and 192x256 macro tiles, ragged on both sides: tiled result, row-major
+    result and row-major left-hand side. Small integers: every sum is exact (and
+    below 2^8, so that a bf16 result is as well)."""
+    import torch
+    g = torch.Generator(device="cuda").manual_seed(M + N)
+    for K, fused in ((192, ({}, {"fuse_unpack": True}, {"fuse_pack_lhs": True})), (216, ({}, {"fuse_unpack": True}))):
+        a = torch.randint(-1, 2, (M, K), generator=g, device="cuda")
+        b = torch.randint(-1, 2, (K, N), generator=g, device="cuda")
+        want = a.double() @ b.double()
+        assert want.abs().max() < 256
+        ad, bd = a.to(getattr(torch, dt)).reshape(-1), b.to(getattr(torch, dt)).reshape(-1)
+        for kw in fused:
+            c = torch.zeros(M * N, dtype=getattr(torch, out_dt), device="cuda")
+            uk.matmul_data_tiled(ad, bd, c, M, N, K, type_flag, tile="dynamic", **kw)
+            assert uk.last_kernel_path() == "mmt4d:mfma" or kw, uk.last_kernel_path()
+            assert torch.equal(c.double().view(M, N), want), (K, kw)
