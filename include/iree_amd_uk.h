@@ -622,6 +622,23 @@ IREE_AMD_UK_EXPORT int iree_amd_uk_matmul_packed_rhs(
     iree_amd_uk_index_t N, iree_amd_uk_index_t K, int32_t K0, uint32_t flags,
     float out_scale, void* stream);
 
+/* The whole data-tiled matmul of a small problem as one launch: what
+ * pack(A), pack(B, inner and outer transposed), [pack(C)], mmt4d and unpack do
+ * (REF compiler/src/iree/compiler/Codegen/Common/CPU/CPULowerToUKernels.cpp:339-480).
+ *   c[m][n] (+)= sum_k a[m][k] * b[k][n]
+ * a is M x K, b K x N, c M x N, all row-major and tight, element types as in
+ * `flags` (an IREE_AMD_UK_FLAG_MMT4D_TYPE_*, optionally ACCUMULATE). lhs, rhs and
+ * out receive the packed operands and the packed result in tiles of M0 x K0,
+ * N0 x K0 and M0 x N0, as the chain leaves them; a null one is not written.
+ * Returns IREE_AMD_UK_STATUS_NOT_FOUND, with no error recorded and nothing
+ * written, for what it does not serve (large problems, which the chain runs
+ * faster; tiles without a matrix-core kernel; buffers that overlap): run the
+ * chain then. Allocates nothing. */
+IREE_AMD_UK_EXPORT int iree_amd_uk_matmul_data_tiled(
+    const void* a, const void* b, void* c, void* lhs, void* rhs, void* out, iree_amd_uk_index_t M,
+    iree_amd_uk_index_t N, iree_amd_uk_index_t K, int32_t M0, int32_t N0, int32_t K0, uint32_t flags,
+    void* stream);
+
 /* `batch` problems of iree_amd_uk_matmul_packed_rhs (a batch matmul on
  * row-major left-hand sides, every entry with packed weights of its own, or
  * rhs_batch_stride = 0 for shared ones), strides in elements as above. One
@@ -702,7 +719,7 @@ IREE_AMD_UK_EXPORT int iree_amd_uk_release_scratch(void);
 IREE_AMD_UK_EXPORT const char* iree_amd_uk_last_error(void);
 /* Name of the kernel family that served the calling thread's last mmt4d or
  * dequant_matmul_i4 call: "mmt4d:mfma", "mmt4d:mfma-narrow",
- * "mmt4d:mfma-widened-s4", "mmt4d:mfma-s16-planes", "mmt4d:element-wise",
+ * "mmt4d:mfma-one-launch" (iree_amd_uk_matmul_data_tiled), "mmt4d:mfma-widened-s4", "mmt4d:mfma-s16-planes", "mmt4d:element-wise",
  * "dequant_i4:mfma", "dequant_i4:gemv", "dequant_i4:reassociated",
  * "dequant_i4:element-wise" ("" before the first call). A static string. No
  * counterpart in the reference, whose tile-function choice is visible through

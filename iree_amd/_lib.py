@@ -137,6 +137,8 @@ def _declare(lib):
     lib.iree_amd_uk_mmt4d_unpack.restype = C.c_int
     lib.iree_amd_uk_mmt4d_unpack.argtypes = [vp, i64, i64, vp, i64, i64, vp, i64, i64, i64, i64,
                                              i64, i64, i64, C.c_int32, C.c_uint32, C.c_float, vp]
+    lib.iree_amd_uk_matmul_data_tiled.restype = C.c_int
+    lib.iree_amd_uk_matmul_data_tiled.argtypes = [vp] * 6 + [i64, i64, i64, i32, i32, i32, u32, vp]
     lib.iree_amd_uk_matmul_packed_rhs.restype = C.c_int
     lib.iree_amd_uk_matmul_packed_rhs.argtypes = [vp, i64, i64, vp, i64, i64, vp, i64, i64,
                                                   i64, i64, i64, C.c_int32, C.c_uint32, C.c_float, vp]

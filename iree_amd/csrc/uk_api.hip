@@ -852,6 +852,15 @@ extern "C" int iree_amd_uk_batch_matmul_packed_rhs(
                                 stream);
 }
 
+extern "C" int iree_amd_uk_matmul_data_tiled(
+    const void* a, const void* b, void* c, void* lhs, void* rhs, void* out, iree_amd_uk_index_t M,
+    iree_amd_uk_index_t N, iree_amd_uk_index_t K, int32_t M0, int32_t N0, int32_t K0, uint32_t flags,
+    void* stream) {
+  const int st = launch_matmul_rowmajor(a, b, c, lhs, rhs, out, M, N, K, M0, N0, K0, flags, (hipStream_t)stream);
+  if (st != IREE_AMD_UK_STATUS_NOT_FOUND) note_kernel_path("mmt4d:mfma-one-launch");
+  return st;
+}
+
 extern "C" int iree_amd_uk_scale_f32(void* buf_f32, iree_amd_uk_index_t n, float scale,
                                      void* stream) {
   if (n < 0) return fail(IREE_AMD_UK_STATUS_INVALID_ARGUMENT, "scale_f32: negative n");

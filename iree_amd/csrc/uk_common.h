@@ -106,6 +106,10 @@ int launch_mmt4d_unpack_mfma(const iree_amd_uk_mmt4d_params_t& p, int64_t out_ro
 int launch_matmul_packed_rhs_mfma(const iree_amd_uk_mmt4d_params_t& p, int64_t out_rows,
                                   int64_t out_cols, float out_scale, int64_t batch, int64_t lhs_batch_stride,
                                   int64_t rhs_batch_stride, int64_t out_batch_stride, hipStream_t s);
+// The whole chain of a small data-tiled matmul as one launch (uk_matmul_rowmajor.hip);
+// NOT_FOUND when the caller has to run the chain.
+int launch_matmul_rowmajor(const void* a, const void* b, void* c, void* lhs, void* rhs, void* out, int64_t M,
+                           int64_t N, int64_t K, int M0, int N0, int K0, uint32_t flags, hipStream_t s);
 int launch_mmt4d_silu_mul_mfma(const iree_amd_uk_mmt4d_params_t& p, float gate_scale,
                                float up_scale, float inv_out_scale, hipStream_t s);
 

@@ -1,0 +1,402 @@
+// The whole data-tiled matmul (pack, pack, [pack C,] mmt4d, unpack) of a small
+// problem as ONE launch.
+//
+// Contract: include/iree_amd_uk.h, iree_amd_uk_matmul_data_tiled. The sequence
+// it stands for is the reference's
+// (compiler/src/iree/compiler/Codegen/Common/CPU/CPULowerToUKernels.cpp:339-480).
+//
+// What bounds such a call is not work but launches: a chain of 4 or 5 kernels
+// that depend on each other costs about 5 us for each whatever it does. Here the
+// first workgroups multiply straight from the row-major operands, the ones
+// after them write the packed operands, which nothing in the launch waits for,
+// and the matmul's epilogue stores both the tiles of the result and the matrix.
+//
+// Among other calls on one stream: f16 81x19x41 21.1 us as the chain, 6.6 here; i8
+// 1024^3 21.0, 11.4.
+//
+// Multiplying workgroups: 4 waves on kRows x kRows of the result, 64 KiB of
+// operands per K-step (128 KiB / kRows bytes of K), fetched for the next
+// step while this one is multiplied: a wide step because a step costs a round
+// trip to memory, and these problems have too few workgroups to hide it.
+// An operand row of a step is kChunks chunks of 16 bytes of consecutive K in
+// LDS, permuted within 16 by a hash of the row: fragment reads (16 consecutive
+// rows, one chunk) and the stores of the right-hand side (rows 4 apart) hit 16
+// different bank groups each. The right-hand side, whose rows run along N,
+// is turned in registers: a thread loads 4 columns of the 16 / element-size
+// rows of a chunk and stores 4 chunks.
+//   kRows = 64: each wave a 32x32 quarter.
+//   kRows = 32: each wave all of it for a quarter of K, summed in LDS in wave
+//   order; four times as many workgroups and half as many steps.
+#include <type_traits>
+
+#include "uk_common.h"
+#include "uk_mfma_cfg.h"
+
+namespace uk {
+namespace {
+
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+
+// f32 on 16 rows: four v_mfma_f32_16x16x4_f32, element e of a lane's 16 bytes
+// for the e-th; both operands pair the same way, so every k meets its partner.
+struct F32Cfg16 {
+  typedef floatx4 frag_t;
+  typedef floatx4 acc_t;
+  typedef float out_t;
+  static constexpr int kElemBytes = 4;
+  __device__ static acc_t mfma(frag_t a, frag_t b, acc_t c) {
+#pragma unroll
+    for (int e = 0; e < 4; ++e) c = __builtin_amdgcn_mfma_f32_16x16x4f32(a[e], b[e], c, 0, 0, 0);
+    return c;
+  }
+};
+
+struct RowMajorArgs {
+  const char* a;       // M x K
+  const char* b;       // K x N
+  char* c;             // M x N
+  char* lhs;           // packed operands and result; null: not wanted
+  char* rhs;
+  char* out;
+  int M, N, K, M0, N0, M1, N1, K1;
+  int tiles_n, product_blocks, lhs_blocks;
+  int accumulate;
+};
+
+// A 128-bit value moved down by `bytes` (0 to 15), zeros from above.
+__device__ __forceinline__ u32x4 shift_down(u32x4 v, int bytes) {
+  union { u32x4 v; unsigned __int128 x; } u;
+  u.v = v;
+  u.x >>= 8 * bytes;
+  return u.v;
+}
+
+// Loads never leave the matrix and never branch: what lies past the end of a
+// row is the 16 bytes (or 4 elements) that end there, moved down when they are
+// stored; what lies past the last row is that row, replaced by zeros then. So
+// all loads of a step are in flight together. (Rows of K are at least a chunk
+// long, rows of N 4 elements.)
+template <int kElemBytes>
+__device__ __forceinline__ u32x4 load_chunk(const char* row, int k, int K) {
+  constexpr int E = 16 / kElemBytes;
+  u32x4 v;
+  __builtin_memcpy(&v, row + (int64_t)(k + E <= K ? k : K - E) * kElemBytes, 16);   // (one load, aligned or not)
+  return v;
+}
+template <int kElemBytes>
+__device__ __forceinline__ u32x4 settle_chunk(u32x4 v, int k, int K, bool row_exists) {
+  constexpr int E = 16 / kElemBytes;
+  if (!row_exists || k >= K) return u32x4{0, 0, 0, 0};
+  return k + E <= K ? v : shift_down(v, (k + E - K) * kElemBytes);
+}
+
+// Four consecutive elements of a row, in kElemBytes dwords.
+template <int kElemBytes>
+struct Four { uint32_t d[kElemBytes]; };
+template <int kElemBytes>
+__device__ __forceinline__ Four<kElemBytes> settle_four(Four<kElemBytes> r, int n, int N, bool row_exists) {
+  if (!row_exists || n >= N) return Four<kElemBytes>{};
+  if (n + 4 <= N) return r;
+  u32x4 v = {0, 0, 0, 0};
+#pragma unroll
+  for (int i = 0; i < kElemBytes; ++i) v[i] = r.d[i];
+  v = shift_down(v, (n + 4 - N) * kElemBytes);
+#pragma unroll
+  for (int i = 0; i < kElemBytes; ++i) r.d[i] = v[i];
+  return r;
+}
+
+// Chunk of column e (0 to 3) from the 16 / kElemBytes rows of a four-column strip.
+template <int kElemBytes>
+__device__ __forceinline__ u32x4 column_chunk(const Four<kElemBytes>* rows, int e) {
+  u32x4 v;
+  if constexpr (kElemBytes == 4) {
+#pragma unroll
+    for (int q = 0; q < 4; ++q) v[q] = rows[q].d[e];
+  } else if constexpr (kElemBytes == 2) {
+    const uint32_t sel = e & 1 ? 0x07060302u : 0x05040100u;
+#pragma unroll
+    for (int q = 0; q < 4; ++q) v[q] = __builtin_amdgcn_perm(rows[2 * q + 1].d[e / 2], rows[2 * q].d[e / 2], sel);
+  } else {
+    const uint32_t sel = 0x0c0c0400u + 0x0101u * e;   // byte e of the second operand, then of the first
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      const uint32_t lo = __builtin_amdgcn_perm(rows[4 * q + 1].d[0], rows[4 * q].d[0], sel);
+      const uint32_t hi = __builtin_amdgcn_perm(rows[4 * q + 3].d[0], rows[4 * q + 2].d[0], sel);
+      v[q] = lo | hi << 16;
+    }
+  }
+  return v;
+}
+
+// One workgroup's 256 chunks of a packed operand. Chunk r of the buffer is row
+// i0 of the tile (i1, k1).
+template <int kElemBytes>
+__device__ void pack_block(const RowMajorArgs& p, int block) {
+  constexpr int E = 16 / kElemBytes;
+  const bool is_lhs = block < p.lhs_blocks;
+  const uint32_t r = (uint32_t)(is_lhs ? block : block - p.lhs_blocks) * 256 + threadIdx.x;
+  const uint32_t T0 = is_lhs ? p.M0 : p.N0, K1 = p.K1;
+  if (r >= T0 * K1 * (uint32_t)(is_lhs ? p.M1 : p.N1)) return;
+  const uint32_t tile = r / T0, i0 = r - tile * T0;
+  const uint32_t i1 = tile / K1, k1 = tile - i1 * K1;
+  const int i = (int)(i1 * T0 + i0), k = (int)k1 * E;
+  u32x4 v = {0, 0, 0, 0};
+  if (is_lhs) {
+    if (i < p.M)
+      v = settle_chunk<kElemBytes>(load_chunk<kElemBytes>(p.a + (int64_t)i * p.K * kElemBytes, k, p.K), k, p.K, true);
+    *(u32x4*)(p.lhs + (int64_t)r * 16) = v;
+  } else {
+    typedef typename std::conditional<kElemBytes == 1, uint8_t,
+                                      typename std::conditional<kElemBytes == 2, uint16_t, uint32_t>::type>::type elem_t;
+    if (i < p.N) {
+      const elem_t* q = (const elem_t*)p.b + i;
+      elem_t x[E];
+#pragma unroll
+      for (int e = 0; e < E; ++e) x[e] = q[(int64_t)(k + e < p.K ? k + e : p.K - 1) * p.N];
+#pragma unroll
+      for (int e = 0; e < E; ++e)
+        v[e * kElemBytes / 4] |= (k + e < p.K ? (uint32_t)x[e] : 0u) << (8 * (e * kElemBytes % 4));
+    }
+    *(u32x4*)(p.rhs + (int64_t)r * 16) = v;
+  }
+}
+
+template <typename Cfg, int kRows>
+__global__ __launch_bounds__(256, 2) void matmul_rowmajor_kernel(RowMajorArgs p) {
+  constexpr int kElemBytes = Cfg::kElemBytes;
+  constexpr int E = 16 / kElemBytes;            // elements of a chunk
+  constexpr int kChunks = 2048 / kRows;         // chunks of a row per step
+  constexpr int kStep = kChunks * E;            // elements of K per step
+  constexpr int kGroups = kRows / 4;            // four-column strips of the right-hand side
+  typedef typename Cfg::frag_t frag_t;
+  typedef typename Cfg::acc_t acc_t;
+  typedef typename Cfg::out_t out_t;
+  __shared__ u32x4 tile_a[2048], tile_b[2048];
+  if ((int)blockIdx.x >= p.product_blocks) {
+    pack_block<kElemBytes>(p, (int)blockIdx.x - p.product_blocks);
+    return;
+  }
+  const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
+  const int m_base = (int)blockIdx.x / p.tiles_n * kRows, n_base = (int)blockIdx.x % p.tiles_n * kRows;
+  auto place = [](int row, int chunk) { return row * kChunks + (chunk ^ ((row + (row >> 4)) & 15)); };
+
+  // what this thread fetches of a step: chunk t % kChunks of 8 rows of A, and
+  // two strips of 4 columns x E rows of B
+  u32x4 next_a[8];
+  Four<kElemBytes> next_b[2][E];
+  const int my_row = m_base + t / kChunks, my_n = n_base + t % kGroups * 4;
+  uint32_t row_at[8];                           // element offsets, 32 bits (operands of up to 64 MiB)
+#pragma unroll
+  for (int j = 0; j < 8; ++j) {
+    const int row = my_row + j * (kRows / 8);
+    row_at[j] = (uint32_t)(row < p.M ? row : p.M - 1) * p.K;
+  }
+  const uint32_t col_at = my_n + 4 <= p.N ? my_n : p.N - 4, last_row = (uint32_t)(p.K - 1) * p.N;
+  auto fetch = [&](int k_base) {
+    const int ka = k_base + t % kChunks * E;
+    const uint32_t at = ka + E <= p.K ? ka : p.K - E;
+#pragma unroll
+    for (int j = 0; j < 8; ++j) __builtin_memcpy(&next_a[j], p.a + (row_at[j] + at) * kElemBytes, 16);
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+      const uint32_t k_row = (uint32_t)(k_base + (t / kGroups + j * (256 / kGroups)) * E) * p.N;
+#pragma unroll
+      for (int e = 0; e < E; ++e) {
+        const uint32_t r = k_row + (uint32_t)e * p.N;
+        __builtin_memcpy(&next_b[j][e], p.b + ((r < last_row ? r : last_row) + col_at) * kElemBytes, 4 * kElemBytes);
+      }
+    }
+  };
+  fetch(0);
+
+  // The wave's 2 x 2 blocks of 16x16: element r of a lane is row 4 (lane / 16) + r,
+  // column lane % 16.
+  const int wm = kRows == 64 ? wave / 2 * 32 : 0, wn = kRows == 64 ? wave % 2 * 32 : 0;
+  const bool owner = kRows == 64 || wave == 0;   // stores the result
+  // A step has sums of its own, one for every other instruction, which are added
+  // to the whole at its end, and the old result last of all: the rounding error
+  // of a sum grows with the number of terms it takes one by one.
+  acc_t acc[2][2] = {}, old[2][2] = {};
+  out_t* const c = (out_t*)p.c;
+  if (p.accumulate && owner) {
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+      for (int j = 0; j < 2; ++j)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          const int m = m_base + wm + i * 16 + lane / 16 * 4 + r, n = n_base + wn + j * 16 + lane % 16;
+          if (m < p.M && n < p.N) old[i][j][r] = c[(int64_t)m * p.N + n];
+        }
+  }
+
+  for (int k_base = 0; k_base < p.K; k_base += kStep) {
+    const int left = p.K - k_base;
+    const int subs = left >= kStep ? kChunks / 4 : (left + 4 * E - 1) / (4 * E);   // of 4 chunks: one instruction's K
+    if (k_base) __syncthreads();
+    if (t % kChunks < subs * 4) {
+#pragma unroll
+      for (int j = 0; j < 8; ++j)
+        tile_a[place(t / kChunks + j * (kRows / 8), t % kChunks)] = settle_chunk<kElemBytes>(
+            next_a[j], k_base + t % kChunks * E, p.K, my_row + j * (kRows / 8) < p.M);
+    }
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+      const int chunk = t / kGroups + j * (256 / kGroups), k = k_base + chunk * E;
+      if (chunk < subs * 4) {
+        if (k + E > p.K || my_n + 4 > p.N) {
+#pragma unroll
+          for (int e = 0; e < E; ++e) next_b[j][e] = settle_four<kElemBytes>(next_b[j][e], my_n, p.N, k + e < p.K);
+        }
+#pragma unroll
+        for (int e = 0; e < 4; ++e) tile_b[place(t % kGroups * 4 + e, chunk)] = column_chunk<kElemBytes>(next_b[j], e);
+      }
+    }
+    __syncthreads();
+    if (k_base + kStep < p.K) fetch(k_base + kStep);
+    acc_t part[2][2][2] = {};
+    auto multiply = [&](int s, acc_t (&sum)[2][2]) {
+      union { u32x4 u; frag_t f; } fa[2], fb[2];
+#pragma unroll
+      for (int i = 0; i < 2; ++i) {
+        fa[i].u = tile_a[place(wm + i * 16 + lane % 16, s * 4 + lane / 16)];
+        fb[i].u = tile_b[place(wn + i * 16 + lane % 16, s * 4 + lane / 16)];
+      }
+#pragma unroll
+      for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int j = 0; j < 2; ++j) sum[i][j] = Cfg::mfma(fa[i].f, fb[j].f, sum[i][j]);
+    };
+    constexpr int kApart = kRows == 64 ? 1 : 4;   // (kRows = 32: a wave takes every fourth)
+    for (int s = kRows == 64 ? 0 : wave; s < subs; s += 2 * kApart) {
+      multiply(s, part[0]);
+      if (s + kApart < subs) multiply(s + kApart, part[1]);
+    }
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+      for (int j = 0; j < 2; ++j) acc[i][j] += part[0][i][j] + part[1][i][j];
+  }
+
+  if constexpr (kRows == 32) {
+    // the quarters of K, in wave order
+    acc_t* const part = (acc_t*)tile_a;           // [wave - 1][block][lane]
+    __syncthreads();
+    if (wave > 0) {
+#pragma unroll
+      for (int i = 0; i < 4; ++i) part[((wave - 1) * 4 + i) * 64 + lane] = acc[i / 2][i % 2];
+    }
+    __syncthreads();
+    if (wave > 0) return;
+#pragma unroll
+    for (int w = 0; w < 3; ++w)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) acc[i / 2][i % 2] += part[(w * 4 + i) * 64 + lane];
+  }
+  out_t* const out = (out_t*)p.out;
+#pragma unroll
+  for (int j = 0; j < 2; ++j) {
+    const int n = n_base + wn + j * 16 + lane % 16;
+    const int n1 = (int)((uint32_t)n / (uint32_t)p.N0), n0 = n - n1 * p.N0;
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int m = m_base + wm + i * 16 + lane / 16 * 4 + r;
+        const out_t v = (out_t)(acc[i][j][r] + old[i][j][r]);
+        if (m < p.M && n < p.N) c[(int64_t)m * p.N + n] = v;
+        if (out) {
+          const int m1 = (int)((uint32_t)m / (uint32_t)p.M0), m0 = m - m1 * p.M0;
+          if (m1 < p.M1 && n1 < p.N1) out[(((int64_t)m1 * p.N1 + n1) * p.M0 + m0) * p.N0 + n0] = v;
+        }
+      }
+  }
+}
+
+// Estimated time in microseconds on kRows = side, and the rule: the launch is
+// taken when the estimate, 10 % added, is below what the chain's launches cost by
+// themselves (5 us each when they follow each other, less 1). A step takes about as
+// long whatever else runs, until a compute unit holds more than one workgroup;
+// then the packed buffers and the result, at 6 TB/s. Measured and estimated, against
+// the chain (i8 1024^3 11.4, 11.7, chain 21.0; f16 81x19x41 6.6, 7.0, 21.1;
+// 512^3 6.8, 7.6, 21.2; 768^3 12.6, 13.5, 21.0; 1024^3 16.0, 17.2, 21.4; 3000x8x1325 13.4,
+// 12.5, 20.7; f32 512^3 10.4, 10.9, 30.4). Beyond the rule the chain's kernels win: f16
+// 2048 x 2048 x 1024 36.8 us here, 28.9 there.
+template <typename Cfg>
+double estimate_us(const RowMajorArgs& p, int side) {
+  constexpr bool kF32 = Cfg::kElemBytes == 4;   // (whose instructions take as long as a step's loads)
+  const double step_us = side == 64 ? (kF32 ? 3.7 : 2.6) : (kF32 ? 2.7 : 2.4);
+  const int64_t rows = (int64_t)p.M1 * p.M0, cols = (int64_t)p.N1 * p.N0;
+  const int64_t groups = ceil_div(rows, (int64_t)side) * ceil_div(cols, (int64_t)side);
+  const int64_t steps = ceil_div((int64_t)p.K * Cfg::kElemBytes, (int64_t)32768 / side);
+  const double load = 0.7 * groups / device_cu_count();
+  const double bytes = (p.lhs ? 32.0 * rows * p.K1 : 0) + (p.rhs ? 32.0 * cols * p.K1 : 0) +
+                       (p.out ? 2.0 : 1.0) * rows * cols * sizeof(typename Cfg::out_t);
+  return 4.5 + steps * step_us * (load > 1 ? load : 1) + bytes / 6e6;
+}
+
+template <typename Cfg>
+int launch(RowMajorArgs p, hipStream_t s) {
+  const int64_t rows = (int64_t)p.M1 * p.M0, cols = (int64_t)p.N1 * p.N0;
+  const double us32 = estimate_us<Cfg>(p, 32), us64 = estimate_us<Cfg>(p, 64);
+  const bool small = us32 < us64;
+  const int launches = (p.lhs != nullptr) + (p.rhs != nullptr) + 1 + (p.out ? 1 + p.accumulate : 0);
+  if ((small ? us32 : us64) * 1.1 > 5.0 * launches - 1.0) return IREE_AMD_UK_STATUS_NOT_FOUND;
+  const int side = small ? 32 : 64;
+  p.tiles_n = (int)ceil_div(cols, (int64_t)side);
+  p.product_blocks = (int)(ceil_div(rows, (int64_t)side) * p.tiles_n);
+  p.lhs_blocks = p.lhs ? (int)ceil_div(rows * p.K1, (int64_t)256) : 0;
+  const int rhs_blocks = p.rhs ? (int)ceil_div(cols * p.K1, (int64_t)256) : 0;
+  const dim3 grid((unsigned)(p.product_blocks + p.lhs_blocks + rhs_blocks)), block(256);
+  if (small) hipLaunchKernelGGL((matmul_rowmajor_kernel<Cfg, 32>), grid, block, 0, s, p);
+  else hipLaunchKernelGGL((matmul_rowmajor_kernel<Cfg, 64>), grid, block, 0, s, p);
+  return check_hip(hipGetLastError(), "matmul_rowmajor launch");
+}
+
+}  // namespace
+
+int launch_matmul_rowmajor(const void* a, const void* b, void* c, void* lhs, void* rhs, void* out, int64_t M,
+                           int64_t N, int64_t K, int M0, int N0, int K0, uint32_t flags, hipStream_t s) {
+  Mmt4dTypeInfo ti;
+  if (!mmt4d_type_info(flags, &ti) || ti.lhs_bits != ti.rhs_bits || ti.lhs_bits < 8) return IREE_AMD_UK_STATUS_NOT_FOUND;
+  const int eb = ti.lhs_bits / 8;
+  if (M <= 0 || N < 4 || K * eb < 16 || M > 65536 || N > 65536 || K > 65536) return IREE_AMD_UK_STATUS_NOT_FOUND;
+  // (tiles that the chain's mmt4d would give to a matrix-core kernel as well:
+  // others sum in the order of the element-wise kernel)
+  const bool narrow = mmt4d_skinny_supported(flags, M0, N0, K0) && (M0 < 32 ? M <= M0 : N <= N0);
+  if (K0 * eb != 16 || !(narrow || mmt4d_mfma_supported(flags, M0, N0, K0))) return IREE_AMD_UK_STATUS_NOT_FOUND;
+  const int64_t M1 = ceil_div(M, (int64_t)M0), N1 = ceil_div(N, (int64_t)N0), K1 = ceil_div(K, (int64_t)K0);
+  if (M1 * M0 * K1 * 16 > (64 << 20) || N1 * N0 * K1 * 16 > (64 << 20) || M1 * M0 * N1 * N0 > (16 << 20))
+    return IREE_AMD_UK_STATUS_NOT_FOUND;
+  // Buffers that share memory: the chain reads an operand completely before
+  // the result is written, this kernel does not.
+  struct Range { uintptr_t at; int64_t bytes; bool written; };
+  const Range r[6] = {{(uintptr_t)a, M * K * eb, false},
+                      {(uintptr_t)b, K * N * eb, false},
+                      {(uintptr_t)c, M * N * ti.out_bytes, true},
+                      {(uintptr_t)lhs, lhs ? M1 * M0 * K1 * 16 : 0, true},
+                      {(uintptr_t)rhs, rhs ? N1 * N0 * K1 * 16 : 0, true},
+                      {(uintptr_t)out, out ? M1 * M0 * N1 * N0 * ti.out_bytes : 0, true}};
+  for (int i = 0; i < 6; ++i)
+    for (int j = 0; j < i; ++j)
+      if ((r[i].written || r[j].written) && r[i].at < r[j].at + r[j].bytes && r[j].at < r[i].at + r[i].bytes)
+        return IREE_AMD_UK_STATUS_NOT_FOUND;
+  if (!a || !b || !c || (uintptr_t)a % eb || (uintptr_t)b % eb || (uintptr_t)c % ti.out_bytes ||
+      (uintptr_t)lhs % 16 || (uintptr_t)rhs % 16 || (uintptr_t)out % ti.out_bytes)
+    return IREE_AMD_UK_STATUS_NOT_FOUND;
+  RowMajorArgs p = {(const char*)a, (const char*)b, (char*)c, (char*)lhs, (char*)rhs, (char*)out,
+                    (int)M, (int)N, (int)K, M0, N0, (int)M1, (int)N1, (int)K1, 0, 0, 0,
+                    (flags & IREE_AMD_UK_FLAG_MMT4D_ACCUMULATE) != 0};
+  switch (flags & IREE_AMD_UK_FLAG_MMT4D_TYPE_MASK) {
+    case IREE_AMD_UK_FLAG_MMT4D_TYPE_F16F16F32: return launch<F16Cfg16>(p, s);
+    case IREE_AMD_UK_FLAG_MMT4D_TYPE_BF16BF16F32: return launch<BF16Cfg16>(p, s);
+    case IREE_AMD_UK_FLAG_MMT4D_TYPE_F16F16F16: return launch<F16F16Cfg16>(p, s);
+    case IREE_AMD_UK_FLAG_MMT4D_TYPE_BF16BF16BF16: return launch<BF16BF16Cfg16>(p, s);
+    case IREE_AMD_UK_FLAG_MMT4D_TYPE_S8S8S32: return launch<S8Cfg16>(p, s);
+    case IREE_AMD_UK_FLAG_MMT4D_TYPE_F32F32F32: return launch<F32Cfg16>(p, s);
+    default: return IREE_AMD_UK_STATUS_NOT_FOUND;
+  }
+}
+
+}  // namespace uk

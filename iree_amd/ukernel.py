@@ -431,12 +431,22 @@ def matmul_data_tiled(a, b, c, M, N, K, mmt4d_type, *, accumulate=False,
         ws["rhs"] = torch.empty(N1 * K1 * N0 * K0, dtype=b.dtype, device=b.device)
     if "out" not in ws and not fuse_unpack:
         ws["out"] = torch.empty(M1 * N1 * M0 * N0, dtype=c.dtype, device=c.device)
+    mm_flags = mmt4d_type | F.MMT4D_ALLOW_GENERIC_FALLBACK_TILE_FUNCTION | \
+        F.MMT4D_SKIP_INTERMEDIATE_ROUNDINGS
+    if not (fuse_unpack and (M0, N0) != (32, 32)) and not (fuse_pack_lhs and K % K0):
+        # (a small problem: all of it as one launch)
+        status = load_library().iree_amd_uk_matmul_data_tiled(
+            _ptr(a), _ptr(b), _ptr(c), None if fuse_pack_lhs else _ptr(ws["lhs"]), _ptr(ws["rhs"]),
+            None if fuse_unpack else _ptr(ws["out"]), M, N, K, M0, N0, K0,
+            mm_flags | (F.MMT4D_ACCUMULATE if accumulate else 0), _stream(None))
+        if status == 0:
+            return ws
+        if status != F.STATUS_NOT_FOUND:
+            _check(status)
     if not fuse_pack_lhs:
         pack(a, ws["lhs"], M, K, M1, K1, M0, K0, 0, in_type)
     pack(b, ws["rhs"], K, N, N1, K1, N0, K0, 0,
          in_type | F.PACK_TRANSPOSE_INNER | F.PACK_TRANSPOSE_OUTER)
-    mm_flags = mmt4d_type | F.MMT4D_ALLOW_GENERIC_FALLBACK_TILE_FUNCTION | \
-        F.MMT4D_SKIP_INTERMEDIATE_ROUNDINGS
     if fuse_pack_lhs:
         if (M0, N0) != (32, 32) or K % K0:
             raise ValueError("fuse_pack_lhs needs 32x32 tiles and K in whole tiles")

@@ -1190,3 +1190,78 @@ def test_medium_macro_tiles(uk, cuda, type_flag, dt, out_dt, M, N):
             uk.matmul_data_tiled(ad, bd, c, M, N, K, type_flag, tile="dynamic", **kw)
             assert uk.last_kernel_path() == "mmt4d:mfma" or kw, uk.last_kernel_path()
             assert torch.equal(c.double().view(M, N), want), (K, kw)
+
+
+@pytest.mark.parametrize("M,N,K,tile", [
+    (1, 32, 48, None), (3, 300, 77, None), (300, 8, 999, None), (81, 19, 41, "dynamic"), (33, 33, 17, "dynamic"),
+    (129, 200, 501, None), (31, 4, 16, "dynamic"), (700, 450, 260, None), (1023, 513, 129, None),
+])
+@pytest.mark.parametrize("type_flag,dt,out_dt", [
+    (F.MMT4D_TYPE_F16F16F32, "float16", "float32"), (F.MMT4D_TYPE_F16F16F16, "float16", "float16"),
+    (F.MMT4D_TYPE_BF16BF16F32, "bfloat16", "float32"), (F.MMT4D_TYPE_BF16BF16BF16, "bfloat16", "bfloat16"),
+    (F.MMT4D_TYPE_S8S8S32, "int8", "int32"), (F.MMT4D_TYPE_F32F32F32, "float32", "float32"),
+])
+def test_small_matmul_in_one_launch(uk, cuda, type_flag, dt, out_dt, M, N, K, tile):
+    """The chain of a small data-tiled matmul as one launch: result and every
+    packed buffer as the calls of the chain leave them. Sizes at and off the
+    edges of the 32 and 64 wide workgroup tiles, of a step of K and of its
+    chunks. Integers of which every partial sum is exact in the result type, and
+    an infinity, which the zeros of a padded tile must not meet."""
+    import torch
+    g = torch.Generator(device="cuda").manual_seed(M + N + K)
+    # (a density that keeps |sums| + |c| below 2^8, the whole numbers of bf16)
+    a = torch.randint(-1, 2, (M, K), generator=g, device="cuda") * (torch.rand(M, K, generator=g, device="cuda") < 0.1)
+    b = torch.randint(-1, 2, (K, N), generator=g, device="cuda")
+    c0 = torch.randint(-9, 10, (M, N), generator=g, device="cuda")
+    exact = a.double() @ b.double()
+    assert exact.abs().max() < 240
+    ad, bd = a.to(getattr(torch, dt)), b.to(getattr(torch, dt))
+    if dt != "int8":
+        ad[M // 2, K - 1], bd[K - 1] = float("inf"), 1
+        exact = ad.double() @ bd.double()
+    for accumulate in (False, True):
+        for form in ({}, {"fuse_unpack": True}):
+            c = c0.to(getattr(torch, out_dt)).contiguous()
+            try:
+                ws = uk.matmul_data_tiled(ad, bd, c, M, N, K, type_flag, accumulate=accumulate, tile=tile, **form)
+            except ValueError:
+                assert form and tile is None and min(M, N) < 32
+                continue
+            assert uk.last_kernel_path() == "mmt4d:mfma-one-launch"
+            want = exact + c0.double() if accumulate else exact
+            assert torch.equal(c.double(), want)
+            M0, N0, K0 = uk.query_matmul_tile_sizes(uk.ukernel._MMT4D_TO_QUERY_OP[type_flag],
+                                                    *(() if tile else (M, N, K)))
+            M1, N1, K1 = -(-M // M0), -(-N // N0), -(-K // K0)
+            in_type, out_type = uk.ukernel._IN_PACK_TYPE[type_flag], uk.ukernel._OUT_PACK_TYPE[type_flag]
+            lhs, rhs = torch.empty_like(ws["lhs"]), torch.empty_like(ws["rhs"])
+            uk.pack(ad, lhs, M, K, M1, K1, M0, K0, 0, in_type)
+            uk.pack(bd, rhs, K, N, N1, K1, N0, K0, 0, in_type | F.PACK_TRANSPOSE_INNER | F.PACK_TRANSPOSE_OUTER)
+            assert torch.equal(ws["lhs"], lhs) and torch.equal(ws["rhs"], rhs)
+            if not form:
+                out = torch.empty_like(ws["out"])
+                uk.pack(c, out, M, N, M1, N1, M0, N0, 0, out_type)
+                back = torch.empty_like(c)
+                uk.unpack(ws["out"], back, M1, N1, M0, N0, M, N, out_type)
+                assert torch.equal(back, c)
+                if dt == "int8":                  # (float padding next to the infinity is 0 * 1 of either sign, or NaN)
+                    assert torch.equal(ws["out"], out)
+
+
+def test_small_matmul_leaves_shared_memory_to_the_chain(uk, cuda):
+    """A result that overlaps an operand, and operands whose rows are shorter
+    than a load: not served by the one launch, and the chain's results."""
+    import torch
+    g = torch.Generator(device="cuda").manual_seed(3)
+    a = torch.randint(-3, 4, (64, 64), generator=g, device="cuda").float()
+    want = a @ a
+    uk.matmul_data_tiled(a, a.clone(), a, 64, 64, 64, F.MMT4D_TYPE_F32F32F32)
+    assert uk.last_kernel_path() != "mmt4d:mfma-one-launch"
+    assert torch.equal(a, want)
+    for M, N, K in ((40, 3, 40), (40, 40, 3), (9, 1, 1)):
+        a = torch.randint(-3, 4, (M, K), generator=g, device="cuda").float()
+        b = torch.randint(-3, 4, (K, N), generator=g, device="cuda").float()
+        c = torch.empty(M, N, device="cuda")
+        uk.matmul_data_tiled(a, b, c, M, N, K, F.MMT4D_TYPE_F32F32F32)
+        assert uk.last_kernel_path() != "mmt4d:mfma-one-launch"
+        assert torch.equal(c, a @ b)
