@@ -622,7 +622,7 @@ IREE_AMD_UK_EXPORT int iree_amd_uk_matmul_packed_rhs(
     iree_amd_uk_index_t N, iree_amd_uk_index_t K, int32_t K0, uint32_t flags,
     float out_scale, void* stream);
 
-/* The whole data-tiled matmul of a small problem as one launch: what
+/* The whole data-tiled matmul of a small problem as one launch or two: what
  * pack(A), pack(B, inner and outer transposed), [pack(C)], mmt4d and unpack do
  * (REF compiler/src/iree/compiler/Codegen/Common/CPU/CPULowerToUKernels.cpp:339-480).
  *   c[m][n] (+)= sum_k a[m][k] * b[k][n]
@@ -633,7 +633,9 @@ IREE_AMD_UK_EXPORT int iree_amd_uk_matmul_packed_rhs(
  * Returns IREE_AMD_UK_STATUS_NOT_FOUND, with no error recorded and nothing
  * written, for what it does not serve (large problems, which the chain runs
  * faster; tiles without a matrix-core kernel; buffers that overlap): run the
- * chain then. Allocates nothing. */
+ * chain then. A long K of few tiles is split over workgroups, whose partial sums
+ * lie in the stream's scratch memory, and takes a second launch; while the
+ * stream is being captured it is not. */
 IREE_AMD_UK_EXPORT int iree_amd_uk_matmul_data_tiled(
     const void* a, const void* b, void* c, void* lhs, void* rhs, void* out, iree_amd_uk_index_t M,
     iree_amd_uk_index_t N, iree_amd_uk_index_t K, int32_t M0, int32_t N0, int32_t K0, uint32_t flags,

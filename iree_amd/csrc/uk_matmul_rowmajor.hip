@@ -1,5 +1,5 @@
 // The whole data-tiled matmul (pack, pack, [pack C,] mmt4d, unpack) of a small
-// problem as ONE launch.
+// problem as ONE launch, or two where K is split.
 //
 // Contract: include/iree_amd_uk.h, iree_amd_uk_matmul_data_tiled. The sequence
 // it stands for is the reference's
@@ -13,6 +13,12 @@
 //
 // Among other calls on one stream: f16 81x19x41 21.1 us as the chain, 6.6 here; i8
 // 1024^3 21.0, 11.4.
+//
+// A step of K costs a workgroup 2.4 to 3.9 us: its 24 loads per thread, many of
+// them of rows 64 bytes long, pass the compute unit's one load path. So a long
+// K of few tiles is dealt to more workgroups, each with its own plane of partial
+// sums, and a second launch adds the planes in order (2 us when it follows):
+// bf16 64x29x3693 35.0 us whole, 8.7 in 8 slices.
 //
 // Multiplying workgroups: 4 waves on kRows x kRows of the result, 64 KiB of
 // operands per K-step (128 KiB / kRows bytes of K), fetched for the next
@@ -61,6 +67,11 @@ struct RowMajorArgs {
   int M, N, K, M0, N0, M1, N1, K1;
   int tiles_n, product_blocks, lhs_blocks;
   int accumulate;
+  // K split: product block t + tiles * i multiplies the elements [i slice_k,
+  // (i + 1) slice_k) of K for tile t into its own plane of partial sums (rows and
+  // columns in whole tiles, accumulator type); partial is null without one.
+  int tiles, slices, slice_k;
+  void* partial;
 };
 
 // A 128-bit value moved down by `bytes` (0 to 15), zeros from above.
@@ -162,6 +173,32 @@ __device__ void pack_block(const RowMajorArgs& p, int block) {
   }
 }
 
+// What the sums of a result type are held in.
+template <typename out_t>
+struct Sum { typedef typename std::conditional<std::is_same<out_t, int32_t>::value, int32_t, float>::type type; };
+
+// Adds the planes of a K split in order, then the old result, and stores the
+// matrix and its tiles: one element per thread.
+template <typename out_t>
+__global__ __launch_bounds__(256) void matmul_rowmajor_sum_kernel(RowMajorArgs p, int rows, int cols) {
+  typedef typename Sum<out_t>::type sum_t;
+  const int64_t at = (int64_t)blockIdx.x * 256 + threadIdx.x, plane = (int64_t)rows * cols;
+  if (at >= plane) return;
+  const int m = (int)(at / cols), n = (int)(at - (int64_t)m * cols);
+  const int m1 = m / p.M0, m0 = m - m1 * p.M0, n1 = n / p.N0, n0 = n - n1 * p.N0;
+  const bool in_matrix = m < p.M && n < p.N, in_tiles = p.out && m1 < p.M1 && n1 < p.N1;
+  if (!in_matrix && !in_tiles) return;
+  const sum_t* part = (const sum_t*)p.partial + at;
+  out_t* const c = (out_t*)p.c + (int64_t)m * p.N + n;
+  const sum_t old = p.accumulate && in_matrix ? (sum_t)*c : (sum_t)0;
+  sum_t sum = 0;
+#pragma unroll 8
+  for (int i = 0; i < p.slices; ++i) sum += part[i * plane];
+  const out_t v = (out_t)(sum + old);
+  if (in_matrix) *c = v;
+  if (in_tiles) ((out_t*)p.out)[(((int64_t)m1 * p.N1 + n1) * p.M0 + m0) * p.N0 + n0] = v;
+}
+
 template <typename Cfg, int kRows>
 __global__ __launch_bounds__(256, 2) void matmul_rowmajor_kernel(RowMajorArgs p) {
   constexpr int kElemBytes = Cfg::kElemBytes;
@@ -178,7 +215,9 @@ __global__ __launch_bounds__(256, 2) void matmul_rowmajor_kernel(RowMajorArgs p)
     return;
   }
   const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
-  const int m_base = (int)blockIdx.x / p.tiles_n * kRows, n_base = (int)blockIdx.x % p.tiles_n * kRows;
+  const int slice = (int)blockIdx.x / p.tiles, tile = (int)blockIdx.x - slice * p.tiles;
+  const int m_base = tile / p.tiles_n * kRows, n_base = tile % p.tiles_n * kRows;
+  const int k_first = slice * p.slice_k, k_end = k_first + p.slice_k < p.K ? k_first + p.slice_k : p.K;
   auto place = [](int row, int chunk) { return row * kChunks + (chunk ^ ((row + (row >> 4)) & 15)); };
 
   // what this thread fetches of a step: chunk t % kChunks of 8 rows of A, and
@@ -208,7 +247,7 @@ __global__ __launch_bounds__(256, 2) void matmul_rowmajor_kernel(RowMajorArgs p)
       }
     }
   };
-  fetch(0);
+  fetch(k_first);
 
   // The wave's 2 x 2 blocks of 16x16: element r of a lane is row 4 (lane / 16) + r,
   // column lane % 16.
@@ -219,7 +258,7 @@ __global__ __launch_bounds__(256, 2) void matmul_rowmajor_kernel(RowMajorArgs p)
   // of a sum grows with the number of terms it takes one by one.
   acc_t acc[2][2] = {}, old[2][2] = {};
   out_t* const c = (out_t*)p.c;
-  if (p.accumulate && owner) {
+  if (p.accumulate && owner && !p.partial) {
 #pragma unroll
     for (int i = 0; i < 2; ++i)
 #pragma unroll
@@ -231,10 +270,10 @@ __global__ __launch_bounds__(256, 2) void matmul_rowmajor_kernel(RowMajorArgs p)
         }
   }
 
-  for (int k_base = 0; k_base < p.K; k_base += kStep) {
-    const int left = p.K - k_base;
+  for (int k_base = k_first; k_base < k_end; k_base += kStep) {
+    const int left = k_end - k_base;
     const int subs = left >= kStep ? kChunks / 4 : (left + 4 * E - 1) / (4 * E);   // of 4 chunks: one instruction's K
-    if (k_base) __syncthreads();
+    if (k_base > k_first) __syncthreads();
     if (t % kChunks < subs * 4) {
 #pragma unroll
       for (int j = 0; j < 8; ++j)
@@ -254,7 +293,7 @@ __global__ __launch_bounds__(256, 2) void matmul_rowmajor_kernel(RowMajorArgs p)
       }
     }
     __syncthreads();
-    if (k_base + kStep < p.K) fetch(k_base + kStep);
+    if (k_base + kStep < k_end) fetch(k_base + kStep);
     acc_t part[2][2][2] = {};
     auto multiply = [&](int s, acc_t (&sum)[2][2]) {
       union { u32x4 u; frag_t f; } fa[2], fb[2];
@@ -294,6 +333,19 @@ __global__ __launch_bounds__(256, 2) void matmul_rowmajor_kernel(RowMajorArgs p)
 #pragma unroll
       for (int i = 0; i < 4; ++i) acc[i / 2][i % 2] += part[(w * 4 + i) * 64 + lane];
   }
+  if (p.partial) {
+    typedef typename Sum<out_t>::type sum_t;
+    const int rows = p.tiles / p.tiles_n * kRows, cols = p.tiles_n * kRows;
+    sum_t* const part = (sum_t*)p.partial + (int64_t)slice * rows * cols;
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+      for (int j = 0; j < 2; ++j)
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+          part[(int64_t)(m_base + wm + i * 16 + lane / 16 * 4 + r) * cols + n_base + wn + j * 16 + lane % 16] = acc[i][j][r];
+    return;
+  }
   out_t* const out = (out_t*)p.out;
 #pragma unroll
   for (int j = 0; j < 2; ++j) {
@@ -314,44 +366,100 @@ __global__ __launch_bounds__(256, 2) void matmul_rowmajor_kernel(RowMajorArgs p)
   }
 }
 
-// Estimated time in microseconds on kRows = side, and the rule: the launch is
-// taken when the estimate, 10 % added, is below what the chain's launches cost by
-// themselves (5 us each when they follow each other, less 1). A step takes about as
-// long whatever else runs, until a compute unit holds more than one workgroup;
-// then the packed buffers and the result, at 6 TB/s. Measured and estimated, against
-// the chain (i8 1024^3 11.4, 11.7, chain 21.0; f16 81x19x41 6.6, 7.0, 21.1;
-// 512^3 6.8, 7.6, 21.2; 768^3 12.6, 13.5, 21.0; 1024^3 16.0, 17.2, 21.4; 3000x8x1325 13.4,
-// 12.5, 20.7; f32 512^3 10.4, 10.9, 30.4). Beyond the rule the chain's kernels win: f16
-// 2048 x 2048 x 1024 36.8 us here, 28.9 there.
+// Estimated time in microseconds on kRows = side with K in `slices`. A step takes
+// about as long whatever else runs, until a compute unit holds more than one
+// workgroup; then the packed buffers and the result, and for a split the planes
+// of sums, written and read, and the second launch. Fitted to 78 problems (f32,
+// 16-bit and i8; 10 to 3900 rows and columns, K 200 to 4000) on both sides and
+// 1 to 16 slices: 12 % off on average, and what it picks is 1.8 % from the best.
 template <typename Cfg>
-double estimate_us(const RowMajorArgs& p, int side) {
+double estimate_us(const RowMajorArgs& p, int side, int slices) {
   constexpr bool kF32 = Cfg::kElemBytes == 4;   // (whose instructions take as long as a step's loads)
-  const double step_us = side == 64 ? (kF32 ? 3.7 : 2.6) : (kF32 ? 2.7 : 2.4);
+  const double step_us = side == 64 ? (kF32 ? 3.9 : 3.0) : 2.8;
   const int64_t rows = (int64_t)p.M1 * p.M0, cols = (int64_t)p.N1 * p.N0;
-  const int64_t groups = ceil_div(rows, (int64_t)side) * ceil_div(cols, (int64_t)side);
+  const int64_t tiles = ceil_div(rows, (int64_t)side) * ceil_div(cols, (int64_t)side);
   const int64_t steps = ceil_div((int64_t)p.K * Cfg::kElemBytes, (int64_t)32768 / side);
-  const double load = 0.7 * groups / device_cu_count();
+  const double load = (double)tiles * slices / device_cu_count();
   const double bytes = (p.lhs ? 32.0 * rows * p.K1 : 0) + (p.rhs ? 32.0 * cols * p.K1 : 0) +
                        (p.out ? 2.0 : 1.0) * rows * cols * sizeof(typename Cfg::out_t);
-  return 4.5 + steps * step_us * (load > 1 ? load : 1) + bytes / 6e6;
+  const double us = 4.3 + ceil_div(steps, (int64_t)slices) * step_us * (load > 1 ? load : 1) + bytes / 5.6e6;
+  return slices > 1 ? us + 1.3 + 4.0 * slices * tiles * side * side / 2.8e6 : us;
+}
+
+// What the chain takes, from below: 5 us a launch when they follow each other,
+// less 1, half a microsecond per MB of packed operands, and what the f32 matmul, which
+// has no K split for so few tiles, takes beyond its launch (f32 172x54x2690 38.8
+// us, estimated 37.4; bf16 1743x286x1222 25.3, 21.5; f16 54x163x733 17.0, 19.1).
+// The rule: the estimate with 10 % added is below it. f16 54x163x733 8.6 us here;
+// bf16 64x29x3693 21.2 as the chain, 35.0 here with K whole, 8.7 in 8 slices; f32
+// 20x589x4022 43.6, 56.0, 13.5; i8 1024^3 18.7 and 11.5. Beyond it the chain wins:
+// bf16 3421x599x980 24.4 as the chain, 36.7 here.
+template <typename Cfg>
+double chain_us(const RowMajorArgs& p) {
+  const int launches = (p.lhs != nullptr) + (p.rhs != nullptr) + 1 + (p.out ? 1 + p.accumulate : 0);
+  const double mb = 16e-6 * p.K1 * ((double)p.M1 * p.M0 + (double)p.N1 * p.N0);
+  const double f32 = Cfg::kElemBytes == 4 ? 4 + 0.004 * p.K : 0;
+  return 5.0 * launches - 1.0 + 0.5 * mb + (f32 < 13 ? f32 : 13);
+}
+
+// The fastest of both sides and 1 to max_slices slices of K; its estimated time.
+template <typename Cfg>
+double choose(const RowMajorArgs& p, int max_slices, int* side, int* slices) {
+  double us = 1e30;
+  for (int try_side = 32; try_side <= 64; try_side += 32) {
+    const int64_t steps = ceil_div((int64_t)p.K * Cfg::kElemBytes, (int64_t)32768 / try_side);
+    for (int n = 1; n <= max_slices && n <= steps; ++n) {
+      const double t = estimate_us<Cfg>(p, try_side, n);
+      if (t < us) { us = t; *side = try_side; *slices = n; }
+    }
+  }
+  return us;
 }
 
 template <typename Cfg>
 int launch(RowMajorArgs p, hipStream_t s) {
   const int64_t rows = (int64_t)p.M1 * p.M0, cols = (int64_t)p.N1 * p.N0;
-  const double us32 = estimate_us<Cfg>(p, 32), us64 = estimate_us<Cfg>(p, 64);
-  const bool small = us32 < us64;
-  const int launches = (p.lhs != nullptr) + (p.rhs != nullptr) + 1 + (p.out ? 1 + p.accumulate : 0);
-  if ((small ? us32 : us64) * 1.1 > 5.0 * launches - 1.0) return IREE_AMD_UK_STATUS_NOT_FOUND;
-  const int side = small ? 32 : 64;
-  p.tiles_n = (int)ceil_div(cols, (int64_t)side);
-  p.product_blocks = (int)(ceil_div(rows, (int64_t)side) * p.tiles_n);
+  const double limit = chain_us<Cfg>(p) / 1.1;
+  int side = 32, slices = 1;
+  if (choose<Cfg>(p, 16, &side, &slices) > limit) return IREE_AMD_UK_STATUS_NOT_FOUND;
+  const int64_t elem_step = 32768 / Cfg::kElemBytes;              // elements of K per step, times the side
+  auto lay_out = [&] {
+    p.tiles_n = (int)ceil_div(cols, (int64_t)side);
+    p.tiles = (int)(ceil_div(rows, (int64_t)side) * p.tiles_n);
+    const int64_t step = elem_step / side;
+    p.slice_k = (int)(ceil_div(ceil_div((int64_t)p.K, step), (int64_t)slices) * step);
+    slices = (int)ceil_div((int64_t)p.K, (int64_t)p.slice_k);     // (no empty last slice)
+  };
+  lay_out();
+  bool may_split = slices > 1;
+  if (may_split) {
+    // (a graph keeps the addresses of its nodes: a call being captured takes no
+    // memory that a later call on the stream may replace)
+    hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+    const bool known = hipStreamIsCapturing(s, &capture) == hipSuccess;
+    if (!known) (void)hipGetLastError();
+    may_split = known && capture == hipStreamCaptureStatusNone;
+  }
+  ScratchLease lease(s, may_split ? (size_t)slices * p.tiles * side * side * 4 : 0);
+  if (slices > 1 && !lease.ptr()) {
+    if (choose<Cfg>(p, 1, &side, &slices) > limit) return IREE_AMD_UK_STATUS_NOT_FOUND;
+    lay_out();
+  }
+  const int64_t plane = (int64_t)p.tiles * side * side;
+  p.slices = slices;
+  p.partial = slices > 1 ? lease.ptr() : nullptr;
+  p.product_blocks = p.tiles * slices;
   p.lhs_blocks = p.lhs ? (int)ceil_div(rows * p.K1, (int64_t)256) : 0;
   const int rhs_blocks = p.rhs ? (int)ceil_div(cols * p.K1, (int64_t)256) : 0;
   const dim3 grid((unsigned)(p.product_blocks + p.lhs_blocks + rhs_blocks)), block(256);
-  if (small) hipLaunchKernelGGL((matmul_rowmajor_kernel<Cfg, 32>), grid, block, 0, s, p);
+  if (side == 32) hipLaunchKernelGGL((matmul_rowmajor_kernel<Cfg, 32>), grid, block, 0, s, p);
   else hipLaunchKernelGGL((matmul_rowmajor_kernel<Cfg, 64>), grid, block, 0, s, p);
-  return check_hip(hipGetLastError(), "matmul_rowmajor launch");
+  const int st = check_hip(hipGetLastError(), "matmul_rowmajor launch");
+  if (st || slices == 1) return st;
+  const int padded_cols = p.tiles_n * side;
+  hipLaunchKernelGGL(matmul_rowmajor_sum_kernel<typename Cfg::out_t>, dim3((unsigned)ceil_div(plane, (int64_t)256)),
+                     block, 0, s, p, (int)(plane / padded_cols), padded_cols);
+  return check_hip(hipGetLastError(), "matmul_rowmajor sum launch");
 }
 
 }  // namespace
@@ -387,7 +495,7 @@ int launch_matmul_rowmajor(const void* a, const void* b, void* c, void* lhs, voi
     return IREE_AMD_UK_STATUS_NOT_FOUND;
   RowMajorArgs p = {(const char*)a, (const char*)b, (char*)c, (char*)lhs, (char*)rhs, (char*)out,
                     (int)M, (int)N, (int)K, M0, N0, (int)M1, (int)N1, (int)K1, 0, 0, 0,
-                    (flags & IREE_AMD_UK_FLAG_MMT4D_ACCUMULATE) != 0};
+                    (flags & IREE_AMD_UK_FLAG_MMT4D_ACCUMULATE) != 0, 0, 1, 0, nullptr};
   switch (flags & IREE_AMD_UK_FLAG_MMT4D_TYPE_MASK) {
     case IREE_AMD_UK_FLAG_MMT4D_TYPE_F16F16F32: return launch<F16Cfg16>(p, s);
     case IREE_AMD_UK_FLAG_MMT4D_TYPE_BF16BF16F32: return launch<BF16Cfg16>(p, s);

@@ -1248,6 +1248,48 @@ def test_small_matmul_in_one_launch(uk, cuda, type_flag, dt, out_dt, M, N, K, ti
                     assert torch.equal(ws["out"], out)
 
 
+@pytest.mark.parametrize("M,N,K,tile", [
+    (11, 25, 3195, None), (64, 29, 3693, "dynamic"), (33, 100, 1030, None), (20, 589, 4022, "dynamic"), (350, 65, 1025, None),
+])
+@pytest.mark.parametrize("type_flag,dt,out_dt", [
+    (F.MMT4D_TYPE_F16F16F32, "float16", "float32"), (F.MMT4D_TYPE_BF16BF16BF16, "bfloat16", "bfloat16"),
+    (F.MMT4D_TYPE_S8S8S32, "int8", "int32"), (F.MMT4D_TYPE_F32F32F32, "float32", "float32"),
+])
+def test_small_matmul_with_k_split(uk, cuda, type_flag, dt, out_dt, M, N, K, tile):
+    """The same with a K long enough to be split over workgroups: last slices of
+    one element and more, of a part of a step, and of whole ones."""
+    test_small_matmul_in_one_launch(uk, cuda, type_flag, dt, out_dt, M, N, K, tile)
+
+
+def test_small_matmul_with_long_k_in_a_graph(uk, cuda):
+    """Captured, the same call keeps no scratch memory: replays after eager
+    calls that grow and use the stream's are what the eager call gives."""
+    import torch
+    M, N, K = 64, 29, 3693
+    g = torch.Generator(device="cuda").manual_seed(4)
+    a = torch.randint(-3, 4, (M, K), generator=g, device="cuda").float()
+    b = torch.randint(-3, 4, (K, N), generator=g, device="cuda").float()
+    c, ws, stream = torch.zeros(M, N, device="cuda"), {}, torch.cuda.Stream()
+    stream.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(stream):
+        uk.matmul_data_tiled(a, b, c, M, N, K, F.MMT4D_TYPE_F32F32F32, workspace=ws)
+    stream.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=stream):
+        uk.matmul_data_tiled(a, b, c, M, N, K, F.MMT4D_TYPE_F32F32F32, workspace=ws)
+    for i in range(3):
+        a.copy_(torch.randint(-3, 4, (M, K), generator=g, device="cuda").float())
+        c.fill_(-1)
+        torch.cuda.synchronize()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(c, (a.double() @ b.double()).float()), i
+        with torch.cuda.stream(stream):
+            uk.matmul_data_tiled(b.t().contiguous(), a.t().contiguous(), torch.empty(N, M, device="cuda"), N, M, K,
+                                 F.MMT4D_TYPE_F32F32F32)
+        stream.synchronize()
+
+
 def test_small_matmul_leaves_shared_memory_to_the_chain(uk, cuda):
     """A result that overlaps an operand, and operands whose rows are shorter
     than a load: not served by the one launch, and the chain's results."""
