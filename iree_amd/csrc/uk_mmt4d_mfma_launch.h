@@ -349,20 +349,36 @@ int launch_estimated(const MfmaArgs& a, hipStream_t s) {
   double best_us = 0;
   const int best = pick(a.M, a.N, &best_us);
   // K over workgroup rows: at most one round, slices of 768 elements and more
-  // of K; it has to win by 3 %.
+  // of K; it has to win by 3 %. iree_amd_uk_mmt4d_noalloc_p runs the same kernels
+  // and refuses a split whose partial sums its array does not hold, so on
+  // operands that it takes such a split is for the large problems that no split
+  // within the array serves (not even two slices fit, both sides from 1024): there
+  // it has to win by 25 %. i8 1792 x 2432 x 16384, three slices: 74 us estimated,
+  // 96 whole. (A smaller problem gains up to a fifth by the estimate from more
+  // slices than fit: the price of serving it. Both rules restated on the CPU over 6
+  // million problems: this one refuses 0.4 %, all of them refused before there
+  // were tiles with a side of 192 as well.)
   if (a.k_slices == 0 && a.batch <= 1) {
-    double split_us = best_us * 0.97;
-    int split_v = 0, split_n = 0;
-    for (int n = 2; n <= 8 && (int64_t)a.ksteps * Cfg::kMfmaK / n >= 768; ++n)
+    struct Split { double us; int v, n; };
+    Split fits = {best_us * 0.97, 0, 0}, any = fits;
+    const int64_t slice_bytes = (int64_t)a.M * a.N * 4096;
+    const bool bounded = !a.lhs_row_major;   // (row-major results split as tiled ones do: the same bits)
+    for (int n = 2; n <= 8 && (int64_t)a.ksteps * Cfg::kMfmaK / n >= 768; ++n) {
+      const int64_t slices = ceil_div((int64_t)a.ksteps, ceil_div((int64_t)a.ksteps, (int64_t)n));   // (as launched)
+      const bool n_fits = !bounded || slices * slice_bytes <= (int64_t)IREE_AMD_UK_NOALLOC_SCRATCH_BYTES;
       for (int v = 0; v < kTilesWithMedium; ++v) {
         const MediumTile& t = kMediumTiles[v];
         const int64_t tiles = ceil_div((int64_t)a.M, (int64_t)2 * t.wm) * ceil_div((int64_t)a.N, (int64_t)2 * t.wn) * n;
         if (tiles > (int64_t)t.occ * cus) continue;
         const double us = estimate_us(a, kOutBytes, v, a.M, a.N, n);
-        if (us < split_us) { split_us = us; split_v = v; split_n = n; }
+        if (us < any.us) any = {us, v, n};
+        if (n_fits && us < fits.us) fits = {us, v, n};
       }
-    if (split_n > 1) {
-      const int st = launch_k_split<Cfg>(a, split_v, split_n, s);
+    }
+    const bool large = 2 * slice_bytes > (int64_t)IREE_AMD_UK_NOALLOC_SCRATCH_BYTES && a.M >= 32 && a.N >= 32;
+    const Split& split = large && any.us * 1.25 <= fits.us ? any : fits;
+    if (split.n > 1) {
+      const int st = launch_k_split<Cfg>(a, split.v, split.n, s);
       if (st != IREE_AMD_UK_STATUS_NOT_FOUND) return st;
     }
   }

@@ -113,6 +113,33 @@ def test_noalloc_mmt4d_on_random_data_and_beyond_the_limit(uk, cuda):
     assert bool((gs[8:] == -5).all()) and bool((gs[:8, 16:] == -5).all())
 
 
+@pytest.mark.parametrize("M1,N1,K1", [(58, 25, 2296), (37, 80, 940), (8, 218, 2012)])
+def test_noalloc_mmt4d_splits_k_no_further_than_its_array_holds(uk, cuda, M1, N1, K1):
+    """More slices than the array holds would be faster by the estimate: the
+    call is served all the same, with the bits of iree_amd_uk_mmt4d_p."""
+    import torch
+    from iree_amd._lib import Mmt4dParams
+    lib = uk.load_library()
+    rng = np.random.default_rng(M1)
+    lhs = torch.from_numpy(rng.integers(-128, 128, M1 * K1 * 512, dtype=np.int8)).cuda()
+    rhs = torch.from_numpy(rng.integers(-128, 128, N1 * K1 * 512, dtype=np.int8)).cuda()
+    stream = C.c_void_p(torch.cuda.current_stream().cuda_stream)
+    results = []
+    for entry in (lib.iree_amd_uk_mmt4d_noalloc_p, lib.iree_amd_uk_mmt4d_p):
+        out = torch.full((M1 * N1 * 1024,), -5, dtype=torch.int32, device=cuda)
+        p = Mmt4dParams(lhs.data_ptr(), 0, K1 * 512, rhs.data_ptr(), 0, K1 * 512, out.data_ptr(), 0, N1 * 1024,
+                        M1, N1, K1, 32, 32, 16, F.MMT4D_TYPE_S8S8S32, None)
+        assert entry(C.byref(p), stream) == 0, lib.iree_amd_uk_last_error()
+        torch.cuda.synchronize()
+        results.append(out)
+    assert torch.equal(results[0], results[1])
+    # one tile against the products themselves (tiles are [row][16 of K])
+    a = lhs.view(M1, K1, 32, 16)[-1].permute(1, 0, 2).reshape(32, -1).cpu().to(torch.int64)
+    b = rhs.view(N1, K1, 32, 16)[-1].permute(1, 0, 2).reshape(32, -1).cpu().to(torch.int64)
+    want = (a.double() @ b.double().T).to(torch.int32)   # (exact: sums stay below 2^53)
+    assert torch.equal(results[0].view(M1, N1, 32, 32)[-1, -1].cpu(), want)
+
+
 def test_noalloc_mmt4d_with_16_bit_operands(uk, cuda):
     """The 16-bit left-hand-side types keep their int8 digit planes and the
     product of the planes in the same array when they fit (4 x 4 and 16 x 16
