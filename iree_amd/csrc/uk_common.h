@@ -136,6 +136,8 @@ int launch_ksplit_reduce(const KSplitReduceArgs& r, hipStream_t s);
 // The object must stay alive until the last launch that uses the memory has
 // been queued: until then the buffer is neither evicted nor replaced. ptr() is
 // nullptr when the memory cannot be had (the call then takes its fallback).
+// While the stream is being captured into a graph only a buffer that is there
+// already is given out, and it is then kept for the graph's replays.
 //
 // A ScratchOverride on the calling thread replaces the cache for the calls made
 // under it: they get `ptr` when they need at most `bytes` and nothing
@@ -158,6 +160,11 @@ class ScratchLease {
   uint64_t id_ = 0;
   bool overflowed_ = false;
 };
+// The call is being captured into a graph, and scratch memory would be the
+// stream's cached buffer, which every other call on the stream uses too: two
+// graphs replayed side by side would share it. Splits that are only taken for
+// speed ask this first.
+bool scratch_under_capture(hipStream_t s);
 // Scratch memory a call cannot do without: the stream's cached buffer when it
 // can be leased, otherwise an allocation of the call's own, made and freed in
 // stream order on the caller's stream (hipMallocAsync / hipFreeAsync: some

@@ -431,15 +431,9 @@ int launch(RowMajorArgs p, hipStream_t s) {
     slices = (int)ceil_div((int64_t)p.K, (int64_t)p.slice_k);     // (no empty last slice)
   };
   lay_out();
-  bool may_split = slices > 1;
-  if (may_split) {
-    // (a graph keeps the addresses of its nodes: a call being captured takes no
-    // memory that a later call on the stream may replace)
-    hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
-    const bool known = hipStreamIsCapturing(s, &capture) == hipSuccess;
-    if (!known) (void)hipGetLastError();
-    may_split = known && capture == hipStreamCaptureStatusNone;
-  }
+  // (a graph keeps the addresses of its nodes: a call being captured takes no
+  // memory that other calls on the stream use too)
+  const bool may_split = slices > 1 && !scratch_under_capture(s);
   ScratchLease lease(s, may_split ? (size_t)slices * p.tiles * side * side * 4 : 0);
   if (slices > 1 && !lease.ptr()) {
     if (choose<Cfg>(p, 1, &side, &slices) > limit) return IREE_AMD_UK_STATUS_NOT_FOUND;

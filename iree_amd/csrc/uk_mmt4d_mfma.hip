@@ -96,7 +96,18 @@ ScratchCache& scratch_cache() {
 struct OverrideState { void* ptr; size_t bytes; bool strict, active; };
 thread_local OverrideState g_override = {nullptr, 0, false, false};
 
+// Whether work on `s` is recorded into a graph. (Where that cannot be told,
+// as for the legacy stream beside another's capture, nothing may be allocated
+// either.)
+bool is_capturing(hipStream_t s) {
+  hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing(s, &status) != hipSuccess) { (void)hipGetLastError(); return true; }
+  return status != hipStreamCaptureStatusNone;
+}
+
 }  // namespace
+
+bool scratch_under_capture(hipStream_t s) { return !g_override.active && is_capturing(s); }
 
 ScratchLease::ScratchLease(hipStream_t s, size_t bytes) {
   if (g_override.active) {
@@ -109,7 +120,7 @@ ScratchLease::ScratchLease(hipStream_t s, size_t bytes) {
   if (s == hipStreamPerThread) return;
   int device = 0;
   if (hipGetDevice(&device) != hipSuccess) { (void)hipGetLastError(); return; }
-  const ScratchCache::Lease lease = scratch_cache().acquire(device, (void*)s, bytes);
+  const ScratchCache::Lease lease = scratch_cache().acquire(device, (void*)s, bytes, bytes != 0 && is_capturing(s));
   ptr_ = lease.ptr;
   id_ = lease.id;
 }

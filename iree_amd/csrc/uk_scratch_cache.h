@@ -14,6 +14,14 @@
 //   * evicted: least recently used first, with a free that waits for the
 //              device, when the table is full (streams come and go),
 //   * released by release_idle() (a plugin's unload).
+//
+// A call that is being captured into a graph is different: nothing can be
+// allocated or freed under it, and the graph keeps the buffer's address for its
+// replays. It gets the buffer only if that exists and is large enough, and from
+// then on the buffer is kept: growing puts it aside instead of freeing it, and
+// it is not evicted. release_idle() frees it with the others. Growing at least
+// doubles, up to the largest size, so what is set aside for a stream stays below
+// twice that.
 #ifndef IREE_AMD_UK_SCRATCH_CACHE_H_
 #define IREE_AMD_UK_SCRATCH_CACHE_H_
 
@@ -46,23 +54,28 @@ class ScratchCache {
 
   // The buffer of (device, stream), at least `bytes` large, or a Lease without
   // a pointer when it cannot be had. Every Lease with an id must be released.
-  Lease acquire(int device, void* stream, size_t bytes) {
+  // `capturing`: the work is being recorded into a graph.
+  Lease acquire(int device, void* stream, size_t bytes, bool capturing = false) {
     Lease none;
     if (bytes == 0 || bytes > max_bytes_) return none;
     std::unique_lock<std::mutex> lock(mutex_);
     for (Entry& e : entries_) {
       if (e.device != device || e.stream != stream) continue;
       if (e.bytes < bytes) {
-        if (e.leases > 0) return none;      // in use: not replaced under its user
+        if (e.leases > 0 || capturing) return none;      // in use: not replaced under its user
         const size_t want = bytes * 2 < max_bytes_ ? bytes * 2 : max_bytes_;
         void* bigger = allocator_.alloc(want, allocator_.user);
         if (!bigger) return none;
-        allocator_.free_ordered(e.ptr, stream, allocator_.user);
+        if (e.captured) set_aside_.push_back(e.ptr);
+        else allocator_.free_ordered(e.ptr, stream, allocator_.user);
         e.ptr = bigger;
         e.bytes = want;
+        e.captured = false;
       }
+      e.captured |= capturing;
       return lease_of(e);
     }
+    if (capturing) return none;
     // A new entry. When the table is full the least recently used idle buffer
     // makes room; it leaves the table here and is freed (a free that waits for
     // the device) only after the lock has been dropped, so that other threads'
@@ -71,9 +84,9 @@ class ScratchCache {
     if (entries_.size() >= max_entries_) {
       size_t victim = entries_.size();
       for (size_t i = 0; i < entries_.size(); ++i)
-        if (entries_[i].leases == 0 && (victim == entries_.size() || entries_[i].last_use < entries_[victim].last_use))
+        if (entries_[i].leases == 0 && !entries_[i].captured && (victim == entries_.size() || entries_[i].last_use < entries_[victim].last_use))
           victim = i;
-      if (victim == entries_.size()) return none;   // every buffer is in use
+      if (victim == entries_.size()) return none;   // every buffer is in use or in a graph
       evicted = entries_[victim].ptr;
       entries_.erase(entries_.begin() + (long)victim);
     }
@@ -87,7 +100,7 @@ class ScratchCache {
     }
     Lease lease;
     if (ptr) {
-      entries_.push_back(Entry{device, stream, ptr, want, 0, 0, next_id_++});
+      entries_.push_back(Entry{device, stream, ptr, want, 0, 0, next_id_++, false});
       lease = lease_of(entries_.back());
     }
     lock.unlock();
@@ -105,11 +118,13 @@ class ScratchCache {
       }
   }
 
-  // Frees every buffer without a lease; returns how many were freed.
+  // Frees every buffer without a lease, those of captured calls as well; returns
+  // how many were freed.
   size_t release_idle() {
     std::vector<void*> idle;
     {
       std::lock_guard<std::mutex> lock(mutex_);
+      idle.swap(set_aside_);
       for (size_t i = 0; i < entries_.size();) {
         if (entries_[i].leases == 0) {
           idle.push_back(entries_[i].ptr);
@@ -138,6 +153,7 @@ class ScratchCache {
     int leases;
     uint64_t last_use;
     uint64_t id;       // survives reordering of the table; a grown buffer keeps it
+    bool captured;     // a graph holds the address of ptr
   };
 
   Lease lease_of(Entry& e) {
@@ -153,6 +169,7 @@ class ScratchCache {
   size_t min_bytes_, max_bytes_, max_entries_;
   std::mutex mutex_;
   std::vector<Entry> entries_;
+  std::vector<void*> set_aside_;   // outgrown buffers that graphs hold
   uint64_t clock_ = 0, next_id_ = 1;
 };
 

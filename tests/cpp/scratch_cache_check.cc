@@ -114,6 +114,36 @@ int main() {
     cache.release(l0);
     CHECK(cache.release_idle() == 1 && c.live.empty());
   }
+  // a call captured into a graph: never an allocation, and the buffer whose
+  // address the graph keeps is neither freed by growth nor evicted
+  {
+    Counting c;
+    uk::ScratchCache cache(allocator(&c), 100, 1000, 2);
+    CHECK(!cache.acquire(0, stream(0), 50, true).ptr && c.allocs == 0);    // no buffer yet
+    auto a = cache.acquire(0, stream(0), 50);
+    cache.release(a);
+    CHECK(!cache.acquire(0, stream(0), 150, true).ptr && c.allocs == 1);   // too small: not grown
+    auto g = cache.acquire(0, stream(0), 60, true);
+    CHECK(g.ptr == a.ptr);
+    cache.release(g);
+    auto bigger = cache.acquire(0, stream(0), 300);                        // 600 bytes
+    CHECK(bigger.ptr && bigger.ptr != g.ptr && c.frees_ordered == 0 && c.live.count(g.ptr) == 1);
+    cache.release(bigger);
+    auto again = cache.acquire(0, stream(0), 700);                         // (no graph holds the 600 bytes)
+    CHECK(again.ptr && c.frees_ordered == 1 && c.live.count(bigger.ptr) == 0);
+    cache.release(again);
+    cache.release(cache.acquire(0, stream(0), 700, true));
+    cache.release(cache.acquire(0, stream(1), 10));
+    cache.release(cache.acquire(0, stream(2), 10));                        // stream 1 went, the captured one did not
+    CHECK(c.live.count(again.ptr) == 1 && c.frees_now == 1 && cache.entry_count() == 2);
+    cache.release(cache.acquire(0, stream(2), 10, true));
+    CHECK(!cache.acquire(0, stream(3), 10).ptr);                           // every buffer is in a graph
+    CHECK(cache.release_idle() == 3 && c.live.empty() && cache.entry_count() == 0);
+    auto fresh = cache.acquire(0, stream(0), 10);
+    CHECK(fresh.ptr);
+    cache.release(fresh);
+    cache.release_idle();
+  }
   // allocation failure leaves the table as it was
   {
     Counting c;

@@ -1261,33 +1261,94 @@ def test_small_matmul_with_k_split(uk, cuda, type_flag, dt, out_dt, M, N, K, til
     test_small_matmul_in_one_launch(uk, cuda, type_flag, dt, out_dt, M, N, K, tile)
 
 
-def test_small_matmul_with_long_k_in_a_graph(uk, cuda):
-    """Captured, the same call keeps no scratch memory: replays after eager
-    calls that grow and use the stream's are what the eager call gives."""
+@pytest.mark.parametrize("type_flag,dt,out_dt", [
+    (F.MMT4D_TYPE_F32F32F32, "float32", "float32"), (F.MMT4D_TYPE_F16F16F32, "float16", "float32"),
+    (F.MMT4D_TYPE_S8S8S32, "int8", "int32"),
+])
+def test_small_matmul_with_long_k_in_a_graph(uk, cuda, type_flag, dt, out_dt):
+    """Captured, the same call takes no scratch memory of its own (16-bit and i8
+    operands run the chain there, whose matmul splits K): replays after eager
+    calls that use the stream's are what the eager call gives."""
     import torch
     M, N, K = 64, 29, 3693
+    dt, out_dt = getattr(torch, dt), getattr(torch, out_dt)
     g = torch.Generator(device="cuda").manual_seed(4)
-    a = torch.randint(-3, 4, (M, K), generator=g, device="cuda").float()
-    b = torch.randint(-3, 4, (K, N), generator=g, device="cuda").float()
-    c, ws, stream = torch.zeros(M, N, device="cuda"), {}, torch.cuda.Stream()
+    a = torch.randint(-3, 4, (M, K), generator=g, device="cuda").to(dt)
+    b = torch.randint(-3, 4, (K, N), generator=g, device="cuda").to(dt)
+    c, ws, stream = torch.zeros(M, N, dtype=out_dt, device="cuda"), {}, torch.cuda.Stream()
     stream.wait_stream(torch.cuda.current_stream())
     with torch.cuda.stream(stream):
-        uk.matmul_data_tiled(a, b, c, M, N, K, F.MMT4D_TYPE_F32F32F32, workspace=ws)
+        uk.matmul_data_tiled(a, b, c, M, N, K, type_flag, workspace=ws)
     stream.synchronize()
     graph = torch.cuda.CUDAGraph()
     with torch.cuda.graph(graph, stream=stream):
-        uk.matmul_data_tiled(a, b, c, M, N, K, F.MMT4D_TYPE_F32F32F32, workspace=ws)
+        uk.matmul_data_tiled(a, b, c, M, N, K, type_flag, workspace=ws)
     for i in range(3):
-        a.copy_(torch.randint(-3, 4, (M, K), generator=g, device="cuda").float())
+        a.copy_(torch.randint(-3, 4, (M, K), generator=g, device="cuda").to(dt))
         c.fill_(-1)
         torch.cuda.synchronize()
         graph.replay()
         torch.cuda.synchronize()
-        assert torch.equal(c, (a.double() @ b.double()).float()), i
+        assert torch.equal(c, (a.double() @ b.double()).to(out_dt)), i
         with torch.cuda.stream(stream):
-            uk.matmul_data_tiled(b.t().contiguous(), a.t().contiguous(), torch.empty(N, M, device="cuda"), N, M, K,
-                                 F.MMT4D_TYPE_F32F32F32)
+            uk.matmul_data_tiled(b.t().contiguous(), a.t().contiguous(), torch.empty(N, M, dtype=out_dt, device="cuda"),
+                                 N, M, K, type_flag)
         stream.synchronize()
+
+
+@pytest.mark.parametrize("type_flag,K0,dt,out_dt", [
+    (F.MMT4D_TYPE_F16F16F32, 8, "float16", "float32"), (F.MMT4D_TYPE_S8S8S32, 16, "int8", "int32"),
+    (F.MMT4D_TYPE_F32F32F32, 4, "float32", "float32"),
+])
+@pytest.mark.parametrize("M0", [32, 2])
+def test_k_split_in_a_graph(uk, cuda, type_flag, K0, dt, out_dt, M0):
+    """A K split whose buffer existed at the capture: replays are right after the
+    stream has grown its buffer, and one captured on a stream without a buffer
+    runs whole. (With f16 and i8, M0 = 32, the second one's K is too short for a
+    split in a capture.) Small integers: exact in any order."""
+    import torch
+    dt, out_dt = getattr(torch, dt), getattr(torch, out_dt)
+    g = torch.Generator(device="cuda").manual_seed(M0 + K0)
+    M1, N1 = (4, 4) if M0 == 32 else (1, 4)
+
+    def problem(K):
+        lhs = torch.randint(-2, 3, (M1, K // K0, M0, K0), generator=g, device="cuda").to(dt)
+        rhs = torch.randint(-2, 3, (N1, K // K0, 32, K0), generator=g, device="cuda").to(dt)
+        return lhs, rhs, torch.zeros(M1, N1, M0, 32, dtype=out_dt, device="cuda")
+
+    def call(lhs, rhs, out):
+        uk.mmt4d(lhs, rhs, out, M1, N1, lhs.shape[1], M0, 32, K0, type_flag)
+
+    def want(lhs, rhs):
+        a = lhs.permute(0, 2, 1, 3).reshape(M1 * M0, -1).double()
+        b = rhs.permute(0, 2, 1, 3).reshape(N1 * 32, -1).double().t().contiguous()
+        return (a @ b).reshape(M1, M0, N1, 32).transpose(1, 2).to(out_dt)
+    warm, cold = torch.cuda.Stream(), torch.cuda.Stream()
+    first, second = problem(8192), problem(1536)
+    torch.cuda.synchronize()
+    with torch.cuda.stream(warm):
+        call(*first)
+    warm.synchronize()
+    graphs = torch.cuda.CUDAGraph(), torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graphs[0], stream=warm):
+        call(*first)
+    with torch.cuda.graph(graphs[1], stream=cold):
+        call(*second)
+    for i in range(3):
+        for graph, (lhs, rhs, out) in zip(graphs, (first, second)):
+            lhs.copy_(torch.randint(-2, 3, lhs.shape, generator=g, device="cuda").to(dt))
+            out.fill_(-1)
+            torch.cuda.synchronize()
+            graph.replay()
+            torch.cuda.synchronize()
+            assert torch.equal(out, want(lhs, rhs)), (i, lhs.shape)
+        # (i8 56 x 76 x 16384 in three slices: 52 MB of partial sums)
+        big = [torch.zeros(m * 1024 * 512, dtype=torch.int8, device="cuda") for m in (56, 76)]
+        torch.cuda.synchronize()
+        with torch.cuda.stream(warm):
+            uk.mmt4d(*big, torch.empty(56 * 76 * 1024, dtype=torch.int32, device="cuda"), 56, 76, 1024, 32, 32, 16,
+                     F.MMT4D_TYPE_S8S8S32)
+        warm.synchronize()
 
 
 def test_small_matmul_leaves_shared_memory_to_the_chain(uk, cuda):
