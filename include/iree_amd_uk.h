@@ -163,7 +163,13 @@ typedef struct iree_amd_uk_mmt4d_params_t {
  * partial sums in a scratch buffer the library allocates once per stream
  * (16 to 512 MiB; kept until iree_amd_uk_release_scratch or, with more than 64
  * streams in use, until it is the least recently used one); every other call
- * allocates nothing. */
+ * allocates nothing. A call that is being captured into a HIP graph allocates
+ * nothing either: it takes the stream's buffer if an earlier call has left one
+ * that is large enough, and otherwise runs whole. (f16, bf16 and i8 tiles with
+ * M0 = 32 split there from 64 matrix-core steps of K and only where the unsplit
+ * tiles leave half of the device idle.) A buffer that a captured call took is
+ * freed by iree_amd_uk_release_scratch alone, after which that graph must not be
+ * replayed; its replays must not overlap other splits of that stream. */
 IREE_AMD_UK_EXPORT int iree_amd_uk_mmt4d(
     const void* lhs_buffer, iree_amd_uk_index_t lhs_offset,
     iree_amd_uk_index_t lhs_stride0, const void* rhs_buffer,
@@ -422,8 +428,10 @@ IREE_AMD_UK_EXPORT int iree_amd_uk_query_matmul_tile_sizes(
  * (two per byte, even group in the low nibble) when ..._ZP_U4 is set. f32
  * accumulation, result rounded to f16 once (RNE). out: f16 [M][N] row-major.
  * Requires K % group_size == 0, group_size % 32 == 0, 1 <= M. A K beyond
- * 4096 is multiplied in slices whose f32 sums go through the stream's scratch
- * buffer (see iree_amd_uk_mmt4d on that buffer).
+ * 4096, and with more than 64 rows a shorter one where that is faster, is
+ * multiplied in slices whose f32 sums go through the stream's scratch buffer
+ * (see iree_amd_uk_mmt4d on that buffer; a call with K <= 4096 and more than 64
+ * rows that is being captured into a graph is not split).
  *===------------------------------------------------------------------------===*/
 #define IREE_AMD_UK_FLAG_DEQUANT_MATMUL_ZP_F16 0x0
 #define IREE_AMD_UK_FLAG_DEQUANT_MATMUL_ZP_U4 0x1

@@ -377,7 +377,14 @@ int launch_estimated(const MfmaArgs& a, hipStream_t s) {
     }
     const bool large = 2 * slice_bytes > (int64_t)IREE_AMD_UK_NOALLOC_SCRATCH_BYTES && a.M >= 32 && a.N >= 32;
     const Split& split = large && any.us * 1.25 <= fits.us ? any : fits;
-    if (split.n > 1) {
+    // A call being captured into a graph splits only a K of 64 steps and more
+    // whose unsplit tiles leave half of the device idle, where the gain is worth
+    // the condition that comes with it (a run before the capture, and no replay
+    // beside the stream's other splits).
+    const MediumTile& whole = kMediumTiles[best];
+    const int64_t whole_tiles = ceil_div((int64_t)a.M, (int64_t)2 * whole.wm) * ceil_div((int64_t)a.N, (int64_t)2 * whole.wn);
+    const bool worth = a.ksteps >= 64 && whole_tiles * 2 <= (int64_t)whole.occ * cus;
+    if (split.n > 1 && (worth || !scratch_under_capture(s))) {
       const int st = launch_k_split<Cfg>(a, split.v, split.n, s);
       if (st != IREE_AMD_UK_STATUS_NOT_FOUND) return st;
     }

@@ -471,34 +471,40 @@ int launch_dequant_gemm_i4(const I4Args& p, hipStream_t s) {
   struct Shape { int wm, wn; };
   static const Shape shapes[] = {{2, 4}, {2, 2}, {1, 4}, {1, 2}, {1, 1}};
   const int cus = device_cu_count();
-  int best = -1, best_slices = 1;
-  double best_cost = 0;
-  for (int v = 0; v < 5; ++v) {
-    const int wm = shapes[v].wm, wn = shapes[v].wn;
-    const int64_t tiles = ceil_div(p.M, wm * 64) * ceil_div(p.N, wn * 64);
-    if (tiles > 0x7FFFFFFF) continue;
-    for (int n = 1; n <= 8; ++n) {
-      if (n > 1 && a.spans / n < 4) break;
-      const int64_t slice_spans = ceil_div(a.spans, n);
-      // workgroups on the busiest compute unit (two of the 64-row ones fit)
-      const int64_t per_cu = ceil_div(tiles * n, (int64_t)cus);
-      const double valu = 680.0 * wm * wn, in = (wm * 4 + wn) * 4096.0 / 29.0;
-      double cost = per_cu * (slice_spans * ((valu > in ? valu : in) + 150) + 6000);
-      if (n > 1) cost += 7000 + (double)p.M * p.N * 4 * (n + 1) / 1500.0;
-      if (best < 0 || cost < best_cost) { best = v; best_slices = n; best_cost = cost; }
+  int best = -1, slices = 1;
+  auto choose = [&](int max_slices) {
+    best = -1;
+    double best_cost = 0;
+    for (int v = 0; v < 5; ++v) {
+      const int wm = shapes[v].wm, wn = shapes[v].wn;
+      const int64_t tiles = ceil_div(p.M, wm * 64) * ceil_div(p.N, wn * 64);
+      if (tiles > 0x7FFFFFFF) continue;
+      for (int n = 1; n <= max_slices; ++n) {
+        if (n > 1 && a.spans / n < 4) break;
+        const int64_t slice_spans = ceil_div(a.spans, n);
+        // workgroups on the busiest compute unit (two of the 64-row ones fit)
+        const int64_t per_cu = ceil_div(tiles * n, (int64_t)cus);
+        const double valu = 680.0 * wm * wn, in = (wm * 4 + wn) * 4096.0 / 29.0;
+        double cost = per_cu * (slice_spans * ((valu > in ? valu : in) + 150) + 6000);
+        if (n > 1) cost += 7000 + (double)p.M * p.N * 4 * (n + 1) / 1500.0;
+        if (best < 0 || cost < best_cost) { best = v; slices = n; best_cost = cost; }
+      }
     }
-  }
+    if (best < 0) return;
+    a.slice_spans = (int)ceil_div(a.spans, slices);
+    slices = (int)ceil_div(a.spans, a.slice_spans);
+  };
+  choose(8);
   if (best < 0) return IREE_AMD_UK_STATUS_NOT_FOUND;
-  int slices = best_slices;
-  a.slice_spans = (int)ceil_div(a.spans, slices);
-  slices = (int)ceil_div(a.spans, a.slice_spans);
+  // A call being captured takes no scratch memory where the kernels for fewer
+  // rows need none (K up to 4096, and what only this kernel serves): it need not
+  // have been made before, and the graph may be replayed beside others.
+  const bool may_split = slices > 1 && ((p.K > 4096 && p.K % 256 == 0) || !scratch_under_capture(s));
+  ScratchLease lease(s, may_split ? (size_t)slices * p.M * p.N * 4 : 0);
+  a.partial = (float*)lease.ptr();
+  if (slices > 1 && !a.partial) choose(1);
   a.tiles_m = (int)ceil_div(p.M, shapes[best].wm * 64);
   a.tiles_n = (int)ceil_div(p.N, shapes[best].wn * 64);
-  ScratchLease lease(s, slices > 1 ? (size_t)slices * p.M * p.N * 4 : 0);
-  if (slices > 1) {
-    a.partial = (float*)lease.ptr();
-    if (!a.partial) { slices = 1; a.slice_spans = a.spans; }
-  }
   int st;
   switch (best) {
     case 0: st = launch_gemm_shape<2, 4>(a, log2_ge, slices, s); break;

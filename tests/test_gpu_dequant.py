@@ -321,3 +321,43 @@ def test_many_rows(uk, cuda, M, N, K, gs):
     oracle's."""
     err, mag = run_case(uk, M, N, K, gs, True, True, seed=M + N + K, want_path="dequant_i4:gemm", repeats=1)
     assert err <= float(np.spacing(np.float16(max(1.0, mag))))
+
+
+@pytest.mark.parametrize("M,N,K", [(128, 1024, 2048), (256, 1024, 4096), (128, 4096, 4096)])
+def test_many_rows_in_a_graph(uk, cuda, M, N, K):
+    """A K of up to 4096, captured on a stream that has run nothing yet (an eager
+    call splits K here): no scratch memory, so replays between calls of the stream
+    that use its buffer are right. Data whose sums are exact in any
+    order (below 2^11 in f16, in quarters)."""
+    import torch
+    g = torch.Generator(device="cuda").manual_seed(M + N)
+    flags = F.DEQUANT_MATMUL_ZP_U4 | F.DEQUANT_MATMUL_W_TILED
+    w = torch.randint(0, 256, (N * K // 2,), generator=g, device="cuda", dtype=torch.uint8)
+    zp = torch.randint(0, 256, (N * K // 256,), generator=g, device="cuda", dtype=torch.uint8)
+    scale = torch.full((N * K // 128,), 0.25, dtype=torch.float16, device="cuda")
+
+    def rows():
+        x = torch.randint(-1, 2, (M, K), generator=g, device="cuda").half()
+        return x * (torch.rand(M, K, generator=g, device="cuda") < 32 / K)
+    x, out = rows(), torch.empty(M * N, dtype=torch.float16, device="cuda")
+    stream = torch.cuda.Stream()
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=stream):
+        uk.dequant_matmul_i4(x, w, scale, zp, out, M, N, K, 128, flags)
+    for i in range(3):
+        x.copy_(rows())
+        want = torch.empty_like(out)
+        with torch.cuda.stream(stream):
+            stream.wait_stream(torch.cuda.default_stream())
+            # (a split K, whose partial sums lie in the stream's buffer)
+            uk.dequant_matmul_i4(torch.randn(100, 14336, generator=g, device="cuda").half(), w.new_zeros(1024 * 7168),
+                                 scale.new_ones(1024 * 112), zp.new_zeros(1024 * 56), out.new_empty(100 * 1024),
+                                 100, 1024, 14336, 128, flags)
+            uk.dequant_matmul_i4(x, w, scale, zp, want, M, N, K, 128, flags)
+        assert uk.last_kernel_path() == "dequant_i4:gemm"
+        out.fill_(-1)
+        torch.cuda.synchronize()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out, want) and want.abs().max() > 1, i
