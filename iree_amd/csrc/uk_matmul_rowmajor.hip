@@ -372,19 +372,27 @@ __global__ __launch_bounds__(256, 2) void matmul_rowmajor_kernel(RowMajorArgs p)
 // of sums, written and read, and the second launch. Fitted to 78 problems (f32,
 // 16-bit and i8; 10 to 3900 rows and columns, K 200 to 4000) on both sides and
 // 1 to 16 slices: 12 % off on average, and what it picks is 1.8 % from the best.
-template <typename Cfg>
-double estimate_us(const RowMajorArgs& p, int side, int slices) {
-  constexpr bool kF32 = Cfg::kElemBytes == 4;   // (whose instructions take as long as a step's loads)
-  const double step_us = side == 64 ? (kF32 ? 3.9 : 3.0) : 2.8;
-  const int64_t rows = (int64_t)p.M1 * p.M0, cols = (int64_t)p.N1 * p.N0;
-  const int64_t tiles = ceil_div(rows, (int64_t)side) * ceil_div(cols, (int64_t)side);
-  const int64_t steps = ceil_div((int64_t)p.K * Cfg::kElemBytes, (int64_t)32768 / side);
-  const double load = (double)tiles * slices / device_cu_count();
-  const double bytes = (p.lhs ? 32.0 * rows * p.K1 : 0) + (p.rhs ? 32.0 * cols * p.K1 : 0) +
-                       (p.out ? 2.0 : 1.0) * rows * cols * sizeof(typename Cfg::out_t);
-  const double us = 4.3 + ceil_div(steps, (int64_t)slices) * step_us * (load > 1 ? load : 1) + bytes / 5.6e6;
-  return slices > 1 ? us + 1.3 + 4.0 * slices * tiles * side * side / 2.8e6 : us;
-}
+struct Estimate {
+  int64_t tiles, steps;
+  double step_us, bytes;
+  template <typename Cfg>
+  static Estimate of(const RowMajorArgs& p, int side) {
+    constexpr bool kF32 = Cfg::kElemBytes == 4;   // (whose instructions take as long as a step's loads)
+    const int64_t rows = (int64_t)p.M1 * p.M0, cols = (int64_t)p.N1 * p.N0;
+    return {ceil_div(rows, (int64_t)side) * ceil_div(cols, (int64_t)side),
+            ceil_div((int64_t)p.K * Cfg::kElemBytes, (int64_t)32768 / side),
+            side == 64 ? (kF32 ? 3.9 : 3.0) : 2.8,
+            (p.lhs ? 32.0 * rows * p.K1 : 0) + (p.rhs ? 32.0 * cols * p.K1 : 0) +
+                (p.out ? 2.0 : 1.0) * rows * cols * sizeof(typename Cfg::out_t)};
+  }
+  double us(int cus, int side, int slices) const {
+    const double load = (double)tiles * slices / cus;
+    const double us = 4.3 + ceil_div(steps, (int64_t)slices) * step_us * (load > 1 ? load : 1) + bytes / 5.6e6;
+    return slices > 1 ? us + 1.3 + 4.0 * slices * tiles * side * side / 2.8e6 : us;
+  }
+  // Below the time of every number of slices.
+  double least_us(int cus) const { return 4.3 + (double)steps * step_us * tiles / cus + bytes / 5.6e6; }
+};
 
 // What the chain takes, from below: 5 us a launch when they follow each other,
 // less 1, half a microsecond per MB of packed operands, and what the f32 matmul, which
@@ -402,18 +410,22 @@ double chain_us(const RowMajorArgs& p) {
   return 5.0 * launches - 1.0 + 0.5 * mb + (f32 < 13 ? f32 : 13);
 }
 
-// The fastest of both sides and 1 to max_slices slices of K; its estimated time.
+// The fastest of both sides and 1 to max_slices slices of K; false when none takes
+// limit_us or less. (A large problem, which is the chain's, is seen by least_us:
+// the estimates of all slices took 0.5 us of every chain.)
 template <typename Cfg>
-double choose(const RowMajorArgs& p, int max_slices, int* side, int* slices) {
-  double us = 1e30;
+bool choose(const RowMajorArgs& p, int max_slices, double limit_us, int* side, int* slices) {
+  const int cus = device_cu_count();
+  bool found = false;
   for (int try_side = 32; try_side <= 64; try_side += 32) {
-    const int64_t steps = ceil_div((int64_t)p.K * Cfg::kElemBytes, (int64_t)32768 / try_side);
-    for (int n = 1; n <= max_slices && n <= steps; ++n) {
-      const double t = estimate_us<Cfg>(p, try_side, n);
-      if (t < us) { us = t; *side = try_side; *slices = n; }
+    const Estimate e = Estimate::of<Cfg>(p, try_side);
+    if (e.least_us(cus) > limit_us) continue;
+    for (int n = 1; n <= max_slices && n <= e.steps; ++n) {
+      const double us = e.us(cus, try_side, n);
+      if (found ? us < limit_us : us <= limit_us) { found = true; limit_us = us; *side = try_side; *slices = n; }
     }
   }
-  return us;
+  return found;
 }
 
 template <typename Cfg>
@@ -421,7 +433,7 @@ int launch(RowMajorArgs p, hipStream_t s) {
   const int64_t rows = (int64_t)p.M1 * p.M0, cols = (int64_t)p.N1 * p.N0;
   const double limit = chain_us<Cfg>(p) / 1.1;
   int side = 32, slices = 1;
-  if (choose<Cfg>(p, 16, &side, &slices) > limit) return IREE_AMD_UK_STATUS_NOT_FOUND;
+  if (!choose<Cfg>(p, 16, limit, &side, &slices)) return IREE_AMD_UK_STATUS_NOT_FOUND;
   const int64_t elem_step = 32768 / Cfg::kElemBytes;              // elements of K per step, times the side
   auto lay_out = [&] {
     p.tiles_n = (int)ceil_div(cols, (int64_t)side);
@@ -436,7 +448,7 @@ int launch(RowMajorArgs p, hipStream_t s) {
   const bool may_split = slices > 1 && !scratch_under_capture(s);
   ScratchLease lease(s, may_split ? (size_t)slices * p.tiles * side * side * 4 : 0);
   if (slices > 1 && !lease.ptr()) {
-    if (choose<Cfg>(p, 1, &side, &slices) > limit) return IREE_AMD_UK_STATUS_NOT_FOUND;
+    if (!choose<Cfg>(p, 1, limit, &side, &slices)) return IREE_AMD_UK_STATUS_NOT_FOUND;
     lay_out();
   }
   const int64_t plane = (int64_t)p.tiles * side * side;

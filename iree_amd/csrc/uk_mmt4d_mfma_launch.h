@@ -231,7 +231,7 @@ int launch_k_split(const MfmaArgs& a, int v, int slices, hipStream_t s) {
 }
 
 // Estimated time in microseconds of the 16-row shapes on macro tile v with K in
-// `slices`, for M x N outer tiles. A step is 64 bytes of K. A workgroup's step
+// `slices`, for M x N outer tiles on `cus` compute units. A step is 64 bytes of K. A workgroup's step
 // takes longer the more of the compute units are busy (power, the L2s), from
 // idle to idle + busy; two workgroups on one compute unit take
 // shared times as long as one; a row-major left-hand side with the weights it
@@ -240,7 +240,9 @@ int launch_k_split(const MfmaArgs& a, int v, int slices, hipStream_t s) {
 // i8; 34 to 4096 rows, 64 to 14336 columns, K 256 to 14336, under sustained
 // load): what the estimate picks is 0.9 % slower than the best of them on
 // average and at most 25 %, 1.2 % on 420 other problems, where the rule before
-// it, on the first four tiles, was at 4.1 %. A bf16 1984 x 4128 x 3008 mmt4d takes
+// it, on the first four tiles, was at 4.1 %. (The caller looks `cus` up: one
+// lookup per estimate took 0.8 us of the host time of a call that splits K, 9.2
+// against 8.4 us.) A bf16 1984 x 4128 x 3008 mmt4d takes
 // 45 us on 192x192 tiles (242 workgroups) and 58 on the best of the first four.
 struct MediumTile { int wm, wn, occ; float idle, busy, shared, row_major; };
 constexpr MediumTile kMediumTiles[kTilesWithMedium] = {
@@ -248,9 +250,8 @@ constexpr MediumTile kMediumTiles[kTilesWithMedium] = {
     {2, 4, 2, 0.255f, 0.177f, 1.856f, 1.126f}, {2, 2, 2, 0.133f, 0.128f, 1.890f, 1.060f},
     {4, 3, 1, 0.354f, 0.275f, 1.0f, 1.112f},   {3, 4, 1, 0.354f, 0.275f, 1.0f, 1.101f},
     {3, 3, 1, 0.258f, 0.245f, 1.0f, 1.083f}};
-inline double estimate_us(const MfmaArgs& a, int out_bytes, int v, int64_t M, int64_t N, int slices) {
+inline double estimate_us(const MfmaArgs& a, int cus, int out_bytes, int v, int64_t M, int64_t N, int slices) {
   const MediumTile& t = kMediumTiles[v];
-  const int cus = device_cu_count();
   const int64_t tiles = ceil_div(M, (int64_t)2 * t.wm) * ceil_div(N, (int64_t)2 * t.wn) * slices *
                         (a.batch > 1 ? a.batch : 1);
   const int64_t slots = (int64_t)t.occ * cus, rounds = tiles / slots, rest = tiles % slots;
@@ -278,8 +279,7 @@ inline double estimate_us(const MfmaArgs& a, int out_bytes, int v, int64_t M, in
 // at least 5 % against best_cost (a launch costs a few microseconds, so only for
 // long K). NOT_FOUND when it is not taken.
 template <typename Cfg, bool kSiluMul, typename Cost, typename Pick>
-int launch_whole_rounds(const MfmaArgs& a, double best_cost, Cost cost_of, Pick pick, hipStream_t s) {
-  const int cus = device_cu_count();
+int launch_whole_rounds(const MfmaArgs& a, int cus, double best_cost, Cost cost_of, Pick pick, hipStream_t s) {
   auto launch = [&](int v, const MfmaArgs& b) -> int { return launch_by_index<Cfg, kSiluMul>(v, b, s); };
   const int64_t rows0 = ceil_div((int64_t)a.M, (int64_t)8);   // macro-tile rows of the large tile
   const int64_t cols0 = ceil_div((int64_t)a.N, (int64_t)8);
@@ -337,7 +337,7 @@ template <typename Cfg>
 int launch_estimated(const MfmaArgs& a, hipStream_t s) {
   constexpr int kOutBytes = (int)sizeof(typename Cfg::out_t);
   const int cus = device_cu_count();
-  auto us_of = [&](int v, int64_t M, int64_t N) -> double { return estimate_us(a, kOutBytes, v, M, N, 1); };
+  auto us_of = [&](int v, int64_t M, int64_t N) -> double { return estimate_us(a, cus, kOutBytes, v, M, N, 1); };
   auto pick = [&](int64_t M, int64_t N, double* out_us) -> int {
     int best = 0;
     for (int v = 0; v < kTilesWithMedium; ++v) {
@@ -370,7 +370,7 @@ int launch_estimated(const MfmaArgs& a, hipStream_t s) {
         const MediumTile& t = kMediumTiles[v];
         const int64_t tiles = ceil_div((int64_t)a.M, (int64_t)2 * t.wm) * ceil_div((int64_t)a.N, (int64_t)2 * t.wn) * n;
         if (tiles > (int64_t)t.occ * cus) continue;
-        const double us = estimate_us(a, kOutBytes, v, a.M, a.N, n);
+        const double us = estimate_us(a, cus, kOutBytes, v, a.M, a.N, n);
         if (us < any.us) any = {us, v, n};
         if (n_fits && us < fits.us) fits = {us, v, n};
       }
@@ -389,7 +389,7 @@ int launch_estimated(const MfmaArgs& a, hipStream_t s) {
       if (st != IREE_AMD_UK_STATUS_NOT_FOUND) return st;
     }
   }
-  const int st = launch_whole_rounds<Cfg, false>(a, best_us, us_of, pick, s);
+  const int st = launch_whole_rounds<Cfg, false>(a, cus, best_us, us_of, pick, s);
   if (st != IREE_AMD_UK_STATUS_NOT_FOUND) return st;
   return launch_by_index<Cfg, false>(best, a, s);
 }
@@ -508,8 +508,8 @@ int launch_cfg(const MfmaArgs& a, hipStream_t s) {
     }
   }
   {
-    const int st = launch_whole_rounds<Cfg, kSiluMul>(a, best_cost, [&](int v, int64_t M, int64_t N) { return cost_of(v, M, N); },
-                                                      pick, s);
+    const int st = launch_whole_rounds<Cfg, kSiluMul>(
+        a, cus, best_cost, [&](int v, int64_t M, int64_t N) { return cost_of(v, M, N); }, pick, s);
     if (st != IREE_AMD_UK_STATUS_NOT_FOUND) return st;
   }
   return launch(best, a);

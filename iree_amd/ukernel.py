@@ -52,7 +52,8 @@ def _stream(stream):
         if _raw_stream is not None:
             return _raw_stream(torch.cuda.current_device())
         stream = torch.cuda.current_stream()
-    return stream.cuda_stream
+    # (a handle that the caller has looked up once for several calls)
+    return stream if type(stream) is int else stream.cuda_stream
 
 
 def mmt4d(lhs_buffer, rhs_buffer, out_buffer, M, N, K, M0, N0, K0, flags, *,
@@ -433,39 +434,40 @@ def matmul_data_tiled(a, b, c, M, N, K, mmt4d_type, *, accumulate=False,
         ws["out"] = torch.empty(M1 * N1 * M0 * N0, dtype=c.dtype, device=c.device)
     mm_flags = mmt4d_type | F.MMT4D_ALLOW_GENERIC_FALLBACK_TILE_FUNCTION | \
         F.MMT4D_SKIP_INTERMEDIATE_ROUNDINGS
+    stream = _stream(None)
     if not (fuse_unpack and (M0, N0) != (32, 32)) and not (fuse_pack_lhs and K % K0):
         # (a small problem: all of it as one launch)
         status = load_library().iree_amd_uk_matmul_data_tiled(
             _ptr(a), _ptr(b), _ptr(c), None if fuse_pack_lhs else _ptr(ws["lhs"]), _ptr(ws["rhs"]),
             None if fuse_unpack else _ptr(ws["out"]), M, N, K, M0, N0, K0,
-            mm_flags | (F.MMT4D_ACCUMULATE if accumulate else 0), _stream(None))
+            mm_flags | (F.MMT4D_ACCUMULATE if accumulate else 0), stream)
         if status == 0:
             return ws
         if status != F.STATUS_NOT_FOUND:
             _check(status)
     if not fuse_pack_lhs:
-        pack(a, ws["lhs"], M, K, M1, K1, M0, K0, 0, in_type)
+        pack(a, ws["lhs"], M, K, M1, K1, M0, K0, 0, in_type, stream=stream)
     pack(b, ws["rhs"], K, N, N1, K1, N0, K0, 0,
-         in_type | F.PACK_TRANSPOSE_INNER | F.PACK_TRANSPOSE_OUTER)
+         in_type | F.PACK_TRANSPOSE_INNER | F.PACK_TRANSPOSE_OUTER, stream=stream)
     if fuse_pack_lhs:
         if (M0, N0) != (32, 32) or K % K0:
             raise ValueError("fuse_pack_lhs needs 32x32 tiles and K in whole tiles")
         if accumulate:
             mm_flags |= F.MMT4D_ACCUMULATE
-        matmul_packed_rhs(a, ws["rhs"], c, M, N, K, K0, mm_flags)
+        matmul_packed_rhs(a, ws["rhs"], c, M, N, K, K0, mm_flags, stream=stream)
         return ws
     if fuse_unpack:
         if (M0, N0) != (32, 32):
             raise ValueError("fuse_unpack needs 32x32 tiles")
         if accumulate:
             mm_flags |= F.MMT4D_ACCUMULATE
-        mmt4d_unpack(ws["lhs"], ws["rhs"], c, M, N, M1, N1, K1, K0, mm_flags)
+        mmt4d_unpack(ws["lhs"], ws["rhs"], c, M, N, M1, N1, K1, K0, mm_flags, stream=stream)
         return ws
     if accumulate:
-        pack(c, ws["out"], M, N, M1, N1, M0, N0, 0, out_type)
+        pack(c, ws["out"], M, N, M1, N1, M0, N0, 0, out_type, stream=stream)
         mm_flags |= F.MMT4D_ACCUMULATE
-    mmt4d(ws["lhs"], ws["rhs"], ws["out"], M1, N1, K1, M0, N0, K0, mm_flags)
-    unpack(ws["out"], c, M1, N1, M0, N0, M, N, out_type)
+    mmt4d(ws["lhs"], ws["rhs"], ws["out"], M1, N1, K1, M0, N0, K0, mm_flags, stream=stream)
+    unpack(ws["out"], c, M1, N1, M0, N0, M, N, out_type, stream=stream)
     return ws
 
 

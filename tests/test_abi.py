@@ -355,3 +355,37 @@ def test_validation_happens_before_any_device_work():
     assert lib.iree_amd_uk_mmt4d_noalloc_p(None, None) == 3
     assert lib.iree_amd_uk_release_scratch() == 0
     assert lib.iree_amd_uk_version() >= 1
+
+
+@pytest.mark.parametrize("form,calls", [
+    ({}, ["pack", "pack", "mmt4d", "unpack"]), ({"accumulate": True}, ["pack", "pack", "pack", "mmt4d", "unpack"]),
+    ({"fuse_unpack": True}, ["pack", "pack", "mmt4d_unpack"]), ({"fuse_pack_lhs": True}, ["pack", "matmul_packed_rhs"]),
+])
+def test_the_chain_looks_its_stream_up_once(monkeypatch, form, calls):
+    """The calls of matmul_data_tiled's chain, recorded by a stand-in for the
+    library that serves no one-launch form: all on the stream found at the start
+    (the lookup takes the host as long as a tenth of a call)."""
+    import types
+
+    import torch
+
+    from iree_amd import ukernel
+    seen, lookups = [], []
+
+    class Library:
+        def __getattr__(self, name):
+            def call(*args):
+                seen.append((name.replace("iree_amd_uk_", ""), args[-1]))
+                return F.STATUS_NOT_FOUND if name == "iree_amd_uk_matmul_data_tiled" else 0
+            return call
+    monkeypatch.setattr(ukernel, "load_library", Library)
+    monkeypatch.setattr(ukernel, "_ptr", lambda t: None if t is None else t.data_ptr())
+    monkeypatch.setattr(ukernel, "_raw_stream", lambda device: lookups.append(device) or 4711)
+    monkeypatch.setattr(torch.cuda, "current_device", lambda: 0)
+    a = torch.zeros(64 * 64)
+    ukernel.matmul_data_tiled(a, a, a.clone(), 64, 64, 64, F.MMT4D_TYPE_F32F32F32, tile=(32, 32, 4), **form)
+    assert seen == [(name, 4711) for name in ["matmul_data_tiled"] + calls]
+    assert len(lookups) == 1
+    # a stream object is taken as before
+    ukernel.scale_f32(a, 1, 1.0, stream=types.SimpleNamespace(cuda_stream=42))
+    assert seen[-1] == ("scale_f32", 42)
