@@ -500,8 +500,14 @@ int launch_cfg(SkinnyArgs a, int chunks, hipStream_t s) {
   // halves: N = 4096, K = 4096 f16 as 256 workgroups of 16 columns 8.4 us, as
   // 128 of 32 with K split over two rows and the launch that adds them 10.85;
   // K = 1024: 4.8 against 7.4).
-  // (a batch whose K is split as well: the planes share that many with their rows)
-  if (a.batch > 1 && chunks > 1) per_plane = (2 * cus + a.batch * chunks - 1) / (a.batch * chunks);
+  // (a batch whose K is split as well: its planes and their rows share one round
+  // of workgroups, two where their slices are short. Values of a decode step, f16:
+  // 32 heads x 4x64x16384, slices of 128 steps, 35.5 us in one round, 37.4 in two;
+  // 32 heads x 1x128x8192, 64 steps, 30.9 and 30.0)
+  if (a.batch > 1 && chunks > 1) {
+    const int want = a.chunk_steps >= 96 ? cus : 2 * cus;
+    per_plane = (want + a.batch * chunks - 1) / (a.batch * chunks);
+  }
   int blocks = a.N < per_plane ? a.N : per_plane;
   if (a.batch <= 1) blocks = a.N * 2 < per_plane ? a.N * 2 : per_plane;
   // K split over workgroup rows: the rows share the compute units, one round in
@@ -612,13 +618,31 @@ int reduce_chunks(const iree_amd_uk_mmt4d_params_t& p, const void* partials, int
 }
 }  // namespace
 
+namespace {
+// Workgroup rows that the K of ONE narrow problem is split over: as many as hold
+// it in registers, and up to 8 where the outer columns alone leave half of the
+// compute units or more idle (`may_spread`), of at least 32 steps.
+int64_t k_chunks(int64_t N, int64_t steps, int max_steps, int cus, bool may_spread) {
+  int64_t chunks = (steps + max_steps - 1) / max_steps;
+  // (column blocks of a launch row: see launch_cfg)
+  const int64_t col_blocks = N * 2 < cus ? N * 2 : cus;
+  if (may_spread && col_blocks * chunks * 2 <= cus && steps >= 64) {
+    int64_t more = cus / col_blocks;
+    if (more > steps / 32) more = steps / 32;
+    if (more > 8) more = 8;
+    if (more > chunks) chunks = more;
+  }
+  return chunks;
+}
+}  // namespace
+
 // `batch` problems of one narrow shape as the planes of one launch, at most
 // 65535 entries and batch strides of whole 16 bytes. A K that one launch row
-// cannot hold in registers is split over workgroup rows as for a single problem
-// (launch_mmt4d_skinny), into more of them where compute units would idle; the
-// partial sums of all entries are then added by one second launch. (The values
-// of a decode step of attention, 32 heads x 1x128x32768 f16, 268 MB: 340 us as
-// 32 single calls of two launches each, 57 as one.)
+// cannot hold in registers is split over workgroup rows exactly as for a single
+// problem (launch_mmt4d_skinny), whatever the batch: an entry has the bits of the
+// single call. The partial sums of all entries are added by one second launch.
+// (The values of a decode step of attention, 32 heads x 1x128x32768 f16, 268 MB:
+// 340 us as 32 single calls of two launches each, 57 as one.)
 int launch_batch_mmt4d_skinny(const iree_amd_uk_mmt4d_params_t& p0, int64_t batch, int64_t lhs_batch_stride,
                               int64_t rhs_batch_stride, int64_t out_batch_stride, hipStream_t s) {
   if (!mmt4d_skinny_supported(p0.flags, p0.M0, p0.N0, p0.K0)) return IREE_AMD_UK_STATUS_NOT_FOUND;
@@ -636,23 +660,15 @@ int launch_batch_mmt4d_skinny(const iree_amd_uk_mmt4d_params_t& p0, int64_t batc
     return IREE_AMD_UK_STATUS_NOT_FOUND;
   const int64_t steps = (k_elems + mk - 1) / mk;   // (the last one may be partial)
   const int max_steps = max_steps_per_launch(mk);
-  const int cus = device_cu_count();
-  int64_t chunks = (steps + max_steps - 1) / max_steps;
-  const int64_t col_blocks = p.N < cus ? p.N : cus;
-  // (a K that fits stays whole even where compute units idle: the second launch
-  // costs more than it gives; 8 heads x 1x128x1216 f16 as part of a decode step
-  // 10.8 us whole, 14.4 as two slices)
-  if (chunks > 1 && col_blocks * batch * chunks * 2 <= cus) {
-    int64_t more = cus / (col_blocks * batch);
-    if (more > steps / 32) more = steps / 32;
-    if (more > 8) more = 8;
-    if (more > chunks) chunks = more;
-  }
   const int64_t elems = p.N * p.M0 * 32;
   const bool transposed = (p.flags & kTransposedOut) != 0;
   const bool dense_out = out_batch_stride == elems &&
                          (!transposed || p.N == 1 || p.out_stride0 == (int64_t)p.M0 * 32);
   const BatchStrides bs = {batch, lhs_batch_stride, rhs_batch_stride, out_batch_stride};
+  // (a K that fits stays whole even where compute units idle: the second launch
+  // costs more than it gives; 8 heads x 1x128x1216 f16 as part of a decode step
+  // 10.8 us whole, 14.4 as two slices)
+  int64_t chunks = steps > max_steps ? k_chunks(p.N, steps, max_steps, device_cu_count(), true) : 1;
   if (chunks > 1 && chunks <= 65535 && dense_out) {
     const int64_t chunk_steps = (steps + chunks - 1) / chunks;
     chunks = (steps + chunk_steps - 1) / chunk_steps;
@@ -691,19 +707,10 @@ int launch_mmt4d_skinny(const iree_amd_uk_mmt4d_params_t& p0, hipStream_t s) {
   // stream's scratch buffer, and a second kernel adds them in row order, after
   // the old result when accumulating. Deterministic; exact for integers, for
   // floats the same sum in another order.
-  const int cus = device_cu_count();
-  int64_t chunks = (steps + max_steps - 1) / max_steps;
   // (partial sums and result are dense arrays there: transposed tiles must
   // follow each other without gaps)
   const bool dense_out = !transposed || p.N == 1 || p.out_stride0 == (int64_t)p.M0 * 32;
-  // (column blocks of a launch row: see launch_cfg)
-  const int64_t col_blocks = p.N * 2 < cus ? p.N * 2 : cus;
-  if (dense_out && col_blocks * chunks * 2 <= cus && steps >= 64) {
-    int64_t more = cus / col_blocks;
-    if (more > steps / 32) more = steps / 32;
-    if (more > 8) more = 8;
-    if (more > chunks) chunks = more;
-  }
+  int64_t chunks = k_chunks(p.N, steps, max_steps, device_cu_count(), dense_out);
   if (chunks > 1 && dense_out) {
     const int64_t chunk_steps = (steps + chunks - 1) / chunks;
     chunks = (steps + chunk_steps - 1) / chunk_steps;

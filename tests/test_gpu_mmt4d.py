@@ -1055,6 +1055,36 @@ def test_batch_of_narrow_tiles_with_a_long_k(uk, cuda, type_flag, tile, batch, s
     assert np.array_equal(gpucase.run_batch_mmt4d(case), case.run_oracle())
 
 
+@pytest.mark.parametrize("type_flag,tile,batch,shape", [
+    (F.MMT4D_TYPE_F16F16F32, (1, 32, 8), 32, (1, 3, 1400)),      # 700 steps of K: 8 slices for one entry
+    (F.MMT4D_TYPE_F16F16F32, (1, 32, 8), 2, (1, 40, 600)),
+    (F.MMT4D_TYPE_BF16BF16BF16, (8, 32, 8), 5, (1, 4, 1201)),
+    (F.MMT4D_TYPE_F8E4M3F8E4M3F32, (2, 32, 16), 9, (1, 2, 4 * 130)),
+    (F.MMT4D_TYPE_F16F16F32, (32, 4, 8), 7, (2, 1, 600)),
+    (F.MMT4D_TYPE_F32F32F32, (1, 32, 4), 6, (1, 5, 1101)),
+])
+@pytest.mark.parametrize("acc", [False, True])
+def test_batch_of_narrow_tiles_with_a_long_k_has_the_bits_of_single_calls(uk, cuda, type_flag, tile, batch, shape, acc):
+    """Data whose sums round: K is cut as for one entry, whatever the batch."""
+    import torch
+    g = torch.Generator(device="cuda").manual_seed(batch + shape[2])
+    (M, N, K), (M0, N0, K0) = shape, tile
+    flags = type_flag | F.MMT4D_SKIP_INTERMEDIATE_ROUNDINGS | (F.MMT4D_ACCUMULATE if acc else 0)
+    dt, out_dt = {F.MMT4D_TYPE_F16F16F32: (torch.float16, torch.float32), F.MMT4D_TYPE_F32F32F32: (torch.float32,) * 2,
+                  F.MMT4D_TYPE_BF16BF16BF16: (torch.bfloat16,) * 2,
+                  F.MMT4D_TYPE_F8E4M3F8E4M3F32: (torch.float8_e4m3fn, torch.float32)}[type_flag]
+    lhs, rhs, old = (torch.randn(batch, n, generator=g, device="cuda")
+                     for n in (M * K * M0 * K0, N * K * N0 * K0, M * N * M0 * N0))
+    lhs, rhs, old = lhs.to(dt), rhs.to(dt), old.to(out_dt)
+    got, want = old.clone(), old.clone()
+    uk.batch_mmt4d(lhs, rhs, got, batch, M, N, K, M0, N0, K0, flags)
+    assert uk.last_kernel_path() == "mmt4d:mfma-narrow"
+    for b in range(batch):
+        uk.mmt4d(lhs[b], rhs[b], want[b], M, N, K, M0, N0, K0, flags)
+    assert want.float().abs().max() > 1
+    assert torch.equal(got.view(torch.uint8), want.view(torch.uint8))
+
+
 def test_batch_mmt4d_degenerate_and_large_batch(uk, cuda):
     rng = np.random.default_rng(8200)
     # batch == 0: nothing is touched
