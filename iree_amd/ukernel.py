@@ -394,6 +394,18 @@ _OUT_PACK_TYPE = {
 }
 
 
+# K of one matrix-core step of a row-major left-hand side (in elements)
+_ROW_MAJOR_STEP = {
+    F.MMT4D_TYPE_F32F32F32: 8,
+    F.MMT4D_TYPE_S8S8S32: 32,
+    F.MMT4D_TYPE_F16F16F32: 32,
+    F.MMT4D_TYPE_F16F16F16: 32,
+    F.MMT4D_TYPE_BF16BF16F32: 32,
+    F.MMT4D_TYPE_BF16BF16BF16: 32,
+    F.MMT4D_TYPE_F8E4M3F8E4M3F32: 64,
+}
+
+
 def _ceil_div(a, b):
     return -(-a // b)
 
@@ -435,8 +447,10 @@ def matmul_data_tiled(a, b, c, M, N, K, mmt4d_type, *, accumulate=False,
     mm_flags = mmt4d_type | F.MMT4D_ALLOW_GENERIC_FALLBACK_TILE_FUNCTION | \
         F.MMT4D_SKIP_INTERMEDIATE_ROUNDINGS
     stream = _stream(None)
-    if not (fuse_unpack and (M0, N0) != (32, 32)) and not (fuse_pack_lhs and K % K0):
-        # (a small problem: all of it as one launch)
+    if not (fuse_unpack and (M0, N0) != (32, 32)) and \
+            not (fuse_pack_lhs and (K % _ROW_MAJOR_STEP[mmt4d_type] or _ptr(a) % 16)):
+        # (a small problem: all of it as one launch; what the chain's matmul on a
+        # row-major left-hand side may refuse is left to it, whatever the size)
         status = load_library().iree_amd_uk_matmul_data_tiled(
             _ptr(a), _ptr(b), _ptr(c), None if fuse_pack_lhs else _ptr(ws["lhs"]), _ptr(ws["rhs"]),
             None if fuse_unpack else _ptr(ws["out"]), M, N, K, M0, N0, K0,

@@ -1381,6 +1381,27 @@ def test_k_split_in_a_graph(uk, cuda, type_flag, K0, dt, out_dt, M0):
         warm.synchronize()
 
 
+@pytest.mark.parametrize("type_flag,dt,out_dt,K", [
+    (F.MMT4D_TYPE_F16F16F32, "float16", "float32", 40), (F.MMT4D_TYPE_BF16BF16BF16, "bfloat16", "bfloat16", 72),
+    (F.MMT4D_TYPE_S8S8S32, "int8", "int32", 80), (F.MMT4D_TYPE_F32F32F32, "float32", "float32", 36),
+])
+def test_small_matmul_on_a_row_major_lhs_has_the_conditions_of_a_large_one(uk, cuda, type_flag, dt, out_dt, K):
+    """K that is not whole matrix-core steps, and rows that are not 16-byte
+    aligned: refused whatever the size."""
+    import torch
+    dt, out_dt = getattr(torch, dt), getattr(torch, out_dt)
+    for M in (64, 2560):
+        c = torch.zeros(M, M, dtype=out_dt, device="cuda")
+        with pytest.raises(uk.UkError):
+            uk.matmul_data_tiled(torch.ones(M, K, device="cuda").to(dt), torch.ones(K, M, device="cuda").to(dt), c,
+                                 M, M, K, type_flag, fuse_pack_lhs=True)
+        a = torch.ones(M * 64 + 1, device="cuda").to(dt)[1:]
+        with pytest.raises(uk.UkError):
+            uk.matmul_data_tiled(a, torch.ones(64, M, device="cuda").to(dt), c, M, M, 64, type_flag, fuse_pack_lhs=True)
+        uk.matmul_data_tiled(a.clone(), torch.ones(64, M, device="cuda").to(dt), c, M, M, 64, type_flag, fuse_pack_lhs=True)
+        assert bool((c == 64).all())
+
+
 def test_small_matmul_leaves_shared_memory_to_the_chain(uk, cuda):
     """A result that overlaps an operand, and operands whose rows are shorter
     than a load: not served by the one launch, and the chain's results."""
