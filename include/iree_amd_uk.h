@@ -732,13 +732,15 @@ IREE_AMD_UK_EXPORT int iree_amd_uk_stream_synchronize(void* stream);
 IREE_AMD_UK_EXPORT int iree_amd_uk_release_scratch(void);
 /* Human-readable text of the calling thread's last non-OK status ("" if none). */
 IREE_AMD_UK_EXPORT const char* iree_amd_uk_last_error(void);
-/* Name of the kernel family that served the calling thread's last mmt4d or
- * dequant_matmul_i4 call: "mmt4d:mfma", "mmt4d:mfma-narrow",
- * "mmt4d:mfma-one-launch" (iree_amd_uk_matmul_data_tiled), "mmt4d:mfma-widened-s4", "mmt4d:mfma-s16-planes", "mmt4d:element-wise",
- * "dequant_i4:mfma", "dequant_i4:gemv", "dequant_i4:reassociated",
- * "dequant_i4:element-wise" ("" before the first call). A static string. No
- * counterpart in the reference, whose tile-function choice is visible through
- * iree_uk_mmt4d_info only. */
+/* Name of the kernel family that served the calling thread's last mmt4d (its
+ * batch and fused forms included, the SiLU one aside) or dequant_matmul_i4 call:
+ * "mmt4d:mfma", "mmt4d:mfma-narrow", "mmt4d:mfma-one-launch"
+ * (iree_amd_uk_matmul_data_tiled), "mmt4d:mfma-widened-s4",
+ * "mmt4d:mfma-s16-planes", "mmt4d:element-wise", "dequant_i4:mfma",
+ * "dequant_i4:gemv", "dequant_i4:gemm", "dequant_i4:reassociated",
+ * "dequant_i4:reassociated-element-wise", "dequant_i4:element-wise" ("" before
+ * the first call). A static string. No counterpart in the reference, whose
+ * tile-function choice is visible through iree_uk_mmt4d_info only. */
 IREE_AMD_UK_EXPORT const char* iree_amd_uk_last_kernel_path(void);
 /* Library version: (major << 16) | minor. */
 IREE_AMD_UK_EXPORT uint32_t iree_amd_uk_version(void);

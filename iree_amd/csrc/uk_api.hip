@@ -292,11 +292,11 @@ extern "C" int iree_amd_uk_batch_mmt4d(const iree_amd_uk_mmt4d_params_t* params,
     // (narrow left-hand sides: the entries of a decode step)
     const int st = launch_batch_mmt4d_skinny(p, batch, lhs_batch_stride, rhs_batch_stride,
                                              out_batch_stride, (hipStream_t)stream);
-    if (st != IREE_AMD_UK_STATUS_NOT_FOUND) return st;
+    if (st != IREE_AMD_UK_STATUS_NOT_FOUND) { note_kernel_path("mmt4d:mfma-narrow"); return st; }
   } else if (p.lhs_buffer && p.rhs_buffer && p.out_buffer && mmt4d_mfma_supported(p.flags, p.M0, p.N0, p.K0)) {
     const int st = launch_batch_mmt4d_mfma(p, batch, lhs_batch_stride, rhs_batch_stride,
                                            out_batch_stride, (hipStream_t)stream);
-    if (st != IREE_AMD_UK_STATUS_NOT_FOUND) return st;
+    if (st != IREE_AMD_UK_STATUS_NOT_FOUND) { note_kernel_path("mmt4d:mfma"); return st; }
   }
   // Otherwise entry by entry, the way the reference lowers the op (batch tiled
   // to 1, then rank-reduced to mmt4d: CPUPrepareUkernels.cpp:23-43,165-245).
@@ -718,6 +718,7 @@ int mmt4d_unpack_impl(
     return fail(IREE_AMD_UK_STATUS_UNIMPLEMENTED,
                 "mmt4d_unpack: needs a type and K0 with a matrix-core kernel, K > 0 and "
                 "16-byte aligned operands");
+  note_kernel_path("mmt4d:mfma");
   return st;
 }
 }  // namespace
@@ -805,6 +806,7 @@ int matmul_packed_rhs_impl(
   // rows of its one narrow tile, reading them and writing the result row-major.
   if (st == IREE_AMD_UK_STATUS_NOT_FOUND && M > 1 && M <= 32 && b.batch == 1 && out_scale == 1.0f)
     st = launch_matmul_rows_skinny(p, M, N, (hipStream_t)stream);
+  const bool narrow = st != IREE_AMD_UK_STATUS_NOT_FOUND;
   if (st == IREE_AMD_UK_STATUS_NOT_FOUND && mmt4d_mfma_supported(flags, 32, 32, K0))
     st = launch_matmul_packed_rhs_mfma(p, M, N, out_scale, b.batch, b.lhs, b.rhs, b.out, (hipStream_t)stream);
   if (st == IREE_AMD_UK_STATUS_NOT_FOUND && b.batch > 1) {
@@ -820,6 +822,7 @@ int matmul_packed_rhs_impl(
     return fail(IREE_AMD_UK_STATUS_UNIMPLEMENTED,
                 "matmul_packed_rhs: needs a type and K0 with a matrix-core kernel, K > 0 in whole "
                 "matrix-core steps and 16-byte aligned rows and tiles");
+  note_kernel_path(narrow ? "mmt4d:mfma-narrow" : "mmt4d:mfma");
   return st;
 }
 }  // namespace

@@ -1085,6 +1085,27 @@ def test_batch_of_narrow_tiles_with_a_long_k_has_the_bits_of_single_calls(uk, cu
     assert torch.equal(got.view(torch.uint8), want.view(torch.uint8))
 
 
+def test_kernel_path_of_the_batch_and_fused_forms(uk, cuda):
+    """Each after a call that another kernel family serves."""
+    import torch
+    K1, t = 8, F.MMT4D_TYPE_F16F16F32
+    a = torch.ones(2 * 64 * K1 * 8, dtype=torch.float16, device="cuda")
+    out = torch.zeros(2 * 64 * 64, device="cuda")
+
+    def path(call):
+        uk.mmt4d(a, a, out, 1, 1, 1, 3, 5, 2, t | F.MMT4D_ALLOW_GENERIC_FALLBACK_TILE_FUNCTION)
+        assert uk.last_kernel_path() == "mmt4d:element-wise"
+        call()
+        return uk.last_kernel_path()
+    assert path(lambda: uk.batch_mmt4d(a, a, out, 2, 2, 2, K1, 32, 32, 8, t)) == "mmt4d:mfma"
+    assert path(lambda: uk.batch_mmt4d(a, a, out, 2, 1, 2, K1, 4, 32, 8, t)) == "mmt4d:mfma-narrow"
+    assert path(lambda: uk.mmt4d_unpack(a, a, out, 50, 60, 2, 2, K1, 8, t)) == "mmt4d:mfma"
+    assert path(lambda: uk.batch_mmt4d_unpack(a, a, out, 2, 50, 60, 2, 2, K1, 8, t)) == "mmt4d:mfma"
+    assert path(lambda: uk.matmul_packed_rhs(a, a, out, 50, 60, 64, 8, t)) == "mmt4d:mfma"
+    assert path(lambda: uk.matmul_packed_rhs(a, a, out, 1, 64, 64, 8, t)) == "mmt4d:mfma-narrow"
+    assert path(lambda: uk.batch_matmul_packed_rhs(a, a, out, 2, 1, 64, 64, 8, t)) == "mmt4d:mfma-narrow"
+
+
 def test_batch_mmt4d_degenerate_and_large_batch(uk, cuda):
     rng = np.random.default_rng(8200)
     # batch == 0: nothing is touched
