@@ -600,20 +600,28 @@ def extras(args, torch, iree_amd, F, synth, lhs, rhs, out, ex):
     del c_two
     del a, b, c, ws
 
-    # the small i8 configuration, 1024^3 on row-major operands (2 packs, mmt4d,
-    # unpack = 4 launches): a latency figure, far too small for a roofline claim
+    # the small i8 configuration, 1024^3 on row-major operands, as the chain (2
+    # packs, mmt4d, unpack = 4 launches) and as the one launch that a call takes
+    # by itself: latency figures, far too small for a roofline claim
     n1k = 1024
     a8 = torch.from_numpy(synth.uniform_int8(1, n1k * n1k)).cuda()
     b8 = torch.from_numpy(synth.uniform_int8(2, n1k * n1k)).cuda()
     c8 = torch.zeros(n1k * n1k, dtype=torch.int32, device="cuda")
-    ws8 = iree_amd.matmul_data_tiled(a8, b8, c8, n1k, n1k, n1k, F.MMT4D_TYPE_S8S8S32)
-    _, t = gpu_time(torch, lambda: iree_amd.matmul_data_tiled(a8, b8, c8, n1k, n1k, n1k,
-                                                              F.MMT4D_TYPE_S8S8S32, workspace=ws8),
-                    steps, warm)
+    ws8 = iree_amd.matmul_data_tiled(a8, b8, c8, n1k, n1k, n1k, F.MMT4D_TYPE_S8S8S32, one_launch=False)
+    _, t = gpu_time(torch, lambda: iree_amd.matmul_data_tiled(a8, b8, c8, n1k, n1k, n1k, F.MMT4D_TYPE_S8S8S32,
+                                                              workspace=ws8, one_launch=False), steps, warm)
     ex["matmul_i8_1024_chain_us"] = round(t * 1e6, 1)
-    # the same product as one launch: right-hand side packed ahead of time,
-    # left-hand side read row-major, row-major result
+    assert iree_amd.last_kernel_path() == "mmt4d:mfma", iree_amd.last_kernel_path()
     c8_chain = c8.clone()
+    c8.fill_(0)
+    _, t = gpu_time(torch, lambda: iree_amd.matmul_data_tiled(a8, b8, c8, n1k, n1k, n1k, F.MMT4D_TYPE_S8S8S32,
+                                                              workspace=ws8), steps, warm)
+    ex["matmul_i8_1024_one_launch_us"] = round(t * 1e6, 1)
+    assert iree_amd.last_kernel_path() == "mmt4d:mfma-one-launch", iree_amd.last_kernel_path()
+    assert torch.equal(c8, c8_chain), "the one launch of an i8 matmul differs from the chain"
+    # the same product with the right-hand side packed ahead of time, left-hand
+    # side read row-major, row-major result
+    c8.fill_(0)
     _, t = gpu_time(torch, lambda: iree_amd.matmul_packed_rhs(a8, ws8["rhs"], c8, n1k, n1k, n1k, 16,
                                                               F.MMT4D_TYPE_S8S8S32), steps, warm)
     ex["matmul_i8_1024_one_kernel_us"] = round(t * 1e6, 1)
@@ -976,9 +984,9 @@ def run_only(args, torch, iree_amd, F, synth, mm_step):
         a8 = torch.from_numpy(synth.uniform_int8(1, n1k * n1k)).cuda()
         b8 = torch.from_numpy(synth.uniform_int8(2, n1k * n1k)).cuda()
         c8 = torch.zeros(n1k * n1k, dtype=torch.int32, device="cuda")
-        ws8 = iree_amd.matmul_data_tiled(a8, b8, c8, n1k, n1k, n1k, F.MMT4D_TYPE_S8S8S32)
+        ws8 = iree_amd.matmul_data_tiled(a8, b8, c8, n1k, n1k, n1k, F.MMT4D_TYPE_S8S8S32, one_launch=False)
         fn = lambda: iree_amd.matmul_data_tiled(a8, b8, c8, n1k, n1k, n1k, F.MMT4D_TYPE_S8S8S32,  # noqa: E731
-                                                workspace=ws8)
+                                                workspace=ws8, one_launch=False)
     elif args.only == "pack_transpose":
         # the right-hand side of the 4096^3 f16 matmul given as B[K][N]: 32x8 tiles, inner and outer
         # transposed; 8 rotating buffer sets (512 MiB) so that the 256 MiB last-level cache serves nothing

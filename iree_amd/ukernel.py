@@ -411,8 +411,11 @@ def _ceil_div(a, b):
 
 
 def matmul_data_tiled(a, b, c, M, N, K, mmt4d_type, *, accumulate=False,
-                      tile=None, workspace=None, fuse_unpack=False, fuse_pack_lhs=False):
-    """Row-major C[M][N] (+)= A[M][K] * B[K][N] through pack -> mmt4d -> unpack.
+                      tile=None, workspace=None, fuse_unpack=False, fuse_pack_lhs=False,
+                      one_launch=True):
+    """Row-major C[M][N] (+)= A[M][K] * B[K][N] through pack -> mmt4d -> unpack,
+    or for a small problem as one launch that leaves the same in every buffer
+    (float sums in another order); ``one_launch=False`` always runs the chain.
     With ``fuse_unpack`` the last two (and the pack of C when accumulating) are
     the one kernel ``mmt4d_unpack``; it needs a tile with a matrix-core kernel.
     With ``fuse_pack_lhs`` the matmul also reads A row-major itself
@@ -447,7 +450,7 @@ def matmul_data_tiled(a, b, c, M, N, K, mmt4d_type, *, accumulate=False,
     mm_flags = mmt4d_type | F.MMT4D_ALLOW_GENERIC_FALLBACK_TILE_FUNCTION | \
         F.MMT4D_SKIP_INTERMEDIATE_ROUNDINGS
     stream = _stream(None)
-    if not (fuse_unpack and (M0, N0) != (32, 32)) and \
+    if one_launch and not (fuse_unpack and (M0, N0) != (32, 32)) and \
             not (fuse_pack_lhs and (K % _ROW_MAJOR_STEP[mmt4d_type] or _ptr(a) % 16)):
         # (a small problem: all of it as one launch; what the chain's matmul on a
         # row-major left-hand side may refuse is left to it, whatever the size)

@@ -34,13 +34,16 @@ def _to_dev(x, elem):
     return torch.from_numpy(x.copy()).cuda()
 
 
+@pytest.mark.parametrize("one_launch", [False, True])
 @pytest.mark.parametrize("shapes_id", ["small", "large"])
 @pytest.mark.parametrize("name", sorted(E.TYPES))
-def test_e2e_matmul_suite(uk, cuda, name, shapes_id):
+def test_e2e_matmul_suite(uk, cuda, name, shapes_id, one_launch):
+    """The chain itself, and what a call takes by default: one launch for all of
+    the suite's sizes but the rows shorter than one of its loads."""
     import torch
     type_flag, in_elem, out_elem = E.TYPES[name]
     o = ukref.oracle()
-    element_wise = []
+    other_paths = []
     for (m, k, n, accumulate, dynamic, ls, rs, accs) in E.cases(E.SMALL if shapes_id == "small" else E.LARGE):
         lhs, rhs, acc = E.operands(m, k, n, ls, rs, accs, in_elem, out_elem)
         want = np.zeros(m * n, E.NP_DTYPE[out_elem])
@@ -64,20 +67,24 @@ def test_e2e_matmul_suite(uk, cuda, name, shapes_id):
         else:
             assert N0 == 32 and M0 == max(1, 1 << (m - 1).bit_length())
         uk.matmul_data_tiled(_to_dev(lhs, in_elem), _to_dev(rhs, in_elem), c, m, n, k, type_flag,
-                             accumulate=accumulate, tile=tile)
+                             accumulate=accumulate, tile=tile, one_launch=one_launch)
         torch.cuda.synchronize()
         got = c.cpu().numpy().view(E.NP_DTYPE[out_elem])
         assert np.array_equal(got.view(np.uint8), want.view(np.uint8)), \
             (name, (m, k, n), accumulate, "dynamic" if dynamic else "static", (M0, N0, K0))
-        if not uk.last_kernel_path().startswith("mmt4d:mfma"):
-            element_wise.append(((m, k, n), dynamic, (M0, N0, K0), uk.last_kernel_path()))
+        path = "mmt4d:mfma" if (M0, N0) == (32, 32) else "mmt4d:mfma-narrow"
+        if one_launch and n >= 4 and k * np.dtype(E.NP_DTYPE[in_elem]).itemsize >= 16:
+            path = "mmt4d:mfma-one-launch"
+        if uk.last_kernel_path() != path:
+            other_paths.append(((m, k, n), dynamic, (M0, N0, K0), uk.last_kernel_path()))
     # Every case of the suite runs on the matrix cores (a K that is not whole
     # instruction steps ends in a partial step, narrow tiles have their kernel).
-    assert not element_wise, element_wise
+    assert not other_paths, other_paths
 
 
+@pytest.mark.parametrize("one_launch", [False, True])
 @pytest.mark.parametrize("name", sorted(E.TYPES))
-def test_e2e_matmul_suite_with_the_unpack_fused(uk, cuda, name):
+def test_e2e_matmul_suite_with_the_unpack_fused(uk, cuda, name, one_launch):
     """The dynamic-size cases once more with the unpack (and the pack of the
     accumulator) folded into the matmul: the same bits."""
     import torch
@@ -90,7 +97,7 @@ def test_e2e_matmul_suite_with_the_unpack_fused(uk, cuda, name):
         c = _to_dev(acc, out_elem) if acc is not None else \
             torch.full((m * n,), 77, dtype=getattr(torch, TORCH_DTYPE[out_elem]), device="cuda")
         uk.matmul_data_tiled(_to_dev(lhs, in_elem), _to_dev(rhs, in_elem), c, m, n, k, type_flag,
-                             accumulate=accumulate, tile="dynamic", fuse_unpack=True)
+                             accumulate=accumulate, tile="dynamic", fuse_unpack=True, one_launch=one_launch)
         torch.cuda.synchronize()
         got = c.cpu().numpy().view(E.NP_DTYPE[out_elem])
         assert np.array_equal(got.view(np.uint8), want.view(np.uint8)), (name, (m, k, n), accumulate)

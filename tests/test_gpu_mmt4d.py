@@ -372,8 +372,9 @@ def _pack_chain_oracle_i8(A, B, M, N, K):
     return want
 
 
+@pytest.mark.parametrize("one_launch", [False, True])
 @pytest.mark.parametrize("M,N,K", [(1024, 1024, 1024), (123, 456, 789), (81, 19, 41), (1, 1000, 1000)])
-def test_i8_matmul_through_pack_mmt4d_unpack(uk, cuda, M, N, K):
+def test_i8_matmul_through_pack_mmt4d_unpack(uk, cuda, M, N, K, one_launch):
     """linalg.matmul i8 x i8 -> i32 through data tiling, bit-exact against a
     plain row-major integer matmul (shapes: the 1024^3 configuration and ragged
     shapes from the reference's e2e generator,
@@ -383,7 +384,10 @@ def test_i8_matmul_through_pack_mmt4d_unpack(uk, cuda, M, N, K):
     B = synth.uniform_int8(2, K * N)
     c = torch.zeros(M * N, dtype=torch.int32, device="cuda")
     uk.matmul_data_tiled(torch.from_numpy(A).cuda(), torch.from_numpy(B).cuda(), c,
-                         M, N, K, F.MMT4D_TYPE_S8S8S32)
+                         M, N, K, F.MMT4D_TYPE_S8S8S32, one_launch=one_launch)
+    # (one row: narrow tiles)
+    assert uk.last_kernel_path() == ("mmt4d:mfma-one-launch" if one_launch else
+                                     "mmt4d:mfma-narrow" if M == 1 else "mmt4d:mfma")
     torch.cuda.synchronize()
     got = c.cpu().numpy().reshape(M, N)
     want = _pack_chain_oracle_i8(A, B, M, N, K)
@@ -394,24 +398,27 @@ def test_i8_matmul_through_pack_mmt4d_unpack(uk, cuda, M, N, K):
         assert hashlib.sha256(got.tobytes()).hexdigest() == golden["matmul_i8_1024_sha256"]
 
 
-def test_i8_matmul_accumulates_into_seeded_c(uk, cuda):
+@pytest.mark.parametrize("one_launch", [False, True])
+def test_i8_matmul_accumulates_into_seeded_c(uk, cuda, one_launch):
     import torch
     M, N, K = 200, 100, 300
     A, B = synth.uniform_int8(1, M * K), synth.uniform_int8(2, K * N)
     c0 = (synth.splitmix64(3, M * N) >> np.uint64(44)).astype(np.int64).astype(np.int32)
     c = torch.from_numpy(c0.copy()).cuda()
     uk.matmul_data_tiled(torch.from_numpy(A).cuda(), torch.from_numpy(B).cuda(), c,
-                         M, N, K, F.MMT4D_TYPE_S8S8S32, accumulate=True)
+                         M, N, K, F.MMT4D_TYPE_S8S8S32, accumulate=True, one_launch=one_launch)
+    assert uk.last_kernel_path() == ("mmt4d:mfma-one-launch" if one_launch else "mmt4d:mfma")
     want = c0.reshape(M, N) + _pack_chain_oracle_i8(A, B, M, N, K)
     assert np.array_equal(c.cpu().numpy().reshape(M, N), want)
 
 
 @pytest.mark.parametrize("M,N,K", [(1024, 1024, 1024), (123, 456, 800), (40, 1000, 992)])
 @pytest.mark.parametrize("accumulate", [False, True])
-def test_i8_matmul_chain_with_the_fused_forms(uk, cuda, M, N, K, accumulate):
+@pytest.mark.parametrize("one_launch", [False, True])
+def test_i8_matmul_chain_with_the_fused_forms(uk, cuda, M, N, K, accumulate, one_launch):
     """The same chain with the unpack, and then also the pack of A, folded into
-    the matmul (pack of B + mmt4d_unpack, pack of B + matmul_packed_rhs): the
-    exact integer product both ways."""
+    the matmul (pack of B + mmt4d_unpack, pack of B + matmul_packed_rhs), and the
+    one launch that stands for them: the exact integer product each way."""
     import torch
     A, B = synth.uniform_int8(1, M * K), synth.uniform_int8(2, K * N)
     c0 = (synth.splitmix64(3, M * N) >> np.uint64(44)).astype(np.int64).astype(np.int32)
@@ -421,7 +428,10 @@ def test_i8_matmul_chain_with_the_fused_forms(uk, cuda, M, N, K, accumulate):
     for kw in ({"fuse_unpack": True}, {"fuse_pack_lhs": True}):
         c = torch.from_numpy(c0.copy()).cuda() if accumulate else torch.zeros(M * N, dtype=torch.int32, device="cuda")
         uk.matmul_data_tiled(torch.from_numpy(A).cuda(), torch.from_numpy(B).cuda(), c,
-                             M, N, K, F.MMT4D_TYPE_S8S8S32, accumulate=accumulate, **kw)
+                             M, N, K, F.MMT4D_TYPE_S8S8S32, accumulate=accumulate, one_launch=one_launch, **kw)
+        # (1024^3 with the pack of A folded in is two launches, estimated faster than one of them)
+        one = one_launch and (M, kw) != (1024, {"fuse_pack_lhs": True})
+        assert uk.last_kernel_path() == ("mmt4d:mfma-one-launch" if one else "mmt4d:mfma"), kw
         torch.cuda.synchronize()
         assert np.array_equal(c.cpu().numpy().reshape(M, N), want), kw
 
