@@ -742,6 +742,10 @@ IREE_AMD_UK_EXPORT const char* iree_amd_uk_last_error(void);
  * the first call). A static string. No counterpart in the reference, whose
  * tile-function choice is visible through iree_uk_mmt4d_info only. */
 IREE_AMD_UK_EXPORT const char* iree_amd_uk_last_kernel_path(void);
+/* Rows and columns of the macro tile of the calling thread's last "mmt4d:mfma"
+ * launch, and the number of slices of K (1: not split); zeros before the first.
+ * For tests and callers that tune, as the above. */
+IREE_AMD_UK_EXPORT void iree_amd_uk_last_macro_tile(int32_t* rows, int32_t* cols, int32_t* k_slices);
 /* Library version: (major << 16) | minor. */
 IREE_AMD_UK_EXPORT uint32_t iree_amd_uk_version(void);
 

@@ -21,6 +21,7 @@ from .ukernel import (  # noqa: F401
     choose_matmul_tile,
     enumerate_matmul_tiles,
     last_kernel_path,
+    last_macro_tile,
     batch_mmt4d,
     batch_mmt4d_unpack,
     mmt4d,

@@ -178,6 +178,8 @@ def _declare(lib):
     lib.iree_amd_uk_release_scratch.argtypes = []
     lib.iree_amd_uk_last_kernel_path.restype = C.c_char_p
     lib.iree_amd_uk_last_kernel_path.argtypes = []
+    lib.iree_amd_uk_last_macro_tile.restype = None
+    lib.iree_amd_uk_last_macro_tile.argtypes = [C.POINTER(C.c_int32)] * 3
     lib.iree_amd_uk_last_error.restype = C.c_char_p
     lib.iree_amd_uk_last_error.argtypes = []
     lib.iree_amd_uk_version.restype = u32

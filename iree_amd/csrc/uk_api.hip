@@ -21,6 +21,12 @@ int fail(int status, const char* fmt, ...) {
 
 static thread_local const char* g_kernel_path = "";
 void note_kernel_path(const char* name) { g_kernel_path = name; }
+static thread_local int32_t g_macro_tile[3] = {0, 0, 0};
+void note_macro_tile(int rows, int cols, int k_slices) {
+  g_macro_tile[0] = rows;
+  g_macro_tile[1] = cols;
+  g_macro_tile[2] = k_slices;
+}
 
 int check_hip(hipError_t err, const char* what) {
   if (err == hipSuccess) return 0;
@@ -943,4 +949,9 @@ extern "C" int iree_amd_uk_release_scratch(void) {
 }
 extern "C" const char* iree_amd_uk_last_error(void) { return g_last_error; }
 extern "C" const char* iree_amd_uk_last_kernel_path(void) { return g_kernel_path; }
+extern "C" void iree_amd_uk_last_macro_tile(int32_t* rows, int32_t* cols, int32_t* k_slices) {
+  if (rows) *rows = g_macro_tile[0];
+  if (cols) *cols = g_macro_tile[1];
+  if (k_slices) *k_slices = g_macro_tile[2];
+}
 extern "C" uint32_t iree_amd_uk_version(void) { return (0u << 16) | 1u; }

@@ -23,6 +23,8 @@ int fail(int status, const char* fmt, ...) __attribute__((format(printf, 2, 3)))
 // iree_amd_uk_last_kernel_path() (a static string; tests and callers that tune
 // use it to tell a matrix-core kernel from the element-wise one).
 void note_kernel_path(const char* name);
+// Likewise the macro tile of a matrix-core mmt4d launch, for iree_amd_uk_last_macro_tile().
+void note_macro_tile(int rows, int cols, int k_slices);
 
 // Converts a hipError_t of a runtime call or of a kernel launch to a status.
 int check_hip(hipError_t err, const char* what);

@@ -128,6 +128,7 @@ int launch_variant(const MfmaArgs& a0, hipStream_t s) {
   a.tiles_n = (a.N * kPerTile + TN - 1) / TN;
   const int64_t blocks = (int64_t)a.tiles_m * a.tiles_n;
   if (blocks > 0x7FFFFFFF) return IREE_AMD_UK_STATUS_NOT_FOUND;
+  note_macro_tile(TM * Cfg::kRows, TN * Cfg::kRows, a.k_slices > 1 ? a.k_slices : 1);
   // one kernel instance per operand form (the forms the entry points produce)
   constexpr bool kPackedLhs = !RowMajorLhsOnly<Cfg>::value;
   if constexpr (!kSiluMul) {

@@ -34,6 +34,13 @@ def last_kernel_path():
     return load_library().iree_amd_uk_last_kernel_path().decode()
 
 
+def last_macro_tile():
+    """(rows, columns, slices of K) of this thread's last "mmt4d:mfma" launch."""
+    out = [C.c_int32() for _ in range(3)]
+    load_library().iree_amd_uk_last_macro_tile(*map(C.byref, out))
+    return tuple(v.value for v in out)
+
+
 def _ptr(t):
     # (plain ints: the declared argtypes convert them, which is cheaper than
     # building a c_void_p per argument)

@@ -1228,29 +1228,75 @@ def test_batch_forms_of_the_fused_entry_points_match_single_calls(uk, cuda, type
                               lhs_batch_stride=2 * K1 * 32 * K0 + 3, rhs_batch_stride=0)
 
 
-@pytest.mark.parametrize("M,N", [(1981, 4101), (2164, 4101), (2347, 3713)])
+def _expect_macro_tile(uk, *want):
+    """The launcher's choice on 256 compute units."""
+    import torch
+    if torch.cuda.get_device_properties(0).multi_processor_count == 256:
+        assert uk.last_macro_tile() == want
+
+
+@pytest.mark.parametrize("M,N,tile", [(1981, 4101, (192, 192)), (2164, 4101, (256, 192)), (2347, 3713, (192, 256))])
 @pytest.mark.parametrize("type_flag,dt,out_dt", [
     (F.MMT4D_TYPE_F16F16F32, "float16", "float32"), (F.MMT4D_TYPE_BF16BF16BF16, "bfloat16", "bfloat16"),
     (F.MMT4D_TYPE_S8S8S32, "int8", "int32"),
 ])
-def test_medium_macro_tiles(uk, cuda, type_flag, dt, out_dt, M, N):
-    """Sizes for which, on 256 compute units, the launcher takes 192x192, 256x192
-    and 192x256 macro tiles, ragged on both sides: tiled result, row-major
-    result and row-major left-hand side. Small integers: every sum is exact (and
+def test_medium_macro_tiles(uk, cuda, type_flag, dt, out_dt, M, N, tile):
+    """Sizes for which the launcher takes 192x192, 256x192 and 192x256 macro
+    tiles, ragged on both sides: tiled result, row-major result and row-major
+    left-hand side, accumulating or not. Small integers: every sum is exact (and
     below 2^8, so that a bf16 result is as well)."""
     import torch
     g = torch.Generator(device="cuda").manual_seed(M + N)
+    c0 = torch.randint(-9, 10, (M, N), generator=g, device="cuda").to(getattr(torch, out_dt))
     for K, fused in ((192, ({}, {"fuse_unpack": True}, {"fuse_pack_lhs": True})), (216, ({}, {"fuse_unpack": True}))):
         a = torch.randint(-1, 2, (M, K), generator=g, device="cuda")
         b = torch.randint(-1, 2, (K, N), generator=g, device="cuda")
         want = a.double() @ b.double()
-        assert want.abs().max() < 256
+        assert want.abs().max() < 240
         ad, bd = a.to(getattr(torch, dt)).reshape(-1), b.to(getattr(torch, dt)).reshape(-1)
         for kw in fused:
-            c = torch.zeros(M * N, dtype=getattr(torch, out_dt), device="cuda")
-            uk.matmul_data_tiled(ad, bd, c, M, N, K, type_flag, tile="dynamic", **kw)
-            assert uk.last_kernel_path() == "mmt4d:mfma" or kw, uk.last_kernel_path()
-            assert torch.equal(c.double().view(M, N), want), (K, kw)
+            for accumulate in (False, True):
+                c = c0.clone()
+                uk.matmul_data_tiled(ad, bd, c, M, N, K, type_flag, tile="dynamic", accumulate=accumulate, **kw)
+                assert uk.last_kernel_path() == "mmt4d:mfma"
+                _expect_macro_tile(uk, *tile, 1)
+                assert torch.equal(c.double(), want + c0.double() if accumulate else want), (K, kw, accumulate)
+
+
+@pytest.mark.parametrize("form,M1,N1,steps,batch,tile", [
+    ("batch", 29, 17, 6, 9, (192, 192, 1)), ("batch", 25, 33, 6, 9, (256, 192, 1)), ("batch", 33, 25, 6, 9, (192, 256, 1)),
+    ("tiled", 29, 65, 128, 1, (192, 192, 4)), ("tiled", 55, 73, 160, 1, (256, 192, 2)),
+    ("tiled", 73, 55, 160, 1, (192, 256, 2)),
+    ("row_major", 41, 45, 128, 1, (192, 192, 4)), ("row_major", 73, 25, 256, 1, (256, 192, 5)),
+    ("row_major", 65, 31, 256, 1, (192, 256, 5)),
+])
+@pytest.mark.parametrize("accumulate", [False, True])
+def test_medium_macro_tiles_of_a_batch_and_with_k_split(uk, cuda, form, M1, N1, steps, batch, tile, accumulate):
+    """The same tiles with planes, and with K over workgroup rows, from packed and
+    from row-major left-hand sides (f16, exact sums)."""
+    import torch
+    g = torch.Generator(device="cuda").manual_seed(M1 + N1)
+    K, flags = steps * 32, F.MMT4D_TYPE_F16F16F32 | (F.MMT4D_ACCUMULATE if accumulate else 0)
+    M, N = (M1 * 32, N1 * 32) if form != "row_major" else (M1 * 32 - 5, N1 * 32 - 3)
+    a = torch.randint(-1, 2, (batch, M, K), generator=g, device="cuda").half()
+    b = torch.randint(-1, 2, (batch, N1 * 32, K), generator=g, device="cuda").half()
+    c0 = torch.randint(-9, 10, (batch, M, N), generator=g, device="cuda").float()
+    want = torch.stack([x.float() @ y[:N].float().t().contiguous() for x, y in zip(a, b)])   # (exact: below 2^24)
+    if accumulate:
+        want += c0
+
+    def tiles(x, t1):
+        return x.reshape(batch, -1, 32, x.shape[2] // t1, t1).transpose(2, 3).contiguous()
+    if form == "row_major":
+        c = c0.clone()
+        uk.matmul_packed_rhs(a, tiles(b, 8), c, M, N, K, 8, flags)
+    else:
+        c = tiles(c0, 32)
+        uk.batch_mmt4d(tiles(a, 8), tiles(b, 8), c, batch, M1, N1, K // 8, 32, 32, 8, flags)
+        c = c.transpose(2, 3).reshape(batch, M, N)
+    assert uk.last_kernel_path() == "mmt4d:mfma"
+    _expect_macro_tile(uk, *tile)
+    assert torch.equal(c, want)
 
 
 @pytest.mark.parametrize("M,N,K,tile", [
