@@ -232,8 +232,11 @@ int launch_dequant_matmul_i4(const void* x, const void* w, const void* scale, co
                        ((uintptr_t)scale % 16) == 0 && ((uintptr_t)zp % 16) == 0;
   // More than 64 rows (a prompt): the tiled kernel of uk_quant_gemm.hip, where
   // the kernels below stream the weights again for every 32 rows (N = 14336,
-  // K = 4096: 128 rows 47.3 -> 30.2 us, 512 181 -> 70; at 64 rows the two
-  // measure the same, at 48 20.7 against 23.3).
+  // K = 4096: 128 rows 46.2 -> 29.8 us, 512 183 -> 72). Both sides on 1900 problems
+  // of 33 to 128 rows, times of the kernels below over those of the tiled one: from
+  // 65 rows at least 1.08 with groups of 64 and more and 0.94 with groups of 32 (96
+  // x 7424 x 2048: 18.5 and 19.9 us); at 49 to 64 rows down to 0.85 where there are
+  // many columns (64 x 8192 x 2048: 11.9 and 13.4), up to 1.6 where there are few.
   if (M > 64 && tiled && a.zp_u4 && gs_ok && K % 128 == 0 && size_ok && aligned) {
     a.w_bytes = (uint32_t)w_bytes;
     const int st = launch_dequant_gemm_i4(a, s);
