@@ -21,7 +21,8 @@ typedef int intx4 __attribute__((ext_vector_type(4)));
 
 // kStepUs: measured time in microseconds of one K-step (the instruction's K
 // extent) of a 256x256 macro tile with all compute units busy on MI355X; the
-// launcher's estimates of absolute time start from it.
+// launcher's estimate for a K split starts from it. (The 16-row shapes, which are
+// launched by a fitted estimate of their own, have none.)
 struct F16Cfg {
   static constexpr float kStepUs = 0.40f;
   static constexpr int kRows = 32;     // the instruction's block is kRows x kRows
@@ -56,7 +57,6 @@ struct BF16Cfg {
 // the smaller block costs less energy per flop (with all-zero operands both
 // run at 2.3-2.4).
 struct F16Cfg16 {
-  static constexpr float kStepUs = 0.69f;
   static constexpr int kRows = 16;
   typedef half8 frag_t;
   typedef floatx4 acc_t;
@@ -69,7 +69,6 @@ struct F16Cfg16 {
   }
 };
 struct BF16Cfg16 {
-  static constexpr float kStepUs = 0.69f;
   static constexpr int kRows = 16;
   typedef bf16x8 frag_t;
   typedef floatx4 acc_t;
@@ -135,7 +134,6 @@ struct S8Cfg {
 // sustains 3.47 (both 4.92 on zeros): the smaller block costs less energy per
 // operation, as with f16.
 struct S8Cfg16 {
-  static constexpr float kStepUs = 0.65f;
   static constexpr int kRows = 16;
   typedef int4v frag_t;
   typedef intx4 acc_t;

@@ -395,10 +395,9 @@ int launch_estimated(const MfmaArgs& a, hipStream_t s) {
   return launch_by_index<Cfg, false>(best, a, s);
 }
 
-template <typename Cfg, bool kSiluMul = false>
-int launch_cfg(const MfmaArgs& a, hipStream_t s) {
-  if constexpr (kHasMediumTiles<Cfg, kSiluMul>) return launch_estimated<Cfg>(a, s);
-  // The 32-row shapes (f32, fp8, the SiLU forms, i8 with K in whole 32s only).
+// The 32-row shapes (f32, fp8, the SiLU forms, i8 with K in whole 32s only).
+template <typename Cfg, bool kSiluMul>
+int launch_costed(const MfmaArgs& a, hipStream_t s) {
   // Pick the macro tile. 256x256 (one workgroup per compute unit, all of its
   // registers) has the best operand reuse: 1 KiB of operand per two MFMAs.
   // 256x128 / 128x256 run two workgroups per compute unit, so one workgroup's
@@ -514,6 +513,12 @@ int launch_cfg(const MfmaArgs& a, hipStream_t s) {
     if (st != IREE_AMD_UK_STATUS_NOT_FOUND) return st;
   }
   return launch(best, a);
+}
+
+template <typename Cfg, bool kSiluMul = false>
+int launch_cfg(const MfmaArgs& a, hipStream_t s) {
+  if constexpr (kHasMediumTiles<Cfg, kSiluMul>) return launch_estimated<Cfg>(a, s);
+  else return launch_costed<Cfg, kSiluMul>(a, s);
 }
 
 }  // namespace

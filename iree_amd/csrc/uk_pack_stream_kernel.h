@@ -21,8 +21,8 @@ template <> struct Chunk<4> { typedef u32x4 aligned_t __attribute__((aligned(4))
 // registers: an array indexed at run time is promoted to LDS, and the kernel
 // then reads its workgroup size from the dispatch packet in HOST memory in
 // every edge wave, and loads the elements one after the other. (bf16, 2000 x
-// 3001 into 32x8 tiles 15.5 -> 6.8 us, the same back 16.0 -> 7.1; 2000 x 3008,
-// which has no such chunk, takes 6.9 and 5.9.)
+// 3001 into 32x8 tiles 16.5 -> 5.0 us, the same back 17.4 -> 5.7; 2000 x 3008,
+// which has no such chunk, takes 5.5 and 5.6.)
 
 // v shifted right (towards lower addresses) by 0 <= bytes < 16.
 __device__ __forceinline__ u32x4 shift_chunk_right(u32x4 v, uint32_t bytes) {
