@@ -272,6 +272,34 @@ inline double estimate_us(const MfmaArgs& a, int cus, int out_bytes, int v, int6
          (a.accumulate ? elems * out_bytes / 13.2 : 0.0);
 }
 
+// The same for a K too short for a split (below 1536), where starting a workgroup
+// and storing its result weigh as much as the steps, which that fit did not
+// cover: in the last round a step takes `alone` when it gives a compute unit one
+// workgroup at most and `shared` when it gives two to some, in the rounds before
+// `round`; `start`, `start_shared` and `start_round` are the rest of a workgroup's time.
+// Fitted to every tile on 5320 problems (200 to 4096 rows, 400 to 14336 columns, K
+// 64 to 1535; f16, bf16 and i8): on 5326 others what it picks is 0.8 % slower than
+// the best on average and 5 % in the 95th percentile, where the estimate above is
+// at 1.9 and 14.5 (f16 1710 x 10701 x 64 19.2 us on the best tile, 21.2 on its choice).
+struct ShortKTile { float alone, shared, round, start, start_shared, start_round; };
+constexpr ShortKTile kShortKTiles[kTilesWithMedium] = {
+    {0.614f, 0.0f, 0.726f, 4.31f, 0.0f, 5.84f},    {0.344f, 0.682f, 0.713f, 0.63f, 2.24f, 3.27f},
+    {0.338f, 0.666f, 0.712f, 0.52f, 2.17f, 3.25f}, {0.181f, 0.390f, 0.453f, 0.0f, 0.89f, 2.11f},
+    {0.471f, 0.0f, 0.560f, 2.98f, 0.0f, 4.82f},    {0.466f, 0.0f, 0.545f, 2.96f, 0.0f, 4.86f},
+    {0.376f, 0.0f, 0.460f, 1.84f, 0.0f, 3.97f}};
+inline double estimate_short_k_us(const MfmaArgs& a, int cus, int out_bytes, int v, int64_t M, int64_t N) {
+  const MediumTile& t = kMediumTiles[v];
+  const ShortKTile& c = kShortKTiles[v];
+  const int64_t batch = a.batch > 1 ? a.batch : 1, slots = (int64_t)t.occ * cus;
+  const int64_t tiles = ceil_div(M, (int64_t)2 * t.wm) * ceil_div(N, (int64_t)2 * t.wn) * batch;
+  const int64_t before = ceil_div(tiles, slots) - 1;
+  const bool shared = tiles - before * slots > cus;
+  const double steps = (double)a.ksteps * (a.lhs_row_major ? t.row_major : 1.0);
+  return 4.8 + before * (steps * c.round + c.start_round) +
+         (shared ? steps * c.shared + c.start_shared : steps * c.alone + c.start) +
+         (double)M * N * batch * 1024e-6 * out_bytes * 0.101;
+}
+
 // A last round that fills only part of the device costs a whole round. When
 // the large tile leaves such a round, the longer outer dimension is split:
 // whole rounds of 256x256 tiles first, the remaining rows or columns as a
@@ -338,7 +366,10 @@ template <typename Cfg>
 int launch_estimated(const MfmaArgs& a, hipStream_t s) {
   constexpr int kOutBytes = (int)sizeof(typename Cfg::out_t);
   const int cus = device_cu_count();
-  auto us_of = [&](int v, int64_t M, int64_t N) -> double { return estimate_us(a, cus, kOutBytes, v, M, N, 1); };
+  const bool short_k = (int64_t)a.ksteps * Cfg::kMfmaK < 1536;
+  auto us_of = [&](int v, int64_t M, int64_t N) -> double {
+    return short_k ? estimate_short_k_us(a, cus, kOutBytes, v, M, N) : estimate_us(a, cus, kOutBytes, v, M, N, 1);
+  };
   auto pick = [&](int64_t M, int64_t N, double* out_us) -> int {
     int best = 0;
     for (int v = 0; v < kTilesWithMedium; ++v) {
