@@ -20,7 +20,8 @@ namespace {
 // kAhead: slices whose loads are in flight together. 8 for a small result, which
 // is bounded by the latency of the loads (one after the other, 8 slices of 1x128
 // for 8 heads took 1.3 us longer); 1 for what fills the device, which they only
-// slow down (500 x 4096 in 8 slices, 67 MB: 1.1 us longer with 8).
+// slow down (500 x 4096 in 8 slices, 67 MB: 1.1 us longer with 8), and for fewer
+// than 4 slices (15 x 13312 int4 in 2: 0.1 us longer with 8).
 template <typename AccT, typename OutT, int kAhead>
 __global__ __launch_bounds__(256) void ksplit_reduce_kernel(KSplitReduceArgs r) {
   typedef AccT acc4_t __attribute__((ext_vector_type(4)));
@@ -182,7 +183,7 @@ int launch_ksplit_reduce(const KSplitReduceArgs& r, hipStream_t s) {
   const int64_t groups = r.flat_elems > 0 ? r.flat_elems / 4 : (int64_t)r.M * r.N * 256;
   const int64_t blocks = (groups + 255) / 256;
   if (blocks < 1 || blocks > 0x7FFFFFFF) return IREE_AMD_UK_STATUS_NOT_FOUND;
-  if (blocks <= 2 * (int64_t)device_cu_count()) launch_reduce<8>(r, dim3((unsigned)blocks), s);
+  if (r.slices >= 4 && blocks <= 2 * (int64_t)device_cu_count()) launch_reduce<8>(r, dim3((unsigned)blocks), s);
   else launch_reduce<1>(r, dim3((unsigned)blocks), s);
   return check_hip(hipGetLastError(), "ksplit_reduce launch");
 }
