@@ -620,7 +620,9 @@ IREE_AMD_UK_EXPORT int iree_amd_uk_batch_mmt4d_unpack(
  * otherwise; use the three-call sequence then): K a multiple of the
  * matrix-core K extent (32 for f16/bf16 and i8, 8 for f32, 64 for fp8),
  * K0 as served by iree_amd_uk_mmt4d, 16-byte aligned lhs rows and rhs tiles.
- * Bit-identical to pack + mmt4d + unpack. Up to 24 rows (32 of 1-byte elements: a decode step)
+ * Bit-identical to pack + mmt4d + unpack where neither or both split K alike
+ * (integers always; else float sums come in another order: the split is chosen
+ * for the row-major operand). Up to 24 rows (32 of 1-byte elements: a decode step)
  * with a K of up to 4096 elements of 2 bytes (8192 of 1 byte) run the kernel
  * for narrow left-hand side tiles on the rows themselves (float sums then
  * come in that kernel's order: the bits of mmt4d on M0 = M tiles). With N >= 16384 (and M >= 512) the
@@ -643,6 +645,9 @@ IREE_AMD_UK_EXPORT int iree_amd_uk_matmul_packed_rhs(
  * `flags` (an IREE_AMD_UK_FLAG_MMT4D_TYPE_*, optionally ACCUMULATE). lhs, rhs and
  * out receive the packed operands and the packed result in tiles of M0 x K0,
  * N0 x K0 and M0 x N0, as the chain leaves them; a null one is not written.
+ * Integers have the chain's bits, and so have the packed operands; float sums come
+ * in another order (a captured call's, whose K stays whole, in a third), with an
+ * error no larger.
  * Returns IREE_AMD_UK_STATUS_NOT_FOUND, with no error recorded and nothing
  * written, for what it does not serve (large problems, which the chain runs
  * faster; tiles without a matrix-core kernel; buffers that overlap): run the
