@@ -18,9 +18,11 @@
 // port. Two waves per SIMD then take 2700 cycles where the MFMAs alone are
 // 2048: vector issue bounds the kernel, and a wave tile twice as tall, which
 // would halve the dequantisation, does not fit the registers that vector
-// instructions can reach. Measured at 14336 columns, K = 4096, groups of 128:
-// 128 / 256 / 512 rows 30.2 / 42.6 / 69.8 us, 0.86 PFLOP/s at 512 (as passes of
-// 32 rows over all the weights 47.3 / 91.8 / 181).
+// instructions can reach. (Two waves per SIMD: a workgroup of 128 rows, or two of
+// 64, which fit a compute unit's LDS up to 128 columns, 64 with groups of 32.)
+// Measured at 14336 columns, K = 4096, groups of 128: 128 / 256 / 512 / 2048 rows
+// 29.5 / 42.2 / 70.7 / 286 us, 0.85 PFLOP/s at 512 (as passes of 32 rows over all
+// the weights 46.2 / 91.3 / 183 / 727).
 // K goes in spans of 128:
 //   * weights: a 16-column x 128-k slab is one 16-byte load per lane (the tiled
 //     layout's 1 KiB), straight to registers, one span ahead;
