@@ -218,14 +218,16 @@ IREE_AMD_UK_EXPORT int iree_amd_uk_mmt4d_noalloc_p(
  * Common/CPU/CPUPrepareUkernels.cpp:23-43 tileBatchDimsForBatchMmt4dOp,
  * :165-245 ConvertBatchMmt4DtoMmt4DPattern), so every entry has the result of
  * iree_amd_uk_mmt4d_p on it: exactly for integers; float sums may be added in
- * another order where the single call splits a K that the batch keeps whole.
+ * another order where the single call splits a K that the batch keeps whole (over
+ * workgroups, or over the waves of one: most problems of few tiles).
  * Matrix-core tiles (M0 = 32, and the narrow ones, M = 1 and M0 < 32) whose
  * batch strides are whole 16 bytes run as ONE launch (batch entries are planes
- * of the grid; it allocates nothing). Only a K that the narrow tiles cannot keep
+ * of the grid; it allocates nothing). A K that the narrow tiles cannot keep
  * in registers (more than 4096 elements of 2 bytes, 2048 of 4, 8192 of 1) is
- * split, for every entry as iree_amd_uk_mmt4d_p splits it and with its bits, and
- * takes a second launch and the stream's scratch buffer (see
- * iree_amd_uk_mmt4d). Everything else runs as iree_amd_uk_mmt4d_p entry by
+ * split, for every entry as iree_amd_uk_mmt4d_p splits it and with its bits: over
+ * the waves of a workgroup up to half as much again against at most 256 outer
+ * columns, else over workgroups, which takes a second launch and the stream's
+ * scratch buffer (see iree_amd_uk_mmt4d). Everything else runs as iree_amd_uk_mmt4d_p entry by
  * entry. Entries must not overlap in `out`.
  * batch == 0 does nothing. */
 IREE_AMD_UK_EXPORT int iree_amd_uk_batch_mmt4d(

@@ -7,6 +7,7 @@
 #include "uk_common.h"
 #include "uk_mmt4d_mfma_kernel.h"
 #include "uk_mmt4d_mfma_launch.h"
+#include "uk_mmt4d_wave_split.h"
 #include "uk_scratch_cache.h"
 
 #include <mutex>
@@ -267,6 +268,7 @@ int make_args(const iree_amd_uk_mmt4d_params_t& p, int out_elem_bytes, bool silu
   a.row_major_out = 0; a.out_rows = a.out_cols = 0;
   a.lhs_row_major = 0;
   a.gate_scale = a.up_scale = a.inv_out_scale = a.out_scale = 1.0f;
+  a.other_us = 0.0f;
   return 0;
 }
 }  // namespace
@@ -418,7 +420,57 @@ int launch_matmul_packed_rhs_mfma(const iree_amd_uk_mmt4d_params_t& p, int64_t o
 }
 
 namespace {
-int launch_typed(const iree_amd_uk_mmt4d_params_t& p, const MfmaArgs& a, hipStream_t s) {
+// The call as a problem for the kernel that splits K over the waves of a
+// workgroup. Not served: K0 other than 16 bytes, batches, and more than 64 outer
+// tiles with a K of less than 1 KB (which gain little; entries of a batch, and the
+// kernels exported for a HAL executable, which keep K whole, have the bits of the
+// single call there).
+bool as_few_tiles(const iree_amd_uk_mmt4d_params_t& p, const MfmaArgs& a, bool silu, WaveSplitArgs* out) {
+  Mmt4dTypeInfo ti;
+  mmt4d_type_info(p.flags, &ti);
+  if (a.k_slices != 0 || a.batch > 1 || p.K0 * ti.lhs_bits != 128) return false;
+  const int64_t lhs_outer = a.lhs_row_major ? 32 * a.lhs_stride_bytes : a.lhs_stride_bytes;
+  if (lhs_outer > 0x7FFFFFFF || (p.K < 64 && (int64_t)a.M * a.N > 64)) return false;
+  WaveSplitArgs w = {};
+  w.lhs = a.lhs; w.rhs = a.rhs; w.out = a.out;
+  w.lhs_outer = lhs_outer;
+  w.rhs_outer = a.rhs_stride_bytes;
+  w.lhs_row = a.lhs_row_major ? (int)a.lhs_stride_bytes : 16;
+  w.lhs_chunk = a.lhs_row_major ? 16 : 512;
+  w.rows = a.lhs_row_major ? a.out_rows : a.M * 32;
+  w.outer_cols = a.N;
+  w.k_chunks = (int)p.K;
+  const int64_t out_pitch = silu ? a.out_stride_bytes : a.out_stride_bytes / ti.out_bytes;
+  w.out_outer = a.row_major_out ? 32 * out_pitch : out_pitch;
+  w.out_row = a.row_major_out ? out_pitch : 32;
+  w.out_tile = a.row_major_out ? 32 : 1024;
+  w.out_col = 1;
+  w.out_rows = a.row_major_out ? a.out_rows : w.rows;
+  w.out_cols = a.row_major_out ? a.out_cols : a.N * 32;
+  w.accumulate = a.accumulate; w.silu = silu; w.batch = 1;
+  w.gate_scale = a.gate_scale; w.up_scale = a.up_scale; w.inv_out_scale = a.inv_out_scale; w.out_scale = a.out_scale;
+  *out = w;
+  return true;
+}
+
+// `launch` on the macro tiles, or the kernel for few tiles where that is faster.
+template <typename Launch>
+int launch_faster(const iree_amd_uk_mmt4d_params_t& p, const MfmaArgs& a, bool silu, hipStream_t s, Launch launch) {
+  MfmaArgs b = a;
+  WaveSplitArgs w;
+  WaveSplitChoice few = {-1, 0.0};
+  const uint32_t type = p.flags & IREE_AMD_UK_FLAG_MMT4D_TYPE_MASK;
+  if (as_few_tiles(p, a, silu, &w)) few = choose_wave_split(w, type);
+  // (up to four macro tiles and half a KB to 8 KB of K: it was, on all of 1220
+  // problems, and the estimates of the macro tiles take 0.2 us of a 3.5 us call)
+  if (few.tile >= 0 && p.K >= 32 && p.K <= 512 && ((a.M + 3) / 4) * (int64_t)((a.N + 3) / 4) <= 4)
+    return launch_mmt4d_wave_split(w, type, few.tile, s);
+  b.other_us = few.tile >= 0 ? (float)few.us : 0.0f;
+  const int st = launch(b);
+  return st == kSlowerThanOther ? launch_mmt4d_wave_split(w, type, few.tile, s) : st;
+}
+
+int launch_macro_tiles(const iree_amd_uk_mmt4d_params_t& p, const MfmaArgs& a, hipStream_t s) {
   switch (p.flags & IREE_AMD_UK_FLAG_MMT4D_TYPE_MASK) {
     case IREE_AMD_UK_FLAG_MMT4D_TYPE_F16F16F32: return launch_mfma_f16f16f32(a, s);
     case IREE_AMD_UK_FLAG_MMT4D_TYPE_BF16BF16F32: return launch_mfma_bf16bf16f32(a, s);
@@ -429,6 +481,10 @@ int launch_typed(const iree_amd_uk_mmt4d_params_t& p, const MfmaArgs& a, hipStre
     case IREE_AMD_UK_FLAG_MMT4D_TYPE_BF16BF16BF16: return launch_mfma_bf16bf16bf16(a, s);
     default: return IREE_AMD_UK_STATUS_NOT_FOUND;
   }
+}
+
+int launch_typed(const iree_amd_uk_mmt4d_params_t& p, const MfmaArgs& a, hipStream_t s) {
+  return launch_faster(p, a, false, s, [&](const MfmaArgs& b) { return launch_macro_tiles(p, b, s); });
 }
 }  // namespace
 
@@ -442,12 +498,14 @@ int launch_mmt4d_silu_mul_mfma(const iree_amd_uk_mmt4d_params_t& p, float gate_s
   if (st) return st;
   a.gate_scale = gate_scale; a.up_scale = up_scale; a.inv_out_scale = inv_out_scale;
   a.accumulate = 0;
-  switch (p.flags & IREE_AMD_UK_FLAG_MMT4D_TYPE_MASK) {
-    case IREE_AMD_UK_FLAG_MMT4D_TYPE_F16F16F32: return launch_mfma_silu_f16(a, s);
-    case IREE_AMD_UK_FLAG_MMT4D_TYPE_BF16BF16F32: return launch_mfma_silu_bf16(a, s);
-    case IREE_AMD_UK_FLAG_MMT4D_TYPE_F8E4M3F8E4M3F32: return launch_mfma_silu_f8(a, s);
-    default: return IREE_AMD_UK_STATUS_NOT_FOUND;
-  }
+  return launch_faster(p, a, true, s, [&](const MfmaArgs& b) {
+    switch (p.flags & IREE_AMD_UK_FLAG_MMT4D_TYPE_MASK) {
+      case IREE_AMD_UK_FLAG_MMT4D_TYPE_F16F16F32: return launch_mfma_silu_f16(b, s);
+      case IREE_AMD_UK_FLAG_MMT4D_TYPE_BF16BF16F32: return launch_mfma_silu_bf16(b, s);
+      case IREE_AMD_UK_FLAG_MMT4D_TYPE_F8E4M3F8E4M3F32: return launch_mfma_silu_f8(b, s);
+      default: return (int)IREE_AMD_UK_STATUS_NOT_FOUND;
+    }
+  });
 }
 
 }  // namespace uk

@@ -106,6 +106,9 @@ struct MfmaArgs {
   int stream_out;
   // macro-tile rows of one column panel of the workgroup order (see tile_coord)
   int panel_rows;
+  // launch side: estimated time in us of another kernel that could serve the
+  // call (0: there is none)
+  float other_us;
 };
 
 namespace {

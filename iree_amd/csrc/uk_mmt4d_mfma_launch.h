@@ -7,6 +7,8 @@
 #ifndef IREE_AMD_UK_MMT4D_MFMA_LAUNCH_H_
 #define IREE_AMD_UK_MMT4D_MFMA_LAUNCH_H_
 
+#include <cmath>
+
 #include "uk_common.h"
 #include "uk_mmt4d_mfma_kernel.h"
 
@@ -24,6 +26,10 @@ int launch_mfma_f8f8f32(const MfmaArgs& a, hipStream_t s);
 int launch_mfma_silu_f16(const MfmaArgs& a, hipStream_t s);
 int launch_mfma_silu_bf16(const MfmaArgs& a, hipStream_t s);
 int launch_mfma_silu_f8(const MfmaArgs& a, hipStream_t s);
+
+// What the launch functions return, having launched nothing, when the call is
+// estimated to take longer here than MfmaArgs::other_us.
+constexpr int kSlowerThanOther = -1;
 
 namespace {
 
@@ -300,6 +306,33 @@ inline double estimate_short_k_us(const MfmaArgs& a, int cus, int out_bytes, int
          (double)M * N * batch * 1024e-6 * out_bytes * 0.101;
 }
 
+// The estimates above rank tiles; against the times themselves (8000 problems of 1 to
+// 800 rows, where they decide against the kernel for few tiles) they are a fifth
+// too long below 8 us and an eighth too short above 20. This straightens them: 9 %
+// off on average.
+inline double straightened_us(double us) { return 0.604 * std::pow(us, 1.181); }
+
+// The 32-row shapes against that kernel: the time of `tiles` workgroups of wm x wn
+// (of the launcher's units, 2 x 2 = 128 x 128) with `steps` of 64 bytes of K each,
+// fitted to the same problems on the tile and slices they ran on (fp8 7 to 13 %
+// off on average, with the SiLU epilogue 7 %, f32 4 %).
+template <typename Cfg, bool kSiluMul>
+double costed_us(const MfmaArgs& a, int wm, int wn, int occ, int64_t tiles, double steps, int slices, int cus) {
+  constexpr bool kF32 = std::is_same<Cfg, F32Cfg>::value;
+  constexpr double kShared = kF32 ? 1.93 : 3.37;
+  const double area = wm * wn / 4.0;
+  const double step = kF32 ? 0.935 * area : 0.163 * area * (a.lhs_row_major ? 1.34 : 1.0);
+  const int64_t slots = (int64_t)occ * cus, before = ceil_div(tiles, slots) - 1;
+  const double out_mb = (double)a.M * a.N * 1024e-6 * (kSiluMul ? 1 : 4);
+  const double us = 3.11 + steps * step * (before * kShared + (tiles - before * slots > cus ? kShared : 1.0)) +
+                    3.96 * before + 0.245 * out_mb + (kSiluMul ? 0.27 * area : 0.0);
+  return slices > 1 ? us + 2.33 + 0.62 * out_mb * slices : us;
+}
+
+// The other kernel's estimate has to be 5 % below this one's (with no margin 75 of
+// 7333 problems got slower by more than 4 %, with it 32, by 16 % at most).
+inline bool other_wins(const MfmaArgs& a, double us) { return a.other_us > 0 && a.other_us < 0.95 * us; }
+
 // A last round that fills only part of the device costs a whole round. When
 // the large tile leaves such a round, the longer outer dimension is split:
 // whole rounds of 256x256 tiles first, the remaining rows or columns as a
@@ -380,6 +413,7 @@ int launch_estimated(const MfmaArgs& a, hipStream_t s) {
   };
   double best_us = 0;
   const int best = pick(a.M, a.N, &best_us);
+  bool split_wins = false;
   // K over workgroup rows: at most one round, slices of 768 elements and more
   // of K; it has to win by 3 %. iree_amd_uk_mmt4d_noalloc_p runs the same kernels
   // and refuses a split whose partial sums its array does not hold, so on
@@ -417,10 +451,13 @@ int launch_estimated(const MfmaArgs& a, hipStream_t s) {
     const int64_t whole_tiles = ceil_div((int64_t)a.M, (int64_t)2 * whole.wm) * ceil_div((int64_t)a.N, (int64_t)2 * whole.wn);
     const bool worth = a.ksteps >= 64 && whole_tiles * 2 <= (int64_t)whole.occ * cus;
     if (split.n > 1 && (worth || !scratch_under_capture(s))) {
+      if (other_wins(a, straightened_us(split.us))) return kSlowerThanOther;
+      split_wins = true;
       const int st = launch_k_split<Cfg>(a, split.v, split.n, s);
       if (st != IREE_AMD_UK_STATUS_NOT_FOUND) return st;
     }
   }
+  if (!split_wins && other_wins(a, straightened_us(best_us))) return kSlowerThanOther;
   const int st = launch_whole_rounds<Cfg, false>(a, cus, best_us, us_of, pick, s);
   if (st != IREE_AMD_UK_STATUS_NOT_FOUND) return st;
   return launch_by_index<Cfg, false>(best, a, s);
@@ -501,6 +538,14 @@ int launch_costed(const MfmaArgs& a, hipStream_t s) {
   auto launch = [&](int v, const MfmaArgs& b) -> int { return launch_by_index<Cfg, kSiluMul>(v, b, s); };
   double best_cost = 0;
   const int best = pick(a.M, a.N, &best_cost);
+  // K-steps of 64 bytes, for the comparison with the kernel for few tiles
+  const double steps = (double)a.ksteps * Cfg::kMfmaK * Cfg::kElemBytes / 64.0;
+  auto other_is_faster = [&](int v, int n) {
+    const Variant& t = variants[v];
+    const int64_t tiles = ceil_div((int64_t)a.M, (int64_t)2 * t.wm) * ceil_div((int64_t)a.N, (int64_t)2 * t.wn) * n;
+    return other_wins(a, costed_us<Cfg, kSiluMul>(a, t.wm, t.wn, t.occ, tiles, steps / n, n, cus));
+  };
+  bool split_wins = false;
   // Few macro tiles and a long K (a few hundred rows against a wide K, as in the
   // down projection of an MLP at small batch) leave most compute units idle:
   // K is then split over workgroup rows. Estimated times in microseconds: cost
@@ -533,11 +578,14 @@ int launch_costed(const MfmaArgs& a, hipStream_t s) {
         }
       }
       if (split_n > 1) {
+        if (other_is_faster(split_v, split_n)) return kSlowerThanOther;
+        split_wins = true;
         const int st = launch_k_split<Cfg>(a, split_v, split_n, s);
         if (st != IREE_AMD_UK_STATUS_NOT_FOUND) return st;
       }
     }
   }
+  if (!split_wins && other_is_faster(best, 1)) return kSlowerThanOther;
   {
     const int st = launch_whole_rounds<Cfg, kSiluMul>(
         a, cus, best_cost, [&](int v, int64_t M, int64_t N) { return cost_of(v, M, N); }, pick, s);

@@ -37,6 +37,7 @@
 
 #include <memory>
 #include "uk_mfma_cfg.h"
+#include "uk_mmt4d_wave_split.h"
 
 #include <type_traits>
 
@@ -636,6 +637,56 @@ int64_t k_chunks(int64_t N, int64_t steps, int max_steps, int cus, bool may_spre
 }
 }  // namespace
 
+namespace {
+// Whether `batch` narrow problems of N outer columns and `chunks` 16-byte pieces of
+// K go to the kernel that splits K over the waves of a workgroup by steps, and N
+// over workgroups by 16 columns (uk_mmt4d_wave_split.hip).
+// K that stays in registers here (up to 8 KB), longer than half a KB: up to two
+// workgroups of 16 columns per compute unit, where that kernel takes 0.79 times as
+// long on average over 487 problems (values of a decode step, 16 heads x 1x64x3232
+// f16, 7.7 -> 3.5 us; 4 rows x 256 x 3456 5.9 -> 4.2), and with more columns this one's
+// longer runs of them win. Longer K, which is split here into slices that a second
+// launch adds: up to 12 KB of K and 256 outer columns, on the shape of an entry
+// alone, so that the entries of a batch have the bits of the single call (fp8 8 rows
+// x 4992 x 15552 36.9 -> 19.5, f16 2 x 128 x 4992 6.1 -> 5.0; beyond 12 KB the few
+// workgroups of a single call take longer: bf16 16 x 480 x 14528 9.1 here, 14.3 there).
+bool few_columns(int64_t N, int64_t chunks, int64_t batch) {
+  if (chunks <= 32) return false;
+  if (chunks <= 512) return batch * N <= device_cu_count();
+  return chunks <= 768 && N <= 256;
+}
+
+// The problem(s) on that kernel; NOT_FOUND where it is not taken.
+int launch_few_columns(const iree_amd_uk_mmt4d_params_t& p, const BatchStrides& b, hipStream_t s) {
+  Mmt4dTypeInfo ti;
+  mmt4d_type_info(p.flags, &ti);
+  const int eb = ti.lhs_bits / 8;
+  if (p.K0 * eb != 16 || !few_columns(p.N, p.K, b.batch)) return IREE_AMD_UK_STATUS_NOT_FOUND;
+  WaveSplitArgs w = {};
+  w.lhs = (const char*)p.lhs_buffer + p.lhs_offset * eb;
+  w.rhs = (const char*)p.rhs_buffer + p.rhs_offset * eb;
+  w.out = (char*)p.out_buffer + p.out_offset * ti.out_bytes;
+  w.lhs_batch = b.lhs * eb; w.rhs_batch = b.rhs * eb; w.out_batch = b.out * ti.out_bytes;
+  w.rhs_outer = p.rhs_stride0 * eb;
+  if (((uintptr_t)w.lhs | (uintptr_t)w.rhs) % 16 || (w.rhs_outer | w.lhs_batch | w.rhs_batch) % 16)
+    return IREE_AMD_UK_STATUS_NOT_FOUND;
+  const bool transposed = (p.flags & kTransposedOut) != 0;
+  w.lhs_row = 16; w.lhs_chunk = p.M0 * 16;
+  w.rows = w.out_rows = p.M0;
+  w.outer_cols = (int)p.N; w.out_cols = (int)p.N * 32;
+  w.k_chunks = (int)p.K;
+  w.out_row = transposed ? 1 : 32;
+  w.out_col = transposed ? p.M0 : 1;
+  w.out_tile = transposed ? p.out_stride0 : (int64_t)p.M0 * 32;
+  w.accumulate = (p.flags & IREE_AMD_UK_FLAG_MMT4D_ACCUMULATE) != 0;
+  w.batch = (int)b.batch;
+  w.out_scale = 1.0f;
+  const uint32_t type = p.flags & IREE_AMD_UK_FLAG_MMT4D_TYPE_MASK;
+  const WaveSplitChoice c = choose_wave_split(w, type);
+  return c.tile < 0 ? (int)IREE_AMD_UK_STATUS_NOT_FOUND : launch_mmt4d_wave_split(w, type, c.tile, s);
+}
+}  // namespace
+
 // `batch` problems of one narrow shape as the planes of one launch, at most
 // 65535 entries and batch strides of whole 16 bytes. A K that one launch row
 // cannot hold in registers is split over workgroup rows exactly as for a single
@@ -658,6 +709,10 @@ int launch_batch_mmt4d_skinny(const iree_amd_uk_mmt4d_params_t& p0, int64_t batc
   // (the kernel counts columns, 32 per outer column, in 32 bits)
   if (p.M != 1 || p.K == 0 || p.N > 0x3FFFFFF || batch > 65535)
     return IREE_AMD_UK_STATUS_NOT_FOUND;
+  {
+    const int st = launch_few_columns(p, BatchStrides{batch, lhs_batch_stride, rhs_batch_stride, out_batch_stride}, s);
+    if (st != IREE_AMD_UK_STATUS_NOT_FOUND) return st;
+  }
   const int64_t steps = (k_elems + mk - 1) / mk;   // (the last one may be partial)
   const int max_steps = max_steps_per_launch(mk);
   const int64_t elems = p.N * p.M0 * 32;
@@ -695,6 +750,10 @@ int launch_mmt4d_skinny(const iree_amd_uk_mmt4d_params_t& p0, hipStream_t s) {
   const int mk = mfma_k_of(p.flags);
   const int64_t k_elems = p.K * p.K0;
   if (p.M != 1 || p.K == 0 || p.N > 0x3FFFFFF) return IREE_AMD_UK_STATUS_NOT_FOUND;
+  {
+    const int st = launch_few_columns(p, BatchStrides{1, 0, 0, 0}, s);
+    if (st != IREE_AMD_UK_STATUS_NOT_FOUND) return st;
+  }
   // (a K that is not whole steps ends in a partial one)
   const int64_t steps = (k_elems + mk - 1) / mk;
   if (steps > 0x7FFFFFFF) return IREE_AMD_UK_STATUS_NOT_FOUND;
@@ -844,20 +903,38 @@ int launch_matmul_rows_skinny(const iree_amd_uk_mmt4d_params_t& p, int64_t M, in
   // which the reduction kernel adds in row order into a result without gaps
   // between its rows.
   const int cus = device_cu_count();
+  const bool few = p.K0 * eb == 16 && few_columns(p.N, p.K, 1);
   int64_t chunks = 1;
-  if (p.N * 2 <= cus && steps >= 64) {
+  if (!few && p.N * 2 <= cus && steps >= 64) {
     chunks = cus / p.N;
     if (chunks > steps / 32) chunks = steps / 32;
     if (chunks > 8) chunks = 8;
     if (chunks < 1) chunks = 1;
   }
-  if (p.N * 2 <= cus && chunks < 2) return IREE_AMD_UK_STATUS_NOT_FOUND;
+  if (!few && p.N * 2 <= cus && chunks < 2) return IREE_AMD_UK_STATUS_NOT_FOUND;
   if (chunks > 1 && (p.out_stride0 != out_cols || (M * out_cols) % 4)) return IREE_AMD_UK_STATUS_NOT_FOUND;
   const char* lhs = (const char*)p.lhs_buffer + p.lhs_offset * eb;
   const char* rhs = (const char*)p.rhs_buffer + p.rhs_offset * eb;
   if (((uintptr_t)lhs | (uintptr_t)rhs) % 16 || (p.rhs_stride0 * eb) % 16 || (p.lhs_stride0 * eb) % 16)
     return IREE_AMD_UK_STATUS_NOT_FOUND;
   if (M * p.lhs_stride0 * eb > 0x7FFFFFFF) return IREE_AMD_UK_STATUS_NOT_FOUND;
+  if (few) {
+    WaveSplitArgs w = {};
+    w.lhs = lhs; w.rhs = rhs;
+    w.out = (char*)p.out_buffer + p.out_offset * ti.out_bytes;
+    w.lhs_outer = 32 * p.lhs_stride0 * eb; w.rhs_outer = p.rhs_stride0 * eb;
+    w.lhs_row = (int)(p.lhs_stride0 * eb); w.lhs_chunk = 16;
+    w.rows = w.out_rows = (int)M;
+    w.outer_cols = (int)p.N; w.out_cols = (int)out_cols;
+    w.k_chunks = (int)p.K;
+    w.out_outer = 32 * p.out_stride0; w.out_row = p.out_stride0; w.out_tile = 32; w.out_col = 1;
+    w.accumulate = (p.flags & IREE_AMD_UK_FLAG_MMT4D_ACCUMULATE) != 0;
+    w.batch = 1;
+    w.out_scale = 1.0f;
+    const uint32_t type = p.flags & IREE_AMD_UK_FLAG_MMT4D_TYPE_MASK;
+    const WaveSplitChoice c = choose_wave_split(w, type);
+    if (c.tile >= 0) return launch_mmt4d_wave_split(w, type, c.tile, s);
+  }
   SkinnyArgs a;
   a.rot_tiles = 0;
   a.lhs = lhs; a.rhs = rhs;

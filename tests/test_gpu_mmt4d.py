@@ -1496,3 +1496,92 @@ def test_small_matmul_leaves_shared_memory_to_the_chain(uk, cuda):
         uk.matmul_data_tiled(a, b, c, M, N, K, F.MMT4D_TYPE_F32F32F32)
         assert uk.last_kernel_path() != "mmt4d:mfma-one-launch"
         assert torch.equal(c, a @ b)
+
+
+# Problems for the kernel that splits K over the waves of a workgroup: rows, columns,
+# 64-byte steps of K, pieces of 16 bytes of K beyond them, tile it takes on 256 compute
+# units (waves without K, a partial last step, steps that just fill and just exceed
+# a round of the pipeline, ragged edges, each tile).
+WAVE_SPLIT = [(5, 32, 8, 0, (16, 16)), (33, 40, 17, 1, (16, 16)), (32, 96, 33, 3, (16, 16)), (800, 160, 65, 1, (16, 32)),
+              (100, 1000, 65, 2, (16, 32)), (70, 1500, 64, 0, (32, 32)), (130, 1400, 97, 0, (32, 32)),
+              (200, 1500, 64, 0, (32, 64)), (800, 1000, 32, 0, (64, 64))]
+
+
+@pytest.mark.parametrize("M,N,steps,pieces,tile", WAVE_SPLIT)
+@pytest.mark.parametrize("type_flag,dt,out_dt,k0", [
+    (F.MMT4D_TYPE_F16F16F32, "float16", "float32", 8), (F.MMT4D_TYPE_BF16BF16BF16, "bfloat16", "bfloat16", 8),
+    (F.MMT4D_TYPE_S8S8S32, "int8", "int32", 16), (F.MMT4D_TYPE_F32F32F32, "float32", "float32", 4),
+    (F.MMT4D_TYPE_F8E4M3F8E4M3F32, "float8_e4m3fn", "float32", 16),
+])
+@pytest.mark.parametrize("accumulate", [False, True])
+def test_few_tiles_with_k_over_the_waves(uk, cuda, type_flag, dt, out_dt, k0, M, N, steps, pieces, tile, accumulate):
+    """Every operand form (tiled, row-major result, row-major left-hand side): exact
+    on small integers (|sums| below 2^8), elements around the matrix untouched."""
+    import torch
+    g = torch.Generator(device="cuda").manual_seed(M + N + steps)
+    dt, out_dt = getattr(torch, dt), getattr(torch, out_dt)
+    flags = type_flag | F.MMT4D_SKIP_INTERMEDIATE_ROUNDINGS | (F.MMT4D_ACCUMULATE if accumulate else 0)
+    K1 = 4 * steps + pieces
+    K, M1, N1 = K1 * k0, -(-M // 32), -(-N // 32)
+    some = 64 / K          # (so many products of a sum are not zero)
+    a = torch.randint(-1, 2, (M1 * 32, K), generator=g, device="cuda") * (torch.rand(M1 * 32, K, generator=g, device="cuda") < some)
+    b = torch.randint(-1, 2, (N1 * 32, K), generator=g, device="cuda")
+    c0 = torch.randint(-9, 10, (M1 * 32, N1 * 32), generator=g, device="cuda").to(out_dt)
+    want = a.double() @ b.double().t().contiguous() + (c0.double() if accumulate else 0)
+    assert want.abs().max() < 256
+
+    def tiles(x, t1):
+        return x.reshape(x.shape[0] // 32, 32, x.shape[1] // t1, t1).transpose(1, 2).contiguous()
+    raw = torch.uint8 if dt is torch.float8_e4m3fn else dt
+    lhs, rhs = tiles(a.to(dt).view(raw), k0), tiles(b.to(dt).view(raw), k0)
+    c = tiles(c0, 32).clone()
+    uk.mmt4d(lhs, rhs, c, M1, N1, K1, 32, 32, k0, flags)
+    assert uk.last_kernel_path() == "mmt4d:mfma"
+    _expect_macro_tile(uk, *tile, 1)
+    assert torch.equal(c.transpose(1, 2).reshape(M1 * 32, N1 * 32).double(), want)
+    c = c0.clone()
+    uk.mmt4d_unpack(lhs, rhs, c, M, N, M1, N1, K1, k0, flags, out_stride0=N1 * 32)
+    _expect_macro_tile(uk, *tile, 1)
+    assert torch.equal(c[:M, :N].double(), want[:M, :N])
+    c[:M, :N] = c0[:M, :N]
+    assert torch.equal(c, c0)
+    if pieces == 0 and M > 32:
+        rows = a[:M].to(dt).view(raw).contiguous()
+        uk.matmul_packed_rhs(rows, rhs, c, M, N, K, k0, flags, out_stride0=N1 * 32)
+        assert torch.equal(c[:M, :N].double(), want[:M, :N])
+        c[:M, :N] = c0[:M, :N]
+        assert torch.equal(c, c0)
+
+
+@pytest.mark.parametrize("M0,N,K1,batch", [(1, 1, 33, 1), (4, 3, 130, 1), (8, 5, 511, 3), (16, 2, 767, 1), (2, 7, 513, 5)])
+@pytest.mark.parametrize("type_flag,dt,out_dt,k0", [
+    (F.MMT4D_TYPE_F16F16F16, "float16", "float16", 8), (F.MMT4D_TYPE_S8S8S32, "int8", "int32", 16),
+    (F.MMT4D_TYPE_F32F32F32, "float32", "float32", 4),
+])
+@pytest.mark.parametrize("accumulate", [False, True])
+def test_few_narrow_columns_with_k_over_the_waves(uk, cuda, type_flag, dt, out_dt, k0, M0, N, K1, batch, accumulate):
+    """Narrow tiles on either side, and planes of them; narrow rows of a row-major matrix."""
+    import torch
+    g = torch.Generator(device="cuda").manual_seed(M0 + N + K1)
+    dt, out_dt = getattr(torch, dt), getattr(torch, out_dt)
+    flags = type_flag | F.MMT4D_SKIP_INTERMEDIATE_ROUNDINGS | (F.MMT4D_ACCUMULATE if accumulate else 0)
+    a = (torch.randint(-1, 2, (batch, K1, M0, k0), generator=g, device="cuda") *
+         (torch.rand(batch, K1, M0, k0, generator=g, device="cuda") < 64 / (K1 * k0))).to(dt)
+    b = torch.randint(-1, 2, (batch, N, K1, 32, k0), generator=g, device="cuda").to(dt)
+    c0 = torch.randint(-9, 10, (batch, N, M0, 32), generator=g, device="cuda").to(out_dt)
+    am = a.transpose(1, 2).reshape(batch, M0, -1).double()
+    bm = b.transpose(2, 3).reshape(batch, N * 32, -1).double().transpose(1, 2).contiguous()
+    want = (am @ bm).reshape(batch, M0, N, 32).transpose(1, 2) + (c0.double() if accumulate else 0)
+    assert want.abs().max() < 256
+    c = c0.clone()
+    uk.batch_mmt4d(a, b, c, batch, 1, N, K1, M0, 32, k0, flags)
+    assert uk.last_kernel_path() == "mmt4d:mfma-narrow" and uk.last_macro_tile()[0] == 16
+    assert torch.equal(c.double(), want)
+    c = c0.transpose(2, 3).contiguous()
+    uk.batch_mmt4d(b, a, c, batch, N, 1, K1, 32, M0, k0, flags)
+    assert torch.equal(c.transpose(2, 3).double(), want)
+    if M0 > 1 and K1 <= 512 and K1 * k0 % 32 == 0:
+        c = c0[0].transpose(0, 1).reshape(M0, N * 32).contiguous()
+        uk.matmul_packed_rhs(am[0].to(dt).contiguous(), b[0], c, M0, N * 32, K1 * k0, k0, flags)
+        assert uk.last_kernel_path() == "mmt4d:mfma-narrow"
+        assert torch.equal(c.reshape(M0, N, 32).transpose(0, 1).double(), want[0])
