@@ -467,10 +467,16 @@ int launch_cfg(SkinnyArgs a, int chunks, hipStream_t s) {
   // the rolling buffer)
   constexpr int kPerWaveSteps = Cfg::kSub == 2 ? 8 : 16;
   const int groups = (a.N + kWaves - 1) / kWaves;
-  if (chunks == 1 && a.chunk_steps <= kPerWaveSteps &&
-      (int64_t)groups * (a.batch > 1 ? a.batch : 1) >= cus) {
-    // a short K and enough outer columns to give every compute unit 8 of
-    // them: one outer column per wave
+  // A short K is not split over the waves where there are enough outer columns, of
+  // all planes together, for a wave to take whole ones: one per compute unit with up
+  // to 4 steps, 1.5 with 8, 3 with 16. Measured on 1200 problems below 8 columns a
+  // compute unit, where this form began before: one to two columns with 4 steps
+  // 0.81 times as long, two to four 0.65, four to eight 0.5 (scores of a decode step, 8
+  // heads x 1x7104x64 f16, 9.0 -> 4.4 us); below the line the other form wins by as much.
+  const int64_t columns = (int64_t)a.N * (a.batch > 1 ? a.batch : 1);
+  const int64_t enough = a.chunk_steps <= 4 ? cus : a.chunk_steps <= 8 ? cus * 3 / 2 : cus * 3;
+  if (chunks == 1 && a.chunk_steps <= kPerWaveSteps && columns >= enough) {
+    // one outer column per wave
     a.steps_per_wave = a.chunk_steps;
     a.stage_wave_bytes = 0;
     // (32 planes of 1024 outer columns, 8 MiB apart: 53.3 -> 51.7 us; other

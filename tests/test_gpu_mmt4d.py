@@ -1585,3 +1585,20 @@ def test_few_narrow_columns_with_k_over_the_waves(uk, cuda, type_flag, dt, out_d
         uk.matmul_packed_rhs(am[0].to(dt).contiguous(), b[0], c, M0, N * 32, K1 * k0, k0, flags)
         assert uk.last_kernel_path() == "mmt4d:mfma-narrow"
         assert torch.equal(c.reshape(M0, N, 32).transpose(0, 1).double(), want[0])
+
+
+@pytest.mark.parametrize("M0,N,batch", [(1, 255, 1), (1, 256, 1), (8, 129, 2), (4, 31, 13), (2, 33, 8)])
+@pytest.mark.parametrize("steps", [1, 4, 5, 8])
+def test_short_k_whole_per_wave(uk, cuda, M0, N, batch, steps):
+    """About one outer column of narrow tiles per compute unit, a K of a few
+    instruction steps: both sides of the line from which a wave takes whole columns."""
+    import torch
+    g = torch.Generator(device="cuda").manual_seed(N + steps)
+    K1 = 2 * steps
+    a = torch.randint(-3, 4, (batch, K1, M0, 8), generator=g, device="cuda").half()
+    b = torch.randint(-3, 4, (batch, N, K1, 32, 8), generator=g, device="cuda").half()
+    c = torch.full((batch, N, M0, 32), -1.0, device="cuda")
+    uk.batch_mmt4d(a, b, c, batch, 1, N, K1, M0, 32, 8, F.MMT4D_TYPE_F16F16F32)
+    am = a.transpose(1, 2).reshape(batch, M0, -1).float()
+    bm = b.transpose(2, 3).reshape(batch, N * 32, -1).float().transpose(1, 2).contiguous()
+    assert torch.equal(c, (am @ bm).reshape(batch, M0, N, 32).transpose(1, 2))
