@@ -646,7 +646,9 @@ IREE_AMD_UK_EXPORT int iree_amd_uk_matmul_packed_rhs(
  * a is M x K, b K x N, c M x N, all row-major and tight, element types as in
  * `flags` (an IREE_AMD_UK_FLAG_MMT4D_TYPE_*, optionally ACCUMULATE). lhs, rhs and
  * out receive the packed operands and the packed result in tiles of M0 x K0,
- * N0 x K0 and M0 x N0, as the chain leaves them; a null one is not written.
+ * N0 x K0 and M0 x N0, as the chain leaves them (the padding of the result's tiles
+ * zeros, also where the chain multiplies padding by an infinity); a null one is not
+ * written.
  * Integers have the chain's bits, and so have the packed operands; float sums come
  * in another order (a captured call's, whose K stays whole, in a third), with an
  * error no larger.

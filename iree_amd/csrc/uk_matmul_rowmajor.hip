@@ -11,28 +11,25 @@
 // after them write the packed operands, which nothing in the launch waits for,
 // and the matmul's epilogue stores both the tiles of the result and the matrix.
 //
-// Among other calls on one stream: f16 81x19x41 with C added 27.1 us as the chain,
-// 7.4 here; i8 1024^3 21.0, 11.4.
+// Among other calls on one stream, as the chain, on tiles of 32 x 32 and 64 x 64 whose
+// waves shared their operands through LDS, and here: f16 81x19x41 with C added 27.1,
+// 8.0, 4.6 us; i8 1024^3 21.0, 12.5, 8.9; f16 1024^3 22.0, 22 to 24, 11.8; f16
+// 2634x35x20 with C added (the chain not timed) 8.8, 3.3.
 //
-// A step of K costs a workgroup 2.4 to 3.9 us: its 24 loads per thread, many of
-// them of rows 64 bytes long, pass the compute unit's one load path. So a long
-// K of few tiles is dealt to more workgroups, each with its own plane of partial
-// sums, and a second launch adds the planes in order (2 us when it follows):
-// bf16 64x29x3693 35.0 us whole, 8.7 in 8 slices.
-//
-// Multiplying workgroups: 4 waves on kRows x kRows of the result, 64 KiB of
-// operands per K-step (128 KiB / kRows bytes of K), fetched for the next
-// step while this one is multiplied: a wide step because a step costs a round
-// trip to memory, and these problems have too few workgroups to hide it.
-// An operand row of a step is kChunks chunks of 16 bytes of consecutive K in
-// LDS, permuted within 16 by a hash of the row: fragment reads (16 consecutive
-// rows, one chunk) and the stores of the right-hand side (rows 4 apart) hit 16
-// different bank groups each. The right-hand side, whose rows run along N,
-// is turned in registers: a thread loads 4 columns of the 16 / element-size
-// rows of a chunk and stores 4 chunks.
-//   kRows = 64: each wave a 32x32 quarter.
-//   kRows = 32: each wave all of it for a quarter of K, summed in LDS in wave
-//   order; four times as many workgroups and half as many steps.
+// Multiplying workgroups: 16 or 32 rows x 64 columns of the result, K dealt to 8
+// waves in steps of 64 bytes. A wave fetches its own steps straight into
+// registers, two ahead, and waits for no other until the sums meet in LDS. A lane
+// loads 4 columns of the 16 / element-size rows of the right-hand side that make a
+// piece of a matrix-core operand, and turns them in registers into a piece of
+// each column: column 4 i + y of the tile is column i of operand y, so that the
+// sums of a lane are 4 consecutive columns again. Sharing the operands cost more
+// than it saved: a step of 32 KB took 2.4 to 3.9 us, most of it waiting.
+// What bounds it now: 3 to 3.5 us for a launch of one step, then the intake of the
+// compute units that have work (loads of twice the columns gave the same times).
+// A long K of few tiles is dealt to more workgroups, each with its own plane of
+// partial sums, and a second launch adds the planes in order (2 us when it follows):
+// bf16 64x29x3693 16.3 us whole, 7.1 in 8 slices (35.0 as the chain).
+#include <cmath>
 #include <type_traits>
 
 #include "uk_common.h"
@@ -57,6 +54,8 @@ struct F32Cfg16 {
   }
 };
 
+constexpr int kThreads = 512;
+
 struct RowMajorArgs {
   const char* a;       // M x K
   const char* b;       // K x N
@@ -74,12 +73,13 @@ struct RowMajorArgs {
   void* partial;
 };
 
-// A 128-bit value moved down by `bytes` (0 to 15), zeros from above.
+// The bytes of a lane's piece move down by `bytes` (0 to 15), zeros from above.
 __device__ __forceinline__ u32x4 shift_down(u32x4 v, int bytes) {
-  union { u32x4 v; unsigned __int128 x; } u;
-  u.v = v;
-  u.x >>= 8 * bytes;
-  return u.v;
+  const u32x4 a = bytes & 8 ? u32x4{v[2], v[3], 0, 0} : v;
+  const u32x4 b = bytes & 4 ? u32x4{a[1], a[2], a[3], 0} : a;
+  const uint32_t r = bytes & 3;
+  return u32x4{__builtin_amdgcn_alignbyte(b[1], b[0], r), __builtin_amdgcn_alignbyte(b[2], b[1], r),
+               __builtin_amdgcn_alignbyte(b[3], b[2], r), b[3] >> (8 * r)};
 }
 
 // Loads never leave the matrix and never branch: what lies past the end of a
@@ -101,23 +101,11 @@ __device__ __forceinline__ u32x4 settle_chunk(u32x4 v, int k, int K, bool row_ex
   return k + E <= K ? v : shift_down(v, (k + E - K) * kElemBytes);
 }
 
-// Four consecutive elements of a row, in kElemBytes dwords.
+// Four consecutive elements of a row.
 template <int kElemBytes>
 struct Four { uint32_t d[kElemBytes]; };
-template <int kElemBytes>
-__device__ __forceinline__ Four<kElemBytes> settle_four(Four<kElemBytes> r, int n, int N, bool row_exists) {
-  if (!row_exists || n >= N) return Four<kElemBytes>{};
-  if (n + 4 <= N) return r;
-  u32x4 v = {0, 0, 0, 0};
-#pragma unroll
-  for (int i = 0; i < kElemBytes; ++i) v[i] = r.d[i];
-  v = shift_down(v, (n + 4 - N) * kElemBytes);
-#pragma unroll
-  for (int i = 0; i < kElemBytes; ++i) r.d[i] = v[i];
-  return r;
-}
 
-// Chunk of column e (0 to 3) from the 16 / kElemBytes rows of a four-column strip.
+// The piece of column e from the 16 / kElemBytes rows of a strip of 4 columns.
 template <int kElemBytes>
 __device__ __forceinline__ u32x4 column_chunk(const Four<kElemBytes>* rows, int e) {
   u32x4 v;
@@ -140,13 +128,13 @@ __device__ __forceinline__ u32x4 column_chunk(const Four<kElemBytes>* rows, int 
   return v;
 }
 
-// One workgroup's 256 chunks of a packed operand. Chunk r of the buffer is row
+// One workgroup's 512 chunks of a packed operand. Chunk r of the buffer is row
 // i0 of the tile (i1, k1).
 template <int kElemBytes>
 __device__ void pack_block(const RowMajorArgs& p, int block) {
   constexpr int E = 16 / kElemBytes;
   const bool is_lhs = block < p.lhs_blocks;
-  const uint32_t r = (uint32_t)(is_lhs ? block : block - p.lhs_blocks) * 256 + threadIdx.x;
+  const uint32_t r = (uint32_t)(is_lhs ? block : block - p.lhs_blocks) * kThreads + threadIdx.x;
   const uint32_t T0 = is_lhs ? p.M0 : p.N0, K1 = p.K1;
   if (r >= T0 * K1 * (uint32_t)(is_lhs ? p.M1 : p.N1)) return;
   const uint32_t tile = r / T0, i0 = r - tile * T0;
@@ -194,235 +182,322 @@ __global__ __launch_bounds__(256) void matmul_rowmajor_sum_kernel(RowMajorArgs p
   sum_t sum = 0;
 #pragma unroll 8
   for (int i = 0; i < p.slices; ++i) sum += part[i * plane];
-  const out_t v = (out_t)(sum + old);
+  const out_t v = in_matrix ? (out_t)(sum + old) : (out_t)0;   // (padding of the tiles: zeros)
   if (in_matrix) *c = v;
   if (in_tiles) ((out_t*)p.out)[(((int64_t)m1 * p.N1 + n1) * p.M0 + m0) * p.N0 + n0] = v;
 }
 
-template <typename Cfg, int kRows>
-__global__ __launch_bounds__(256, 2) void matmul_rowmajor_kernel(RowMajorArgs p) {
+constexpr int kWaves = 8;
+constexpr uint32_t kNowhere = 0x80000000u;   // past the end of every descriptor: the load gives zeros
+
+// One workgroup: 16 MB rows x 64 columns of the result (of a slice of K).
+template <typename Cfg, int MB>
+__device__ __forceinline__ void multiply_tile(const RowMajorArgs& p) {
   constexpr int kElemBytes = Cfg::kElemBytes;
-  constexpr int E = 16 / kElemBytes;            // elements of a chunk
-  constexpr int kChunks = 2048 / kRows;         // chunks of a row per step
-  constexpr int kStep = kChunks * E;            // elements of K per step
-  constexpr int kGroups = kRows / 4;            // four-column strips of the right-hand side
+  constexpr int E = 16 / kElemBytes;            // elements of a piece, rows of the right-hand side per lane and step
+  constexpr int kStep = 4 * E;                  // elements of K per step
   typedef typename Cfg::frag_t frag_t;
   typedef typename Cfg::acc_t acc_t;
   typedef typename Cfg::out_t out_t;
-  __shared__ u32x4 tile_a[2048], tile_b[2048];
-  if ((int)blockIdx.x >= p.product_blocks) {
-    pack_block<kElemBytes>(p, (int)blockIdx.x - p.product_blocks);
-    return;
-  }
-  const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
+  typedef typename Sum<out_t>::type sum_t;
+  typedef sum_t sum4_t __attribute__((ext_vector_type(4)));
+  typedef sum_t sum4_unaligned_t __attribute__((ext_vector_type(4), aligned(4)));
+  typedef out_t out4_t __attribute__((ext_vector_type(4), aligned(sizeof(out_t))));
+  constexpr int F = MB * 4;                     // rows of a lane, 4 columns each
+  constexpr int D = 2;                          // steps in flight
+  typedef Four<kElemBytes> columns_t;
+  __shared__ sum4_t sums[kWaves][F][64];
+  __shared__ u32x4 turn[kWaves][MB][64];
+  const int lane = threadIdx.x & 63, l16 = lane & 15, kc = lane >> 4;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int slice = (int)blockIdx.x / p.tiles, tile = (int)blockIdx.x - slice * p.tiles;
-  const int m_base = tile / p.tiles_n * kRows, n_base = tile % p.tiles_n * kRows;
+  const int m_base = tile / p.tiles_n * (MB * 16), n_base = tile % p.tiles_n * 64;
   const int k_first = slice * p.slice_k, k_end = k_first + p.slice_k < p.K ? k_first + p.slice_k : p.K;
-  auto place = [](int row, int chunk) { return row * kChunks + (chunk ^ ((row + (row >> 4)) & 15)); };
-
-  // what this thread fetches of a step: chunk t % kChunks of 8 rows of A, and
-  // two strips of 4 columns x E rows of B
-  u32x4 next_a[8];
-  Four<kElemBytes> next_b[2][E];
-  const int my_row = m_base + t / kChunks, my_n = n_base + t % kGroups * 4;
-  uint32_t row_at[8];                           // element offsets, 32 bits (operands of up to 64 MiB)
+  // This lane's columns: 4 of them, from n on; past the last ones the last ones again.
+  const int n = n_base + l16 * 4, n_at = n + 4 <= p.N ? n : p.N - 4;
+  const __amdgpu_buffer_rsrc_t a_src = __builtin_amdgcn_make_buffer_rsrc((void*)p.a, 0, 0x7FFFFFFF, 0x00020000);
+  const __amdgpu_buffer_rsrc_t b_src = __builtin_amdgcn_make_buffer_rsrc((void*)p.b, 0, 0x7FFFFFFF, 0x00020000);
+  // (32-bit offsets: operands of up to 64 MiB)
+  // The row and piece of a block of A that this lane fetches: the lanes of a quad the
+  // 64 bytes of one row (of four rows they would be four requests). A block goes
+  // through LDS into operand order, the pieces of row r rotated by r / 4 there.
+  const int a_row = lane >> 2, a_piece = ((lane & 3) - (lane >> 4)) & 3;
+  uint32_t a_at[MB];
 #pragma unroll
-  for (int j = 0; j < 8; ++j) {
-    const int row = my_row + j * (kRows / 8);
-    row_at[j] = (uint32_t)(row < p.M ? row : p.M - 1) * p.K;
+  for (int x = 0; x < MB; ++x) {
+    const int row = m_base + x * 16 + a_row;
+    a_at[x] = (uint32_t)((row < p.M ? row : p.M - 1) * p.K + k_first + a_piece * E) * kElemBytes;
   }
-  const uint32_t col_at = my_n + 4 <= p.N ? my_n : p.N - 4, last_row = (uint32_t)(p.K - 1) * p.N;
-  auto fetch = [&](int k_base) {
-    const int ka = k_base + t % kChunks * E;
-    const uint32_t at = ka + E <= p.K ? ka : p.K - E;
+  const uint32_t b_row = (uint32_t)p.N * kElemBytes;
+  const uint32_t b_at = (uint32_t)(k_first + kc * E) * b_row + (uint32_t)n_at * kElemBytes;
+
+  // what a step fetches: a piece of MB rows of A, 4 columns of E rows of B
+  struct Step {
+    u32x4 a[MB];
+    columns_t b[E];
+  };
+  auto load_columns = [&](uint32_t at, uint32_t more) -> columns_t {
+    columns_t r;
+    if constexpr (kElemBytes == 1) {
+      r.d[0] = __builtin_amdgcn_raw_buffer_load_b32(b_src, at, more, 0);
+    } else if constexpr (kElemBytes == 2) {
+      const auto v = __builtin_amdgcn_raw_buffer_load_b64(b_src, at, more, 0);
+      r.d[0] = v[0]; r.d[1] = v[1];
+    } else {
+      const auto v = __builtin_amdgcn_raw_buffer_load_b128(b_src, at, more, 0);
 #pragma unroll
-    for (int j = 0; j < 8; ++j) __builtin_memcpy(&next_a[j], p.a + (row_at[j] + at) * kElemBytes, 16);
+      for (int i = 0; i < 4; ++i) r.d[i] = v[i];
+    }
+    return r;
+  };
+  const int steps = (k_end - k_first) / kStep, tail = (k_end - k_first) % kStep;   // whole steps, elements left over
+  // Steps are dealt to the waves one by one (the fewer a wave adds up one after the
+  // other, the smaller the rounding error); what is past the last whole one is not
+  // fetched.
+  auto load = [&](Step& s, int i) {
+    const int step = i * kWaves + wave;
+    const bool exists = step < steps;
 #pragma unroll
-    for (int j = 0; j < 2; ++j) {
-      const uint32_t k_row = (uint32_t)(k_base + (t / kGroups + j * (256 / kGroups)) * E) * p.N;
+    for (int e = 0; e < E; ++e) s.b[e] = load_columns(exists ? b_at : kNowhere, exists ? (uint32_t)(step * kStep + e) * b_row : 0);
 #pragma unroll
-      for (int e = 0; e < E; ++e) {
-        const uint32_t r = k_row + (uint32_t)e * p.N;
-        __builtin_memcpy(&next_b[j][e], p.b + ((r < last_row ? r : last_row) + col_at) * kElemBytes, 4 * kElemBytes);
+    for (int x = 0; x < MB; ++x)
+      s.a[x] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(a_src, exists ? a_at[x] : kNowhere,
+                                                                              exists ? step * 64 : 0, 0));
+  };
+  acc_t acc[MB][4];
+#pragma unroll
+  for (int x = 0; x < MB; ++x)
+#pragma unroll
+    for (int y = 0; y < 4; ++y) acc[x][y] = acc_t{0, 0, 0, 0};
+  auto multiply = [&](const Step& s) {
+    // (a wave's LDS accesses are served in order)
+    u32x4 fa[MB];
+#pragma unroll
+    for (int x = 0; x < MB; ++x) turn[wave][x][lane] = s.a[x];
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+#pragma unroll
+    for (int x = 0; x < MB; ++x) fa[x] = turn[wave][x][l16 * 4 + ((kc + (l16 >> 2)) & 3)];
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+#pragma unroll
+    for (int y = 0; y < 4; ++y) {
+      const frag_t fb = __builtin_bit_cast(frag_t, column_chunk<kElemBytes>(s.b, y));
+#pragma unroll
+      for (int x = 0; x < MB; ++x) {
+        // (f32, four instructions a step: each step has a sum of its own, for the
+        // rounding error; 1.05 times as large on average without)
+        if constexpr (kElemBytes == 4) acc[x][y] += Cfg::mfma(__builtin_bit_cast(frag_t, fa[x]), fb, acc_t{0, 0, 0, 0});
+        else acc[x][y] = Cfg::mfma(__builtin_bit_cast(frag_t, fa[x]), fb, acc[x][y]);
       }
     }
   };
-  fetch(k_first);
-
-  // The wave's 2 x 2 blocks of 16x16: element r of a lane is row 4 (lane / 16) + r,
-  // column lane % 16.
-  const int wm = kRows == 64 ? wave / 2 * 32 : 0, wn = kRows == 64 ? wave % 2 * 32 : 0;
-  const bool owner = kRows == 64 || wave == 0;   // stores the result
-  // A step has sums of its own, one for every other instruction, which are added
-  // to the whole at its end, and the old result last of all: the rounding error
-  // of a sum grows with the number of terms it takes one by one.
-  acc_t acc[2][2] = {}, old[2][2] = {};
+  // Row f of a lane after the sums.
+  auto row_of = [&](int f) { return m_base + f / 4 * 16 + kc * 4 + f % 4; };
+  constexpr int kOwn = (F + kWaves - 1) / kWaves;
+  sum4_t old[kOwn];
   out_t* const c = (out_t*)p.c;
-  if (p.accumulate && owner && !p.partial) {
 #pragma unroll
-    for (int i = 0; i < 2; ++i)
+  for (int o = 0; o < kOwn; ++o) {
+    old[o] = sum4_t{0, 0, 0, 0};
+    const int f = o * kWaves + wave;
+    if (p.accumulate && !p.partial && f < F && row_of(f) < p.M) {
+      const out4_t v = *(const out4_t*)(c + (int64_t)row_of(f) * p.N + n_at);
 #pragma unroll
-      for (int j = 0; j < 2; ++j)
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          const int m = m_base + wm + i * 16 + lane / 16 * 4 + r, n = n_base + wn + j * 16 + lane % 16;
-          if (m < p.M && n < p.N) old[i][j][r] = c[(int64_t)m * p.N + n];
-        }
+      for (int e = 0; e < 4; ++e) old[o][e] = (sum_t)v[e];
+    }
   }
-
-  for (int k_base = k_first; k_base < k_end; k_base += kStep) {
-    const int left = k_end - k_base;
-    const int subs = left >= kStep ? kChunks / 4 : (left + 4 * E - 1) / (4 * E);   // of 4 chunks: one instruction's K
-    if (k_base > k_first) __syncthreads();
-    if (t % kChunks < subs * 4) {
+  // The step that ends inside itself: pieces that cross the end of K are those that
+  // end there, moved down; rows past it the last one, replaced by zeros.
+  const bool has_tail = tail > 0 && wave == steps % kWaves;
+  const int k_tail = k_first + steps * kStep + kc * E, a_tail = k_first + steps * kStep + a_piece * E;   // (of B, of A)
+  Step last;
+  if (has_tail) {
 #pragma unroll
-      for (int j = 0; j < 8; ++j)
-        tile_a[place(t / kChunks + j * (kRows / 8), t % kChunks)] = settle_chunk<kElemBytes>(
-            next_a[j], k_base + t % kChunks * E, p.K, my_row + j * (kRows / 8) < p.M);
+    for (int x = 0; x < MB; ++x) {
+      const int back = a_tail + E <= p.K ? 0 : a_tail + E - p.K;
+      last.a[x] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(
+                                                a_src, a_at[x] + (uint32_t)(steps * 64 - back * kElemBytes), 0, 0));
     }
 #pragma unroll
-    for (int j = 0; j < 2; ++j) {
-      const int chunk = t / kGroups + j * (256 / kGroups), k = k_base + chunk * E;
-      if (chunk < subs * 4) {
-        if (k + E > p.K || my_n + 4 > p.N) {
+    for (int e = 0; e < E; ++e) {
+      const int k = k_tail + e < k_end ? k_tail + e : k_end - 1;
+      last.b[e] = load_columns((uint32_t)k * b_row + (uint32_t)n_at * kElemBytes, 0);
+    }
+  }
+  Step ring[D];
+  const int rounds = steps > wave ? (steps - wave - 1) / kWaves + 1 : 0;      // steps of this wave
+  if (rounds > 0) {
+    Step ring[D];
 #pragma unroll
-          for (int e = 0; e < E; ++e) next_b[j][e] = settle_four<kElemBytes>(next_b[j][e], my_n, p.N, k + e < p.K);
-        }
+    for (int d = 0; d < D; ++d) load(ring[d], d);
+#pragma unroll 1
+    for (int i = 0; i + D < rounds; i += D) {
 #pragma unroll
-        for (int e = 0; e < 4; ++e) tile_b[place(t % kGroups * 4 + e, chunk)] = column_chunk<kElemBytes>(next_b[j], e);
+      for (int d = 0; d < D; ++d) {
+        __builtin_amdgcn_sched_barrier(0);
+        multiply(ring[d]);
+        __builtin_amdgcn_sched_barrier(0);
+        load(ring[d], i + D + d);
       }
     }
-    __syncthreads();
-    if (k_base + kStep < k_end) fetch(k_base + kStep);
-    acc_t part[2][2][2] = {};
-    auto multiply = [&](int s, acc_t (&sum)[2][2]) {
-      union { u32x4 u; frag_t f; } fa[2], fb[2];
+    __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-      for (int i = 0; i < 2; ++i) {
-        fa[i].u = tile_a[place(wm + i * 16 + lane % 16, s * 4 + lane / 16)];
-        fb[i].u = tile_b[place(wn + i * 16 + lane % 16, s * 4 + lane / 16)];
-      }
+    for (int d = 0; d < D; ++d) multiply(ring[d]);
+  }
+  if (has_tail) {
+    const int left = k_end - k_tail;            // rows of this lane's that exist
 #pragma unroll
-      for (int i = 0; i < 2; ++i)
-#pragma unroll
-        for (int j = 0; j < 2; ++j) sum[i][j] = Cfg::mfma(fa[i].f, fb[j].f, sum[i][j]);
-    };
-    constexpr int kApart = kRows == 64 ? 1 : 4;   // (kRows = 32: a wave takes every fourth)
-    for (int s = kRows == 64 ? 0 : wave; s < subs; s += 2 * kApart) {
-      multiply(s, part[0]);
-      if (s + kApart < subs) multiply(s + kApart, part[1]);
+    for (int x = 0; x < MB; ++x) {
+      const int back = a_tail + E <= p.K ? 0 : a_tail + E - p.K;
+      last.a[x] = a_tail < p.K ? shift_down(last.a[x], back * kElemBytes & 15) : u32x4{0, 0, 0, 0};
     }
 #pragma unroll
-    for (int i = 0; i < 2; ++i)
-#pragma unroll
-      for (int j = 0; j < 2; ++j) acc[i][j] += part[0][i][j] + part[1][i][j];
+    for (int e = 0; e < E; ++e)
+      if (e >= left) last.b[e] = columns_t{};
+    multiply(last);
   }
-
-  if constexpr (kRows == 32) {
-    // the quarters of K, in wave order
-    acc_t* const part = (acc_t*)tile_a;           // [wave - 1][block][lane]
-    __syncthreads();
-    if (wave > 0) {
+  // ---- the waves' sums, by twos, then the old result --------------------
 #pragma unroll
-      for (int i = 0; i < 4; ++i) part[((wave - 1) * 4 + i) * 64 + lane] = acc[i / 2][i % 2];
-    }
-    __syncthreads();
-    if (wave > 0) return;
+  for (int x = 0; x < MB; ++x)
 #pragma unroll
-    for (int w = 0; w < 3; ++w)
-#pragma unroll
-      for (int i = 0; i < 4; ++i) acc[i / 2][i % 2] += part[(w * 4 + i) * 64 + lane];
-  }
-  if (p.partial) {
-    typedef typename Sum<out_t>::type sum_t;
-    const int rows = p.tiles / p.tiles_n * kRows, cols = p.tiles_n * kRows;
-    sum_t* const part = (sum_t*)p.partial + (int64_t)slice * rows * cols;
-#pragma unroll
-    for (int i = 0; i < 2; ++i)
-#pragma unroll
-      for (int j = 0; j < 2; ++j)
-#pragma unroll
-        for (int r = 0; r < 4; ++r)
-          part[(int64_t)(m_base + wm + i * 16 + lane / 16 * 4 + r) * cols + n_base + wn + j * 16 + lane % 16] = acc[i][j][r];
-    return;
-  }
+    for (int r = 0; r < 4; ++r)
+      sums[wave][x * 4 + r][lane] = sum4_t{acc[x][0][r], acc[x][1][r], acc[x][2][r], acc[x][3][r]};
+  __syncthreads();
   out_t* const out = (out_t*)p.out;
 #pragma unroll
-  for (int j = 0; j < 2; ++j) {
-    const int n = n_base + wn + j * 16 + lane % 16;
-    const int n1 = (int)((uint32_t)n / (uint32_t)p.N0), n0 = n - n1 * p.N0;
+  for (int o = 0; o < kOwn; ++o) {
+    const int f = o * kWaves + wave;
+    if (f >= F) break;
+    const int m = row_of(f);
+    sum4_t part[kWaves];
 #pragma unroll
-    for (int i = 0; i < 2; ++i)
+    for (int w = 0; w < kWaves; ++w) part[w] = sums[w][f][lane];
 #pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int m = m_base + wm + i * 16 + lane / 16 * 4 + r;
-        const out_t v = (out_t)(acc[i][j][r] + old[i][j][r]);
-        if (m < p.M && n < p.N) c[(int64_t)m * p.N + n] = v;
-        if (out) {
-          const int m1 = (int)((uint32_t)m / (uint32_t)p.M0), m0 = m - m1 * p.M0;
-          if (m1 < p.M1 && n1 < p.N1) out[(((int64_t)m1 * p.N1 + n1) * p.M0 + m0) * p.N0 + n0] = v;
-        }
+    for (int apart = 1; apart < kWaves; apart *= 2)
+#pragma unroll
+      for (int w = 0; w < kWaves; w += 2 * apart) part[w] += part[w + apart];
+    sum4_t sum = part[0];
+    if (p.partial) {
+      const int64_t cols = (int64_t)p.tiles_n * 64, rows = (int64_t)p.tiles / p.tiles_n * (MB * 16);
+      if (n < p.N) *(sum4_unaligned_t*)((sum_t*)p.partial + ((int64_t)slice * rows + m) * cols + n_at) = sum;
+      continue;
+    }
+    sum += old[o];
+    out4_t v;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) v[e] = (out_t)sum[e];
+    // (a repeated column is stored by the lane whose own it is: the others may be in
+    // another workgroup, which then adds to it as well)
+    const bool own = n_at == n;
+    if (m < p.M && n < p.N) {
+      out_t* const dst = c + (int64_t)m * p.N + n_at;
+      if (own) {
+        *(out4_t*)dst = v;
+      } else {
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+          if (n_at + e >= n) dst[e] = v[e];
       }
+    }
+    if (out) {
+      const int m1 = (int)((uint32_t)m / (uint32_t)p.M0), m0 = m - m1 * p.M0;
+      if (m1 >= p.M1) continue;
+      if (m >= p.M) v = out4_t{(out_t)0, (out_t)0, (out_t)0, (out_t)0};      // (padding of the tiles: zeros)
+      auto place = [&](int col) -> out_t* {
+        const int n1 = (int)((uint32_t)col / (uint32_t)p.N0), n0 = col - n1 * p.N0;
+        return out + (((int64_t)m1 * p.N1 + n1) * p.M0 + m0) * p.N0 + n0;
+      };
+      if (p.N0 % 4 == 0 && own) {
+        *(out4_t*)place(n) = v;
+        continue;
+      }
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        if (n < p.N && n_at + e >= n) *place(n_at + e) = v[e];
+        const int at = n + e;
+        if (at >= p.N && at < p.N1 * p.N0) *place(at) = (out_t)0;
+      }
+    }
   }
 }
 
-// Estimated time in microseconds on kRows = side with K in `slices`. A step takes
-// about as long whatever else runs, until a compute unit holds more than one
-// workgroup; then the packed buffers and the result, and for a split the planes
-// of sums, written and read, and the second launch. Fitted to 78 problems (f32,
-// 16-bit and i8; 10 to 3900 rows and columns, K 200 to 4000) on both sides and
-// 1 to 16 slices: 12 % off on average, and what it picks is 1.8 % from the best.
+template <typename Cfg, int MB>
+__global__ __launch_bounds__(kThreads, 4) void matmul_rowmajor_kernel(RowMajorArgs p) {
+  if ((int)blockIdx.x >= p.product_blocks) {
+    pack_block<Cfg::kElemBytes>(p, (int)blockIdx.x - p.product_blocks);
+    return;
+  }
+  multiply_tile<Cfg, MB>(p);
+}
+
+// Estimated time in microseconds on 16 mb rows x 64 columns with K in `slices`: the
+// first round of workgroups, one per compute unit, each further one, an eighth of the
+// steps of all of them (by element size), the result, C, and for a split the planes
+// of sums and the launch that adds them. Fitted to half of 1300 problems (8 to 4096
+// rows and columns, K 16 to 4096, six types) on 1 to 16 slices; on the other half
+// 12 % off on average, and what it picks is 1 % from the best.
+struct Shape {
+  float first, round, step4, step1, step2, hidden, store, add, split, plane;
+};
+constexpr Shape kShapes[2] = {{3.47f, 0.30f, 0.82f, 0.99f, 0.78f, 0.26f, 0.42f, 0.18f, 2.10f, 1.12f},
+                              {3.68f, 0.17f, 1.28f, 1.54f, 0.95f, 0.05f, 0.39f, 0.22f, 1.91f, 1.11f}};
+
 struct Estimate {
-  int64_t tiles, steps;
-  double step_us, bytes;
+  double groups, steps, step_us, other;
+  const Shape& t;
+  int cus;
   template <typename Cfg>
-  static Estimate of(const RowMajorArgs& p, int side) {
-    constexpr bool kF32 = Cfg::kElemBytes == 4;   // (whose instructions take as long as a step's loads)
-    const int64_t rows = (int64_t)p.M1 * p.M0, cols = (int64_t)p.N1 * p.N0;
-    return {ceil_div(rows, (int64_t)side) * ceil_div(cols, (int64_t)side),
-            ceil_div((int64_t)p.K * Cfg::kElemBytes, (int64_t)32768 / side),
-            side == 64 ? (kF32 ? 3.9 : 3.0) : 2.8,
-            (p.lhs ? 32.0 * rows * p.K1 : 0) + (p.rhs ? 32.0 * cols * p.K1 : 0) +
-                (p.out ? 2.0 : 1.0) * rows * cols * sizeof(typename Cfg::out_t)};
+  static Estimate of(const RowMajorArgs& p, int mb, int cus) {
+    const Shape& t = kShapes[mb - 1];
+    const int rows = p.M1 * p.M0, cols = p.N1 * p.N0;
+    const double groups = (double)((rows + 16 * mb - 1) / (16 * mb)) * ((cols + 63) / 64);
+    const double result = (double)rows * cols * sizeof(typename Cfg::out_t) * 1e-6 * (p.out ? 2 : 1);
+    return {groups, std::ceil(p.K * (Cfg::kElemBytes / 64.0)),
+            (Cfg::kElemBytes == 4 ? t.step4 : Cfg::kElemBytes == 1 ? t.step1 : t.step2) / 8.0,
+            result * t.store + (p.accumulate ? t.add : 0.0), t, cus};
   }
-  double us(int cus, int side, int slices) const {
-    const double load = (double)tiles * slices / cus;
-    const double us = 4.3 + ceil_div(steps, (int64_t)slices) * step_us * (load > 1 ? load : 1) + bytes / 5.6e6;
-    return slices > 1 ? us + 1.3 + 4.0 * slices * tiles * side * side / 2.8e6 : us;
+  double us(int mb, int slices) const {
+    const double rounds = std::ceil(groups * slices / cus), stream = rounds * std::ceil(steps / slices) * step_us;
+    const double us = t.first + t.round * (rounds - 1) + (stream > t.hidden ? stream - t.hidden : 0.0) + other;
+    return slices > 1 ? us + t.split + t.plane * groups * slices * mb * 4096e-6 : us;
   }
-  // Below the time of every number of slices.
-  double least_us(int cus) const { return 4.3 + (double)steps * step_us * tiles / cus + bytes / 5.6e6; }
 };
 
-// What the chain takes, from below: 5 us a launch when they follow each other,
-// less 1, half a microsecond per MB of packed operands, and what the f32 matmul, which
-// has no K split for so few tiles, takes beyond its launch (f32 172x54x2690 38.8
-// us, estimated 37.4; bf16 1743x286x1222 25.3, 21.5; f16 54x163x733 17.0, 19.1).
-// The rule: the estimate with 10 % added is below it. f16 54x163x733 8.6 us here;
-// bf16 64x29x3693 21.2 as the chain, 35.0 here with K whole, 8.7 in 8 slices; f32
-// 20x589x4022 43.6, 56.0, 13.5; i8 1024^3 18.7 and 11.5. Beyond it the chain wins:
-// bf16 3421x599x980 24.4 as the chain, 36.7 here.
+// What the chain takes: its launches, the packed operands and the result, the
+// matrix instructions, and a share of K (fitted to the same problems, 11 % off on
+// average). The rule: the estimate of one launch is below 0.9 of it; on the other half
+// of the problems that is 1.1 % from the better of the two on average, and one call
+// slower by more than 5 % (f32 2458x1795x18 17.6 us as the chain, 19.3 here).
+// A chain that does not pack A (its matmul reads the matrix, so there are two
+// launches) was not among them; its estimate is from below.
 template <typename Cfg>
 double chain_us(const RowMajorArgs& p) {
   const int launches = (p.lhs != nullptr) + (p.rhs != nullptr) + 1 + (p.out ? 1 + p.accumulate : 0);
-  const double mb = 16e-6 * p.K1 * ((double)p.M1 * p.M0 + (double)p.N1 * p.N0);
-  const double f32 = Cfg::kElemBytes == 4 ? 4 + 0.004 * p.K : 0;
-  return 5.0 * launches - 1.0 + 0.5 * mb + (f32 < 13 ? f32 : 13);
+  const double rows = (double)p.M1 * p.M0, cols = (double)p.N1 * p.N0, bytes = (double)p.K * Cfg::kElemBytes;
+  if (!p.lhs) {
+    const double f32 = Cfg::kElemBytes == 4 ? 4 + 0.004 * p.K : 0;
+    return 5.0 * launches - 1.0 + 0.5e-6 * (rows + cols) * bytes + (f32 < 13 ? f32 : 13);
+  }
+  const double giga = Cfg::kElemBytes == 4 ? 16.1 : Cfg::kElemBytes == 1 ? 3.0 : 2.8;
+  return 3.17 + 2.40 * launches + 0.48e-6 * (rows + cols) * bytes + 0.62e-6 * rows * cols * sizeof(typename Cfg::out_t) +
+         giga * 1e-9 * rows * cols * p.K + 0.16e-3 * bytes;
 }
 
-// The fastest of both sides and 1 to max_slices slices of K; false when none takes
-// limit_us or less. (A large problem, which is the chain's, is seen by least_us:
-// the estimates of all slices took 0.5 us of every chain.)
+// The fastest of both shapes and 1 to max_slices slices of K; false when none takes
+// limit_us or less.
 template <typename Cfg>
-bool choose(const RowMajorArgs& p, int max_slices, double limit_us, int* side, int* slices) {
+bool choose(const RowMajorArgs& p, int max_slices, double limit_us, int* mb, int* slices) {
   const int cus = device_cu_count();
   bool found = false;
-  for (int try_side = 32; try_side <= 64; try_side += 32) {
-    const Estimate e = Estimate::of<Cfg>(p, try_side);
-    if (e.least_us(cus) > limit_us) continue;
-    for (int n = 1; n <= max_slices && n <= e.steps; ++n) {
-      const double us = e.us(cus, try_side, n);
-      if (found ? us < limit_us : us <= limit_us) { found = true; limit_us = us; *side = try_side; *slices = n; }
+  for (int rows = 1; rows <= 2; ++rows) {
+    const Estimate e = Estimate::of<Cfg>(p, rows, cus);
+    for (int n = 1; n <= max_slices && (n == 1 || n * 8 <= e.steps); n *= 2) {
+      const double us = e.us(rows, n);
+      if (us <= limit_us) { found = true; limit_us = us; *mb = rows; *slices = n; }
+      if (e.groups * n >= 4 * cus) break;
     }
   }
   return found;
@@ -430,41 +505,40 @@ bool choose(const RowMajorArgs& p, int max_slices, double limit_us, int* side, i
 
 template <typename Cfg>
 int launch(RowMajorArgs p, hipStream_t s) {
+  constexpr int kStep = 64 / Cfg::kElemBytes;                     // elements of K per step
   const int64_t rows = (int64_t)p.M1 * p.M0, cols = (int64_t)p.N1 * p.N0;
-  const double limit = chain_us<Cfg>(p) / 1.1;
-  int side = 32, slices = 1;
-  if (!choose<Cfg>(p, 16, limit, &side, &slices)) return IREE_AMD_UK_STATUS_NOT_FOUND;
-  const int64_t elem_step = 32768 / Cfg::kElemBytes;              // elements of K per step, times the side
+  const double limit = 0.9 * chain_us<Cfg>(p);
+  int mb = 1, slices = 1;
+  if (!choose<Cfg>(p, 16, limit, &mb, &slices)) return IREE_AMD_UK_STATUS_NOT_FOUND;
   auto lay_out = [&] {
-    p.tiles_n = (int)ceil_div(cols, (int64_t)side);
-    p.tiles = (int)(ceil_div(rows, (int64_t)side) * p.tiles_n);
-    const int64_t step = elem_step / side;
-    p.slice_k = (int)(ceil_div(ceil_div((int64_t)p.K, step), (int64_t)slices) * step);
+    p.tiles_n = (int)ceil_div(cols, (int64_t)64);
+    p.tiles = (int)(ceil_div(rows, (int64_t)mb * 16) * p.tiles_n);
+    p.slice_k = (int)ceil_div(ceil_div((int64_t)p.K, (int64_t)kStep), (int64_t)slices) * kStep;
     slices = (int)ceil_div((int64_t)p.K, (int64_t)p.slice_k);     // (no empty last slice)
   };
   lay_out();
   // (a graph keeps the addresses of its nodes: a call being captured takes no
   // memory that other calls on the stream use too)
   const bool may_split = slices > 1 && !scratch_under_capture(s);
-  ScratchLease lease(s, may_split ? (size_t)slices * p.tiles * side * side * 4 : 0);
+  ScratchLease lease(s, may_split ? (size_t)slices * p.tiles * mb * 4096 : 0);
   if (slices > 1 && !lease.ptr()) {
-    if (!choose<Cfg>(p, 1, limit, &side, &slices)) return IREE_AMD_UK_STATUS_NOT_FOUND;
+    if (!choose<Cfg>(p, 1, limit, &mb, &slices)) return IREE_AMD_UK_STATUS_NOT_FOUND;
     lay_out();
   }
-  const int64_t plane = (int64_t)p.tiles * side * side;
+  const int64_t plane = (int64_t)p.tiles * mb * 1024;
   p.slices = slices;
   p.partial = slices > 1 ? lease.ptr() : nullptr;
   p.product_blocks = p.tiles * slices;
-  p.lhs_blocks = p.lhs ? (int)ceil_div(rows * p.K1, (int64_t)256) : 0;
-  const int rhs_blocks = p.rhs ? (int)ceil_div(cols * p.K1, (int64_t)256) : 0;
-  const dim3 grid((unsigned)(p.product_blocks + p.lhs_blocks + rhs_blocks)), block(256);
-  if (side == 32) hipLaunchKernelGGL((matmul_rowmajor_kernel<Cfg, 32>), grid, block, 0, s, p);
-  else hipLaunchKernelGGL((matmul_rowmajor_kernel<Cfg, 64>), grid, block, 0, s, p);
+  p.lhs_blocks = p.lhs ? (int)ceil_div(rows * p.K1, (int64_t)kThreads) : 0;
+  const int rhs_blocks = p.rhs ? (int)ceil_div(cols * p.K1, (int64_t)kThreads) : 0;
+  const dim3 grid((unsigned)(p.product_blocks + p.lhs_blocks + rhs_blocks));
+  if (mb == 1) hipLaunchKernelGGL((matmul_rowmajor_kernel<Cfg, 1>), grid, dim3(kThreads), 0, s, p);
+  else hipLaunchKernelGGL((matmul_rowmajor_kernel<Cfg, 2>), grid, dim3(kThreads), 0, s, p);
   const int st = check_hip(hipGetLastError(), "matmul_rowmajor launch");
   if (st || slices == 1) return st;
-  const int padded_cols = p.tiles_n * side;
+  const int padded_cols = p.tiles_n * 64;
   hipLaunchKernelGGL(matmul_rowmajor_sum_kernel<typename Cfg::out_t>, dim3((unsigned)ceil_div(plane, (int64_t)256)),
-                     block, 0, s, p, (int)(plane / padded_cols), padded_cols);
+                     dim3(256), 0, s, p, (int)(plane / padded_cols), padded_cols);
   return check_hip(hipGetLastError(), "matmul_rowmajor sum launch");
 }
 

@@ -1602,3 +1602,29 @@ def test_short_k_whole_per_wave(uk, cuda, M0, N, batch, steps):
     am = a.transpose(1, 2).reshape(batch, M0, -1).float()
     bm = b.transpose(2, 3).reshape(batch, N * 32, -1).float().transpose(1, 2).contiguous()
     assert torch.equal(c, (am @ bm).reshape(batch, M0, N, 32).transpose(1, 2))
+
+
+@pytest.mark.parametrize("M,N,K", [(4, 4, 16), (17, 65, 33), (48, 67, 1056), (33, 129, 97), (16, 194, 2081)])
+@pytest.mark.parametrize("type_flag,dt,out_dt", [
+    (F.MMT4D_TYPE_BF16BF16F32, "bfloat16", "float32"), (F.MMT4D_TYPE_S8S8S32, "int8", "int32"),
+    (F.MMT4D_TYPE_F32F32F32, "float32", "float32"),
+])
+def test_small_matmul_columns_that_two_lanes_hold(uk, cuda, type_flag, dt, out_dt, M, N, K):
+    """N a little over whole 64s (and 4s): the last lane's four columns reach back into
+    those of the lane, or the workgroup, before it, which alone may add them to C; K a
+    little over whole steps and rounds of the waves."""
+    import torch
+    g = torch.Generator(device="cuda").manual_seed(M + N + K)
+    a = torch.randint(-3, 4, (M, K), generator=g, device="cuda").to(getattr(torch, dt))
+    b = torch.randint(-3, 4, (K, N), generator=g, device="cuda").to(getattr(torch, dt))
+    c0 = torch.randint(-99, 100, (M, N), generator=g, device="cuda").to(getattr(torch, out_dt))
+    want = a.double() @ b.double() + c0.double()
+    for tile in ("dynamic", None):
+        c = c0.clone()
+        ws = uk.matmul_data_tiled(a, b, c, M, N, K, type_flag, accumulate=True, tile=tile)
+        assert uk.last_kernel_path() == "mmt4d:mfma-one-launch"
+        assert torch.equal(c.double(), want)
+        M0, N0, K0 = uk.query_matmul_tile_sizes(uk.ukernel._MMT4D_TO_QUERY_OP[type_flag], *(() if tile else (M, N, K)))
+        out = torch.empty_like(ws["out"])
+        uk.pack(c, out, M, N, -(-M // M0), -(-N // N0), M0, N0, 0, uk.ukernel._OUT_PACK_TYPE[type_flag])
+        assert torch.equal(ws["out"], out)
