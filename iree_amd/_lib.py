@@ -5,6 +5,8 @@ The library must have been built (``python -m iree_amd.build`` or
 stale library raises.
 """
 import ctypes as C
+import importlib.machinery
+import importlib.util
 import os
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
@@ -213,6 +215,24 @@ def _declare(lib):
     lib.iree_amd_hal_executable_release.argtypes = [vp]
 
 
+def _bind_builtins(lib):
+    """Puts csrc/uk_python.so's builtins in the place of the ctypes functions that
+    they stand for (the same arguments, less time per call); the one of
+    query_matmul_tile_sizes, which returns the tile, is lib.matmul_tile."""
+    path = os.path.join(_HERE, "csrc", "uk_python.so")
+    if not os.path.exists(path):
+        raise RuntimeError(
+            f"{path} is missing: the extension has not been built "
+            "(run `python -m iree_amd.build`).")
+    loader = importlib.machinery.ExtensionFileLoader("uk_python", path)
+    module = importlib.util.module_from_spec(importlib.util.spec_from_loader("uk_python", loader))
+    loader.exec_module(module)
+    for name in module.names():
+        function = getattr(lib, name)
+        builtin = module.bind(name, C.cast(function, C.c_void_p).value, function)
+        setattr(lib, "matmul_tile" if name == "iree_amd_uk_query_matmul_tile_sizes" else name, builtin)
+
+
 def load_library():
     """Returns the loaded C-ABI library; raises if it has not been built."""
     global _lib
@@ -224,5 +244,6 @@ def load_library():
                 "(run `python -m iree_amd.build`). There is no CPU fallback.")
         lib = C.CDLL(path)
         _declare(lib)
+        _bind_builtins(lib)
         _lib = lib
     return _lib

@@ -1,5 +1,6 @@
-"""Builds the C-ABI library (iree_amd/csrc/libiree_amd_uk.so) and the code
-object of the mmt4d kernels for a HAL executable
+"""Builds the C-ABI library (iree_amd/csrc/libiree_amd_uk.so), its calls as
+builtins of this interpreter (iree_amd/csrc/uk_python.so) and the code object of
+the mmt4d kernels for a HAL executable
 (iree_amd/hal/mi355x_kernels_gfx950.co) for gfx950.
 
     python -m iree_amd.build            # incremental
@@ -16,7 +17,7 @@ CSRC = os.path.join(HERE, "csrc")
 
 
 def build(force=False, jobs=8, quiet=False):
-    cmd = ["make", "-C", CSRC, f"-j{jobs}"]
+    cmd = ["make", "-C", CSRC, f"-j{jobs}", f"PYTHON={sys.executable}"]
     if force:
         cmd.append("-B")
     out = subprocess.DEVNULL if quiet else None
@@ -26,6 +27,8 @@ def build(force=False, jobs=8, quiet=False):
         raise RuntimeError("build finished but libiree_amd_uk.so is missing")
     if not os.path.exists(os.path.join(HERE, "hal", "mi355x_kernels_gfx950.co")):
         raise RuntimeError("build finished but hal/mi355x_kernels_gfx950.co is missing")
+    if not os.path.exists(os.path.join(CSRC, "uk_python.so")):
+        raise RuntimeError("build finished but uk_python.so is missing")
     return lib
 
 

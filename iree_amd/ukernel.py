@@ -186,8 +186,12 @@ def query_matmul_tile_sizes(operation, M=_INT64_MIN, N=_INT64_MIN, K=_INT64_MIN)
     (``_INT64_MIN`` = dynamic): at most one of M0 and N0 is narrowed, the one of
     the smaller static size (the reference's chooseMatmulTile,
     CPUMaterializeEncodingPass.cpp:296-303)."""
+    lib = load_library()
+    tile = lib.matmul_tile(operation, M, N, K)
+    if tile is not None:
+        return tile
     out = MatmulTile()
-    _check(load_library().iree_amd_uk_query_matmul_tile_sizes(operation, M, N, K, C.byref(out)))
+    _check(lib.iree_amd_uk_query_matmul_tile_sizes(operation, M, N, K, C.byref(out)))
     return out.M, out.N, out.K
 
 

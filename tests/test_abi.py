@@ -389,3 +389,42 @@ def test_the_chain_looks_its_stream_up_once(monkeypatch, form, calls):
     # a stream object is taken as before
     ukernel.scale_f32(a, 1, 1.0, stream=types.SimpleNamespace(cuda_stream=42))
     assert seen[-1] == ("scale_f32", 42)
+
+
+@pytest.mark.parametrize("values", [
+    (16, 0, 8, None, -1, 1 << 63, 32, -(1 << 63), 5, 1, 2, 3, 4, -6, -7, 0x102, 0.3, 64),
+    (None, 1 << 40, (1 << 70) + 3, 16, 0, 8, (1 << 64) - 16, 7, 9, 2, 3, 4, 5, 6, (1 << 32) + 2, -1, float("-inf"), None),
+    (C.c_void_p(16), 0, True, 16, 0, 8, 32, 0, 8, C.c_int64(2), 3, 4, 5, 6, 7, 8, 1, C.c_void_p(64)),
+    (16, 0, 8, 16, 0, 8, 32, 0, 8, 2, 3, 4, 5, 6, 7, 8, C.c_float(2.5), 0),
+    (16, 0, 8.0, 16, 0, 8, 32, 0, 8, 2, 3, 4, 5, 6, 7, 8, 1.0, 0), (1, 2), (16,) * 19,
+], ids=["plain", "wide", "ctypes", "ctypes_float", "refused", "too_few", "too_many"])
+def test_builtins_pass_their_arguments_as_ctypes_does(values):
+    """The builtin of a C-ABI function with every kind of argument (pointer, 64- and
+    32-bit ints, float), over a recorder in its place: the same arguments arrive, or
+    the same error leaves, as with the ctypes function alone."""
+    import importlib.machinery
+    import importlib.util
+    path = os.path.join(ROOT, "iree_amd", "csrc", "uk_python.so")
+    loader = importlib.machinery.ExtensionFileLoader("uk_python", path)
+    module = importlib.util.module_from_spec(importlib.util.spec_from_loader("uk_python", loader))
+    loader.exec_module(module)
+    vp, i64, i32, u32 = C.c_void_p, C.c_int64, C.c_int32, C.c_uint32
+    types = [vp, i64, i64] * 3 + [i64] * 5 + [i32, u32, C.c_float, vp]
+    assert iree_amd.load_library().iree_amd_uk_mmt4d_unpack and len(types) == 18
+    seen = []
+
+    def record(*args):
+        seen.append(args)
+        return 11
+    function = C.CFUNCTYPE(C.c_int, *types)(record)
+    builtin = module.bind("iree_amd_uk_mmt4d_unpack", C.cast(function, vp).value, function)
+
+    def outcome(f):
+        try:
+            return f(*values)
+        except (TypeError, C.ArgumentError) as e:
+            return type(e), str(e)
+    assert outcome(function) == outcome(builtin)
+    assert len(seen) in (0, 2) and seen[:1] == seen[1:]
+    with pytest.raises(KeyError):
+        module.bind("iree_amd_uk_version", 16, function)
