@@ -34,7 +34,14 @@ __host__ __device__ inline FastDiv make_fastdiv(uint32_t d) {
 // one 128-bit store. Lanes of a wave take 64 consecutive matrix columns, so
 // every load instruction reads 64 consecutive elements of a row and the stores
 // of a wave are whole tiles (or whole rows of chunks of a tile); a wave walks
-// kTransUnroll consecutive row groups so that enough loads are in flight.
+// kTransUnroll consecutive row groups so that enough loads are in flight. What
+// bounds it is memory. A form with dword loads (4 / ES columns a lane, a quarter or
+// half of the load instructions) took the 1- and 2-byte elements of aligned rows
+// before and is slower: it leaves a quarter of the waves, and each of its stores
+// touches lines that it fills only over 4 instructions. Measured, that form -> this
+// one, i8: 8192 x 8192 in rotation 42.0 -> 30.6 us, 4096 x 14336 38.6 -> 26.5, 1024 x
+// 1024 5.5 -> 3.8, and where columns end inside a wave 3000 x 4100 18.1 -> 9.2, 3001 x
+// 300 14.2 -> 5.2; f16 2000 x 600 and 1024 x 1024 within 0.3 us of each other.
 //---------------------------------------------------------------------------
 constexpr int kTransUnroll = 4;
 
@@ -117,93 +124,11 @@ __device__ __forceinline__ void pack_transpose_body(const TransArgs& a) {
   }
 }
 
-// The same for 1- and 2-byte elements with dword loads: a thread takes W = 4 / ES
-// adjacent columns (one dword of every row) and builds W chunks, so that a
-// wave's load instruction reads 256 bytes of a row instead of 64 or 128. The
-// kernel above is bound by the rate at which a compute unit takes load
-// instructions (f16 4096 x 4096 into 32x8 tiles: 17.2 -> 15.8 us). Needs rows
-// that start on 4-byte boundaries and tiles of whole W columns (the host
-// checks); a wave covers 64 W columns.
-template <int ES>
-__device__ __forceinline__ void pack_transpose_wide_body(const TransArgs& a) {
-  static_assert(ES == 1 || ES == 2, "32-bit elements are dwords already");
-  constexpr int CE = 16 / ES, W = 4 / ES;
-  typedef typename Chunk<ES>::elem_t elem_t;
-  const uint32_t lane = threadIdx.x & 63;
-  const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  uint32_t bx, by;
-  {
-    constexpr uint32_t kXcds = 8;
-    const uint32_t total = a.blocks_x * a.blocks_y;
-    const uint32_t per = total / kXcds, rem = total % kXcds;
-    const uint32_t xcd = blockIdx.x % kXcds, idx = blockIdx.x / kXcds;
-    const uint32_t logical = xcd * per + (xcd < rem ? xcd : rem) + idx;
-    by = logical / a.blocks_x;
-    bx = logical - by * a.blocks_x;
-  }
-  const int64_t c = ((int64_t)bx * 64 + lane) * W;           // first of this thread's columns
-  const int64_t g0 = ((int64_t)by * 4 + wave) * kTransUnroll;  // first row group of this wave
-  if (g0 >= a.row_groups) return;
-  const bool col_in_tiles = c < a.padded_cols;   // (tiles are whole W columns: all of them or none)
-  const uint32_t cc = col_in_tiles ? (uint32_t)c : 0;
-  const uint32_t ocol = a.by_tile_cols.div(cc), d2 = cc - ocol * a.tile_cols;
-  char* out_col = a.tiled + (int64_t)ocol * a.t_stride_ocol_bytes + (int64_t)d2 * a.tile_rows * ES;
-  const uint32_t pad = (uint32_t)(elem_t)a.padding;
-  const bool interior = (int64_t)(bx + 1) * 64 * W <= a.m_size1 &&
-                        (g0 + kTransUnroll) * CE <= a.m_size0 && g0 + kTransUnroll <= a.row_groups;
-  uint32_t v[kTransUnroll][CE];     // the W elements of one row, first column in the low bits
-  if (interior) {
-    const char* src = a.mat + g0 * CE * a.m_pitch_bytes + c * ES;
-#pragma unroll
-    for (int u = 0; u < kTransUnroll; ++u)
-#pragma unroll
-      for (int i = 0; i < CE; ++i) v[u][i] = *(const uint32_t*)(src + (int64_t)(u * CE + i) * a.m_pitch_bytes);
-  } else {
-#pragma unroll
-    for (int u = 0; u < kTransUnroll; ++u)
-#pragma unroll
-      for (int i = 0; i < CE; ++i) {
-        const int64_t r = (g0 + u) * CE + i;
-        uint32_t d = 0;
-#pragma unroll
-        for (int w = 0; w < W; ++w) {
-          const uint32_t e = (r < a.m_size0 && c + w < a.m_size1)
-                                 ? (uint32_t)*(const elem_t*)(a.mat + r * a.m_pitch_bytes + (c + w) * ES) : pad;
-          d |= e << (8 * ES * w);
-        }
-        v[u][i] = d;
-      }
-  }
-  if (!col_in_tiles) return;
-#pragma unroll
-  for (int u = 0; u < kTransUnroll; ++u) {
-    const int64_t g = g0 + u;
-    if (g >= a.row_groups) break;
-    int64_t orow;
-    uint32_t grp;
-    if (g < 0x7FFFFFFF) {
-      orow = a.by_groups.div((uint32_t)g);
-      grp = (uint32_t)g - (uint32_t)orow * a.groups_per_tile;
-    } else {
-      orow = g / a.groups_per_tile;
-      grp = (uint32_t)(g - orow * a.groups_per_tile);
-    }
-    char* dst = out_col + orow * a.t_stride_orow_bytes + (int64_t)grp * 16;
-#pragma unroll
-    for (int w = 0; w < W; ++w) {
-      union { elem_t e[CE]; u32x4 vec; } chunk;
-#pragma unroll
-      for (int i = 0; i < CE; ++i) chunk.e[i] = (elem_t)(v[u][i] >> (8 * ES * w));
-      *(u32x4*)(dst + (int64_t)w * a.tile_rows * ES) = chunk.vec;
-    }
-  }
-}
-
 // 2-byte elements, whole rows of 16 bytes per lane: a wave covers 512 columns
 // of the 8 matrix rows of one row group with 8 load instructions of 1 KiB each
-// (the streaming pack's rate; the dword kernel above needs 32 for the same
-// bytes). A lane then holds an 8 x 8 block, transposes it in registers (one
-// byte permute per dword) into the 8 chunks of its 8 columns, and the wave
+// (the streaming pack's rate; the kernel above needs 64 for the same bytes). A
+// lane then holds an 8 x 8 block, transposes it in registers (one byte permute
+// per dword) into the 8 chunks of its 8 columns, and the wave
 // passes the chunks through its 8 KiB of LDS so that store instruction s takes
 // columns 64 s .. 64 s + 63, one per lane: 1 KiB of whole tiles per store where
 // the lane's own 8 chunks would be 64 pieces of 16 bytes 128 bytes apart. LDS
@@ -211,7 +136,7 @@ __device__ __forceinline__ void pack_transpose_wide_body(const TransArgs& a) {
 // writes (lanes 128 bytes apart) and the reads (8 lanes per 128 bytes, two
 // source lanes per 16) then touch every bank once per 16 lanes.
 // kLdsUnroll row groups per wave, all loaded before the first is stored (4:
-// 13.4 us for f16 4096 x 4096 into 32x8 tiles, 1: 14.3; the dword kernel 15.8).
+// 13.4 us for f16 4096 x 4096 into 32x8 tiles, 1: 14.3; the kernel above 17.0).
 template <int ES, int kLdsUnroll>
 __device__ __forceinline__ void pack_transpose_lds_body(const TransArgs& a) {
   static_assert(ES == 2, "2-byte elements");
