@@ -639,25 +639,26 @@ IREE_AMD_UK_EXPORT int iree_amd_uk_matmul_packed_rhs(
     iree_amd_uk_index_t N, iree_amd_uk_index_t K, int32_t K0, uint32_t flags,
     float out_scale, void* stream);
 
-/* The whole data-tiled matmul of a small problem as one launch or two: what
- * pack(A), pack(B, inner and outer transposed), [pack(C)], mmt4d and unpack do
+/* The whole data-tiled matmul: what pack(A), pack(B, inner and outer transposed),
+ * [pack(C)], mmt4d and unpack do (a small problem as one launch or two, another in full
+ * tiles as that chain with both operands packed by one launch)
  * (REF compiler/src/iree/compiler/Codegen/Common/CPU/CPULowerToUKernels.cpp:339-480).
  *   c[m][n] (+)= sum_k a[m][k] * b[k][n]
  * a is M x K, b K x N, c M x N, all row-major and tight, element types as in
  * `flags` (an IREE_AMD_UK_FLAG_MMT4D_TYPE_*, optionally ACCUMULATE). lhs, rhs and
  * out receive the packed operands and the packed result in tiles of M0 x K0,
  * N0 x K0 and M0 x N0, as the chain leaves them (the padding of the result's tiles
- * zeros, also where the chain multiplies padding by an infinity); a null one is not
- * written.
- * Integers have the chain's bits, and so have the packed operands; float sums come
- * in another order (a captured call's, whose K stays whole, in a third), with an
- * error no larger.
+ * of a small problem zeros, also where the chain multiplies padding by an infinity); a
+ * null one is not written.
+ * Integers have the chain's bits, and so have the packed operands; float sums of a
+ * small problem come in another order (a captured call's, whose K stays whole, in a
+ * third), with an error no larger.
  * Returns IREE_AMD_UK_STATUS_NOT_FOUND, with no error recorded and nothing
- * written, for what it does not serve (large problems, which the chain runs
- * faster; tiles without a matrix-core kernel; buffers that overlap): run the
- * chain then. A long K of few tiles is split over workgroups, whose partial sums
- * lie in the stream's scratch memory, and takes a second launch; while the
- * stream is being captured it is not. */
+ * written, for what it does not serve (a null lhs or rhs of a large problem; tiles
+ * without a matrix-core kernel; buffers that overlap): run the chain then. A long K
+ * of few tiles is split over workgroups, whose partial sums lie in the stream's
+ * scratch memory, and takes a second launch; while the stream is being captured it
+ * is not. */
 IREE_AMD_UK_EXPORT int iree_amd_uk_matmul_data_tiled(
     const void* a, const void* b, void* c, void* lhs, void* rhs, void* out, iree_amd_uk_index_t M,
     iree_amd_uk_index_t N, iree_amd_uk_index_t K, int32_t M0, int32_t N0, int32_t K0, uint32_t flags,

@@ -866,7 +866,9 @@ extern "C" int iree_amd_uk_matmul_data_tiled(
     iree_amd_uk_index_t N, iree_amd_uk_index_t K, int32_t M0, int32_t N0, int32_t K0, uint32_t flags,
     void* stream) {
   const int st = launch_matmul_rowmajor(a, b, c, lhs, rhs, out, M, N, K, M0, N0, K0, flags, (hipStream_t)stream);
-  if (st != IREE_AMD_UK_STATUS_NOT_FOUND) note_kernel_path("mmt4d:mfma-one-launch");
+  if (st == IREE_AMD_UK_STATUS_NOT_FOUND)
+    return launch_matmul_chain(a, b, c, lhs, rhs, out, M, N, K, M0, N0, K0, flags, (hipStream_t)stream);
+  note_kernel_path("mmt4d:mfma-one-launch");
   return st;
 }
 

@@ -112,6 +112,10 @@ int launch_matmul_packed_rhs_mfma(const iree_amd_uk_mmt4d_params_t& p, int64_t o
 // NOT_FOUND when the caller has to run the chain.
 int launch_matmul_rowmajor(const void* a, const void* b, void* c, void* lhs, void* rhs, void* out, int64_t M,
                            int64_t N, int64_t K, int M0, int N0, int K0, uint32_t flags, hipStream_t s);
+// The chain itself for full tiles, with both operands packed in one launch;
+// NOT_FOUND, with nothing launched, where the caller has to run it step by step.
+int launch_matmul_chain(const void* a, const void* b, void* c, void* lhs, void* rhs, void* out, int64_t M, int64_t N,
+                        int64_t K, int M0, int N0, int K0, uint32_t flags, hipStream_t s);
 int launch_mmt4d_silu_mul_mfma(const iree_amd_uk_mmt4d_params_t& p, float gate_scale,
                                float up_scale, float inv_out_scale, hipStream_t s);
 
@@ -216,6 +220,10 @@ int scratch_overflow_status(const char* what, size_t bytes);
 size_t scratch_release_idle();
 
 int launch_pack(const iree_amd_uk_pack_params_t& p, hipStream_t s);
+// Row-major a[M][K] and b[K][N] of es-byte elements into tiles of M0 x K0 and N0 x K0
+// (b transposed) in one launch; NOT_FOUND, with nothing launched, where two are right.
+int launch_pack_operands(const void* a, const void* b, void* lhs, void* rhs, int64_t M, int64_t N, int64_t K, int M0,
+                         int N0, int K0, int es, hipStream_t s);
 int launch_unpack(const iree_amd_uk_unpack_params_t& p, hipStream_t s);
 
 int launch_dequant_matmul_i4(const void* x, const void* w, const void* scale,

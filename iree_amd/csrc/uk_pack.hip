@@ -255,16 +255,22 @@ bool pow2_eligible(const StreamArgs& a, int es) {
   return true;
 }
 
-template <int ES, bool kPack>
-int launch_stream_pow2(const StreamArgs& a, hipStream_t s) {
+Pow2Args pow2_args(const StreamArgs& a, int es) {
   Pow2Args p;
   p.mat = a.mat; p.tiled = a.tiled;
-  p.m_size0 = a.m_size0; p.m_size1 = a.m_size1; p.m_pitch_bytes = a.m_stride0 * ES;
+  p.m_size0 = a.m_size0; p.m_size1 = a.m_size1; p.m_pitch_bytes = a.m_stride0 * es;
   p.t_stride_row_bytes = a.t_stride_row_bytes; p.t_stride_col_bytes = a.t_stride_col_bytes;
   p.padded_rows = a.padded_rows;
   p.chunks_per_row = a.chunks_per_row; p.padded_chunks_per_row = a.padded_chunks_per_row;
   p.log2_tile_rows = a.log2_tile_rows; p.log2_cpr = a.log2_cpr;
   p.padding = a.padding;
+  p.blocks_x = p.blocks_y = 0;
+  return p;
+}
+
+template <int ES, bool kPack>
+int launch_stream_pow2(const StreamArgs& a, hipStream_t s) {
+  Pow2Args p = pow2_args(a, ES);
   const int64_t cols = kPack ? a.padded_chunks_per_row : a.chunks_per_row;
   const int64_t rows = kPack ? a.padded_rows : a.m_size0;
   // Tiles whose rows are a single chunk (f16 32x8, i8 32x16, f32 32x4: the
@@ -331,6 +337,26 @@ int launch_unpack_transpose(TransArgs a, hipStream_t s) {
   a.blocks_x = (uint32_t)bx; a.blocks_y = (uint32_t)by;
   hipLaunchKernelGGL((unpack_transpose_kernel<ES>), dim3((unsigned)(bx * by)), dim3(256), 0, s, a);
   return check_hip(hipGetLastError(), "unpack_transpose launch");
+}
+
+// Rows and columns are the matrix's; ce: elements of a chunk.
+TransArgs trans_args(const char* mat, char* tiled, int64_t size0, int64_t size1, int64_t pitch_bytes, int64_t outer_rows,
+                     int64_t outer_cols, int tile_rows, int tile_cols, int64_t stride_orow_bytes,
+                     int64_t stride_ocol_bytes, uint64_t padding, int ce) {
+  TransArgs a;
+  a.mat = mat; a.tiled = tiled;
+  a.m_size0 = size0; a.m_size1 = size1; a.m_pitch_bytes = pitch_bytes;
+  a.tile_rows = tile_rows; a.tile_cols = tile_cols;
+  a.groups_per_tile = tile_rows / ce;
+  a.row_groups = outer_rows * a.groups_per_tile;
+  a.padded_cols = outer_cols * tile_cols;
+  a.t_stride_orow_bytes = stride_orow_bytes;
+  a.t_stride_ocol_bytes = stride_ocol_bytes;
+  a.by_tile_cols = make_fastdiv((uint32_t)tile_cols);
+  a.by_groups = make_fastdiv((uint32_t)a.groups_per_tile);
+  a.padding = padding;
+  a.blocks_x = a.blocks_y = 0;
+  return a;
 }
 
 template <int ES>
@@ -476,7 +502,55 @@ int launch_generic(K kernel, const PackArgs& a, int64_t total, hipStream_t s, co
   return check_hip(hipGetLastError(), what);
 }
 
+// Both operands of a matmul in one launch: workgroups 0 .. lhs_blocks - 1 the
+// streaming pack of A, the rest the transposing pack of B. Each pass is short beside
+// a launch and its drain (A of the 1999 x 4099 x 3001 bf16 matmul 7.6 us, B 11.5 for
+// 24 and 49 MB).
+template <int ES>
+__global__ __launch_bounds__(256) void pack_operands_kernel(Pow2Args lhs, uint32_t lhs_blocks, TransArgs rhs) {
+  if (blockIdx.x < lhs_blocks) stream_pow2_body<ES, true, true, true, 8, 1, 1, 4>(lhs, blockIdx.x);
+  else pack_transpose_body<ES>(rhs, blockIdx.x - lhs_blocks);
+}
+
+template <int ES>
+int launch_operands(Pow2Args lhs, TransArgs rhs, hipStream_t s) {
+  const int64_t lx = ceil_div((int64_t)lhs.padded_chunks_per_row, (int64_t)8), ly = ceil_div(lhs.padded_rows, (int64_t)32);
+  const int64_t rx = ceil_div(rhs.padded_cols, (int64_t)64), ry = ceil_div(rhs.row_groups, (int64_t)(4 * kTransUnroll));
+  if (lx * ly + rx * ry > 0x7FFFFFFF) return IREE_AMD_UK_STATUS_NOT_FOUND;
+  lhs.blocks_x = (uint32_t)lx; lhs.blocks_y = (uint32_t)ly;
+  rhs.blocks_x = (uint32_t)rx; rhs.blocks_y = (uint32_t)ry;
+  hipLaunchKernelGGL((pack_operands_kernel<ES>), dim3((unsigned)(lx * ly + rx * ry)), dim3(256), 0, s, lhs,
+                     (uint32_t)(lx * ly), rhs);
+  return check_hip(hipGetLastError(), "pack_operands launch");
+}
+
 }  // namespace
+
+int launch_pack_operands(const void* a, const void* b, void* lhs, void* rhs, int64_t M, int64_t N, int64_t K, int M0,
+                         int N0, int K0, int es, hipStream_t s) {
+  const int ce = 16 / es;
+  if (K0 != ce || M0 < 8 || N0 < 1 || (uintptr_t)a % es || (uintptr_t)b % es || (uintptr_t)lhs % 16 || (uintptr_t)rhs % 16 ||
+      M < 1 || N < 1 || K < 1 || M >= 1 << 30 || N >= 1 << 30 || K >= 1 << 30)
+    return IREE_AMD_UK_STATUS_NOT_FOUND;
+  const int64_t M1 = ceil_div(M, (int64_t)M0), N1 = ceil_div(N, (int64_t)N0), K1 = ceil_div(K, (int64_t)K0);
+  // (rows 8 KiB apart and multiples of it: 2-byte elements read column by column then
+  // meet in few memory channels, 17.0 us for f16 4096 x 4096, where the kernel that
+  // exchanges them through LDS takes 13.6; other pitches are equal or slower there)
+  if (es == 2 && N * es % 8192 == 0) return IREE_AMD_UK_STATUS_NOT_FOUND;
+  StreamArgs sa;
+  sa.mat = (const char*)a; sa.tiled = (char*)lhs;
+  sa.m_size0 = M; sa.m_size1 = K; sa.m_stride0 = K;
+  sa.outer_rows = M1; sa.outer_cols = K1;
+  sa.t_stride_row = K1 * M0 * K0; sa.t_stride_col = (int64_t)M0 * K0;
+  sa.tile_rows = M0; sa.tile_cols = K0; sa.padding = 0;
+  fill_stream_geometry(&sa, es);
+  if (!stream_eligible(es, 1, 0, M0, K0, K1, K, lhs, sa.t_stride_row, sa.t_stride_col) || !pow2_eligible(sa, es))
+    return IREE_AMD_UK_STATUS_NOT_FOUND;
+  const TransArgs ta = trans_args((const char*)b, (char*)rhs, K, N, N * es, K1, N1, K0, N0, (int64_t)N0 * 16,
+                                  K1 * N0 * 16, 0, ce);
+  const Pow2Args pa = pow2_args(sa, es);
+  return es == 1 ? launch_operands<1>(pa, ta, s) : es == 2 ? launch_operands<2>(pa, ta, s) : launch_operands<4>(pa, ta, s);
+}
 
 int launch_pack(const iree_amd_uk_pack_params_t& p, hipStream_t s) {
   const int es = pack_elem_bytes(p.flags);
@@ -514,21 +588,10 @@ int launch_pack(const iree_amd_uk_pack_params_t& p, hipStream_t s) {
   if (ti && p.in_stride1 == 1 && p.out_size3 > 0 && p.out_size3 % ce == 0 && p.out_size2 > 0 &&
       ((uintptr_t)out % 16) == 0 && (p.out_stride0 * es) % 16 == 0 && (tile_elems * es) % 16 == 0 &&
       p.in_size1 < (1ll << 31) && (to ? p.out_size0 : p.out_size1) * p.out_size2 < (1ll << 31)) {
-    TransArgs a;
-    a.mat = in; a.tiled = out;
-    a.m_size0 = p.in_size0; a.m_size1 = p.in_size1; a.m_pitch_bytes = p.in_stride0 * es;
-    a.tile_rows = (int)p.out_size3; a.tile_cols = (int)p.out_size2;
-    a.groups_per_tile = a.tile_rows / ce;
-    const int64_t outer_rows = to ? p.out_size1 : p.out_size0;
-    const int64_t outer_cols = to ? p.out_size0 : p.out_size1;
-    a.row_groups = outer_rows * a.groups_per_tile;
-    a.padded_cols = outer_cols * a.tile_cols;
-    a.t_stride_orow_bytes = (to ? tile_elems : p.out_stride0) * es;
-    a.t_stride_ocol_bytes = (to ? p.out_stride0 : tile_elems) * es;
-    a.by_tile_cols = make_fastdiv((uint32_t)a.tile_cols);
-    a.by_groups = make_fastdiv((uint32_t)a.groups_per_tile);
-    a.padding = p.padding_value;
-    a.blocks_x = a.blocks_y = 0;
+    const TransArgs a = trans_args(in, out, p.in_size0, p.in_size1, p.in_stride0 * es, to ? p.out_size1 : p.out_size0,
+                                   to ? p.out_size0 : p.out_size1, (int)p.out_size3, (int)p.out_size2,
+                                   (to ? tile_elems : p.out_stride0) * es, (to ? p.out_stride0 : tile_elems) * es,
+                                   p.padding_value, ce);
     int st = es == 1 ? launch_pack_transpose<1>(a, s)
            : es == 2 ? launch_pack_transpose<2>(a, s)
                      : launch_pack_transpose<4>(a, s);

@@ -138,7 +138,7 @@ struct Pow2Args {
 // workgroups.
 template <int ES, bool kPack, bool kNtLoad = true, bool kNtStore = kPack, int kBlockRows = kPow2Rows,
           int kStreamUnroll = kPow2Unroll, int kWX = kPow2WavesX, int kWaves = kPow2Waves>
-__device__ __forceinline__ void stream_pow2_body(const Pow2Args a) {
+__device__ __forceinline__ void stream_pow2_body(const Pow2Args a, const uint32_t block = blockIdx.x) {
   constexpr int CE = 16 / ES;
   constexpr int kBlockChunks = 64 / kBlockRows;
   constexpr int kRows = kBlockRows * kStreamUnroll;
@@ -153,7 +153,7 @@ __device__ __forceinline__ void stream_pow2_body(const Pow2Args a) {
     constexpr uint32_t kXcds = 8;
     const uint32_t total = a.blocks_x * a.blocks_y;
     const uint32_t per = total / kXcds, rem = total % kXcds;
-    const uint32_t xcd = blockIdx.x % kXcds, idx = blockIdx.x / kXcds;
+    const uint32_t xcd = block % kXcds, idx = block / kXcds;
     const uint32_t logical = xcd * per + (xcd < rem ? xcd : rem) + idx;
     by = logical / a.blocks_x;
     bx = logical - by * a.blocks_x;

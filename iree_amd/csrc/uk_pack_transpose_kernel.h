@@ -60,7 +60,7 @@ struct TransArgs {
 };
 
 template <int ES>
-__device__ __forceinline__ void pack_transpose_body(const TransArgs& a) {
+__device__ __forceinline__ void pack_transpose_body(const TransArgs& a, const uint32_t block = blockIdx.x) {
   constexpr int CE = 16 / ES;
   typedef typename Chunk<ES>::elem_t elem_t;
   const uint32_t lane = threadIdx.x & 63;
@@ -71,7 +71,7 @@ __device__ __forceinline__ void pack_transpose_body(const TransArgs& a) {
     constexpr uint32_t kXcds = 8;
     const uint32_t total = a.blocks_x * a.blocks_y;
     const uint32_t per = total / kXcds, rem = total % kXcds;
-    const uint32_t xcd = blockIdx.x % kXcds, idx = blockIdx.x / kXcds;
+    const uint32_t xcd = block % kXcds, idx = block / kXcds;
     const uint32_t logical = xcd * per + (xcd < rem ? xcd : rem) + idx;
     by = logical / a.blocks_x;
     bx = logical - by * a.blocks_x;

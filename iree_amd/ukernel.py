@@ -426,7 +426,8 @@ def matmul_data_tiled(a, b, c, M, N, K, mmt4d_type, *, accumulate=False,
                       one_launch=True):
     """Row-major C[M][N] (+)= A[M][K] * B[K][N] through pack -> mmt4d -> unpack,
     or for a small problem as one launch that leaves the same in every buffer
-    (float sums in another order); ``one_launch=False`` always runs the chain.
+    (float sums in another order); ``one_launch=False`` always runs the chain,
+    one call for each step.
     With ``fuse_unpack`` the last two (and the pack of C when accumulating) are
     the one kernel ``mmt4d_unpack``; it needs a tile with a matrix-core kernel.
     With ``fuse_pack_lhs`` the matmul also reads A row-major itself
@@ -463,8 +464,9 @@ def matmul_data_tiled(a, b, c, M, N, K, mmt4d_type, *, accumulate=False,
     stream = _stream(None)
     if one_launch and not (fuse_unpack and (M0, N0) != (32, 32)) and \
             not (fuse_pack_lhs and (K % _ROW_MAJOR_STEP[mmt4d_type] or _ptr(a) % 16)):
-        # (a small problem: all of it as one launch; what the chain's matmul on a
-        # row-major left-hand side may refuse is left to it, whatever the size)
+        # (a small problem: all of it as one launch; another in full tiles: the chain with
+        # both packs in one launch; what the chain's matmul on a row-major left-hand side
+        # may refuse is left to it, whatever the size)
         status = load_library().iree_amd_uk_matmul_data_tiled(
             _ptr(a), _ptr(b), _ptr(c), None if fuse_pack_lhs else _ptr(ws["lhs"]), _ptr(ws["rhs"]),
             None if fuse_unpack else _ptr(ws["out"]), M, N, K, M0, N0, K0,

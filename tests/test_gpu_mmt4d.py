@@ -1628,3 +1628,28 @@ def test_small_matmul_columns_that_two_lanes_hold(uk, cuda, type_flag, dt, out_d
         out = torch.empty_like(ws["out"])
         uk.pack(c, out, M, N, -(-M // M0), -(-N // N0), M0, N0, 0, uk.ukernel._OUT_PACK_TYPE[type_flag])
         assert torch.equal(ws["out"], out)
+
+
+@pytest.mark.parametrize("type_flag,dt,out_dt,M,N,K", [
+    (F.MMT4D_TYPE_S8S8S32, "int8", "int32", 1500, 1501, 1502),
+    (F.MMT4D_TYPE_S8S8S32, "int8", "int32", 2017, 2049, 1537),
+    (F.MMT4D_TYPE_F16F16F32, "float16", "float32", 2049, 1537, 1031),
+    (F.MMT4D_TYPE_F16F16F32, "float16", "float32", 1025, 4096, 2048),   # (B through LDS: two packs)
+    (F.MMT4D_TYPE_BF16BF16BF16, "bfloat16", "bfloat16", 1999, 2053, 1777),
+    (F.MMT4D_TYPE_F32F32F32, "float32", "float32", 2001, 1733, 1030),
+], ids=lambda v: str(v))
+def test_chain_with_both_operands_packed_together(uk, cuda, type_flag, dt, out_dt, M, N, K):
+    """Sizes beyond the small problems' kernel, with ragged last tiles, columns and rows of
+    K: every buffer has the bits that the chain run step by step leaves."""
+    import torch
+    g = torch.Generator(device="cuda").manual_seed(M + N + K)
+    a = torch.randint(-5, 6, (M * K,), generator=g, device="cuda").to(getattr(torch, dt))
+    b = torch.randint(-5, 6, (K * N,), generator=g, device="cuda").to(getattr(torch, dt))
+    c0 = torch.randint(-99, 100, (M * N,), generator=g, device="cuda").to(getattr(torch, out_dt))
+    for kw in ({}, {"accumulate": True}, {"fuse_unpack": True}, {"fuse_unpack": True, "accumulate": True}):
+        c, step = c0.clone(), c0.clone()
+        ws = uk.matmul_data_tiled(a, b, c, M, N, K, type_flag, **kw)
+        assert uk.last_kernel_path() == "mmt4d:mfma", kw
+        chain = uk.matmul_data_tiled(a, b, step, M, N, K, type_flag, one_launch=False, **kw)
+        assert torch.equal(c, step), kw
+        assert ws.keys() == chain.keys() and all(torch.equal(ws[k], chain[k]) for k in ws), kw
