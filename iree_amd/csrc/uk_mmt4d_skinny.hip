@@ -89,6 +89,7 @@ struct SkinnyArgs {
   int64_t lhs_row_pitch_bytes;
   int64_t out_row_pitch_elems;
   int out_cols;
+  float out_scale;   // of that matrix (float results)
   // per-wave form with batch planes: plane z starts rot_tiles * z outer columns on
   int rot_tiles;
 };
@@ -383,7 +384,8 @@ __global__ __launch_bounds__(kThreads) void mmt4d_skinny_kernel(SkinnyArgs a) {
         if (rows_out && j * 32 + nn >= a.out_cols) continue;
         const int v = ((nn >> 3) << 2) | (nn & 3), l = mm + 32 * ((nn >> 2) & 1);
         const int64_t at = rows_out ? mm * a.out_row_pitch_elems + nn : e;
-        const sum_t sum = (a.accumulate ? (sum_t)tile[at] : (sum_t)0) + mine[v][l];
+        sum_t sum = (a.accumulate ? (sum_t)tile[at] : (sum_t)0) + mine[v][l];
+        if constexpr (rows_out && std::is_floating_point<sum_t>::value) sum *= a.out_scale;
         tile[at] = (store_t)sum;
       }
       __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
@@ -412,6 +414,7 @@ __global__ __launch_bounds__(kThreads) void mmt4d_skinny_kernel(SkinnyArgs a) {
         sum_t sum = a.accumulate ? (sum_t)tile[at] : (sum_t)0;
 #pragma unroll
         for (int w = 0; w < kWaves; ++w) sum += buf[w][v][l];
+        if constexpr (rows_out && std::is_floating_point<sum_t>::value) sum *= a.out_scale;
         tile[at] = (store_t)sum;
       }
     }
@@ -850,6 +853,7 @@ int launch_chunk(const iree_amd_uk_mmt4d_params_t& p, int chunks, int chunk_step
   a.chunk_out_elems = 0;
   a.lhs_row_pitch_bytes = 0;
   a.out_row_pitch_elems = 0;
+  a.out_scale = 1.0f;
   a.out_cols = 0;
   a.batch = 1;
   a.lhs_batch_bytes = a.rhs_batch_bytes = a.out_batch_bytes = 0;
@@ -884,12 +888,13 @@ int launch_chunk(const iree_amd_uk_mmt4d_params_t& p, int chunks, int chunk_step
 // The whole linear layer on a few rows: out[M][out_cols] (+)= lhs[M][K] * rhs,
 // lhs and out row-major (`p` describes them as iree_amd_uk_matmul_packed_rhs
 // does: lhs_stride0 and out_stride0 are row pitches in elements), rhs packed
-// 32 x K0 tiles, 1 < M <= 32. One launch of the kernel above with the rows of
+// 32 x K0 tiles, 1 <= M <= 32, float results times out_scale. One launch of the kernel above with the rows of
 // the matrix as the rows of its single narrow tile; NOT_FOUND for what that
 // launch cannot take (a K that one launch row cannot hold in registers, too
-// few outer columns to be worth it, operands that are not 16-byte aligned).
-int launch_matmul_rows_skinny(const iree_amd_uk_mmt4d_params_t& p, int64_t M, int64_t out_cols, hipStream_t s) {
-  if (M < 2 || M > 32 || !mmt4d_skinny_supported(p.flags, 16, 32, p.K0)) return IREE_AMD_UK_STATUS_NOT_FOUND;
+// few outer columns to be worth it, a scale and K split over workgroups, operands that are not 16-byte aligned).
+int launch_matmul_rows_skinny(const iree_amd_uk_mmt4d_params_t& p, int64_t M, int64_t out_cols, float out_scale,
+                              hipStream_t s) {
+  if (M < 1 || M > 32 || !mmt4d_skinny_supported(p.flags, 16, 32, p.K0)) return IREE_AMD_UK_STATUS_NOT_FOUND;
   const int mk = mfma_k_of(p.flags);
   Mmt4dTypeInfo ti;
   mmt4d_type_info(p.flags, &ti);
@@ -918,7 +923,7 @@ int launch_matmul_rows_skinny(const iree_amd_uk_mmt4d_params_t& p, int64_t M, in
     if (chunks < 1) chunks = 1;
   }
   if (!few && p.N * 2 <= cus && chunks < 2) return IREE_AMD_UK_STATUS_NOT_FOUND;
-  if (chunks > 1 && (p.out_stride0 != out_cols || (M * out_cols) % 4)) return IREE_AMD_UK_STATUS_NOT_FOUND;
+  if (chunks > 1 && (p.out_stride0 != out_cols || (M * out_cols) % 4 || out_scale != 1.0f)) return IREE_AMD_UK_STATUS_NOT_FOUND;
   const char* lhs = (const char*)p.lhs_buffer + p.lhs_offset * eb;
   const char* rhs = (const char*)p.rhs_buffer + p.rhs_offset * eb;
   if (((uintptr_t)lhs | (uintptr_t)rhs) % 16 || (p.rhs_stride0 * eb) % 16 || (p.lhs_stride0 * eb) % 16)
@@ -936,7 +941,7 @@ int launch_matmul_rows_skinny(const iree_amd_uk_mmt4d_params_t& p, int64_t M, in
     w.out_outer = 32 * p.out_stride0; w.out_row = p.out_stride0; w.out_tile = 32; w.out_col = 1;
     w.accumulate = (p.flags & IREE_AMD_UK_FLAG_MMT4D_ACCUMULATE) != 0;
     w.batch = 1;
-    w.out_scale = 1.0f;
+    w.out_scale = out_scale;
     const uint32_t type = p.flags & IREE_AMD_UK_FLAG_MMT4D_TYPE_MASK;
     const WaveSplitChoice c = choose_wave_split(w, type);
     if (c.tile >= 0) return launch_mmt4d_wave_split(w, type, c.tile, s);
@@ -959,6 +964,7 @@ int launch_matmul_rows_skinny(const iree_amd_uk_mmt4d_params_t& p, int64_t M, in
   a.chunk_out_elems = 0;
   a.lhs_row_pitch_bytes = p.lhs_stride0 * eb;
   a.out_row_pitch_elems = p.out_stride0;
+  a.out_scale = out_scale;
   a.out_cols = (int)out_cols;
   a.batch = 1;
   a.lhs_batch_bytes = a.rhs_batch_bytes = a.out_batch_bytes = 0;

@@ -1653,3 +1653,32 @@ def test_chain_with_both_operands_packed_together(uk, cuda, type_flag, dt, out_d
         chain = uk.matmul_data_tiled(a, b, step, M, N, K, type_flag, one_launch=False, **kw)
         assert torch.equal(c, step), kw
         assert ws.keys() == chain.keys() and all(torch.equal(ws[k], chain[k]) for k in ws), kw
+
+
+@pytest.mark.parametrize("M", [1, 2, 24, 32])
+@pytest.mark.parametrize("type_flag,dt,K0", [(F.MMT4D_TYPE_F8E4M3F8E4M3F32, "uint8", 16),
+                                             (F.MMT4D_TYPE_F16F16F32, "float16", 8)], ids=["fp8", "f16"])
+@pytest.mark.parametrize("N,K", [(8219, 1024), (14315, 4096), (1003, 2048), (4111, 2048)])
+def test_few_rows_with_a_scaled_result(uk, cuda, type_flag, dt, K0, N, K, M):
+    """A few rows whose result is scaled, N inside a tile: the narrow kernels (more columns
+    than they need, and fewer, with K over the waves) give the unscaled call's sums
+    times the scale, in f32: the same bits."""
+    import torch
+    g = torch.Generator(device="cuda").manual_seed(M + N + K)
+    tiles = -(-N // 32) * 32
+
+    def values(n):
+        v = torch.randint(-4, 5, (n,), generator=g, device="cuda").float()
+        return v.to(torch.float8_e4m3fn).view(torch.uint8) if dt == "uint8" else v.half()
+    x, w = values(M * K), values(tiles * K)
+    plain, scaled = torch.full((M * N + 64,), 7.0, device="cuda"), torch.full((M * N + 64,), 7.0, device="cuda")
+    uk.matmul_packed_rhs(x, w, plain, M, N, K, K0, type_flag)
+    if M <= 24 or dt == "uint8":
+        assert uk.last_kernel_path() == "mmt4d:mfma-narrow"
+    uk.matmul_packed_rhs(x, w, scaled, M, N, K, K0, type_flag, out_scale=0.37)
+    decode = (lambda t: t.view(torch.float8_e4m3fn).double()) if dt == "uint8" else (lambda t: t.double())
+    rhs = decode(w).view(-1, K // K0, 32, K0).permute(0, 2, 1, 3).reshape(tiles, K)[:N]
+    want = decode(x).view(M, K) @ rhs.T
+    assert torch.equal(plain[:M * N].view(M, N).double(), want)                 # (whole numbers: exact in f32)
+    assert torch.equal(scaled[:M * N], plain[:M * N] * torch.tensor(0.37, device="cuda"))
+    assert (plain[M * N:] == 7.0).all() and (scaled[M * N:] == 7.0).all()
