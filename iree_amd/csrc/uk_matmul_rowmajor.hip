@@ -105,6 +105,20 @@ __device__ __forceinline__ u32x4 settle_chunk(u32x4 v, int k, int K, bool row_ex
 template <int kElemBytes>
 struct Four { uint32_t d[kElemBytes]; };
 
+// (of the matrix on tiles of 64 x 64: what lies past its ends, zeros)
+template <int kElemBytes>
+__device__ __forceinline__ Four<kElemBytes> settle_four(Four<kElemBytes> r, int n, int N, bool row_exists) {
+  if (!row_exists || n >= N) return Four<kElemBytes>{};
+  if (n + 4 <= N) return r;
+  u32x4 v = {0, 0, 0, 0};
+#pragma unroll
+  for (int i = 0; i < kElemBytes; ++i) v[i] = r.d[i];
+  v = shift_down(v, (n + 4 - N) * kElemBytes);
+#pragma unroll
+  for (int i = 0; i < kElemBytes; ++i) r.d[i] = v[i];
+  return r;
+}
+
 // The piece of column e from the 16 / kElemBytes rows of a strip of 4 columns.
 template <int kElemBytes>
 __device__ __forceinline__ u32x4 column_chunk(const Four<kElemBytes>* rows, int e) {
@@ -128,13 +142,13 @@ __device__ __forceinline__ u32x4 column_chunk(const Four<kElemBytes>* rows, int 
   return v;
 }
 
-// One workgroup's 512 chunks of a packed operand. Chunk r of the buffer is row
+// One workgroup's kBlock chunks of a packed operand. Chunk r of the buffer is row
 // i0 of the tile (i1, k1).
-template <int kElemBytes>
+template <int kElemBytes, int kBlock = kThreads>
 __device__ void pack_block(const RowMajorArgs& p, int block) {
   constexpr int E = 16 / kElemBytes;
   const bool is_lhs = block < p.lhs_blocks;
-  const uint32_t r = (uint32_t)(is_lhs ? block : block - p.lhs_blocks) * kThreads + threadIdx.x;
+  const uint32_t r = (uint32_t)(is_lhs ? block : block - p.lhs_blocks) * kBlock + threadIdx.x;
   const uint32_t T0 = is_lhs ? p.M0 : p.N0, K1 = p.K1;
   if (r >= T0 * K1 * (uint32_t)(is_lhs ? p.M1 : p.N1)) return;
   const uint32_t tile = r / T0, i0 = r - tile * T0;
@@ -433,6 +447,149 @@ __global__ __launch_bounds__(kThreads, 4) void matmul_rowmajor_kernel(RowMajorAr
   multiply_tile<Cfg, MB>(p);
 }
 
+// The same on 64 x 64 of the result per workgroup: 4 waves, each a 32 x 32 quarter of it
+// for all of K, which comes in steps of 512 bytes through LDS (64 KiB of both operands;
+// chunk c of row r lies at c ^ hash(r) within 16, so that fragment reads, 16 rows of one
+// chunk, and the turned stores hit 16 bank groups). The kernel above sums its 8 waves
+// through LDS whatever K is; where K is a step or two and the result large, that is
+// most of its time. Which of them: square_is_faster.
+template <typename Cfg>
+__global__ __launch_bounds__(256, 2) void matmul_rowmajor_square_kernel(RowMajorArgs p) {
+  constexpr int kRows = 64;
+  constexpr int kElemBytes = Cfg::kElemBytes;
+  constexpr int E = 16 / kElemBytes;            // elements of a chunk
+  constexpr int kChunks = 2048 / kRows;         // chunks of a row per step
+  constexpr int kStep = kChunks * E;            // elements of K per step
+  constexpr int kGroups = kRows / 4;            // four-column strips of the right-hand side
+  typedef typename Cfg::frag_t frag_t;
+  typedef typename Cfg::acc_t acc_t;
+  typedef typename Cfg::out_t out_t;
+  __shared__ u32x4 tile_a[2048], tile_b[2048];
+  if ((int)blockIdx.x >= p.product_blocks) {
+    pack_block<kElemBytes, 256>(p, (int)blockIdx.x - p.product_blocks);
+    return;
+  }
+  const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
+  const int tile = (int)blockIdx.x;
+  const int m_base = tile / p.tiles_n * kRows, n_base = tile % p.tiles_n * kRows;
+  auto place = [](int row, int chunk) { return row * kChunks + (chunk ^ ((row + (row >> 4)) & 15)); };
+
+  // what this thread fetches of a step: chunk t % kChunks of 8 rows of A, and
+  // two strips of 4 columns x E rows of B
+  u32x4 next_a[8];
+  Four<kElemBytes> next_b[2][E];
+  const int my_row = m_base + t / kChunks, my_n = n_base + t % kGroups * 4;
+  uint32_t row_at[8];                           // element offsets, 32 bits (operands of up to 64 MiB)
+#pragma unroll
+  for (int j = 0; j < 8; ++j) {
+    const int row = my_row + j * (kRows / 8);
+    row_at[j] = (uint32_t)(row < p.M ? row : p.M - 1) * p.K;
+  }
+  const uint32_t col_at = my_n + 4 <= p.N ? my_n : p.N - 4, last_row = (uint32_t)(p.K - 1) * p.N;
+  auto fetch = [&](int k_base) {
+    const int ka = k_base + t % kChunks * E;
+    const uint32_t at = ka + E <= p.K ? ka : p.K - E;
+#pragma unroll
+    for (int j = 0; j < 8; ++j) __builtin_memcpy(&next_a[j], p.a + (row_at[j] + at) * kElemBytes, 16);
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+      const uint32_t k_row = (uint32_t)(k_base + (t / kGroups + j * (256 / kGroups)) * E) * p.N;
+#pragma unroll
+      for (int e = 0; e < E; ++e) {
+        const uint32_t r = k_row + (uint32_t)e * p.N;
+        __builtin_memcpy(&next_b[j][e], p.b + ((r < last_row ? r : last_row) + col_at) * kElemBytes, 4 * kElemBytes);
+      }
+    }
+  };
+  fetch(0);
+
+  // The wave's 2 x 2 blocks of 16x16: element r of a lane is row 4 (lane / 16) + r,
+  // column lane % 16.
+  const int wm = wave / 2 * 32, wn = wave % 2 * 32;
+  // A step has sums of its own, one for every other instruction, which are added
+  // to the whole at its end, and the old result last of all: the rounding error
+  // of a sum grows with the number of terms it takes one by one.
+  acc_t acc[2][2] = {}, old[2][2] = {};
+  out_t* const c = (out_t*)p.c;
+  if (p.accumulate) {
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+      for (int j = 0; j < 2; ++j)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          const int m = m_base + wm + i * 16 + lane / 16 * 4 + r, n = n_base + wn + j * 16 + lane % 16;
+          if (m < p.M && n < p.N) old[i][j][r] = c[(int64_t)m * p.N + n];
+        }
+  }
+
+  for (int k_base = 0; k_base < p.K; k_base += kStep) {
+    const int left = p.K - k_base;
+    const int subs = left >= kStep ? kChunks / 4 : (left + 4 * E - 1) / (4 * E);   // of 4 chunks: one instruction's K
+    if (k_base > 0) __syncthreads();
+    if (t % kChunks < subs * 4) {
+#pragma unroll
+      for (int j = 0; j < 8; ++j)
+        tile_a[place(t / kChunks + j * (kRows / 8), t % kChunks)] = settle_chunk<kElemBytes>(
+            next_a[j], k_base + t % kChunks * E, p.K, my_row + j * (kRows / 8) < p.M);
+    }
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+      const int chunk = t / kGroups + j * (256 / kGroups), k = k_base + chunk * E;
+      if (chunk < subs * 4) {
+        if (k + E > p.K || my_n + 4 > p.N) {
+#pragma unroll
+          for (int e = 0; e < E; ++e) next_b[j][e] = settle_four<kElemBytes>(next_b[j][e], my_n, p.N, k + e < p.K);
+        }
+#pragma unroll
+        for (int e = 0; e < 4; ++e) tile_b[place(t % kGroups * 4 + e, chunk)] = column_chunk<kElemBytes>(next_b[j], e);
+      }
+    }
+    __syncthreads();
+    if (k_base + kStep < p.K) fetch(k_base + kStep);
+    acc_t part[2][2][2] = {};
+    auto multiply = [&](int s, acc_t (&sum)[2][2]) {
+      union { u32x4 u; frag_t f; } fa[2], fb[2];
+#pragma unroll
+      for (int i = 0; i < 2; ++i) {
+        fa[i].u = tile_a[place(wm + i * 16 + lane % 16, s * 4 + lane / 16)];
+        fb[i].u = tile_b[place(wn + i * 16 + lane % 16, s * 4 + lane / 16)];
+      }
+#pragma unroll
+      for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int j = 0; j < 2; ++j) sum[i][j] = Cfg::mfma(fa[i].f, fb[j].f, sum[i][j]);
+    };
+    for (int s = 0; s < subs; s += 2) {
+      multiply(s, part[0]);
+      if (s + 1 < subs) multiply(s + 1, part[1]);
+    }
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+      for (int j = 0; j < 2; ++j) acc[i][j] += part[0][i][j] + part[1][i][j];
+  }
+
+  out_t* const out = (out_t*)p.out;
+#pragma unroll
+  for (int j = 0; j < 2; ++j) {
+    const int n = n_base + wn + j * 16 + lane % 16;
+    const int n1 = (int)((uint32_t)n / (uint32_t)p.N0), n0 = n - n1 * p.N0;
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int m = m_base + wm + i * 16 + lane / 16 * 4 + r;
+        const out_t v = (out_t)(acc[i][j][r] + old[i][j][r]);
+        if (m < p.M && n < p.N) c[(int64_t)m * p.N + n] = v;
+        if (out) {
+          const int m1 = (int)((uint32_t)m / (uint32_t)p.M0), m0 = m - m1 * p.M0;
+          if (m1 < p.M1 && n1 < p.N1) out[(((int64_t)m1 * p.N1 + n1) * p.M0 + m0) * p.N0 + n0] = v;
+        }
+      }
+  }
+}
+
 // Estimated time in microseconds on 16 mb rows x 64 columns with K in `slices`: the
 // first round of workgroups, one per compute unit, each further one, an eighth of the
 // steps of all of them (by element size), the result, C, and for a split the planes
@@ -503,6 +660,32 @@ bool choose(const RowMajorArgs& p, int max_slices, double limit_us, int* mb, int
   return found;
 }
 
+// Results of a workgroup on 64 x 64 for every compute unit and more, and a K of one step of
+// that kernel, f32 (four matrix instructions for the others' one) one and a half. With
+// the packed result stored beside it both are bound by the stores, but for f32. Measured
+// (16 or 32 x 64, 64 x 64), us: f32 1200x1500x100 16.1, 12.5, without the packed result
+// 14.6, 9.9; 651x2125x158 16.5, 15.7 and 14.4, 13.1; 900x1300x300 17.2, 20.9; without the
+// packed result i8 700x2100x500 9.9, 8.4, f16 1200x1500x100 7.4, 7.0; with it 11.0, 10.9
+// and 9.2, 9.7.
+template <typename Cfg>
+bool square_is_faster(const RowMajorArgs& p) {
+  const int64_t tiles = ceil_div((int64_t)p.M1 * p.M0, (int64_t)64) * ceil_div((int64_t)p.N1 * p.N0, (int64_t)64);
+  const int bytes = p.K * Cfg::kElemBytes;
+  return tiles >= device_cu_count() && (Cfg::kElemBytes == 4 ? bytes <= 768 : !p.out && bytes <= 512);
+}
+
+template <typename Cfg>
+int launch_square(RowMajorArgs p, hipStream_t s) {
+  const int64_t rows = (int64_t)p.M1 * p.M0, cols = (int64_t)p.N1 * p.N0;
+  p.tiles_n = (int)ceil_div(cols, (int64_t)64);
+  p.tiles = p.product_blocks = (int)(ceil_div(rows, (int64_t)64) * p.tiles_n);
+  p.lhs_blocks = p.lhs ? (int)ceil_div(rows * p.K1, (int64_t)256) : 0;
+  const int rhs_blocks = p.rhs ? (int)ceil_div(cols * p.K1, (int64_t)256) : 0;
+  hipLaunchKernelGGL(matmul_rowmajor_square_kernel<Cfg>, dim3((unsigned)(p.product_blocks + p.lhs_blocks + rhs_blocks)),
+                     dim3(256), 0, s, p);
+  return check_hip(hipGetLastError(), "matmul_rowmajor launch");
+}
+
 template <typename Cfg>
 int launch(RowMajorArgs p, hipStream_t s) {
   constexpr int kStep = 64 / Cfg::kElemBytes;                     // elements of K per step
@@ -514,6 +697,7 @@ int launch(RowMajorArgs p, hipStream_t s) {
   const double limit = together && chain < 24.0 ? chain - 2.4 : 0.9 * chain;
   int mb = 1, slices = 1;
   if (!choose<Cfg>(p, 16, limit, &mb, &slices)) return IREE_AMD_UK_STATUS_NOT_FOUND;
+  if (square_is_faster<Cfg>(p)) return launch_square<Cfg>(p, s);
   auto lay_out = [&] {
     p.tiles_n = (int)ceil_div(cols, (int64_t)64);
     p.tiles = (int)(ceil_div(rows, (int64_t)mb * 16) * p.tiles_n);
