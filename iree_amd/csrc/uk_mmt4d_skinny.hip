@@ -113,7 +113,10 @@ __global__ __launch_bounds__(kThreads) void mmt4d_skinny_kernel(SkinnyArgs a) {
   typedef typename Cfg::frag_t frag_t;
   typedef typename Cfg::acc_t acc_t;
   typedef typename Cfg::out_t out_t;
-  constexpr int kDepth = (SP % kDepthMax == 0) ? kDepthMax : 8;
+  // (fp8: a block is two registers' worth of the others, and 16 of them beside 16
+  // steps of the left-hand side spilled: N = 10587, K = 7424, 4 rows 36 us, with 8
+  // of them 17)
+  constexpr int kDepth = (SP % kDepthMax == 0 && Cfg::kSub == 1) ? kDepthMax : 8;
   static_assert(SP % kDepth == 0, "the rolling buffer must divide the steps of a tile");
   // partial sums keep the accumulator's type (f32, or s32 for integer inputs)
   typedef typename std::conditional<std::is_same<out_t, int32_t>::value, int32_t, float>::type sum_t;
@@ -653,15 +656,16 @@ namespace {
 // K that stays in registers here (up to 8 KB), longer than half a KB: up to two
 // workgroups of 16 columns per compute unit, where that kernel takes 0.79 times as
 // long on average over 487 problems (values of a decode step, 16 heads x 1x64x3232
-// f16, 7.7 -> 3.5 us; 4 rows x 256 x 3456 5.9 -> 4.2), and with more columns this one's
-// longer runs of them win. Longer K, which is split here into slices that a second
+// f16, 7.7 -> 3.5 us; 4 rows x 256 x 3456 5.9 -> 4.2), one beyond 6.25 KB (i8 4 rows x
+// 4160 x 7424, two of them 10.3, here 9.3), and with more columns this one's longer
+// runs of them win. Longer K, which is split here into slices that a second
 // launch adds: up to 12 KB of K and 256 outer columns, on the shape of an entry
 // alone, so that the entries of a batch have the bits of the single call (fp8 8 rows
 // x 4992 x 15552 36.9 -> 19.5, f16 2 x 128 x 4992 6.1 -> 5.0; beyond 12 KB the few
 // workgroups of a single call take longer: bf16 16 x 480 x 14528 9.1 here, 14.3 there).
 bool few_columns(int64_t N, int64_t chunks, int64_t batch) {
   if (chunks <= 32) return false;
-  if (chunks <= 512) return batch * N <= device_cu_count();
+  if (chunks <= 512) return batch * N * (chunks <= 400 ? 1 : 2) <= device_cu_count();
   return chunks <= 768 && N <= 256;
 }
 
@@ -906,6 +910,11 @@ int launch_matmul_rows_skinny(const iree_amd_uk_mmt4d_params_t& p, int64_t M, in
   // elements at 32 rows 15.1 (i8) and 16.7 (fp8) against 17.2 and 17.0)
   if (eb > 1 && M > 24) return IREE_AMD_UK_STATUS_NOT_FOUND;
   const int64_t steps = k_elems / mk;
+  // (fp8, more outer columns than compute units, macro tiles against this kernel at
+  // N = 10587: K = 1024 6.9 and 7.9 us, 1536 8.7 and 8.4; more than 16 rows and K = 4608
+  // 15.7 and 16.8, 6144 19.0 and 18.9)
+  if (mk == 64 && p.N > device_cu_count() && (steps < 20 || (M > 16 && steps > 64 && steps < 96)))
+    return IREE_AMD_UK_STATUS_NOT_FOUND;
   // (a K longer than one launch row keeps in registers goes to the macro-tile
   // kernel with its K split, which measures as fast or faster there)
   if (steps > max_steps_per_launch(mk)) return IREE_AMD_UK_STATUS_NOT_FOUND;
