@@ -505,7 +505,7 @@ int launch_generic(K kernel, const PackArgs& a, int64_t total, hipStream_t s, co
 // Both operands of a matmul in one launch: workgroups 0 .. lhs_blocks - 1 the
 // streaming pack of A, the rest the transposing pack of B. Each pass is short beside
 // a launch and its drain (A of the 1999 x 4099 x 3001 bf16 matmul 7.6 us, B 11.5 for
-// 24 and 49 MB).
+// 24 and 49 MB; together 17.7, and 3 us less of the whole call).
 template <int ES>
 __global__ __launch_bounds__(256) void pack_operands_kernel(Pow2Args lhs, uint32_t lhs_blocks, TransArgs rhs) {
   if (blockIdx.x < lhs_blocks) stream_pow2_body<ES, true, true, true, 8, 1, 1, 4>(lhs, blockIdx.x);
