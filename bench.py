@@ -424,7 +424,9 @@ def extras(args, torch, iree_amd, F, synth, lhs, rhs, out, ex):
             iree_amd.mmt4d(lb, rb, o1, bt, bt, bk, 32, 32, 8, F.MMT4D_TYPE_F16F16F32,
                            lhs_offset=b * Bs * Bs, rhs_offset=b * Bs * Bs, out_offset=b * Bs * Bs)
     _, t1 = gpu_time(torch, one_by_one, max(steps // 4, 2), 1)
-    assert torch.equal(ob.view(torch.int32), o1.view(torch.int32)), "batch_mmt4d differs from per-entry mmt4d"
+    # (the single call deals K over the waves of a workgroup, the batch keeps it whole:
+    # sums of 1024 products in another order, sqrt(1024) * 2^-24 = 2e-6 of their size)
+    assert ((ob - o1).norm() <= 1e-5 * ob.norm()).item(), "batch_mmt4d differs from per-entry mmt4d"
     ex["batch_mmt4d_f16_16x1024_tflops"] = round(2.0 * Bn * Bs ** 3 / t / 1e12, 1)
     ex["batch_mmt4d_f16_16x1024_entry_by_entry_tflops"] = round(2.0 * Bn * Bs ** 3 / t1 / 1e12, 1)
     del lb, rb, ob, o1
