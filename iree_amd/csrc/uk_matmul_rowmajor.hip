@@ -580,8 +580,9 @@ __global__ __launch_bounds__(256, 2) void matmul_rowmajor_square_kernel(RowMajor
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
         const int m = m_base + wm + i * 16 + lane / 16 * 4 + r;
-        const out_t v = (out_t)(acc[i][j][r] + old[i][j][r]);
-        if (m < p.M && n < p.N) c[(int64_t)m * p.N + n] = v;
+        const bool in_matrix = m < p.M && n < p.N;
+        const out_t v = in_matrix ? (out_t)(acc[i][j][r] + old[i][j][r]) : (out_t)0;   // (padding of the tiles: zeros)
+        if (in_matrix) c[(int64_t)m * p.N + n] = v;
         if (out) {
           const int m1 = (int)((uint32_t)m / (uint32_t)p.M0), m0 = m - m1 * p.M0;
           if (m1 < p.M1 && n1 < p.N1) out[(((int64_t)m1 * p.N1 + n1) * p.M0 + m0) * p.N0 + n0] = v;

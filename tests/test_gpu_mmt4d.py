@@ -1705,3 +1705,26 @@ def test_large_result_of_a_short_k(uk, cuda, type_flag, dt, out_dt, M, N, K):
         chain = uk.matmul_data_tiled(a, b, step, M, N, K, type_flag, one_launch=False, **kw)
         assert torch.equal(c, step), kw
         assert ws.keys() == chain.keys() and all(torch.equal(ws[k], chain[k]) for k in ws), kw
+
+
+@pytest.mark.parametrize("type_flag,dt", [(F.MMT4D_TYPE_F32F32F32, "float32"), (F.MMT4D_TYPE_BF16BF16F32, "bfloat16")])
+@pytest.mark.parametrize("M,N,K", [(1025, 1027, 191), (81, 19, 41), (200, 136, 264)])
+def test_infinities_do_not_reach_the_padding(uk, cuda, type_flag, dt, M, N, K):
+    """An infinity and a NaN in either operand of a small problem, also in the last step
+    of K: where they belong in the matrix, and zeros in the padding of the packed
+    result (1025 x 1027 x 191 f32: the kernel on 64 x 64 tiles)."""
+    import torch
+    g = torch.Generator(device="cuda").manual_seed(M + N + K)
+    a = torch.randint(1, 4, (M, K), generator=g, device="cuda").to(getattr(torch, dt))
+    b = torch.randint(1, 4, (K, N), generator=g, device="cuda").to(getattr(torch, dt))
+    a[3, K - 1], a[M - 1, 0], b[K - 1, N - 1], b[5, 7] = float("inf"), float("nan"), float("-inf"), float("inf")
+    want = a.double() @ b.double()
+    for accumulate in (False, True):
+        c = torch.full((M, N), 2.0, device="cuda")
+        ws = uk.matmul_data_tiled(a, b, c, M, N, K, type_flag, accumulate=accumulate)
+        assert uk.last_kernel_path() == "mmt4d:mfma-one-launch"
+        assert torch.equal(c.double().nan_to_num(1e9, 2e9, 3e9), (want + 2 * accumulate).nan_to_num(1e9, 2e9, 3e9))
+        M0, N0, _ = uk.query_matmul_tile_sizes(uk.ukernel._MMT4D_TO_QUERY_OP[type_flag], M, N, K)
+        out = torch.empty_like(ws["out"])
+        uk.pack(c, out, M, N, -(-M // M0), -(-N // N0), M0, N0, 0, uk.ukernel._OUT_PACK_TYPE[type_flag])
+        assert torch.equal(ws["out"].view(torch.int32), out.view(torch.int32))
