@@ -359,8 +359,10 @@ int launch_type(const WaveSplitArgs& a, int v, hipStream_t s) {
 WaveSplitChoice choose_wave_split(const WaveSplitArgs& a, uint32_t type) {
   WaveSplitChoice best = {-1, 0.0};
   const bool f32 = type == IREE_AMD_UK_FLAG_MMT4D_TYPE_F32F32F32, f8 = type == IREE_AMD_UK_FLAG_MMT4D_TYPE_F8E4M3F8E4M3F32;
-  // (32-bit offsets within a workgroup's tile and along K)
-  if ((a.silu && !f8) || a.lhs_outer > (1 << 28) || a.rhs_outer > (1 << 28) || a.k_chunks < 1 || a.k_chunks > (1 << 18) ||
+  // (unsigned 32-bit offsets within a workgroup's tile and along K: outer rows or columns
+  // that run backwards are the other kernels')
+  if ((a.silu && !f8) || a.lhs_outer < 0 || a.rhs_outer < 0 || a.lhs_outer > (1 << 28) || a.rhs_outer > (1 << 28) ||
+      a.k_chunks < 1 || a.k_chunks > (1 << 18) ||
       a.rows < 1 || a.rows > (1 << 24) || a.outer_cols < 1 || a.outer_cols > (1 << 20))
     return best;
   const bool half_out = type == IREE_AMD_UK_FLAG_MMT4D_TYPE_F16F16F16 || type == IREE_AMD_UK_FLAG_MMT4D_TYPE_BF16BF16BF16;

@@ -1728,3 +1728,36 @@ def test_infinities_do_not_reach_the_padding(uk, cuda, type_flag, dt, M, N, K):
         out = torch.empty_like(ws["out"])
         uk.pack(c, out, M, N, -(-M // M0), -(-N // N0), M0, N0, 0, uk.ukernel._OUT_PACK_TYPE[type_flag])
         assert torch.equal(ws["out"].view(torch.int32), out.view(torch.int32))
+
+
+@pytest.mark.parametrize("M1,N1,steps,tile", [(7, 47, 64, (32, 64)), (25, 32, 32, (64, 64))])
+@pytest.mark.parametrize("backwards", ["lhs", "rhs"])
+def test_outer_rows_that_run_backwards(uk, cuda, M1, N1, steps, tile, backwards):
+    """A negative pitch of the outer rows or columns, at sizes whose forward form runs on
+    tiles of few problems that span two of them: the macro tiles', with the same
+    (exact) sums; narrow tiles against outer columns that run backwards as well."""
+    import torch
+    g = torch.Generator(device="cuda").manual_seed(M1 + N1)
+    K1 = 4 * steps
+    lhs = torch.randint(-2, 3, (M1, K1, 32, 8), generator=g, device="cuda").half()
+    rhs = torch.randint(-2, 3, (N1, K1, 32, 8), generator=g, device="cuda").half()
+    want, got = (torch.zeros(M1, N1, 32, 32, device="cuda") for _ in range(2))
+    uk.mmt4d(lhs, rhs, want, M1, N1, K1, 32, 32, 8, F.MMT4D_TYPE_F16F16F32)
+    _expect_macro_tile(uk, *tile, 1)
+    pitch = K1 * 256
+    if backwards == "lhs":
+        uk.mmt4d(lhs.flip(0).contiguous(), rhs, got, M1, N1, K1, 32, 32, 8, F.MMT4D_TYPE_F16F16F32,
+                 lhs_offset=(M1 - 1) * pitch, lhs_stride0=-pitch)
+    else:
+        uk.mmt4d(lhs, rhs.flip(0).contiguous(), got, M1, N1, K1, 32, 32, 8, F.MMT4D_TYPE_F16F16F32,
+                 rhs_offset=(N1 - 1) * pitch, rhs_stride0=-pitch)
+    assert uk.last_kernel_path() == "mmt4d:mfma" and uk.last_macro_tile()[0] >= 128
+    assert torch.equal(got, want)
+    assert torch.equal(want[0, 0], lhs[0].transpose(0, 1).reshape(32, -1).float() @ rhs[0].transpose(0, 1).reshape(32, -1).float().T)
+    if backwards == "rhs":
+        rows = lhs[0, :, :4].contiguous()               # (four rows as a narrow tile)
+        want, got = (torch.zeros(N1, 4, 32, device="cuda") for _ in range(2))
+        uk.mmt4d(rows, rhs, want, 1, N1, K1, 4, 32, 8, F.MMT4D_TYPE_F16F16F32)
+        uk.mmt4d(rows, rhs.flip(0).contiguous(), got, 1, N1, K1, 4, 32, 8, F.MMT4D_TYPE_F16F16F32,
+                 rhs_offset=(N1 - 1) * pitch, rhs_stride0=-pitch)
+        assert torch.equal(got, want) and want.abs().max() > 0
