@@ -269,6 +269,7 @@ int make_args(const iree_amd_uk_mmt4d_params_t& p, int out_elem_bytes, bool silu
   a.lhs_row_major = 0;
   a.gate_scale = a.up_scale = a.inv_out_scale = a.out_scale = 1.0f;
   a.other_us = 0.0f;
+  a.compare_only = false;
   return 0;
 }
 }  // namespace
@@ -453,21 +454,35 @@ bool as_few_tiles(const iree_amd_uk_mmt4d_params_t& p, const MfmaArgs& a, bool s
   return true;
 }
 
+// The call on the kernel for few tiles: its best tile there (tile < 0: not served),
+// and whether that needs no comparison.
+struct FewTiles {
+  WaveSplitArgs args;
+  WaveSplitChoice choice;
+  bool certain;
+};
+FewTiles consider_few_tiles(const iree_amd_uk_mmt4d_params_t& p, const MfmaArgs& a, bool silu) {
+  FewTiles few;
+  few.choice = {-1, 0.0};
+  if (as_few_tiles(p, a, silu, &few.args))
+    few.choice = choose_wave_split(few.args, p.flags & IREE_AMD_UK_FLAG_MMT4D_TYPE_MASK);
+  // (up to four macro tiles and half a KB to 8 KB of K: it was faster, on all of 1220
+  // problems, and the estimates of the macro tiles take 0.2 us of a 3.5 us call)
+  few.certain = few.choice.tile >= 0 && p.K >= 32 && p.K <= 512 && ((a.M + 3) / 4) * (int64_t)((a.N + 3) / 4) <= 4;
+  return few;
+}
+int launch_few_tiles(const iree_amd_uk_mmt4d_params_t& p, const FewTiles& few, hipStream_t s) {
+  return launch_mmt4d_wave_split(few.args, p.flags & IREE_AMD_UK_FLAG_MMT4D_TYPE_MASK, few.choice.tile, s);
+}
+
 // `launch` on the macro tiles, or the kernel for few tiles where that is faster.
 template <typename Launch>
-int launch_faster(const iree_amd_uk_mmt4d_params_t& p, const MfmaArgs& a, bool silu, hipStream_t s, Launch launch) {
+int launch_faster(const iree_amd_uk_mmt4d_params_t& p, const MfmaArgs& a, const FewTiles& few, hipStream_t s, Launch launch) {
+  if (few.certain) return launch_few_tiles(p, few, s);
   MfmaArgs b = a;
-  WaveSplitArgs w;
-  WaveSplitChoice few = {-1, 0.0};
-  const uint32_t type = p.flags & IREE_AMD_UK_FLAG_MMT4D_TYPE_MASK;
-  if (as_few_tiles(p, a, silu, &w)) few = choose_wave_split(w, type);
-  // (up to four macro tiles and half a KB to 8 KB of K: it was, on all of 1220
-  // problems, and the estimates of the macro tiles take 0.2 us of a 3.5 us call)
-  if (few.tile >= 0 && p.K >= 32 && p.K <= 512 && ((a.M + 3) / 4) * (int64_t)((a.N + 3) / 4) <= 4)
-    return launch_mmt4d_wave_split(w, type, few.tile, s);
-  b.other_us = few.tile >= 0 ? (float)few.us : 0.0f;
+  b.other_us = few.choice.tile >= 0 ? (float)few.choice.us : 0.0f;
   const int st = launch(b);
-  return st == kSlowerThanOther ? launch_mmt4d_wave_split(w, type, few.tile, s) : st;
+  return st == kSlowerThanOther ? launch_few_tiles(p, few, s) : st;
 }
 
 int launch_macro_tiles(const iree_amd_uk_mmt4d_params_t& p, const MfmaArgs& a, hipStream_t s) {
@@ -484,7 +499,8 @@ int launch_macro_tiles(const iree_amd_uk_mmt4d_params_t& p, const MfmaArgs& a, h
 }
 
 int launch_typed(const iree_amd_uk_mmt4d_params_t& p, const MfmaArgs& a, hipStream_t s) {
-  return launch_faster(p, a, false, s, [&](const MfmaArgs& b) { return launch_macro_tiles(p, b, s); });
+  return launch_faster(p, a, consider_few_tiles(p, a, false), s,
+                       [&](const MfmaArgs& b) { return launch_macro_tiles(p, b, s); });
 }
 }  // namespace
 
@@ -498,14 +514,29 @@ int launch_mmt4d_silu_mul_mfma(const iree_amd_uk_mmt4d_params_t& p, float gate_s
   if (st) return st;
   a.gate_scale = gate_scale; a.up_scale = up_scale; a.inv_out_scale = inv_out_scale;
   a.accumulate = 0;
-  return launch_faster(p, a, true, s, [&](const MfmaArgs& b) {
+  auto launch = [&](const MfmaArgs& b) {
     switch (p.flags & IREE_AMD_UK_FLAG_MMT4D_TYPE_MASK) {
       case IREE_AMD_UK_FLAG_MMT4D_TYPE_F16F16F32: return launch_mfma_silu_f16(b, s);
       case IREE_AMD_UK_FLAG_MMT4D_TYPE_BF16BF16F32: return launch_mfma_silu_bf16(b, s);
       case IREE_AMD_UK_FLAG_MMT4D_TYPE_F8E4M3F8E4M3F32: return launch_mfma_silu_f8(b, s);
       default: return (int)IREE_AMD_UK_STATUS_NOT_FOUND;
     }
-  });
+  };
+  const FewTiles few = consider_few_tiles(p, a, true);
+  if (few.choice.tile >= 0 && !few.certain) {
+    // (fp8) The kernel of the plain mmt4d on these operands, whose sums have the same
+    // bits then; the estimates of the two forms, each for itself, differed on 1 % of
+    // the problems. Where the plain one splits K over workgroups, which this form
+    // does not, it goes by its own.
+    MfmaArgs plain = a;
+    plain.compare_only = true;
+    const FewTiles of_plain = consider_few_tiles(p, a, false);
+    plain.other_us = (float)of_plain.choice.us;
+    const int st = launch_mfma_f8f8f32(plain, s);
+    if (st == kSlowerThanOther) return launch_few_tiles(p, few, s);
+    if (st != kSplitsK) return launch(a);
+  }
+  return launch_faster(p, a, few, s, launch);
 }
 
 }  // namespace uk

@@ -30,6 +30,8 @@ int launch_mfma_silu_f8(const MfmaArgs& a, hipStream_t s);
 // What the launch functions return, having launched nothing, when the call is
 // estimated to take longer here than MfmaArgs::other_us.
 constexpr int kSlowerThanOther = -1;
+// And what launch_costed returns for MfmaArgs::compare_only where it would split K.
+constexpr int kSplitsK = -2;
 
 namespace {
 
@@ -579,6 +581,7 @@ int launch_costed(const MfmaArgs& a, hipStream_t s) {
       }
       if (split_n > 1) {
         if (other_is_faster(split_v, split_n)) return kSlowerThanOther;
+        if (a.compare_only) return kSplitsK;
         split_wins = true;
         const int st = launch_k_split<Cfg>(a, split_v, split_n, s);
         if (st != IREE_AMD_UK_STATUS_NOT_FOUND) return st;
@@ -586,6 +589,7 @@ int launch_costed(const MfmaArgs& a, hipStream_t s) {
     }
   }
   if (!split_wins && other_is_faster(best, 1)) return kSlowerThanOther;
+  if (a.compare_only) return 0;
   {
     const int st = launch_whole_rounds<Cfg, kSiluMul>(
         a, cus, best_cost, [&](int v, int64_t M, int64_t N) { return cost_of(v, M, N); }, pick, s);

@@ -335,6 +335,36 @@ def test_fused_gate_up_silu_matches_unfused(uk, cuda, type_flag, K0, M1, P, K1):
     assert np.all(got[:, P * 1024:] == 0xEE)
 
 
+@pytest.mark.parametrize("M1,P,K1,tile", [
+    (1, 9, 250, None), (3, 56, 112, (32, 64)), (3, 56, 130, (32, 64)), (7, 42, 101, (64, 64)), (22, 19, 127, (64, 64)),
+    # (where the two forms' own estimates would take different kernels)
+    (3, 99, 230, (128, 128)), (4, 96, 104, (128, 128)), (2, 118, 164, (128, 128)),
+])
+def test_gate_up_silu_of_few_tiles_has_the_bits_of_mmt4d(uk, cuda, M1, P, K1, tile):
+    """The fused form on the kernel that deals K to the waves (tiles of two and four
+    16-column blocks a side, K of several rounds of its pipeline) and near the line to
+    the macro tiles: the bytes of plain mmt4d followed by silu_mul_quantize_tiled on
+    operands whose fp8 sums depend on their order, so both run the same kernel."""
+    import torch
+    type_flag, K0 = F.MMT4D_TYPE_F8E4M3F8E4M3F32, 16
+    g = torch.Generator(device="cuda").manual_seed(M1 * 100 + P + K1)
+    lhs, rhs = (torch.randn(n * K1 * 32 * K0, generator=g, device="cuda").to(torch.float8_e4m3fn).view(torch.uint8)
+                for n in (M1, 2 * P))
+    scale, out_scale = (K1 * K0) ** -0.5, 8.0       # (gate and up about N(0, 1), the product within e4m3)
+    fused, want = (torch.zeros(M1 * P * 1024, dtype=torch.uint8, device="cuda") for _ in range(2))
+    uk.mmt4d_silu_mul_f8e4m3(lhs, rhs, fused, M1, 2 * P, K1, K0, type_flag, scale, scale, out_scale)
+    on = uk.last_macro_tile()
+    if tile and torch.cuda.get_device_properties(0).multi_processor_count == 256:
+        assert on == (*tile, 1)
+    acc = torch.zeros(M1 * 2 * P * 1024, dtype=torch.float32, device="cuda")
+    uk.mmt4d(lhs, rhs, acc, M1, 2 * P, K1, 32, 32, K0, type_flag)
+    assert (uk.last_macro_tile()[0] < 128) == (on[0] < 128)
+    a4 = acc.view(M1, P, 2, 1024)
+    split = torch.cat([a4[:, :, 0], a4[:, :, 1]], dim=1).contiguous()     # [M1][gate tiles | up tiles]
+    uk.silu_mul_quantize_tiled(split, 2 * P * 1024, 0, P, want, P * 1024, M1, P, scale, scale, out_scale)
+    assert torch.equal(fused, want) and want.unique().numel() > 100
+
+
 def test_fused_gate_up_silu_invalid_arguments(uk, cuda):
     import torch
     t = torch.zeros(4096, dtype=torch.uint8, device="cuda")
