@@ -626,10 +626,10 @@ IREE_AMD_UK_EXPORT int iree_amd_uk_batch_mmt4d_unpack(
  * (integers always; else float sums come in another order: the split is chosen
  * for the row-major operand). Up to 24 rows (32 of 1-byte elements: a decode step)
  * with a K of up to 4096 elements of 2 bytes (8192 of 1 byte) run the kernel
- * for narrow left-hand side tiles on the rows themselves (float sums then
- * come in that kernel's order: the bits of mmt4d on M0 = M tiles). With N >= 16384 (and M >= 512) the
- * left-hand side is packed into the stream's scratch buffer first (see
- * iree_amd_uk_mmt4d on that buffer). */
+ * for narrow left-hand side tiles on the rows themselves from 8193 columns on (float
+ * sums then come in that kernel's order: the bits of mmt4d on M0 = M tiles), with
+ * fewer columns or a scaled result where it is the faster. With N >= 16384 (and M >= 512) the left-hand side is packed into the stream's
+ * scratch buffer first (see iree_amd_uk_mmt4d on that buffer). */
 IREE_AMD_UK_EXPORT int iree_amd_uk_matmul_packed_rhs(
     const void* lhs_buffer, iree_amd_uk_index_t lhs_offset,
     iree_amd_uk_index_t lhs_stride0, const void* rhs_buffer,

@@ -910,10 +910,10 @@ int launch_matmul_rows_skinny(const iree_amd_uk_mmt4d_params_t& p, int64_t M, in
   // elements at 32 rows 15.1 (i8) and 16.7 (fp8) against 17.2 and 17.0)
   if (eb > 1 && M > 24) return IREE_AMD_UK_STATUS_NOT_FOUND;
   const int64_t steps = k_elems / mk;
-  // (fp8, more outer columns than compute units, macro tiles against this kernel at
+  // (fp8 with a scaled result, more outer columns than compute units, macro tiles against this kernel at
   // N = 10587: K = 1024 6.9 and 7.9 us, 1536 8.7 and 8.4; more than 16 rows and K = 4608
   // 15.7 and 16.8, 6144 19.0 and 18.9)
-  if (mk == 64 && p.N > device_cu_count() && (steps < 20 || (M > 16 && steps > 64 && steps < 96)))
+  if (out_scale != 1.0f && mk == 64 && p.N > device_cu_count() && (steps < 20 || (M > 16 && steps > 64 && steps < 96)))
     return IREE_AMD_UK_STATUS_NOT_FOUND;
   // (a K longer than one launch row keeps in registers goes to the macro-tile
   // kernel with its K split, which measures as fast or faster there)

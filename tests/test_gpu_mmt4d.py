@@ -1761,3 +1761,17 @@ def test_outer_rows_that_run_backwards(uk, cuda, M1, N1, steps, tile, backwards)
         uk.mmt4d(rows, rhs.flip(0).contiguous(), got, 1, N1, K1, 4, 32, 8, F.MMT4D_TYPE_F16F16F32,
                  rhs_offset=(N1 - 1) * pitch, rhs_stride0=-pitch)
         assert torch.equal(got, want) and want.abs().max() > 0
+
+
+@pytest.mark.parametrize("M,N1,K", [(2, 257, 64), (8, 260, 1024), (24, 700, 1216), (20, 260, 4608), (31, 300, 5120)])
+def test_few_fp8_rows_have_the_bits_of_narrow_tiles(uk, cuda, M, N1, K):
+    """An unscaled result of a few fp8 rows and many columns: the bits of mmt4d on tiles
+    of as many rows, whatever K, on operands whose fp8 sums depend on their order."""
+    import torch
+    g = torch.Generator(device="cuda").manual_seed(M + N1 + K)
+    x, w = (torch.randn(n, generator=g, device="cuda").to(torch.float8_e4m3fn).view(torch.uint8) for n in (M * K, N1 * 32 * K))
+    y, tiles = torch.empty(M, N1 * 32, device="cuda"), torch.empty(N1, M, 32, device="cuda")
+    uk.matmul_packed_rhs(x, w, y, M, N1 * 32, K, 16, F.MMT4D_TYPE_F8E4M3F8E4M3F32)
+    assert uk.last_kernel_path() == "mmt4d:mfma-narrow"
+    uk.mmt4d(x.view(M, K // 16, 16).transpose(0, 1).contiguous(), w, tiles, 1, N1, K // 16, M, 32, 16, F.MMT4D_TYPE_F8E4M3F8E4M3F32)
+    assert torch.equal(tiles.transpose(0, 1).reshape(M, -1), y)
