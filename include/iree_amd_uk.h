@@ -628,7 +628,8 @@ IREE_AMD_UK_EXPORT int iree_amd_uk_batch_mmt4d_unpack(
  * with a K of up to 4096 elements of 2 bytes (8192 of 1 byte) run the kernel
  * for narrow left-hand side tiles on the rows themselves from 8193 columns on (float
  * sums then come in that kernel's order: the bits of mmt4d on M0 = M tiles), with
- * fewer columns or a scaled result where it is the faster. With N >= 16384 (and M >= 512) the left-hand side is packed into the stream's
+ * fewer columns, a scaled result, or one row that ends inside a tile, where it is the
+ * faster. With N >= 16384 (and M >= 512) the left-hand side is packed into the stream's
  * scratch buffer first (see iree_amd_uk_mmt4d on that buffer). */
 IREE_AMD_UK_EXPORT int iree_amd_uk_matmul_packed_rhs(
     const void* lhs_buffer, iree_amd_uk_index_t lhs_offset,

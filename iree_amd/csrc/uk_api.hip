@@ -810,9 +810,9 @@ int matmul_packed_rhs_impl(
   }
   // A few rows (to 32; one row too whose result is scaled or ends inside a tile):
   // the same kernel with the rows of the matrix as the rows of its one narrow tile,
-  // reading them and writing the result row-major. (A scaled result went to the
-  // macro tiles before: fp8, N = 14336, K = 4096, 4 rows 17.0 us there, 13.0 here;
-  // 1 row 17.1 and 12.8; N = 11008, K = 2048, 24 rows 11.1 and 10.4.)
+  // reading them and writing the result row-major, where that is the faster for a
+  // scaled one (fp8, N = 14336, K = 4096, 4 rows 17.0 us on the macro tiles, 13.0
+  // here; 1 row 17.1 and 12.8).
   if (st == IREE_AMD_UK_STATUS_NOT_FOUND && M >= 1 && M <= 32 && b.batch == 1)
     st = launch_matmul_rows_skinny(p, M, N, out_scale, (hipStream_t)stream);
   const bool narrow = st != IREE_AMD_UK_STATUS_NOT_FOUND;

@@ -889,6 +889,31 @@ int launch_chunk(const iree_amd_uk_mmt4d_params_t& p, int chunks, int chunk_step
 }
 }  // namespace
 
+namespace {
+// Whether the launch below takes a result of M rows that is scaled, or that is one row
+// which ends inside a tile, from the other kernels for the same call (an unscaled one
+// of more rows it always takes). Up to 256 outer columns it wins unless K is so short
+// that the launch is all there is. Beyond that the others take a short K, whose sums
+// over the waves cost more than its loads, 769 to 1024 outer columns (a 128-column
+// tile on nearly every compute unit: f16 20 rows x 32224 x 3968 38.0 and 44.0 us here)
+// and, for fp8, a K from 4097 to 6143 of more than 8 rows or 512 outer columns, which
+// they split; f32 waits for its instructions, of whose rows half are idle here.
+// Measured on 2500 problems (1 to 32 rows, 4 to 1100 outer columns, K of 128 to 8192
+// bytes, weights from memory), and on 2500 others 0.4 % from the faster of the two
+// on average, where taking all but a few of fp8 was at 3.2 % (f16 24 rows x 10491 x 96
+// 3.9 us on the others, 6.2 here; fp8 20 x 30656 x 1280 10.8 and 16.4, 12 x 12091 x 3264
+// 14.8 and 11.6).
+bool scaled_rows_are_faster(int eb, bool fp8, int64_t M, int64_t outer_cols, int64_t k_bytes) {
+  if (outer_cols <= 256) return k_bytes > 512 || eb == 4 || (!fp8 && M <= 8 && k_bytes > 256);
+  if (eb == 4) return k_bytes > 512 && k_bytes <= 1024;
+  const bool middle = outer_cols > 384 && outer_cols <= 768;
+  if (!fp8) return middle ? k_bytes > 1024 : k_bytes >= 2048 && (M <= 8 || outer_cols <= 768 || outer_cols > 1024);
+  if (k_bytes <= 4096)
+    return (k_bytes > 3072 && (M <= 16 || outer_cols <= 768)) || (k_bytes > 1400 && middle && outer_cols <= 512);
+  return (M <= 8 && outer_cols <= 512) || (k_bytes >= 6144 && (M <= 8 || middle));
+}
+}  // namespace
+
 // The whole linear layer on a few rows: out[M][out_cols] (+)= lhs[M][K] * rhs,
 // lhs and out row-major (`p` describes them as iree_amd_uk_matmul_packed_rhs
 // does: lhs_stride0 and out_stride0 are row pitches in elements), rhs packed
@@ -910,10 +935,7 @@ int launch_matmul_rows_skinny(const iree_amd_uk_mmt4d_params_t& p, int64_t M, in
   // elements at 32 rows 15.1 (i8) and 16.7 (fp8) against 17.2 and 17.0)
   if (eb > 1 && M > 24) return IREE_AMD_UK_STATUS_NOT_FOUND;
   const int64_t steps = k_elems / mk;
-  // (fp8 with a scaled result, more outer columns than compute units, macro tiles against this kernel at
-  // N = 10587: K = 1024 6.9 and 7.9 us, 1536 8.7 and 8.4; more than 16 rows and K = 4608
-  // 15.7 and 16.8, 6144 19.0 and 18.9)
-  if (out_scale != 1.0f && mk == 64 && p.N > device_cu_count() && (steps < 20 || (M > 16 && steps > 64 && steps < 96)))
+  if ((out_scale != 1.0f || M == 1) && !scaled_rows_are_faster(eb, mk == 64, M, p.N, k_elems * eb))
     return IREE_AMD_UK_STATUS_NOT_FOUND;
   // (a K longer than one launch row keeps in registers goes to the macro-tile
   // kernel with its K split, which measures as fast or faster there)

@@ -1775,3 +1775,28 @@ def test_few_fp8_rows_have_the_bits_of_narrow_tiles(uk, cuda, M, N1, K):
     assert uk.last_kernel_path() == "mmt4d:mfma-narrow"
     uk.mmt4d(x.view(M, K // 16, 16).transpose(0, 1).contiguous(), w, tiles, 1, N1, K // 16, M, 32, 16, F.MMT4D_TYPE_F8E4M3F8E4M3F32)
     assert torch.equal(tiles.transpose(0, 1).reshape(M, -1), y)
+
+
+@pytest.mark.parametrize("type_flag,dt,M,N,K,narrow", [
+    (F.MMT4D_TYPE_F16F16F32, "float16", 24, 10491, 96, False), (F.MMT4D_TYPE_F16F16F32, "float16", 8, 10491, 1056, True),
+    (F.MMT4D_TYPE_F16F16F32, "float16", 9, 30000, 1056, False), (F.MMT4D_TYPE_F16F16F32, "float16", 1, 12347, 544, True),
+    (F.MMT4D_TYPE_F8E4M3F8E4M3F32, "float8_e4m3fn", 20, 30656, 1280, False),
+    (F.MMT4D_TYPE_F8E4M3F8E4M3F32, "float8_e4m3fn", 12, 12091, 3264, True),
+    (F.MMT4D_TYPE_F8E4M3F8E4M3F32, "float8_e4m3fn", 9, 8300, 4608, False), (F.MMT4D_TYPE_F32F32F32, "float32", 3, 9001, 264, False),
+])
+def test_scaled_rows_on_either_kernel(uk, cuda, type_flag, dt, M, N, K, narrow):
+    """Both sides of the rule that gives a scaled result of a few rows to the narrow
+    kernel: exact sums of small integers times a power of two."""
+    import torch
+    g = torch.Generator(device="cuda").manual_seed(M + N + K)
+    dt, N1 = getattr(torch, dt), -(-N // 32)
+    k0 = 16 // dt.itemsize
+    x = torch.randint(-3, 4, (M, K), generator=g, device="cuda")
+    w = torch.randint(-3, 4, (N1, K // k0, 32, k0), generator=g, device="cuda")
+    raw = torch.uint8 if dt.itemsize == 1 else dt
+    y = torch.full((M * N + 64,), 7.0, device="cuda")
+    uk.matmul_packed_rhs(x.to(dt).view(raw), w.to(dt).view(raw), y, M, N, K, k0, type_flag, out_scale=0.125)
+    if torch.cuda.get_device_properties(0).multi_processor_count == 256:
+        assert (uk.last_kernel_path() == "mmt4d:mfma-narrow") == narrow
+    want = x.double() @ w.transpose(1, 2).reshape(N1 * 32, K)[:N].double().T.contiguous() * 0.125
+    assert torch.equal(y[:M * N].view(M, N).double(), want) and (y[M * N:] == 7.0).all()
