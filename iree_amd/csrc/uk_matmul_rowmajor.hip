@@ -452,7 +452,7 @@ __global__ __launch_bounds__(kThreads, 4) void matmul_rowmajor_kernel(RowMajorAr
 // chunk c of row r lies at c ^ hash(r) within 16, so that fragment reads, 16 rows of one
 // chunk, and the turned stores hit 16 bank groups). The kernel above sums its 8 waves
 // through LDS whatever K is; where K is a step or two and the result large, that is
-// most of its time. Which of them: square_is_faster.
+// most of its time. Which of them: square_us.
 template <typename Cfg>
 __global__ __launch_bounds__(256, 2) void matmul_rowmajor_square_kernel(RowMajorArgs p) {
   constexpr int kRows = 64;
@@ -626,9 +626,14 @@ struct Estimate {
 
 // What the chain takes: its launches, the packed operands and the result, the
 // matrix instructions, and a share of K (fitted to the same problems, 11 % off on
-// average). The rule: the estimate of one launch is below 0.9 of it; on the other half
-// of the problems that is 1.1 % from the better of the two on average, and one call
-// slower by more than 5 % (f32 2458x1795x18 17.6 us as the chain, 19.3 here).
+// average). Without a packed result (the matmul writes the matrix, and reads the old one
+// when it accumulates) a byte of the result costs a third. The rule: the estimate of one
+// launch is below 0.9 of it. On 2500 other problems (4 to 4200 rows and columns, K 16
+// to 4200) that is 0.4 % from the best of all three on average, 2 % on 1500 of 200
+// rows and columns and more with a K of up to 1200 bytes, where the fastest change with
+// every further round of workgroups (43 of these took over 15 % longer than on the
+// kernels before when both results were taken for two: f16 2945x3940x145 20.9 us as
+// the chain, 32.7 on 64 x 64 tiles; now 3 do).
 // A chain that does not pack A (its matmul reads the matrix, so there are two
 // launches) was not among them; its estimate is from below.
 template <typename Cfg>
@@ -640,39 +645,44 @@ double chain_us(const RowMajorArgs& p) {
     return 5.0 * launches - 1.0 + 0.5e-6 * (rows + cols) * bytes + (f32 < 13 ? f32 : 13);
   }
   const double giga = Cfg::kElemBytes == 4 ? 16.1 : Cfg::kElemBytes == 1 ? 3.0 : 2.8;
-  return 3.17 + 2.40 * launches + 0.48e-6 * (rows + cols) * bytes + 0.62e-6 * rows * cols * sizeof(typename Cfg::out_t) +
+  const double store = p.out ? 0.62 : p.accumulate ? 0.35 : 0.2;
+  return 3.17 + 2.40 * launches + 0.48e-6 * (rows + cols) * bytes + store * 1e-6 * rows * cols * sizeof(typename Cfg::out_t) +
          giga * 1e-9 * rows * cols * p.K + 0.16e-3 * bytes;
 }
 
-// The fastest of both shapes and 1 to max_slices slices of K; false when none takes
-// limit_us or less.
+// The fastest of both shapes and 1 to max_slices slices of K, whose time replaces *us;
+// false when none takes *us or less.
 template <typename Cfg>
-bool choose(const RowMajorArgs& p, int max_slices, double limit_us, int* mb, int* slices) {
+bool choose(const RowMajorArgs& p, int max_slices, double* us, int* mb, int* slices) {
   const int cus = device_cu_count();
+  // (f32 of a short K: its results, several hundred rows and columns, took 1.2 times as long)
+  const double longer = Cfg::kElemBytes == 4 && p.K <= 300 ? 1.2 : 1.0;
   bool found = false;
   for (int rows = 1; rows <= 2; ++rows) {
     const Estimate e = Estimate::of<Cfg>(p, rows, cus);
     for (int n = 1; n <= max_slices && (n == 1 || n * 8 <= e.steps); n *= 2) {
-      const double us = e.us(rows, n);
-      if (us <= limit_us) { found = true; limit_us = us; *mb = rows; *slices = n; }
+      const double t = longer * e.us(rows, n);
+      if (t <= *us) { found = true; *us = t; *mb = rows; *slices = n; }
       if (e.groups * n >= 4 * cus) break;
     }
   }
   return found;
 }
 
-// Results of a workgroup on 64 x 64 for every compute unit and more, and a K of one step of
-// that kernel, f32 (four matrix instructions for the others' one) one and a half. With
-// the packed result stored beside it both are bound by the stores, but for f32. Measured
-// (16 or 32 x 64, 64 x 64), us: f32 1200x1500x100 16.1, 12.5, without the packed result
-// 14.6, 9.9; 651x2125x158 16.5, 15.7 and 14.4, 13.1; 900x1300x300 17.2, 20.9; without the
-// packed result i8 700x2100x500 9.9, 8.4, f16 1200x1500x100 7.4, 7.0; with it 11.0, 10.9
-// and 9.2, 9.7.
+// The kernel on 64 x 64: workgroups beyond one per compute unit run one after the
+// other, each with a fixed part and its share of K; the result, C and the packed
+// operands. Fitted to 2000 problems of up to 1200 bytes of K, 8 to 9 % off on average.
+// 16-bit types have no such kernel: it was the best for 13 of 525 of theirs, f32 203 of 482
+// (1200x1500x100 16.1 us on 16 or 32 x 64, 12.5 here; 900x1300x300 17.2 and 20.9).
 template <typename Cfg>
-bool square_is_faster(const RowMajorArgs& p) {
-  const int64_t tiles = ceil_div((int64_t)p.M1 * p.M0, (int64_t)64) * ceil_div((int64_t)p.N1 * p.N0, (int64_t)64);
-  const int bytes = p.K * Cfg::kElemBytes;
-  return tiles >= device_cu_count() && (Cfg::kElemBytes == 4 ? bytes <= 768 : !p.out && bytes <= 512);
+double square_us(const RowMajorArgs& p) {
+  constexpr bool kF32 = Cfg::kElemBytes == 4;
+  const double rows = (double)p.M1 * p.M0, cols = (double)p.N1 * p.N0, bytes = (double)p.K * Cfg::kElemBytes;
+  const double load = std::fmax(1.0, std::ceil(rows / 64) * std::ceil(cols / 64) / device_cu_count());
+  const double out_mb = rows * cols * 4e-6;
+  return (kF32 ? 3.82 : 4.50) + load * ((kF32 ? 0.32 : 0.81) + (kF32 ? 3.47 : 2.49) / 512 * bytes) +
+         (p.out ? 1.36 : 0.0) + (kF32 ? 0.205 : 0.221) * out_mb * (p.out ? 2 : 1) + (p.accumulate ? 0.42 * out_mb : 0.0) +
+         (kF32 ? 0.62e-6 : 0.45e-6) * (rows + cols) * bytes;
 }
 
 template <typename Cfg>
@@ -695,10 +705,14 @@ int launch(RowMajorArgs p, hipStream_t s) {
   // they take 2.0 to 3.5 us less: 1500 x 1501 x 1502 int8 26.4 -> 22.9 us in all)
   const double chain = chain_us<Cfg>(p);
   const bool together = p.lhs && p.rhs && p.M0 == 32 && p.N0 == 32 && (Cfg::kElemBytes != 2 || p.N % 4096 != 0);
-  const double limit = together && chain < 24.0 ? chain - 2.4 : 0.9 * chain;
+  const double limit = together && p.out && chain < 24.0 ? chain - 2.4 : 0.9 * chain;
   int mb = 1, slices = 1;
-  if (!choose<Cfg>(p, 16, limit, &mb, &slices)) return IREE_AMD_UK_STATUS_NOT_FOUND;
-  if (square_is_faster<Cfg>(p)) return launch_square<Cfg>(p, s);
+  double us = limit;
+  const bool found = choose<Cfg>(p, 16, &us, &mb, &slices);
+  if constexpr (Cfg::kElemBytes != 2) {
+    if (p.K * Cfg::kElemBytes <= 1200 && square_us<Cfg>(p) < us) return launch_square<Cfg>(p, s);
+  }
+  if (!found) return IREE_AMD_UK_STATUS_NOT_FOUND;
   auto lay_out = [&] {
     p.tiles_n = (int)ceil_div(cols, (int64_t)64);
     p.tiles = (int)(ceil_div(rows, (int64_t)mb * 16) * p.tiles_n);
@@ -711,7 +725,8 @@ int launch(RowMajorArgs p, hipStream_t s) {
   const bool may_split = slices > 1 && !scratch_under_capture(s);
   ScratchLease lease(s, may_split ? (size_t)slices * p.tiles * mb * 4096 : 0);
   if (slices > 1 && !lease.ptr()) {
-    if (!choose<Cfg>(p, 1, limit, &mb, &slices)) return IREE_AMD_UK_STATUS_NOT_FOUND;
+    us = limit;
+    if (!choose<Cfg>(p, 1, &us, &mb, &slices)) return IREE_AMD_UK_STATUS_NOT_FOUND;
     lay_out();
   }
   const int64_t plane = (int64_t)p.tiles * mb * 1024;

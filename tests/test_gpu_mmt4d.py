@@ -1800,3 +1800,26 @@ def test_scaled_rows_on_either_kernel(uk, cuda, type_flag, dt, M, N, K, narrow):
         assert (uk.last_kernel_path() == "mmt4d:mfma-narrow") == narrow
     want = x.double() @ w.transpose(1, 2).reshape(N1 * 32, K)[:N].double().T.contiguous() * 0.125
     assert torch.equal(y[:M * N].view(M, N).double(), want) and (y[M * N:] == 7.0).all()
+
+
+@pytest.mark.parametrize("type_flag,dt,out_dt,M,N,K,path", [
+    (F.MMT4D_TYPE_F16F16F32, "float16", "float32", 2945, 3940, 145, "mmt4d:mfma"),
+    (F.MMT4D_TYPE_S8S8S32, "int8", "int32", 3357, 3403, 44, "mmt4d:mfma"),
+    (F.MMT4D_TYPE_F16F16F32, "float16", "float32", 1200, 1500, 100, "mmt4d:mfma-one-launch"),
+    (F.MMT4D_TYPE_F32F32F32, "float32", "float32", 692, 1150, 96, "mmt4d:mfma-one-launch"),
+    (F.MMT4D_TYPE_S8S8S32, "int8", "int32", 1669, 974, 300, "mmt4d:mfma-one-launch"),
+])
+def test_large_result_of_a_short_k_without_its_packed_form(uk, cuda, type_flag, dt, out_dt, M, N, K, path):
+    """The result is stored once: from some size on the chain of two launches is the
+    faster, below it the kernels on 16, 32 or 64 x 64."""
+    import torch
+    g = torch.Generator(device="cuda").manual_seed(M + N + K)
+    a = torch.randint(-2, 3, (M * K,), generator=g, device="cuda").to(getattr(torch, dt))
+    b = torch.randint(-2, 3, (K * N,), generator=g, device="cuda").to(getattr(torch, dt))
+    c = torch.zeros(M * N, dtype=getattr(torch, out_dt), device="cuda")
+    step = c.clone()
+    uk.matmul_data_tiled(a, b, c, M, N, K, type_flag, fuse_unpack=True)
+    if torch.cuda.get_device_properties(0).multi_processor_count == 256:
+        assert uk.last_kernel_path() == path
+    uk.matmul_data_tiled(a, b, step, M, N, K, type_flag, fuse_unpack=True, one_launch=False)
+    assert torch.equal(c, step)
