@@ -415,7 +415,6 @@ int launch_estimated(const MfmaArgs& a, hipStream_t s) {
   };
   double best_us = 0;
   const int best = pick(a.M, a.N, &best_us);
-  bool split_wins = false;
   // K over workgroup rows: at most one round, slices of 768 elements and more
   // of K; it has to win by 3 %. iree_amd_uk_mmt4d_noalloc_p runs the same kernels
   // and refuses a split whose partial sums its array does not hold, so on
@@ -454,12 +453,11 @@ int launch_estimated(const MfmaArgs& a, hipStream_t s) {
     const bool worth = a.ksteps >= 64 && whole_tiles * 2 <= (int64_t)whole.occ * cus;
     if (split.n > 1 && (worth || !scratch_under_capture(s))) {
       if (other_wins(a, straightened_us(split.us))) return kSlowerThanOther;
-      split_wins = true;
       const int st = launch_k_split<Cfg>(a, split.v, split.n, s);
-      if (st != IREE_AMD_UK_STATUS_NOT_FOUND) return st;
+      if (st != IREE_AMD_UK_STATUS_NOT_FOUND) return st;     // (without scratch memory: whole, or the other kernel)
     }
   }
-  if (!split_wins && other_wins(a, straightened_us(best_us))) return kSlowerThanOther;
+  if (other_wins(a, straightened_us(best_us))) return kSlowerThanOther;
   const int st = launch_whole_rounds<Cfg, false>(a, cus, best_us, us_of, pick, s);
   if (st != IREE_AMD_UK_STATUS_NOT_FOUND) return st;
   return launch_by_index<Cfg, false>(best, a, s);
@@ -547,7 +545,6 @@ int launch_costed(const MfmaArgs& a, hipStream_t s) {
     const int64_t tiles = ceil_div((int64_t)a.M, (int64_t)2 * t.wm) * ceil_div((int64_t)a.N, (int64_t)2 * t.wn) * n;
     return other_wins(a, costed_us<Cfg, kSiluMul>(a, t.wm, t.wn, t.occ, tiles, steps / n, n, cus));
   };
-  bool split_wins = false;
   // Few macro tiles and a long K (a few hundred rows against a wide K, as in the
   // down projection of an MLP at small batch) leave most compute units idle:
   // K is then split over workgroup rows. Estimated times in microseconds: cost
@@ -582,13 +579,12 @@ int launch_costed(const MfmaArgs& a, hipStream_t s) {
       if (split_n > 1) {
         if (other_is_faster(split_v, split_n)) return kSlowerThanOther;
         if (a.compare_only) return kSplitsK;
-        split_wins = true;
         const int st = launch_k_split<Cfg>(a, split_v, split_n, s);
-        if (st != IREE_AMD_UK_STATUS_NOT_FOUND) return st;
+        if (st != IREE_AMD_UK_STATUS_NOT_FOUND) return st;   // (without scratch memory: whole, or the other kernel)
       }
     }
   }
-  if (!split_wins && other_is_faster(best, 1)) return kSlowerThanOther;
+  if (other_is_faster(best, 1)) return kSlowerThanOther;
   if (a.compare_only) return 0;
   {
     const int st = launch_whole_rounds<Cfg, kSiluMul>(

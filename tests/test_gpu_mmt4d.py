@@ -1823,3 +1823,31 @@ def test_large_result_of_a_short_k_without_its_packed_form(uk, cuda, type_flag, 
         assert uk.last_kernel_path() == path
     uk.matmul_data_tiled(a, b, step, M, N, K, type_flag, fuse_unpack=True, one_launch=False)
     assert torch.equal(c, step)
+
+
+@pytest.mark.parametrize("type_flag,dt,M1,N1,K1", [
+    (F.MMT4D_TYPE_S8S8S32, "int8", 3, 181, 560), (F.MMT4D_TYPE_F16F16F32, "float16", 4, 193, 245),
+    (F.MMT4D_TYPE_F8E4M3F8E4M3F32, "float8_e4m3fn", 1, 69, 1136), (F.MMT4D_TYPE_F32F32F32, "float32", 22, 31, 1046),
+])
+def test_k_split_without_scratch_memory(uk, cuda, type_flag, dt, M1, N1, K1):
+    """Problems whose K is split over workgroups, on a stream that gets no scratch
+    memory (the per-thread one): the kernel for few tiles, which needs none, where that
+    beats the whole macro tiles; exact sums of small integers on both."""
+    import torch
+    import types
+    g = torch.Generator(device="cuda").manual_seed(M1 + N1 + K1)
+    dt = getattr(torch, dt)
+    k0 = 16 // dt.itemsize
+    raw = torch.uint8 if dt is torch.float8_e4m3fn else dt
+    lhs, rhs = (torch.randint(-1, 2, (n, K1, 32, k0), generator=g, device="cuda").to(dt).view(raw) for n in (M1, N1))
+    want, got = (torch.zeros(M1, N1, 32, 32, dtype=torch.int32 if dt is torch.int8 else torch.float32, device="cuda") for _ in range(2))
+    on_256 = torch.cuda.get_device_properties(0).multi_processor_count == 256
+    uk.mmt4d(lhs, rhs, want, M1, N1, K1, 32, 32, k0, type_flag)
+    assert uk.last_macro_tile()[2] > 1 or not on_256
+    torch.cuda.synchronize()
+    uk.mmt4d(lhs, rhs, got, M1, N1, K1, 32, 32, k0, type_flag, stream=types.SimpleNamespace(cuda_stream=2))
+    assert uk.last_macro_tile()[0] < 128 or not on_256
+    torch.cuda.synchronize()
+    assert torch.equal(got, want)
+    row, col = lhs.view(dt)[0].transpose(0, 1).reshape(32, -1), rhs.view(dt)[N1 - 1].transpose(0, 1).reshape(32, -1)
+    assert torch.equal(got[0, N1 - 1].double(), row.double() @ col.double().T.contiguous())
