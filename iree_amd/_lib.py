@@ -8,6 +8,8 @@ import ctypes as C
 import importlib.machinery
 import importlib.util
 import os
+import sys
+import sysconfig
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
 _LIB_NAME = "libiree_amd_uk.so"
@@ -218,12 +220,14 @@ def _declare(lib):
 def _bind_builtins(lib):
     """Puts csrc/uk_python.so's builtins in the place of the ctypes functions that
     they stand for (the same arguments, less time per call); the one of
-    query_matmul_tile_sizes, which returns the tile, is lib.matmul_tile."""
+    query_matmul_tile_sizes, which returns the tile, is lib.matmul_tile. Where that
+    module was not built (it needs Python's headers), or the interpreter cannot load
+    it (its ABI is CPython's limited one of 3.10), the ctypes functions stay."""
     path = os.path.join(_HERE, "csrc", "uk_python.so")
-    if not os.path.exists(path):
-        raise RuntimeError(
-            f"{path} is missing: the extension has not been built "
-            "(run `python -m iree_amd.build`).")
+    lib.matmul_tile = lambda *args: None
+    if not os.path.exists(path) or sys.implementation.name != "cpython" or sys.version_info < (3, 10) or \
+            sysconfig.get_config_var("Py_GIL_DISABLED"):
+        return
     loader = importlib.machinery.ExtensionFileLoader("uk_python", path)
     module = importlib.util.module_from_spec(importlib.util.spec_from_loader("uk_python", loader))
     loader.exec_module(module)

@@ -1,5 +1,5 @@
 """Builds the C-ABI library (iree_amd/csrc/libiree_amd_uk.so), its calls as
-builtins of this interpreter (iree_amd/csrc/uk_python.so) and the code object of
+builtins of CPython (iree_amd/csrc/uk_python.so) and the code object of
 the mmt4d kernels for a HAL executable
 (iree_amd/hal/mi355x_kernels_gfx950.co) for gfx950.
 
@@ -17,7 +17,7 @@ CSRC = os.path.join(HERE, "csrc")
 
 
 def build(force=False, jobs=8, quiet=False):
-    cmd = ["make", "-C", CSRC, f"-j{jobs}", f"PYTHON={sys.executable}"]
+    cmd = ["make", "-C", CSRC, f"-j{jobs}", "all", "python", f"PYTHON={sys.executable}"]
     if force:
         cmd.append("-B")
     out = subprocess.DEVNULL if quiet else None

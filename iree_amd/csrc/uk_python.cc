@@ -8,7 +8,9 @@
 // it stands, so everything that was accepted is, and what is refused is refused by
 // the same code. The interpreter lock is released around the function, as ctypes does.
 // The module links against neither the library nor torch: bind() receives addresses.
+// It keeps to the limited API, so that one binary serves every CPython from 3.10 on.
 #define PY_SSIZE_T_CLEAN
+#define Py_LIMITED_API 0x030A0000
 #include <Python.h>
 
 #include <stdint.h>
@@ -36,12 +38,24 @@ bool convert(PyObject* v, T& out) {
     out = (T)(uintptr_t)PyLong_AsUnsignedLongLongMask(v);
   } else if constexpr (std::is_floating_point<T>::value) {
     if (!PyFloat_CheckExact(v)) return false;
-    out = (T)PyFloat_AS_DOUBLE(v);
+    out = (T)PyFloat_AsDouble(v);
   } else {
     if (!PyLong_CheckExact(v)) return false;
     out = (T)PyLong_AsUnsignedLongLongMask(v);
   }
   return true;
+}
+
+PyObject* pass_on(const Bound* b, PyObject* const* args, Py_ssize_t n) {
+  PyObject* tuple = PyTuple_New(n);
+  if (!tuple) return nullptr;
+  for (Py_ssize_t i = 0; i < n; ++i) {
+    Py_INCREF(args[i]);
+    PyTuple_SetItem(tuple, i, args[i]);      // (takes the reference)
+  }
+  PyObject* result = PyObject_CallObject(b->ctypes_function, tuple);
+  Py_DECREF(tuple);
+  return result;
 }
 
 template <typename Function>
@@ -51,8 +65,7 @@ struct Entry<int (*)(A...)> {
   template <size_t... I>
   static PyObject* run(const Bound* b, PyObject* const* args, Py_ssize_t n, std::index_sequence<I...>) {
     std::tuple<std::remove_const_t<A>...> a;
-    if (n != (Py_ssize_t)sizeof...(A) || !(convert(args[I], std::get<I>(a)) && ...))
-      return PyObject_Vectorcall(b->ctypes_function, args, (size_t)n, nullptr);
+    if (n != (Py_ssize_t)sizeof...(A) || !(convert(args[I], std::get<I>(a)) && ...)) return pass_on(b, args, n);
     int status;
     Py_BEGIN_ALLOW_THREADS
     status = ((int (*)(A...))b->function)(std::get<I>(a)...);
@@ -123,7 +136,7 @@ void release(PyObject* capsule) {
 
 // bind(name, address, ctypes function): the builtin.
 PyObject* bind(PyObject*, PyObject* const* args, Py_ssize_t n) {
-  const char* name = n == 3 ? PyUnicode_AsUTF8(args[0]) : nullptr;
+  const char* name = n == 3 ? PyUnicode_AsUTF8AndSize(args[0], nullptr) : nullptr;
   void* function = name && PyLong_CheckExact(args[1]) ? PyLong_AsVoidPtr(args[1]) : nullptr;
   if (!function) {
     if (!PyErr_Occurred()) PyErr_SetString(PyExc_TypeError, "bind(name, address, function) expected");

@@ -5,6 +5,7 @@ import ctypes as C
 import os
 import re
 import subprocess
+import sys
 import tempfile
 
 import pytest
@@ -428,3 +429,21 @@ def test_builtins_pass_their_arguments_as_ctypes_does(values):
     assert len(seen) in (0, 2) and seen[:1] == seen[1:]
     with pytest.raises(KeyError):
         module.bind("iree_amd_uk_version", 16, function)
+
+
+def test_without_the_builtins_the_ctypes_functions_stay(monkeypatch):
+    """Where uk_python.so was not built, or the interpreter is not one that it was built
+    for, the library loads and its calls are the ctypes functions."""
+    from iree_amd import _lib
+    want = iree_amd.query_matmul_tile_sizes(F.QUERY_OP_MATMUL_I8I8I32, 5, 100, 100)
+    exists = os.path.exists
+    for name, value in ((os.path, lambda path: not path.endswith("uk_python.so") and exists(path)), (sys, (3, 9, 0))):
+        with monkeypatch.context() as m:
+            m.setattr(name, "exists" if name is os.path else "version_info", value)
+            lib = C.CDLL(_lib.library_path())
+            _lib._declare(lib)
+            _lib._bind_builtins(lib)
+            assert isinstance(lib.iree_amd_uk_mmt4d, lib._FuncPtr)
+            m.setattr(_lib, "_lib", lib)
+            assert iree_amd.query_matmul_tile_sizes(F.QUERY_OP_MATMUL_I8I8I32, 5, 100, 100) == want
+    assert not isinstance(iree_amd.load_library().iree_amd_uk_mmt4d, lib._FuncPtr)
