@@ -821,7 +821,9 @@ KSPLIT_TYPES = [(F.MMT4D_TYPE_S8S8S32, 16, 32), (F.MMT4D_TYPE_F16F16F32, 8, 32),
 def test_k_split_shapes_bit_exact(uk, cuda, type_flag, K0, mfma_k):
     """Outer shapes of a few tiles with 70 to 200 matrix-core K-steps (plus a
     partial last one where K0 allows it), tiled result, with and without
-    accumulate: the bits of the oracle (every partial sum is exact)."""
+    accumulate: the bits of the oracle (every partial sum is exact). K0 of 16 bytes
+    runs on the kernel that deals K to the waves, K0 of 32 splits K over workgroups
+    (as the problems of test_forms_of_a_k_split do)."""
     rng = np.random.default_rng(9100 + type_flag + K0)
     tps = mfma_k // K0
     for (M, N, steps), acc in itertools.product([(8, 16, 128), (3, 5, 70), (1, 40, 200)], (False, True)):
@@ -838,9 +840,9 @@ def test_k_split_shapes_bit_exact(uk, cuda, type_flag, K0, mfma_k):
                                                     (F.MMT4D_TYPE_F32F32F32, 4, 8, np.float32)])
 @pytest.mark.parametrize("accumulate", [False, True])
 def test_k_split_row_major_forms_equal_the_three_call_chain(uk, cuda, type_flag, K0, mfma_k, dt, accumulate):
-    """The fused forms on a K-split shape (200 x 333, 96 K-steps) with random
-    data: mmt4d_unpack and matmul_packed_rhs give the bits of pack + mmt4d +
-    unpack (all three split alike and add the slices in the same order), and
+    """The fused forms on a shape whose K is dealt to waves (200 x 333, 96 K-steps) with
+    random data: mmt4d_unpack and matmul_packed_rhs give the bits of pack + mmt4d +
+    unpack (all three deal K alike and add the sums in the same order), and
     within the stated tolerance of a float64 matmul."""
     import torch
     M, N, K = 200, 333, 96 * mfma_k
@@ -896,8 +898,8 @@ def test_k_split_scratch_grows_and_is_kept_per_stream(uk, cuda):
     streams = [torch.cuda.Stream(), torch.cuda.Stream()]
     rng = np.random.default_rng(5)
     jobs = []
-    # 16 MiB is the smallest buffer: 4 slices of 40 x 40 tiles need 26 MiB, 4 of 64 x 48 need 50
-    for idx, (M1, N1, K1) in enumerate([(2, 3, 256), (40, 40, 256), (1, 2, 512), (64, 48, 256), (40, 40, 256)]):
+    # 16 MiB is the smallest buffer: 4 slices of 8 x 128 tiles need 16, 5 of 40 x 40 31, 3 of 56 x 76 49
+    for idx, (M1, N1, K1) in enumerate([(8, 128, 896), (40, 40, 1024), (24, 24, 1024), (56, 76, 1024), (40, 40, 1024)]):
         A = rng.integers(-128, 128, (M1 * 32, K1 * 16), dtype=np.int8)
         B = rng.integers(-128, 128, (N1 * 32, K1 * 16), dtype=np.int8)
         a_dev, b_dev = torch.from_numpy(A).cuda(), torch.from_numpy(B).cuda()
@@ -914,13 +916,14 @@ def test_k_split_scratch_grows_and_is_kept_per_stream(uk, cuda):
             with torch.cuda.stream(st):
                 uk.matmul_packed_rhs(a_dev, rhs, out, M1 * 32, N1 * 32, K1 * 16, 16, F.MMT4D_TYPE_S8S8S32,
                                      stream=st)
+            assert uk.last_macro_tile()[2] > 1 or torch.cuda.get_device_properties(0).multi_processor_count != 256
             outs.append(out)
         jobs.append((A, B, outs, a_dev, rhs))
     torch.cuda.synchronize()
-    for A, B, outs, _, _ in jobs:
-        want = A.astype(np.int32) @ B.astype(np.int32).T
+    for A, B, outs, a_dev, _ in jobs:
+        want = (a_dev.double() @ torch.from_numpy(B).cuda().double().T.contiguous()).int()     # (exact)
         for out in outs:
-            assert np.array_equal(out.cpu().numpy().reshape(want.shape), want)
+            assert torch.equal(out.view(want.shape), want)
     # the cached buffers can be given back (what a plugin's unload does) and
     # come back on demand
     lib = uk.load_library()
@@ -1410,13 +1413,14 @@ def test_small_matmul_with_long_k_in_a_graph(uk, cuda, type_flag, dt, out_dt):
 @pytest.mark.parametrize("M0", [32, 2])
 def test_k_split_in_a_graph(uk, cuda, type_flag, K0, dt, out_dt, M0):
     """A K split whose buffer existed at the capture: replays are right after the
-    stream has grown its buffer, and one captured on a stream without a buffer
-    runs whole. (With f16 and i8, M0 = 32, the second one's K is too short for a
-    split in a capture.) Small integers: exact in any order."""
+    stream has grown its buffer, and one captured on a stream without a buffer, of a
+    shorter K, runs whole (M0 = 32: or on the kernel for few tiles). Small integers:
+    exact in any order."""
     import torch
     dt, out_dt = getattr(torch, dt), getattr(torch, out_dt)
     g = torch.Generator(device="cuda").manual_seed(M0 + K0)
-    M1, N1 = (4, 4) if M0 == 32 else (1, 4)
+    # (narrow: beyond what the kernel for few tiles takes; that one notes its tile, this one does not)
+    M1, N1, long_k = {8: (10, 66, 8208), 16: (3, 181, 8960), 4: (22, 31, 4184)}[K0] if M0 == 32 else (1, 4, 1024 * K0)
 
     def problem(K):
         lhs = torch.randint(-2, 3, (M1, K // K0, M0, K0), generator=g, device="cuda").to(dt)
@@ -1431,10 +1435,14 @@ def test_k_split_in_a_graph(uk, cuda, type_flag, K0, dt, out_dt, M0):
         b = rhs.permute(0, 2, 1, 3).reshape(N1 * 32, -1).double().t().contiguous()
         return (a @ b).reshape(M1, M0, N1, 32).transpose(1, 2).to(out_dt)
     warm, cold = torch.cuda.Stream(), torch.cuda.Stream()
-    first, second = problem(8192), problem(1536)
+    first, second = problem(long_k), problem(1536)
     torch.cuda.synchronize()
     with torch.cuda.stream(warm):
+        before = uk.last_macro_tile()
         call(*first)
+    tile = uk.last_macro_tile()
+    if torch.cuda.get_device_properties(0).multi_processor_count == 256:
+        assert tile[2] > 1 if M0 == 32 else tile == before
     warm.synchronize()
     graphs = torch.cuda.CUDAGraph(), torch.cuda.CUDAGraph()
     with torch.cuda.graph(graphs[0], stream=warm):
@@ -1851,3 +1859,95 @@ def test_k_split_without_scratch_memory(uk, cuda, type_flag, dt, M1, N1, K1):
     assert torch.equal(got, want)
     row, col = lhs.view(dt)[0].transpose(0, 1).reshape(32, -1), rhs.view(dt)[N1 - 1].transpose(0, 1).reshape(32, -1)
     assert torch.equal(got[0, N1 - 1].double(), row.double() @ col.double().T.contiguous())
+
+
+@pytest.mark.parametrize("type_flag,dt,M1,N1,K1", [
+    (F.MMT4D_TYPE_S8S8S32, "int8", 3, 181, 560), (F.MMT4D_TYPE_F16F16F32, "float16", 10, 66, 1027),
+    (F.MMT4D_TYPE_F8E4M3F8E4M3F32, "float8_e4m3fn", 1, 69, 1137), (F.MMT4D_TYPE_F32F32F32, "float32", 22, 31, 1047),
+])
+@pytest.mark.parametrize("accumulate", [False, True])
+def test_forms_of_a_k_split(uk, cuda, type_flag, dt, M1, N1, K1, accumulate):
+    """Problems that K is split for (a last slice and a last step that are not whole):
+    mmt4d, its fused unpack on a ragged matrix and the entry point that allocates
+    nothing split alike, with the same bits, within the rounding of f32 sums (fp8:
+    of its instruction, 2e-5 of the terms) of a float64 product."""
+    import torch
+    lib = uk.load_library()
+    g = torch.Generator(device="cuda").manual_seed(M1 + N1 + K1)
+    dt = getattr(torch, dt)
+    k0, out_dt = 16 // dt.itemsize, torch.int32 if dt is torch.int8 else torch.float32
+    raw = torch.uint8 if dt is torch.float8_e4m3fn else dt
+    lhs, rhs = ((torch.randint(-128, 128, (n, K1, 32, k0), generator=g, device="cuda") if dt is torch.int8 else
+                 torch.randn(n, K1, 32, k0, generator=g, device="cuda")).to(dt).view(raw) for n in (M1, N1))
+    init = torch.randint(-9, 10, (M1, N1, 32, 32), generator=g, device="cuda").to(out_dt)
+    flags = type_flag | (F.MMT4D_ACCUMULATE if accumulate else 0)
+    tiled, other = init.clone(), init.clone()
+    uk.mmt4d(lhs, rhs, tiled, M1, N1, K1, 32, 32, k0, flags)
+    split = uk.last_macro_tile()
+    assert split[2] > 1 or torch.cuda.get_device_properties(0).multi_processor_count != 256
+    p = uk._lib.Mmt4dParams(lhs.data_ptr(), 0, K1 * 32 * k0, rhs.data_ptr(), 0, K1 * 32 * k0, other.data_ptr(), 0, N1 * 1024,
+                            M1, N1, K1, 32, 32, k0, flags, None)
+    assert lib.iree_amd_uk_mmt4d_noalloc_p(C.byref(p), C.c_void_p(torch.cuda.current_stream().cuda_stream)) == 0
+    assert uk.last_macro_tile() == split and torch.equal(other, tiled)
+    M, N = M1 * 32 - 5, N1 * 32 - 7
+    matrix = tiled.transpose(1, 2).reshape(M1 * 32, N1 * 32)
+    fused = init.transpose(1, 2).reshape(M1 * 32, N1 * 32)[:M, :N].contiguous()
+    uk.mmt4d_unpack(lhs, rhs, fused, M, N, M1, N1, K1, k0, flags)
+    assert uk.last_macro_tile() == split and torch.equal(fused, matrix[:M, :N])
+    a, b = (t.view(dt).transpose(1, 2).reshape(-1, K1 * k0).double() for t in (lhs, rhs))
+    want = a @ b.T.contiguous() + (init.transpose(1, 2).reshape(M1 * 32, -1).double() if accumulate else 0)
+    if dt is torch.int8:
+        assert torch.equal(matrix.double(), want)
+    else:
+        size = a.abs() @ b.abs().T.contiguous() + 9
+        assert ((matrix.double() - want).abs() <= (2e-5 if dt is torch.float8_e4m3fn else 2e-6) * size).all()
+
+
+@pytest.mark.parametrize("form", ["tiled", "row_major", "narrow"])
+@pytest.mark.parametrize("type_flag,dt", [(F.MMT4D_TYPE_F16F16F32, "float16"), (F.MMT4D_TYPE_BF16BF16F32, "bfloat16"),
+                                          (F.MMT4D_TYPE_F32F32F32, "float32"), (F.MMT4D_TYPE_F8E4M3F8E4M3F32, "float8_e4m3fn")])
+@pytest.mark.parametrize("M,N1,K1", [(33, 3, 69), (70, 47, 132), (130, 44, 388), (200, 47, 260)])
+def test_few_tiles_on_random_data_with_infinities(uk, cuda, type_flag, dt, form, M, N1, K1):
+    """K dealt to the waves, K and rows that end inside the tile, operands N(0, 1): within
+    the rounding of f32 sums (2e-6 of the sum of the terms' sizes; fp8: of its
+    instruction, 2e-5) of a float64 product; an infinity and a NaN (fp8: a NaN) in the
+    last existing row, column and K, and only where they belong."""
+    import torch
+    g = torch.Generator(device="cuda").manual_seed(M + N1 + K1)
+    dt = getattr(torch, dt)
+    k0, fp8 = 16 // dt.itemsize, dt is torch.float8_e4m3fn
+    if form == "narrow":
+        M, N1, K1 = M // 12, min(N1, 5), K1 // 4 * 4 + 3
+    elif form == "row_major":
+        K1 = K1 // 4 * 4                # (whole matrix-core steps)
+    N, K, M1 = N1 * 32 - 3, K1 * k0, -(-M // 32)
+    a, b = torch.randn(M, K, generator=g, device="cuda"), torch.randn(N1 * 32, K, generator=g, device="cuda")
+    a[M - 1, K - 1], b[N - 1, K - 1], a[0, 5] = float("nan" if fp8 else "inf"), float("nan"), float("nan" if fp8 else "-inf")
+    a, b = a.to(dt), b.to(dt)
+    raw = torch.uint8 if fp8 else dt
+    rhs = b.view(raw).view(N1, 32, K1, k0).transpose(1, 2).contiguous()
+    c = torch.full((M1 * 32 + 1, N1 * 32), 7.0, device="cuda")
+    if form == "narrow":
+        lhs = a.view(raw).view(M, K1, k0).transpose(0, 1).contiguous()
+        out = torch.zeros(N1, M, 32, device="cuda")
+        uk.mmt4d(lhs, rhs, out, 1, N1, K1, M, 32, k0, type_flag)
+        got = out.transpose(0, 1).reshape(M, -1)[:, :N]
+    else:
+        if form == "row_major":
+            uk.matmul_packed_rhs(a.view(raw), rhs, c, M, N, K, k0, type_flag, out_stride0=N1 * 32)
+        else:
+            lhs = torch.zeros(M1 * 32, K, dtype=raw, device="cuda")
+            lhs[:M] = a.view(raw)
+            lhs = lhs.view(M1, 32, K1, k0).transpose(1, 2).contiguous()
+            uk.mmt4d_unpack(lhs, rhs, c, M, N, M1, N1, K1, k0, type_flag, out_stride0=N1 * 32)
+        assert (c[M:] == 7.0).all() and (c[:M, N:] == 7.0).all()
+        got = c[:M, :N]
+    if torch.cuda.get_device_properties(0).multi_processor_count == 256:
+        assert uk.last_macro_tile()[0] < 128
+    a, b = a.double(), b.double()[:N]
+    want = a @ b.T.contiguous()
+    assert torch.equal(got.isnan(), want.isnan()) and torch.equal(got.isinf(), want.isinf())
+    assert torch.equal(got[got.isinf()].double(), want[want.isinf()]) and want.isnan().sum() >= M
+    finite = want.isfinite()
+    size = a.nan_to_num(0, 0, 0).abs() @ b.nan_to_num(0, 0, 0).abs().T.contiguous()
+    assert ((got.double() - want).abs() <= (2e-5 if fp8 else 2e-6) * size)[finite].all() and finite.sum() >= (M - 2) * (N - 1)

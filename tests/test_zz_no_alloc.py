@@ -25,8 +25,9 @@ def _run(entry, case, lhs, rhs, out_init):
 
 def test_noalloc_mmt4d_equals_the_allocating_entry_point(uk, cuda):
     """Two calls in a row per type, the second with a smaller input (the array
-    keeps the first call's partial sums): K-split shapes, whose kernels use the
-    scratch memory, and one unsplit shape. Bit-exact against
+    keeps the first call's partial sums): shapes of few tiles, whose K is dealt to
+    waves, narrow ones, whose K split uses the scratch memory, and one unsplit shape
+    (K splits of full tiles: test_forms_of_a_k_split). Bit-exact against
     iree_amd_uk_mmt4d_p (the same kernels and the same split, so even float
     sums agree to the bit) and against the oracle on exact inputs; no device
     memory is allocated by the calls."""
@@ -37,7 +38,7 @@ def test_noalloc_mmt4d_equals_the_allocating_entry_point(uk, cuda):
                                   (F.MMT4D_TYPE_F8E4M3F8E4M3F32, 16, 64)):
         tps = mfma_k // K0
         # (outer rows, outer columns, matrix-core K steps): 8 x 16 x 128 and
-        # 3 x 5 x 70 split K; 20 x 20 x 12 does not; the narrow tile splits K
+        # 3 x 5 x 70 deal K to waves; 20 x 20 x 12 does not; the narrow tile splits K
         # through the dense form of the same buffer
         shapes = [(8, 16, 128, 32, True), (3, 5, 70, 32, False), (20, 20, 12, 32, True),
                   (1, 40, 600, 8, False), (1, 9, 300, 8, True)]
@@ -60,7 +61,7 @@ def test_noalloc_mmt4d_equals_the_allocating_entry_point(uk, cuda):
 
 
 def test_noalloc_mmt4d_on_random_data_and_beyond_the_limit(uk, cuda):
-    """N(0,1) f16 operands on a K-split shape: the bits of iree_amd_uk_mmt4d_p
+    """N(0,1) f16 operands on shapes of few tiles: the bits of iree_amd_uk_mmt4d_p
     and within 1e-2 relative / 1e-3 absolute of the float64 oracle. A K split
     whose partial sums exceed the array is refused with RESOURCE_EXHAUSTED
     before anything runs; the next call works."""
