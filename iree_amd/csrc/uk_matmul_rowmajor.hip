@@ -341,7 +341,6 @@ __device__ __forceinline__ void multiply_tile(const RowMajorArgs& p) {
       last.b[e] = load_columns((uint32_t)k * b_row + (uint32_t)n_at * kElemBytes, 0);
     }
   }
-  Step ring[D];
   const int rounds = steps > wave ? (steps - wave - 1) / kWaves + 1 : 0;      // steps of this wave
   if (rounds > 0) {
     Step ring[D];
