@@ -219,7 +219,8 @@ IREE_AMD_UK_EXPORT int iree_amd_uk_mmt4d_noalloc_p(
  * :165-245 ConvertBatchMmt4DtoMmt4DPattern), so every entry has the result of
  * iree_amd_uk_mmt4d_p on it: exactly for integers; float sums may be added in
  * another order where the single call splits a K that the batch keeps whole (over
- * workgroups, or over the waves of one: most problems of few tiles).
+ * workgroups, or over the waves of one: most problems of few tiles) or the other way
+ * round (narrow tiles, whose columns are counted over all entries).
  * Matrix-core tiles (M0 = 32, and the narrow ones, M = 1 and M0 < 32) whose
  * batch strides are whole 16 bytes run as ONE launch (batch entries are planes
  * of the grid; it allocates nothing). A K that the narrow tiles cannot keep
@@ -622,9 +623,9 @@ IREE_AMD_UK_EXPORT int iree_amd_uk_batch_mmt4d_unpack(
  * otherwise; use the three-call sequence then): K a multiple of the
  * matrix-core K extent (32 for f16/bf16 and i8, 8 for f32, 64 for fp8),
  * K0 as served by iree_amd_uk_mmt4d, 16-byte aligned lhs rows and rhs tiles.
- * Bit-identical to pack + mmt4d + unpack where neither or both split K alike
- * (integers always; else float sums come in another order: the split is chosen
- * for the row-major operand). Up to 24 rows (32 of 1-byte elements: a decode step)
+ * Bit-identical to pack + mmt4d + unpack where neither or both split K alike, over
+ * workgroups or the waves of one (integers always; else float sums come in another
+ * order: the split is chosen for the row-major operand). Up to 24 rows (32 of 1-byte elements: a decode step)
  * with a K of up to 4096 elements of 2 bytes (8192 of 1 byte) run the kernel
  * for narrow left-hand side tiles on the rows themselves from 8193 columns on (float
  * sums then come in that kernel's order: the bits of mmt4d on M0 = M tiles), with
@@ -655,8 +656,11 @@ IREE_AMD_UK_EXPORT int iree_amd_uk_matmul_packed_rhs(
  * small problem come in another order (a captured call's, whose K stays whole, in a
  * third), with an error no larger.
  * Returns IREE_AMD_UK_STATUS_NOT_FOUND, with no error recorded and nothing
- * written, for what it does not serve (a null lhs or rhs of a large problem; tiles
- * without a matrix-core kernel; buffers that overlap): run the chain then. A long K
+ * written, for what it does not serve: run the chain then. That is a null lhs or
+ * rhs, or a narrow tile, of a large problem; 2-byte elements whose rows of b are whole
+ * 8 KiB, of a large problem; tiles without a matrix-core kernel; buffers that
+ * overlap; operands or results that are not aligned to their elements, lhs and rhs
+ * to 16 bytes. A long K
  * of few tiles is split over workgroups, whose partial sums lie in the stream's
  * scratch memory, and takes a second launch; while the stream is being captured it
  * is not. */

@@ -11,10 +11,10 @@
 // after them write the packed operands, which nothing in the launch waits for,
 // and the matmul's epilogue stores both the tiles of the result and the matrix.
 //
-// Among other calls on one stream, as the chain, on tiles of 32 x 32 and 64 x 64 whose
-// waves shared their operands through LDS, and here: f16 81x19x41 with C added 27.1,
-// 8.0, 4.6 us; i8 1024^3 21.0, 12.5, 8.9; f16 1024^3 22.0, 22 to 24, 11.8; f16
-// 2634x35x20 with C added (the chain not timed) 8.8, 3.3.
+// Called again and again on one stream, operands in the last-level cache, as the chain
+// step by step, on tiles of 32 x 32 and 64 x 64 whose waves shared their operands
+// through LDS, and here: f16 81x19x41 with C added 16.9, 7.5, 4.4 us; i8 1024^3 15.8,
+// 10.6, 7.4; f16 1024^3 18.4, 22 to 24, 10.3; f16 2634x35x20 with C added 16.2, 8.2, 4.3.
 //
 // Multiplying workgroups: 16 or 32 rows x 64 columns of the result, K dealt to 8
 // waves in steps of 64 bytes. A wave fetches its own steps straight into
@@ -28,7 +28,7 @@
 // compute units that have work (loads of twice the columns gave the same times).
 // A long K of few tiles is dealt to more workgroups, each with its own plane of
 // partial sums, and a second launch adds the planes in order (2 us when it follows):
-// bf16 64x29x3693 16.3 us whole, 7.1 in 8 slices (35.0 as the chain).
+// bf16 64x29x3693 11.7 us whole, 6.7 in slices (14.3 as the chain).
 #include <cmath>
 #include <type_traits>
 

@@ -663,6 +663,8 @@ namespace {
 // alone, so that the entries of a batch have the bits of the single call (fp8 8 rows
 // x 4992 x 15552 36.9 -> 19.5, f16 2 x 128 x 4992 6.1 -> 5.0; beyond 12 KB the few
 // workgroups of a single call take longer: bf16 16 x 480 x 14528 9.1 here, 14.3 there).
+// (Lines of measured times: that kernel's estimate picks its tile for these calls, and
+// is not compared with one of this kernel, of which there is none.)
 bool few_columns(int64_t N, int64_t chunks, int64_t batch) {
   if (chunks <= 32) return false;
   if (chunks <= 512) return batch * N * (chunks <= 400 ? 1 : 2) <= device_cu_count();

@@ -14,9 +14,11 @@
 // tile.
 //
 // What bounds it: 3.5 us for a launch of one step; then what one compute unit
-// takes in while the operands come from beyond its L2, 60 to 110 GB/s (8 to 10 us
-// per MB of packed operands, whose size decides the tile). Before and after, among
-// other calls: bf16 128x608x1184 10.7 -> 4.0 us, 64x64x768 7.9 -> 3.5, f16 2208x160x1984
+// takes in while the operands come from beyond its L2: packed ones 8 to 10 us per MB
+// by the fit below (100 to 125 GB/s; f16 512x512 on 256 workgroups 100 from K = 1024 to
+// 2048, 70 from there to 4096), row-major ones 13 to 17 (60 to 80 GB/s). That size
+// decides the tile. Before and after, among other calls, operands in the last-level
+// cache: bf16 128x608x1184 10.7 -> 4.0 us, 64x64x768 7.9 -> 3.5, f16 2208x160x1984
 // 14.7 -> 8.0, 1024^3 10.8 -> 7.2; a linear layer of fp8 42x2602x5760 12.6 -> 7.1, f16
 // 32x3117x1152 10.7 -> 5.0, 84 rows of bf16 1024x4288 13.0 -> 8.2; f32 416x971x1071
 // with its packing 31.4 -> 22.8.
