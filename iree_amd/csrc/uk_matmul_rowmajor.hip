@@ -595,10 +595,15 @@ __global__ __launch_bounds__(256, 2) void matmul_rowmajor_square_kernel(RowMajor
 // steps of all of them (by element size), the result, C, and for a split the planes
 // of sums and the launch that adds them. Fitted to half of 1300 problems (8 to 4096
 // rows and columns, K 16 to 4096, six types) on 1 to 16 slices; on the other half
-// 12 % off on average, and what it picks is 1 % from the best.
+// 12 % off on average, and what it picks is 1 % from the best. A B beyond the 4 MB of an
+// L2 comes from behind it, and in part for every row of workgroups anew, which those
+// problems hardly had: with kBehind and kAgain 30 of 16328 others took over 20 % longer than
+// as the chain, without them 102 (bf16 281x3489x3988 63.3 us in one launch, 38.4 as the
+// chain; f16 45x4023x3840 38.1 and 27.3).
 struct Shape {
   float first, round, step4, step1, step2, hidden, store, add, split, plane;
 };
+constexpr double kL2Mb = 4.0, kBehind = 0.4, kAgain = 0.08;       // (us per MB)
 constexpr Shape kShapes[2] = {{3.47f, 0.30f, 0.82f, 0.99f, 0.78f, 0.26f, 0.42f, 0.18f, 2.10f, 1.12f},
                               {3.68f, 0.17f, 1.28f, 1.54f, 0.95f, 0.05f, 0.39f, 0.22f, 1.91f, 1.11f}};
 
@@ -612,9 +617,11 @@ struct Estimate {
     const int rows = p.M1 * p.M0, cols = p.N1 * p.N0;
     const double groups = (double)((rows + 16 * mb - 1) / (16 * mb)) * ((cols + 63) / 64);
     const double result = (double)rows * cols * sizeof(typename Cfg::out_t) * 1e-6 * (p.out ? 2 : 1);
+    const double b_mb = 1e-6 * cols * p.K * Cfg::kElemBytes, over = std::fmax(b_mb - kL2Mb, 0.0);
+    const double again = kBehind * over + kAgain * std::fmin(over / kL2Mb, 1.0) * b_mb * ((rows + 16 * mb - 1) / (16 * mb));
     return {groups, std::ceil(p.K * (Cfg::kElemBytes / 64.0)),
             (Cfg::kElemBytes == 4 ? t.step4 : Cfg::kElemBytes == 1 ? t.step1 : t.step2) / 8.0,
-            result * t.store + (p.accumulate ? t.add : 0.0), t, cus};
+            result * t.store + again + (p.accumulate ? t.add : 0.0), t, cus};
   }
   double us(int mb, int slices) const {
     const double rounds = std::ceil(groups * slices / cus), stream = rounds * std::ceil(steps / slices) * step_us;

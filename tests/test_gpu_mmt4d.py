@@ -1951,3 +1951,25 @@ def test_few_tiles_on_random_data_with_infinities(uk, cuda, type_flag, dt, form,
     finite = want.isfinite()
     size = a.nan_to_num(0, 0, 0).abs() @ b.nan_to_num(0, 0, 0).abs().T.contiguous()
     assert ((got.double() - want).abs() <= (2e-5 if fp8 else 2e-6) * size)[finite].all() and finite.sum() >= (M - 2) * (N - 1)
+
+
+@pytest.mark.parametrize("type_flag,dt,M,N,K,fuse,path", [
+    (F.MMT4D_TYPE_BF16BF16F32, "bfloat16", 281, 3489, 3988, False, "mmt4d:mfma"),
+    (F.MMT4D_TYPE_F16F16F32, "float16", 45, 4023, 3840, True, "mmt4d:mfma"),
+    (F.MMT4D_TYPE_S8S8S32, "int8", 165, 3798, 3432, False, "mmt4d:mfma"),
+    (F.MMT4D_TYPE_F16F16F32, "float16", 45, 423, 3840, True, "mmt4d:mfma-one-launch"),
+])
+def test_wide_b_of_a_long_k(uk, cuda, type_flag, dt, M, N, K, fuse, path):
+    """A B that an L2 does not hold, which one launch fetches for every row of its
+    workgroups anew: the chain, with the same exact sums."""
+    import torch
+    g = torch.Generator(device="cuda").manual_seed(M + N + K)
+    a = torch.randint(-2, 3, (M * K,), generator=g, device="cuda").to(getattr(torch, dt))
+    b = torch.randint(-2, 3, (K * N,), generator=g, device="cuda").to(getattr(torch, dt))
+    c = torch.zeros(M * N, dtype=torch.int32 if dt == "int8" else torch.float32, device="cuda")
+    step = c.clone()
+    uk.matmul_data_tiled(a, b, c, M, N, K, type_flag, fuse_unpack=fuse)
+    if torch.cuda.get_device_properties(0).multi_processor_count == 256:
+        assert uk.last_kernel_path() == path
+    uk.matmul_data_tiled(a, b, step, M, N, K, type_flag, fuse_unpack=fuse, one_launch=False)
+    assert torch.equal(c, step)
