@@ -678,6 +678,9 @@ bool choose(const RowMajorArgs& p, int max_slices, double* us, int* mb, int* sli
 // The kernel on 64 x 64: workgroups beyond one per compute unit run one after the
 // other, each with a fixed part and its share of K; the result, C and the packed
 // operands. Fitted to 2000 problems of up to 1200 bytes of K, 8 to 9 % off on average.
+// (int8: a result beyond 8 MB costs more than that, by 0.2 us per MB stored; of 3400 other
+// problems 22 took over 20 % longer than as the chain without it, 7 with it: 4016x3477x16 35.2
+// us as the chain, 46.6 here, 3069x2476x45 26.4 and 30.2.)
 // 16-bit types have no such kernel: it was the best for 13 of 525 of theirs, f32 203 of 482
 // (1200x1500x100 16.1 us on 16 or 32 x 64, 12.5 here; 900x1300x300 17.2 and 20.9).
 template <typename Cfg>
@@ -688,7 +691,7 @@ double square_us(const RowMajorArgs& p) {
   const double out_mb = rows * cols * 4e-6;
   return (kF32 ? 3.82 : 4.50) + load * ((kF32 ? 0.32 : 0.81) + (kF32 ? 3.47 : 2.49) / 512 * bytes) +
          (p.out ? 1.36 : 0.0) + (kF32 ? 0.205 : 0.221) * out_mb * (p.out ? 2 : 1) + (p.accumulate ? 0.42 * out_mb : 0.0) +
-         (kF32 ? 0.62e-6 : 0.45e-6) * (rows + cols) * bytes;
+         (kF32 ? 0.62e-6 : 0.45e-6) * (rows + cols) * bytes + (kF32 ? 0.0 : 0.2 * std::fmax(0.0, out_mb * (p.out ? 2 : 1) - 8));
 }
 
 template <typename Cfg>

@@ -1958,10 +1958,13 @@ def test_few_tiles_on_random_data_with_infinities(uk, cuda, type_flag, dt, form,
     (F.MMT4D_TYPE_F16F16F32, "float16", 45, 4023, 3840, True, "mmt4d:mfma"),
     (F.MMT4D_TYPE_S8S8S32, "int8", 165, 3798, 3432, False, "mmt4d:mfma"),
     (F.MMT4D_TYPE_F16F16F32, "float16", 45, 423, 3840, True, "mmt4d:mfma-one-launch"),
+    (F.MMT4D_TYPE_S8S8S32, "int8", 4016, 3477, 16, False, "mmt4d:mfma"),
+    (F.MMT4D_TYPE_S8S8S32, "int8", 816, 977, 16, False, "mmt4d:mfma-one-launch"),
 ])
-def test_wide_b_of_a_long_k(uk, cuda, type_flag, dt, M, N, K, fuse, path):
+def test_wide_b_or_large_result_is_the_chain_s(uk, cuda, type_flag, dt, M, N, K, fuse, path):
     """A B that an L2 does not hold, which one launch fetches for every row of its
-    workgroups anew: the chain, with the same exact sums."""
+    workgroups anew, and int8 results that are most of the call: the chain, with the same
+    exact sums."""
     import torch
     g = torch.Generator(device="cuda").manual_seed(M + N + K)
     a = torch.randint(-2, 3, (M * K,), generator=g, device="cuda").to(getattr(torch, dt))
