@@ -107,9 +107,9 @@ struct MfmaArgs {
   // macro-tile rows of one column panel of the workgroup order (see tile_coord)
   int panel_rows;
   // launch side: estimated time in us of another kernel that could serve the
-  // call (0: there is none); whether only to compare with it, launching nothing
-  // (fp8 and f32)
-  float other_us;
+  // call (0: there is none), against a K split and against whole K; whether only to
+  // compare with it, launching nothing (fp8 and f32)
+  float other_us, other_whole_us;
   bool compare_only;
 };
 

@@ -333,7 +333,10 @@ double costed_us(const MfmaArgs& a, int wm, int wn, int occ, int64_t tiles, doub
 
 // The other kernel's estimate has to be 5 % below this one's (with no margin 75 of
 // 7333 problems got slower by more than 4 %, with it 32, by 16 % at most).
-inline bool other_wins(const MfmaArgs& a, double us) { return a.other_us > 0 && a.other_us < 0.95 * us; }
+inline bool other_wins(const MfmaArgs& a, double us, bool whole) {
+  const float other = whole ? a.other_whole_us : a.other_us;
+  return other > 0 && other < 0.95 * us;
+}
 
 // A last round that fills only part of the device costs a whole round. When
 // the large tile leaves such a round, the longer outer dimension is split:
@@ -452,12 +455,12 @@ int launch_estimated(const MfmaArgs& a, hipStream_t s) {
     const int64_t whole_tiles = ceil_div((int64_t)a.M, (int64_t)2 * whole.wm) * ceil_div((int64_t)a.N, (int64_t)2 * whole.wn);
     const bool worth = a.ksteps >= 64 && whole_tiles * 2 <= (int64_t)whole.occ * cus;
     if (split.n > 1 && (worth || !scratch_under_capture(s))) {
-      if (other_wins(a, straightened_us(split.us))) return kSlowerThanOther;
+      if (other_wins(a, straightened_us(split.us), false)) return kSlowerThanOther;
       const int st = launch_k_split<Cfg>(a, split.v, split.n, s);
       if (st != IREE_AMD_UK_STATUS_NOT_FOUND) return st;     // (without scratch memory: whole, or the other kernel)
     }
   }
-  if (other_wins(a, straightened_us(best_us))) return kSlowerThanOther;
+  if (other_wins(a, straightened_us(best_us), true)) return kSlowerThanOther;
   const int st = launch_whole_rounds<Cfg, false>(a, cus, best_us, us_of, pick, s);
   if (st != IREE_AMD_UK_STATUS_NOT_FOUND) return st;
   return launch_by_index<Cfg, false>(best, a, s);
@@ -543,7 +546,7 @@ int launch_costed(const MfmaArgs& a, hipStream_t s) {
   auto other_is_faster = [&](int v, int n) {
     const Variant& t = variants[v];
     const int64_t tiles = ceil_div((int64_t)a.M, (int64_t)2 * t.wm) * ceil_div((int64_t)a.N, (int64_t)2 * t.wn) * n;
-    return other_wins(a, costed_us<Cfg, kSiluMul>(a, t.wm, t.wn, t.occ, tiles, steps / n, n, cus));
+    return other_wins(a, costed_us<Cfg, kSiluMul>(a, t.wm, t.wn, t.occ, tiles, steps / n, n, cus), n == 1);
   };
   // Few macro tiles and a long K (a few hundred rows against a wide K, as in the
   // down projection of an MLP at small batch) leave most compute units idle:

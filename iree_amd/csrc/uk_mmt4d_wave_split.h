@@ -30,9 +30,10 @@ struct WaveSplitArgs {
   int tiles_m, tiles_n;        // (set by the launch)
 };
 
-// The best tile for a problem and its estimated time; tile < 0: not served. The
-// caller compares it with what else serves the call.
-struct WaveSplitChoice { int tile; double us; };
+// The best tile for a problem, its estimated time and whether each of its workgroups
+// has a compute unit; tile < 0: not served. The caller compares it with what else
+// serves the call.
+struct WaveSplitChoice { int tile; double us; bool one_round; };
 WaveSplitChoice choose_wave_split(const WaveSplitArgs& a, uint32_t type);
 int launch_mmt4d_wave_split(const WaveSplitArgs& a, uint32_t type, int tile, hipStream_t s);
 

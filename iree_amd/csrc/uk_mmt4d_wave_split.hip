@@ -359,7 +359,7 @@ int launch_type(const WaveSplitArgs& a, int v, hipStream_t s) {
 }  // namespace
 
 WaveSplitChoice choose_wave_split(const WaveSplitArgs& a, uint32_t type) {
-  WaveSplitChoice best = {-1, 0.0};
+  WaveSplitChoice best = {-1, 0.0, false};
   const bool f32 = type == IREE_AMD_UK_FLAG_MMT4D_TYPE_F32F32F32, f8 = type == IREE_AMD_UK_FLAG_MMT4D_TYPE_F8E4M3F8E4M3F32;
   // (unsigned 32-bit offsets within a workgroup's tile and along K: outer rows or columns
   // that run backwards are the other kernels')
@@ -373,8 +373,11 @@ WaveSplitChoice choose_wave_split(const WaveSplitArgs& a, uint32_t type) {
   for (int v = 0; v < kTiles; ++v) {
     if (a.silu && kTile[v].nb == 1) continue;             // (gate and up columns side by side)
     const double us = estimate_us(a, f32, out_bytes, kTile[v], cus);
-    if (best.tile < 0 || us < best.us) best = {v, us};
+    if (best.tile < 0 || us < best.us) best = {v, us, false};
   }
+  if (best.tile >= 0)
+    best.one_round = ceil_div((int64_t)a.rows, (int64_t)(kTile[best.tile].mb * 16)) *
+                         ceil_div((int64_t)a.outer_cols * 2, (int64_t)kTile[best.tile].nb) * a.batch <= cus;
   return best;
 }
 
