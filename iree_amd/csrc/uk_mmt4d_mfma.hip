@@ -466,9 +466,10 @@ FewTiles consider_few_tiles(const iree_amd_uk_mmt4d_params_t& p, const MfmaArgs&
   few.choice = {-1, 0.0, false};
   if (as_few_tiles(p, a, silu, &few.args))
     few.choice = choose_wave_split(few.args, p.flags & IREE_AMD_UK_FLAG_MMT4D_TYPE_MASK);
-  // (up to four macro tiles and half a KB to 8 KB of K: it was faster, on all of 1220
-  // problems, and the estimates of the macro tiles take 0.2 us of a 3.5 us call)
-  few.certain = few.choice.tile >= 0 && p.K >= 32 && p.K <= 512 && ((a.M + 3) / 4) * (int64_t)((a.N + 3) / 4) <= 4;
+  // (up to four macro tiles and 8 KB of K, or less than half a KB of K: it was no slower on
+  // all of 1220 and of 4000 problems, and the estimates of the macro tiles take 0.2 us of a
+  // 3.5 us call, of both forms 0.3)
+  few.certain = few.choice.tile >= 0 && (p.K < 32 || (p.K <= 512 && ((a.M + 3) / 4) * (int64_t)((a.N + 3) / 4) <= 4));
   return few;
 }
 // The time to compare with macro tiles that keep K whole. The estimates of both were
