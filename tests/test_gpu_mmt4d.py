@@ -1960,6 +1960,7 @@ def test_few_tiles_on_random_data_with_infinities(uk, cuda, type_flag, dt, form,
     (F.MMT4D_TYPE_S8S8S32, "int8", 165, 3798, 3432, False, "mmt4d:mfma"),
     (F.MMT4D_TYPE_F16F16F32, "float16", 45, 423, 3840, True, "mmt4d:mfma-one-launch"),
     (F.MMT4D_TYPE_S8S8S32, "int8", 4016, 3477, 16, False, "mmt4d:mfma"),
+    (F.MMT4D_TYPE_F32F32F32, "float32", 531, 2782, 605, False, "mmt4d:mfma-one-launch"),
     (F.MMT4D_TYPE_S8S8S32, "int8", 816, 977, 16, False, "mmt4d:mfma-one-launch"),
 ])
 def test_wide_b_or_large_result_is_the_chain_s(uk, cuda, type_flag, dt, M, N, K, fuse, path):
