@@ -480,7 +480,11 @@ int launch_cfg(SkinnyArgs a, int chunks, hipStream_t s) {
   // 0.81 times as long, two to four 0.65, four to eight 0.5 (scores of a decode step, 8
   // heads x 1x7104x64 f16, 9.0 -> 4.4 us); below the line the other form wins by as much.
   const int64_t columns = (int64_t)a.N * (a.batch > 1 ? a.batch : 1);
-  const int64_t enough = a.chunk_steps <= 4 ? cus : a.chunk_steps <= 8 ? cus * 3 / 2 : cus * 3;
+  // (More than 12 rows of one problem with up to 4 steps are bound by their results, which a
+  // wave then stores by itself: f16 24 rows x 9137 x 64 6.4 us in the other form, 7.4 here; they
+  // keep the line of 8 columns.)
+  const bool many_rows = a.M0 > 12 && a.batch <= 1;
+  const int64_t enough = a.chunk_steps <= 4 ? (many_rows ? cus * 8 - 7 : cus) : a.chunk_steps <= 8 ? cus * 3 / 2 : cus * 3;
   if (chunks == 1 && a.chunk_steps <= kPerWaveSteps && columns >= enough) {
     // one outer column per wave
     a.steps_per_wave = a.chunk_steps;

@@ -1595,7 +1595,7 @@ def test_few_narrow_columns_with_k_over_the_waves(uk, cuda, type_flag, dt, out_d
         assert torch.equal(c.reshape(M0, N, 32).transpose(0, 1).double(), want[0])
 
 
-@pytest.mark.parametrize("M0,N,batch", [(1, 255, 1), (1, 256, 1), (8, 129, 2), (4, 31, 13), (2, 33, 8)])
+@pytest.mark.parametrize("M0,N,batch", [(1, 255, 1), (1, 256, 1), (8, 129, 2), (4, 31, 13), (2, 33, 8), (16, 300, 1)])
 @pytest.mark.parametrize("steps", [1, 4, 5, 8])
 def test_short_k_whole_per_wave(uk, cuda, M0, N, batch, steps):
     """About one outer column of narrow tiles per compute unit, a K of a few
