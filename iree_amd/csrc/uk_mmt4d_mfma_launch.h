@@ -329,12 +329,13 @@ double costed_us(const MfmaArgs& a, int wm, int wn, int occ, int64_t tiles, doub
   const double us = 3.11 + steps * step * (before * kShared + (tiles - before * slots > cus ? kShared : 1.0)) +
                     3.96 * before + 0.245 * out_mb + (kSiluMul ? 0.27 * area : 0.0);
   if (slices == 1) return us;
-  // (f32: beyond 12 MB of partial sums a third of that; without it 21 of 5000 problems whose
-  // K is split went to the kernel for few tiles and took over 10 % longer there, with it 8:
-  // a linear layer of 1461 rows 576 -> 1472 40.5 us split, 49.1
-  // there)
+  // (f32 with up to 256 elements of K per slice: beyond 12 MB of partial sums a third of that;
+  // without it 21 of 5000 problems whose K is split went to the kernel for few tiles and took
+  // over 10 % longer there, with it 11: a linear layer of 1461 rows 576 -> 1472 40.5 us split,
+  // 49.1 there. Longer slices hide no less of the sums than the fit says: 400 rows 7040 -> 3392
+  // 213 us split, 165 there.)
   const double sums_mb = out_mb * slices;
-  return us + 2.33 + 0.62 * sums_mb - (kF32 && sums_mb > 12 ? 0.4 * (sums_mb - 12) : 0.0);
+  return us + 2.33 + 0.62 * sums_mb - (kF32 && steps <= 16 && sums_mb > 12 ? 0.4 * (sums_mb - 12) : 0.0);
 }
 
 // The other kernel's estimate has to be 5 % below this one's (with no margin 75 of
