@@ -333,9 +333,10 @@ double costed_us(const MfmaArgs& a, int wm, int wn, int occ, int64_t tiles, doub
   // without it 21 of 5000 problems whose K is split went to the kernel for few tiles and took
   // over 10 % longer there, with it 11: a linear layer of 1461 rows 576 -> 1472 40.5 us split,
   // 49.1 there. Longer slices hide no less of the sums than the fit says: 400 rows 7040 -> 3392
-  // 213 us split, 165 there.)
+  // 213 us split, 165 there. Nor where iree_amd_uk_mmt4d_noalloc_p would have to refuse the split.)
   const double sums_mb = out_mb * slices;
-  return us + 2.33 + 0.62 * sums_mb - (kF32 && steps <= 16 && sums_mb > 12 ? 0.4 * (sums_mb - 12) : 0.0);
+  const bool less = kF32 && steps <= 16 && sums_mb > 12 && (a.lhs_row_major || sums_mb * 1e6 <= IREE_AMD_UK_NOALLOC_SCRATCH_BYTES);
+  return us + 2.33 + 0.62 * sums_mb - (less ? 0.4 * (sums_mb - 12) : 0.0);
 }
 
 // The other kernel's estimate has to be 5 % below this one's (with no margin 75 of
@@ -464,8 +465,10 @@ int launch_estimated(const MfmaArgs& a, hipStream_t s) {
     if (split.n > 1 && (worth || !scratch_under_capture(s))) {
       // (16-bit types in 8 slices, K from 6144: the other kernel has to be 15 % below. Of 1934 such
       // problems 43 then take over 5 % longer there, with 5 % it was 100, f16 32 rows 10688 -> 2112
-      // 18.3 us split and 23.6 there; 1.5 and 1.3 % from the faster one on average)
-      const double against = Cfg::kElemBytes == 2 && split.n == 8 ? 0.9 : 1.0;
+      // 18.3 us split and 23.6 there; 1.5 and 1.3 % from the faster one on average. Not a split that
+      // iree_amd_uk_mmt4d_noalloc_p refuses.)
+      const bool later = Cfg::kElemBytes == 2 && split.n == 8 && 8 * slice_bytes <= (int64_t)IREE_AMD_UK_NOALLOC_SCRATCH_BYTES;
+      const double against = later ? 0.9 : 1.0;
       if (other_wins(a, against * straightened_us(split.us), false)) return kSlowerThanOther;
       const int st = launch_k_split<Cfg>(a, split.v, split.n, s);
       if (st != IREE_AMD_UK_STATUS_NOT_FOUND) return st;     // (without scratch memory: whole, or the other kernel)

@@ -1864,7 +1864,7 @@ def test_k_split_without_scratch_memory(uk, cuda, type_flag, dt, M1, N1, K1):
 @pytest.mark.parametrize("type_flag,dt,M1,N1,K1", [
     (F.MMT4D_TYPE_S8S8S32, "int8", 3, 181, 560), (F.MMT4D_TYPE_F16F16F32, "float16", 10, 66, 1027),
     (F.MMT4D_TYPE_F8E4M3F8E4M3F32, "float8_e4m3fn", 1, 69, 1137), (F.MMT4D_TYPE_F32F32F32, "float32", 22, 31, 1047),
-    (F.MMT4D_TYPE_F32F32F32, "float32", 20, 159, 301),
+    (F.MMT4D_TYPE_F32F32F32, "float32", 48, 50, 181),
     (F.MMT4D_TYPE_F16F16F32, "float16", 8, 10, 1580),
 ])
 @pytest.mark.parametrize("accumulate", [False, True])
