@@ -636,7 +636,7 @@ struct Estimate {
 // matrix instructions, and a share of K (fitted to the same problems, 11 % off on
 // average). Without a packed result (the matmul writes the matrix, and reads the old one
 // when it accumulates) a byte of the result costs a third. The rule: the estimate of one
-// launch is below 0.9 of it (f32: 1.1). On 2500 other problems (4 to 4200 rows and columns, K 16
+// launch is below 0.9 of it (f32, not too large: 1.1). On 2500 other problems (4 to 4200 rows and columns, K 16
 // to 4200) that is 0.4 % from the best of all three on average, 2 % on 1500 of 200
 // rows and columns and more with a K of up to 1200 bytes, where the fastest change with
 // every further round of workgroups (43 of these took over 15 % longer than on the
@@ -716,10 +716,11 @@ int launch(RowMajorArgs p, hipStream_t s) {
   // they take 2.0 to 3.5 us less: 1500 x 1501 x 1502 int8 26.4 -> 22.9 us in all)
   const double chain = chain_us<Cfg>(p);
   const bool together = p.lhs && p.rhs && p.M0 == 32 && p.N0 == 32 && (Cfg::kElemBytes != 2 || p.N % 4096 != 0);
-  // (f32: its chain takes longer than estimated; on 2343 problems 2.6 % from the best kernel on
-  // average and 7 over 20 % longer than as the chain, with 0.9 of it 3.3 % and none, and
-  // 531x2782x605 42.0 us as the chain, 27.8 in one launch)
-  const double limit = together && p.out && chain < 24.0 ? chain - 2.4 : (Cfg::kElemBytes == 4 ? 1.1 : 0.9) * chain;
+  // (f32: its chain takes longer than estimated, for results of up to 3 million elements; on
+  // 2343 problems 2.6 % from the best kernel on average and 5 over 20 % longer than as the
+  // chain, with 0.9 of it 3.1 % and 4, and 531x2782x605 42.0 us as the chain, 27.8 in one launch)
+  const bool slow_chain = Cfg::kElemBytes == 4 && rows * cols <= 3000000;
+  const double limit = together && p.out && chain < 24.0 ? chain - 2.4 : (slow_chain ? 1.1 : 0.9) * chain;
   int mb = 1, slices = 1;
   double us = limit;
   const bool found = choose<Cfg>(p, 16, &us, &mb, &slices);
