@@ -908,15 +908,19 @@ namespace {
 // bytes, weights from memory), and on 2500 others 0.4 % from the faster of the two
 // on average, where taking all but a few of fp8 was at 3.2 % (f16 24 rows x 10491 x 96
 // 3.9 us on the others, 6.2 here; fp8 20 x 30656 x 1280 10.8 and 16.4, 12 x 12091 x 3264
-// 14.8 and 11.6).
+// 14.8 and 11.6). The lines of up to 8 rows, of f32 and just below 384 outer columns are from
+// 900 more (bf16 1 x 11580 x 960 11.3 and 6.9, f32 1 x 10198 x 128 10.8 and 7.8, fp8 4 x 11712 x
+// 2368 10.1 and 7.0).
 bool scaled_rows_are_faster(int eb, bool fp8, int64_t M, int64_t outer_cols, int64_t k_bytes) {
   if (outer_cols <= 256) return k_bytes > 512 || eb == 4 || (!fp8 && M <= 8 && k_bytes > 256);
-  if (eb == 4) return k_bytes > 512 && k_bytes <= 1024;
+  if (eb == 4) return k_bytes >= 512 && k_bytes <= 1024;
   const bool middle = outer_cols > 384 && outer_cols <= 768;
+  if (!fp8 && M <= 8 && outer_cols <= 768) return k_bytes >= 1024;
   if (!fp8) return middle ? k_bytes > 1024 : k_bytes >= 2048 && (M <= 8 || outer_cols <= 768 || outer_cols > 1024);
   if (k_bytes <= 4096)
-    return (k_bytes > 3072 && (M <= 16 || outer_cols <= 768)) || (k_bytes > 1400 && middle && outer_cols <= 512);
-  return (M <= 8 && outer_cols <= 512) || (k_bytes >= 6144 && (M <= 8 || middle));
+    return (k_bytes > 3072 && (M <= 16 || outer_cols <= 768)) || (k_bytes > 1400 && middle && outer_cols <= 512) ||
+           (k_bytes >= 2048 && outer_cols > 360 && outer_cols <= 384);
+  return (M <= 8 && outer_cols <= 512) || (k_bytes >= 6144 && (M <= 8 || (outer_cols > 340 && outer_cols <= 768)));
 }
 }  // namespace
 

@@ -1791,6 +1791,8 @@ def test_few_fp8_rows_have_the_bits_of_narrow_tiles(uk, cuda, M, N1, K):
     (F.MMT4D_TYPE_F8E4M3F8E4M3F32, "float8_e4m3fn", 20, 30656, 1280, False),
     (F.MMT4D_TYPE_F8E4M3F8E4M3F32, "float8_e4m3fn", 12, 12091, 3264, True),
     (F.MMT4D_TYPE_F8E4M3F8E4M3F32, "float8_e4m3fn", 9, 8300, 4608, False), (F.MMT4D_TYPE_F32F32F32, "float32", 3, 9001, 264, False),
+    (F.MMT4D_TYPE_F32F32F32, "float32", 3, 9001, 128, True), (F.MMT4D_TYPE_BF16BF16F32, "bfloat16", 6, 11479, 832, True),
+    (F.MMT4D_TYPE_F8E4M3F8E4M3F32, "float8_e4m3fn", 4, 11712, 2368, True),
 ])
 def test_scaled_rows_on_either_kernel(uk, cuda, type_flag, dt, M, N, K, narrow):
     """Both sides of the rule that gives a scaled result of a few rows to the narrow
