@@ -479,6 +479,18 @@ FewTiles consider_few_tiles(const iree_amd_uk_mmt4d_params_t& p, const MfmaArgs&
 // fp8 128x7808x2848 12.1 us on the macro tiles, 9.1 here; with the SiLU epilogue 14.9 and
 // 9.9 at 128 x 2 x 3104 x 4240).
 float whole_us(const WaveSplitChoice& c) { return (float)(c.one_round ? c.us * (0.95 / 1.3) : c.us); }
+// The time to compare with a K split. 16-bit types on 16 x 32 and 32 x 32 results per workgroup
+// with K from 6144 on, where the estimate is the less certain: a tenth longer (of 934 such
+// problems in 8 slices 32 then take over 5 % longer here, without it 85: f16 32 rows 10688 -> 2112
+// 18.3 us split and 23.6 here; on 16 x 16 results it is too long already: 2 rows 11968 ->
+// 2401 15.5 and 10.7). Not against a split that iree_amd_uk_mmt4d_noalloc_p refuses.
+float split_us(const iree_amd_uk_mmt4d_params_t& p, const MfmaArgs& a, const FewTiles& few) {
+  Mmt4dTypeInfo ti;
+  mmt4d_type_info(p.flags, &ti);
+  const bool longer = ti.lhs_bits == 16 && p.K * p.K0 >= 6144 && (few.choice.tile == 1 || few.choice.tile == 2) &&
+                      (int64_t)a.M * a.N * 4096 * 8 <= (int64_t)IREE_AMD_UK_NOALLOC_SCRATCH_BYTES;
+  return (float)(longer ? few.choice.us / 0.9 : few.choice.us);
+}
 int launch_few_tiles(const iree_amd_uk_mmt4d_params_t& p, const FewTiles& few, hipStream_t s) {
   return launch_mmt4d_wave_split(few.args, p.flags & IREE_AMD_UK_FLAG_MMT4D_TYPE_MASK, few.choice.tile, s);
 }
@@ -489,8 +501,10 @@ int launch_faster(const iree_amd_uk_mmt4d_params_t& p, const MfmaArgs& a, const 
                   Launch launch) {
   if (few.certain) return launch_few_tiles(p, few, s);
   MfmaArgs b = a;
-  b.other_us = few.choice.tile >= 0 ? (float)few.choice.us : 0.0f;
-  b.other_whole_us = few.choice.tile >= 0 && !silu ? whole_us(few.choice) : b.other_us;
+  if (few.choice.tile >= 0) {
+    b.other_us = split_us(p, a, few);
+    b.other_whole_us = silu ? (float)few.choice.us : whole_us(few.choice);
+  }
   const int st = launch(b);
   return st == kSlowerThanOther ? launch_few_tiles(p, few, s) : st;
 }

@@ -463,13 +463,7 @@ int launch_estimated(const MfmaArgs& a, hipStream_t s) {
     const int64_t whole_tiles = ceil_div((int64_t)a.M, (int64_t)2 * whole.wm) * ceil_div((int64_t)a.N, (int64_t)2 * whole.wn);
     const bool worth = a.ksteps >= 64 && whole_tiles * 2 <= (int64_t)whole.occ * cus;
     if (split.n > 1 && (worth || !scratch_under_capture(s))) {
-      // (16-bit types in 8 slices, K from 6144: the other kernel has to be 15 % below. Of 1934 such
-      // problems 43 then take over 5 % longer there, with 5 % it was 100, f16 32 rows 10688 -> 2112
-      // 18.3 us split and 23.6 there; 1.5 and 1.3 % from the faster one on average. Not a split that
-      // iree_amd_uk_mmt4d_noalloc_p refuses.)
-      const bool later = Cfg::kElemBytes == 2 && split.n == 8 && 8 * slice_bytes <= (int64_t)IREE_AMD_UK_NOALLOC_SCRATCH_BYTES;
-      const double against = later ? 0.9 : 1.0;
-      if (other_wins(a, against * straightened_us(split.us), false)) return kSlowerThanOther;
+      if (other_wins(a, straightened_us(split.us), false)) return kSlowerThanOther;
       const int st = launch_k_split<Cfg>(a, split.v, split.n, s);
       if (st != IREE_AMD_UK_STATUS_NOT_FOUND) return st;     // (without scratch memory: whole, or the other kernel)
     }
