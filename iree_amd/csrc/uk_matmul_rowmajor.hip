@@ -636,12 +636,11 @@ struct Estimate {
 // matrix instructions, and a share of K (fitted to the same problems, 11 % off on
 // average). Without a packed result (the matmul writes the matrix, and reads the old one
 // when it accumulates) a byte of the result costs a third. The rule: the estimate of one
-// launch is below 0.9 of it (f32, not too large: 1.1). On 2500 other problems (4 to 4200 rows and columns, K 16
-// to 4200) that is 0.4 % from the best of all three on average, 2 % on 1500 of 200
-// rows and columns and more with a K of up to 1200 bytes, where the fastest change with
-// every further round of workgroups (43 of these took over 15 % longer than on the
-// kernels before when both results were taken for two: f16 2945x3940x145 20.9 us as
-// the chain, 32.7 on 64 x 64 tiles; now 3 do).
+// launch is below 0.9 of it (f32, not too large: 1.1). On 16328 other problems (32 to 4200 rows and
+// columns, K 8 to 4200) that is 1.9 % from the best of all three on average, the noise of the
+// timing among it, and 11 take over 20 % longer than as the chain (f16 2945x3940x145 without
+// a packed result is one that the store counted twice sent to 64 x 64 tiles: 20.9 us as the
+// chain, 32.7 there).
 // A chain that does not pack A (its matmul reads the matrix, so there are two
 // launches) was not among them; its estimate is from below.
 template <typename Cfg>
