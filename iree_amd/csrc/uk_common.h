@@ -214,6 +214,19 @@ class ScratchOverride {
   size_t prev_bytes_;
   bool prev_strict_, prev_active_;
 };
+// While one of these lives, the calling thread's mmt4d stays on the macro tiles: the rows
+// of a problem that is run in blocks then have the sums of the whole one, whatever the size
+// of a block.
+class MacroTilesOnly {
+ public:
+  MacroTilesOnly();
+  ~MacroTilesOnly();
+  MacroTilesOnly(const MacroTilesOnly&) = delete;
+  MacroTilesOnly& operator=(const MacroTilesOnly&) = delete;
+
+ private:
+  bool prev_;
+};
 // Records the error of a request of `bytes` that a strict override cannot
 // serve and returns its status (RESOURCE_EXHAUSTED).
 int scratch_overflow_status(const char* what, size_t bytes);

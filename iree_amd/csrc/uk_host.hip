@@ -313,6 +313,7 @@ int mmt4d_on(iree_amd_uk_host_pool_t* pool, const iree_amd_uk_mmt4d_params_t* pa
       q.M = rows;
       {
         ScratchOverride no_scratch(nullptr, 0, /*strict=*/false);
+        MacroTilesOnly as_whole;
         status = iree_amd_uk_mmt4d_p(&q, slot->stream);
       }
       if (!status) status = check_hip(hipEventRecord(slot->events[b], slot->stream), "hipEventRecord");

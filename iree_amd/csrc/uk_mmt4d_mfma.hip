@@ -461,10 +461,11 @@ struct FewTiles {
   WaveSplitChoice choice;
   bool certain;
 };
+thread_local bool t_macro_tiles_only = false;
 FewTiles consider_few_tiles(const iree_amd_uk_mmt4d_params_t& p, const MfmaArgs& a, bool silu) {
   FewTiles few;
   few.choice = {-1, 0.0, false};
-  if (as_few_tiles(p, a, silu, &few.args))
+  if (!t_macro_tiles_only && as_few_tiles(p, a, silu, &few.args))
     few.choice = choose_wave_split(few.args, p.flags & IREE_AMD_UK_FLAG_MMT4D_TYPE_MASK);
   // (up to four macro tiles and 8 KB of K, or less than half a KB of K: it was no slower on
   // all of 1220 and of 4000 problems, and the estimates of the macro tiles take 0.2 us of a
@@ -527,6 +528,9 @@ int launch_typed(const iree_amd_uk_mmt4d_params_t& p, const MfmaArgs& a, hipStre
                        [&](const MfmaArgs& b) { return launch_macro_tiles(p, b, s); });
 }
 }  // namespace
+
+MacroTilesOnly::MacroTilesOnly() : prev_(t_macro_tiles_only) { t_macro_tiles_only = true; }
+MacroTilesOnly::~MacroTilesOnly() { t_macro_tiles_only = prev_; }
 
 // mmt4d whose epilogue is e4m3(silu(gate) * up): `p.N` counts gate AND up outer
 // columns (interleaved, so it is even); the output has N / 2 outer columns of

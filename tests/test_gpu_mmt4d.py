@@ -1981,3 +1981,29 @@ def test_wide_b_or_large_result_is_the_chain_s(uk, cuda, type_flag, dt, M, N, K,
         assert uk.last_kernel_path() == path
     uk.matmul_data_tiled(a, b, step, M, N, K, type_flag, fuse_unpack=fuse, one_launch=False)
     assert torch.equal(c, step)
+
+
+@pytest.mark.parametrize("type_flag,dt", [(F.MMT4D_TYPE_F16F16F32, "float16"), (F.MMT4D_TYPE_F8E4M3F8E4M3F32, "float8_e4m3fn")])
+def test_host_pointers_in_blocks_of_rows_have_the_bits_of_the_device_call(uk, cuda, type_flag, dt):
+    """A large result is computed in 16 blocks of outer rows (here 8, the last one 7), each of
+    which alone would run on the kernel for few tiles: the sums of the whole problem."""
+    import torch
+    lib = uk.load_library()
+    g = torch.Generator(device="cuda").manual_seed(11)
+    dt = getattr(torch, dt)
+    M1, N1, k0 = 127, 64, 16 // dt.itemsize
+    K1 = 4096 // k0
+    raw = torch.uint8 if dt.itemsize == 1 else dt
+    lhs, rhs = (torch.randn(n * K1 * 32 * k0, generator=g, device="cuda").to(dt).view(raw) for n in (M1, N1))
+    out = torch.zeros(M1 * N1 * 1024, device="cuda")
+    uk.mmt4d(lhs, rhs, out, M1, N1, K1, 32, 32, k0, type_flag)
+    assert uk.last_macro_tile()[0] >= 128 and uk.last_macro_tile()[2] == 1
+    block = torch.zeros(8 * N1 * 1024, device="cuda")
+    uk.mmt4d(lhs, rhs, block, 8, N1, K1, 32, 32, k0, type_flag)
+    if torch.cuda.get_device_properties(0).multi_processor_count == 256:
+        assert uk.last_macro_tile()[0] < 128
+    lh, rh, oh = lhs.cpu().numpy(), rhs.cpu().numpy(), np.zeros(M1 * N1 * 1024, np.float32)
+    p = uk._lib.Mmt4dParams(lh.ctypes.data, 0, K1 * 32 * k0, rh.ctypes.data, 0, K1 * 32 * k0, oh.ctypes.data, 0, N1 * 1024,
+                            M1, N1, K1, 32, 32, k0, type_flag, None)
+    assert lib.iree_amd_uk_mmt4d_host(C.byref(p)) == 0
+    assert np.array_equal(oh, out.cpu().numpy())
