@@ -232,7 +232,7 @@ int launch_dequant_matmul_i4(const void* x, const void* w, const void* scale, co
                        ((uintptr_t)scale % 16) == 0 && ((uintptr_t)zp % 16) == 0;
   // More than 64 rows (a prompt): the tiled kernel of uk_quant_gemm.hip, where
   // the kernels below stream the weights again for every 32 rows (N = 14336,
-  // K = 4096: 128 rows 46.2 -> 29.8 us, 512 183 -> 72). Both sides on 1900 problems
+  // K = 4096: 128 rows 46.2 -> 28.5 us, 512 183 -> 66). Both sides on 1900 problems
   // of 33 to 128 rows, times of the kernels below over those of the tiled one: from
   // 65 rows at least 1.08 with groups of 64 and more and 0.94 with groups of 32 (96
   // x 7424 x 2048: 18.5 and 19.9 us); at 49 to 64 rows down to 0.85 where there are

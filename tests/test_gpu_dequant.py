@@ -323,6 +323,37 @@ def test_many_rows(uk, cuda, M, N, K, gs):
     assert err <= float(np.spacing(np.float16(max(1.0, mag))))
 
 
+@pytest.mark.parametrize("M,N,K,gs", [
+    (257, 13088, 384, 32), (385, 13984, 384, 64), (470, 12320, 384, 128), (257, 13088, 768, 256),   # 128 x 256
+    (65, 10816, 3200, 32), (65, 10976, 3200, 64), (512, 4096, 14336, 128),                          # ... K split
+    (129, 10912, 384, 32), (129, 10912, 384, 64), (129, 10944, 640, 128),                           # 64 x 256
+    (65, 5472, 2176, 32), (65, 4128, 3200, 128),                                                    # ... K split
+    (200, 12320, 256, 64), (129, 10912, 384, 128), (65, 6432, 3200, 64),                            # 64 x 128
+])
+def test_many_rows_wide_tiles(uk, cuda, M, N, K, gs):
+    """The tiles with 128 columns and more: rows and columns past the last whole tile,
+    odd and even numbers of spans, every depth of the rings, whole and split K.
+    Against float64: products exact, f32 sums of up to K terms and one rounding to
+    f16, 2^-11 of the value, and K 2^-24 of the sum of the terms' sizes."""
+    import torch
+    g = torch.Generator(device="cuda").manual_seed(M + N + K + gs)
+    x = torch.randn(M, K, generator=g, device="cuda").half()
+    rows = torch.randint(0, 256, (N, K // 2), generator=g, device="cuda", dtype=torch.uint8)
+    w = torch.empty_like(rows)
+    uk.pack_i4_weights(rows, w, N, K)
+    s = (torch.rand(N, K // gs, generator=g, device="cuda") * 0.015 + 0.005).half()
+    zp = torch.randint(0, 256, (-(-N * (K // gs) // 2),), generator=g, device="cuda", dtype=torch.uint8)
+    out = torch.full((M, N), float("nan"), dtype=torch.float16, device="cuda")
+    uk.dequant_matmul_i4(x, w, s, zp, out, M, N, K, gs, F.DEQUANT_MATMUL_ZP_U4 | F.DEQUANT_MATMUL_W_TILED)
+    assert uk.last_kernel_path() == "dequant_i4:gemm"
+    q = torch.stack([rows & 15, rows >> 4], -1).view(N, K // gs, gs).double()
+    z = torch.stack([zp & 15, zp >> 4], -1).view(-1)[:N * (K // gs)].view(N, K // gs, 1).double()
+    wd = ((q - z) * s.double()[:, :, None]).view(N, K).t().contiguous()
+    want, size = x.double() @ wd, x.double().abs() @ wd.abs()
+    bound = want.abs() * 2.0 ** -11 + size * (K * 2.0 ** -24) + 2.0 ** -24
+    assert bool(((out.double() - want).abs() <= bound).all())
+
+
 @pytest.mark.parametrize("M,N,K", [(128, 1024, 2048), (256, 1024, 4096), (128, 4096, 4096)])
 def test_many_rows_in_a_graph(uk, cuda, M, N, K):
     """A K of up to 4096, captured on a stream that has run nothing yet (an eager
