@@ -106,6 +106,11 @@ int launch_batch_mmt4d_mfma(const iree_amd_uk_mmt4d_params_t& p, int64_t batch, 
 int launch_mmt4d_unpack_mfma(const iree_amd_uk_mmt4d_params_t& p, int64_t out_rows,
                              int64_t out_cols, float out_scale, int64_t batch, int64_t lhs_batch_stride,
                              int64_t rhs_batch_stride, int64_t out_batch_stride, hipStream_t s);
+// The result as an out_rows x out_cols matrix (p.out_*) and, at `tiles`, as the dense
+// tiles that iree_amd_uk_mmt4d writes: an mmt4d and its unpack, and with the accumulate
+// flag, which adds to the matrix, the pack before them. NOT_FOUND as above.
+int launch_mmt4d_and_unpack_mfma(const iree_amd_uk_mmt4d_params_t& p, int64_t out_rows, int64_t out_cols, void* tiles,
+                                 hipStream_t s);
 int launch_matmul_packed_rhs_mfma(const iree_amd_uk_mmt4d_params_t& p, int64_t out_rows,
                                   int64_t out_cols, float out_scale, int64_t batch, int64_t lhs_batch_stride,
                                   int64_t rhs_batch_stride, int64_t out_batch_stride, hipStream_t s);
@@ -131,6 +136,8 @@ struct KSplitReduceArgs {
   void* out;                 // offset applied
   int64_t out_stride_bytes;
   int accumulate, row_major_out, out_rows, out_cols;
+  char* tiles = nullptr;     // row-major result: where it goes as tiles too, or null
+  int64_t tiles_stride_bytes = 0;
   float out_scale;
   int acc_is_float;          // else int32
   int out_kind;              // 0 = accumulator type, 1 = f16, 2 = bf16

@@ -657,6 +657,26 @@ double chain_us(const RowMajorArgs& p) {
          giga * 1e-9 * rows * cols * p.K + 0.16e-3 * bytes;
 }
 
+// The chain on full tiles whose matmul writes C beside the packed result
+// (launch_matmul_chain): two launches. Fitted to 18000 problems (33 to 4096 rows and
+// columns, K 16 to 4096), 11 to 12 % off on average; on 7000 others the faster of the two
+// is taken but for the noise of their timing (4 %), 1.19 times its time in the 99th
+// percentile, where the fit of three launches above left 1.30. f32, whose matrix
+// instructions weigh more than the launches, keeps that one.
+template <typename Cfg>
+bool full_tiles_chain(const RowMajorArgs& p) {
+  return Cfg::kElemBytes != 4 && p.lhs && p.rhs && p.out && p.M0 == 32 && p.N0 == 32;
+}
+template <typename Cfg>
+double full_tiles_chain_us(const RowMajorArgs& p) {
+  constexpr bool kS8 = Cfg::kElemBytes == 1;
+  const double rows = (double)p.M1 * p.M0, cols = (double)p.N1 * p.N0, bytes = (double)p.K * Cfg::kElemBytes;
+  const double out_mb = rows * cols * 1e-6 * sizeof(typename Cfg::out_t);
+  return (kS8 ? 11.1 : 9.6) + (kS8 ? 0.55e-6 : 0.48e-6) * (rows + cols) * bytes + 0.34 * out_mb +
+         (kS8 ? 1.9e-9 : 2.9e-9) * rows * cols * p.K - (kS8 ? 0.79e-3 : 0.2e-3) * bytes +
+         (p.accumulate ? 1.1 + (sizeof(typename Cfg::out_t) == 2 ? 0.8 : 0.43) * out_mb : 0.0);
+}
+
 // The fastest of both shapes and 1 to max_slices slices of K, whose time replaces *us;
 // false when none takes *us or less.
 template <typename Cfg>
@@ -713,13 +733,13 @@ int launch(RowMajorArgs p, hipStream_t s) {
   const int64_t rows = (int64_t)p.M1 * p.M0, cols = (int64_t)p.N1 * p.N0;
   // (the chain as it was fitted packed the operands one after the other; in one launch
   // they take 2.0 to 3.5 us less: 1500 x 1501 x 1502 int8 26.4 -> 22.9 us in all)
-  const double chain = chain_us<Cfg>(p);
+  const double chain = full_tiles_chain<Cfg>(p) ? full_tiles_chain_us<Cfg>(p) : chain_us<Cfg>(p);
   const bool together = p.lhs && p.rhs && p.M0 == 32 && p.N0 == 32 && (Cfg::kElemBytes != 2 || p.N % 4096 != 0);
   // (f32: its chain takes longer than estimated, for results of up to 3 million elements; on
   // 2343 problems 2.6 % from the best kernel on average and 5 over 20 % longer than as the
   // chain, with 0.9 of it 3.1 % and 4, and 531x2782x605 42.0 us as the chain, 27.8 in one launch)
   const bool slow_chain = Cfg::kElemBytes == 4 && rows * cols <= 3000000;
-  const double limit = together && p.out && chain < 24.0 ? chain - 2.4 : (slow_chain ? 1.1 : 0.9) * chain;
+  const double limit = full_tiles_chain<Cfg>(p) ? chain : together && p.out && chain < 24.0 ? chain - 2.4 : (slow_chain ? 1.1 : 0.9) * chain;
   int mb = 1, slices = 1;
   double us = limit;
   const bool found = choose<Cfg>(p, 16, &us, &mb, &slices);
@@ -791,10 +811,35 @@ int launch_matmul_chain(const void* a, const void* b, void* c, void* lhs, void* 
       (uintptr_t)out % ob ||
       share_memory(a, b, c, lhs, rhs, out, M, N, K, eb, ob, M1 * M0 * K1 * 16, N1 * N0 * K1 * 16, M1 * M0 * N1 * N0 * ob))
     return IREE_AMD_UK_STATUS_NOT_FOUND;
-  UK_RETURN_IF_ERROR(launch_pack_operands(a, b, lhs, rhs, M, N, K, M0, N0, K0, eb, s));
+  int packed = launch_pack_operands(a, b, lhs, rhs, M, N, K, M0, N0, K0, eb, s);
+  if (packed == IREE_AMD_UK_STATUS_NOT_FOUND && eb == 2 && N % 4096 == 0 && M0 == 32 && N0 == 32 &&
+      !(((uintptr_t)a | (uintptr_t)b) % 2) && !(((uintptr_t)lhs | (uintptr_t)rhs) % 16)) {
+    // (rows a power of two apart: each operand by the kernel that suits it)
+    const uint32_t type = IREE_AMD_UK_FLAG_PACK_TYPE_F16F16;
+    UK_RETURN_IF_ERROR(iree_amd_uk_pack(a, 0, K, 1, lhs, 0, K1 * M0 * K0, (int64_t)M0 * K0, M, K, M1, K1, M0, K0, 0, type,
+                                        nullptr, s));
+    packed = iree_amd_uk_pack(b, 0, N, 1, rhs, 0, K1 * N0 * K0, (int64_t)N0 * K0, K, N, N1, K1, N0, K0, 0,
+                              type | IREE_AMD_UK_FLAG_PACK_TRANSPOSE_INNER | IREE_AMD_UK_FLAG_PACK_TRANSPOSE_OUTER, nullptr, s);
+  }
+  if (packed) return packed;
   if (!out)
     return iree_amd_uk_mmt4d_unpack(lhs, 0, K1 * M0 * K0, rhs, 0, K1 * N0 * K0, c, 0, N, M, N, M1, N1, K1, K0, flags, 1.0f,
                                     s);
+  if (M0 == 32 && N0 == 32) {
+    // The matmul writes the matrix beside the tiles (and adds to the matrix itself), and
+    // the launch that would read the tiles back (and the one that packs C) is not needed:
+    // bf16 1999 x 4099 x 3001 72.5 -> 69.7 us, f16 2048^3 with f16 results 38.4 -> 34.8,
+    // 1000 x 4000 x 3000 added to C 56.1 -> 49.5, i8 4096^3 96 -> 89, 2000 x 3000 x 1000
+    // 29.6 -> 27.1. What is left of the unpack is its store, at the rate of memory: all
+    // workgroups of a round store at once.
+    const iree_amd_uk_mmt4d_params_t p = {lhs, 0, K1 * M0 * K0, rhs, 0, K1 * N0 * K0, c, 0, N, M1, N1, K1, M0, N0, K0,
+                                          flags, nullptr};
+    const int st = launch_mmt4d_and_unpack_mfma(p, M, N, out, s);
+    if (st != IREE_AMD_UK_STATUS_NOT_FOUND) {
+      if (!st) note_kernel_path("mmt4d:mfma");
+      return st;
+    }
+  }
   const uint32_t copy = ob == 2 ? IREE_AMD_UK_FLAG_PACK_TYPE_F16F16 : IREE_AMD_UK_FLAG_PACK_TYPE_I32I32;
   if (flags & IREE_AMD_UK_FLAG_MMT4D_ACCUMULATE)
     UK_RETURN_IF_ERROR(iree_amd_uk_pack(c, 0, N, 1, out, 0, N1 * M0 * N0, (int64_t)M0 * N0, M, N, M1, N1, M0, N0, 0, copy,

@@ -35,13 +35,14 @@ __global__ __launch_bounds__(256) void ksplit_reduce_kernel(KSplitReduceArgs r) 
   const int row_in_tile = in_tile >> 3, col_in_tile = (in_tile & 7) * 4;
   const int i = (int)(tile / r.N), j = (int)(tile % r.N);
   OutT* dst;
-  int valid = 4;   // leading elements of the group that exist in the result
+  int valid = 4;   // leading elements of the group that exist in the result (0: only in its tiles)
   if (r.flat_elems > 0) {
     dst = (OutT*)r.out + g * 4;
   } else if (r.row_major_out) {
     const int row = i * 32 + row_in_tile, col = j * 32 + col_in_tile;
-    if (row >= r.out_rows || col >= r.out_cols) return;
-    valid = r.out_cols - col < 4 ? r.out_cols - col : 4;
+    const bool exists = row < r.out_rows && col < r.out_cols;
+    if (!exists && !r.tiles) return;
+    valid = !exists ? 0 : r.out_cols - col < 4 ? r.out_cols - col : 4;
     dst = (OutT*)((char*)r.out + (int64_t)row * r.out_stride_bytes) + col;
   } else {
     dst = (OutT*)((char*)r.out + (int64_t)i * r.out_stride_bytes) + (int64_t)j * 1024 + in_tile * 4;
@@ -80,6 +81,7 @@ __global__ __launch_bounds__(256) void ksplit_reduce_kernel(KSplitReduceArgs r) 
   } else {
     for (int e = 0; e < valid; ++e) dst[e] = v[e];
   }
+  if (r.tiles) *(out4_t*)((OutT*)(r.tiles + (int64_t)i * r.tiles_stride_bytes) + (int64_t)j * 1024 + in_tile * 4) = v;
 }
 
 }  // namespace
@@ -266,6 +268,7 @@ int make_args(const iree_amd_uk_mmt4d_params_t& p, int out_elem_bytes, bool silu
   a.accumulate = (p.flags & IREE_AMD_UK_FLAG_MMT4D_ACCUMULATE) != 0;
   a.k0_div = sv.mfma_k / p.K0;
   a.row_major_out = 0; a.out_rows = a.out_cols = 0;
+  a.tiles = nullptr; a.tiles_stride_bytes = 0;
   a.lhs_row_major = 0;
   a.gate_scale = a.up_scale = a.inv_out_scale = a.out_scale = 1.0f;
   a.other_us = a.other_whole_us = 0.0f;
@@ -349,6 +352,22 @@ int launch_mmt4d_unpack_mfma(const iree_amd_uk_mmt4d_params_t& p, int64_t out_ro
   a.out_rows = (int)out_rows;
   a.out_cols = (int)out_cols;
   if (batch > 1) return launch_planes(p, a, batch, lhs_batch_stride, rhs_batch_stride, out_batch_stride, s);
+  return launch_typed(p, a, s);
+}
+
+int launch_mmt4d_and_unpack_mfma(const iree_amd_uk_mmt4d_params_t& p, int64_t out_rows, int64_t out_cols, void* tiles,
+                                 hipStream_t s) {
+  Mmt4dTypeInfo ti;
+  mmt4d_type_info(p.flags, &ti);
+  MfmaArgs a;
+  const int st = make_args(p, ti.out_bytes, false, &a);
+  if (st) return st;
+  if (out_rows > 0x7FFFFFFF || out_cols > 0x7FFFFFFF) return IREE_AMD_UK_STATUS_NOT_FOUND;
+  a.row_major_out = 1;
+  a.out_rows = (int)out_rows;
+  a.out_cols = (int)out_cols;
+  a.tiles = (char*)tiles;
+  a.tiles_stride_bytes = p.N * 1024 * ti.out_bytes;
   return launch_typed(p, a, s);
 }
 
@@ -446,6 +465,8 @@ bool as_few_tiles(const iree_amd_uk_mmt4d_params_t& p, const MfmaArgs& a, bool s
   w.out_row = a.row_major_out ? out_pitch : 32;
   w.out_tile = a.row_major_out ? 32 : 1024;
   w.out_col = 1;
+  w.tiles = a.tiles;
+  w.tiles_outer = a.tiles_stride_bytes / ti.out_bytes;
   w.out_rows = a.row_major_out ? a.out_rows : w.rows;
   w.out_cols = a.row_major_out ? a.out_cols : a.N * 32;
   w.accumulate = a.accumulate; w.silu = silu; w.batch = 1;

@@ -80,6 +80,10 @@ struct MfmaArgs {
   // row-major result (mmt4d fused with the unpack that would follow it): the
   // matrix has out_rows x out_cols elements, out_stride_bytes is its row pitch
   int row_major_out, out_rows, out_cols;
+  // ... and, if not null, where it goes as tiles too, tiles_stride_bytes per outer row:
+  // what the mmt4d would have written before the unpack, padding included
+  char* tiles;
+  int64_t tiles_stride_bytes;
   // row-major left-hand side (the pack of the LHS fused into the loads): lhs is
   // the out_rows x K matrix itself, lhs_stride_bytes its row pitch; the block
   // of (outer row i, K-step ks) is rows 32 i .. 32 i + 31, bytes
@@ -206,7 +210,7 @@ __device__ __forceinline__ void tile_coord(int bid, int tiles_m, int tiles_n, in
 // kForm: which of the operand forms the instance is compiled for: 0 = packed
 // left-hand side, tiled result; 1 = row-major result; 2 = row-major left-hand
 // side and result; 3 = row-major left-hand side, tiled result (the partial
-// sums of a K split). (An instance compiled for one form has constant step sizes
+// sums of a K split); 4 = row-major result, and as tiles too. (An instance compiled for one form has constant step sizes
 // in its loop and one epilogue: measured 2 % (f16) to 6 % (i8) faster at 4096^3
 // than one that reads the form from its arguments.)
 // kStreamOut: the tiled result is not read again soon and may be written past
@@ -215,9 +219,10 @@ __device__ __forceinline__ void tile_coord(int bid, int tiles_m, int tiles_n, in
 template <typename Cfg, int WM, int WN, int kRing, int kSync, bool kSiluMul = false, int kWavesN = 2,
           int kForm = 0, bool kStreamOut = true>
 __device__ __forceinline__ void mmt4d_mfma_body(const MfmaArgs a, const int bid = blockIdx.x) {
-  static_assert(kForm >= 0 && kForm <= 3 && (!kSiluMul || kForm == 0), "unknown operand form");
-  constexpr bool lhs_row_major = kForm >= 2;
-  constexpr bool row_major_out = kForm == 1 || kForm == 2;
+  static_assert(kForm >= 0 && kForm <= 4 && (!kSiluMul || kForm == 0), "unknown operand form");
+  constexpr bool lhs_row_major = kForm == 2 || kForm == 3;
+  constexpr bool row_major_out = kForm == 1 || kForm == 2 || kForm == 4;
+  constexpr bool tiles_too = kForm == 4;
   // kSwap: the MFMAs are issued with the operands exchanged (B fragment first),
   // so that a block's accumulator holds the TRANSPOSE in the instruction's
   // layout and a lane owns 4 consecutive COLUMNS of one row per register group
@@ -388,11 +393,12 @@ __device__ __forceinline__ void mmt4d_mfma_body(const MfmaArgs a, const int bid 
   auto load_acc = [&]() {
     if constexpr (row_major_out) {
       // (rows and columns past the matrix edge are read from the last valid
-      // one: their accumulators are never stored)
+      // one: their accumulators are never stored, or start at zero)
 #pragma unroll
       for (int x = 0; x < WM; ++x) {
         int row = (i_base + wm * WM + x) * R + acc_r;
-        row = row < a.out_rows ? row : a.out_rows - 1;
+        const bool in_rows = row < a.out_rows;
+        row = in_rows ? row : a.out_rows - 1;
         const out_t* src = (const out_t*)(a.out + (int64_t)row * a.out_stride_bytes);
 #pragma unroll
         for (int y = 0; y < WN; ++y)
@@ -402,12 +408,12 @@ __device__ __forceinline__ void mmt4d_mfma_body(const MfmaArgs a, const int bid 
             if (col + 4 <= a.out_cols) {
               const out4_t v4 = *(const out4_t*)(src + col);
 #pragma unroll
-              for (int e = 0; e < 4; ++e) acc[x][y][4 * g + e] = v4[e];
+              for (int e = 0; e < 4; ++e) acc[x][y][4 * g + e] = tiles_too && !in_rows ? (out_t)0 : v4[e];
             } else {
 #pragma unroll
               for (int e = 0; e < 4; ++e) {
                 const int c = col + e < a.out_cols ? col + e : a.out_cols - 1;
-                acc[x][y][4 * g + e] = src[c];
+                acc[x][y][4 * g + e] = tiles_too && !(in_rows && col + e < a.out_cols) ? (out_t)0 : src[c];
               }
             }
           }
@@ -709,7 +715,75 @@ __device__ __forceinline__ void mmt4d_mfma_body(const MfmaArgs a, const int bid 
       }
     return;
   }
+  if constexpr (row_major_out && R == 16 && sizeof(out_t) == 2 && WN % 2 == 0) {
+    // 16-bit results of 16-row blocks: a lane has 4 columns, 8 bytes, of one block. Two
+    // neighbouring blocks of an outer tile exchange lane rows (v_permlane16_swap: the odd
+    // ones of the first register against the even ones of the second), after which lane
+    // group g (of 16) has columns 8 (g / 2) .. + 8 of block g % 2: one store of 16 bytes a
+    // lane for both blocks, 64 bytes of a row, instead of two of 8.
+    typedef out_t out2_t __attribute__((ext_vector_type(2)));
+    typedef out_t out8_t __attribute__((ext_vector_type(8), aligned(sizeof(out_t))));
+    typedef uint32_t words_t __attribute__((ext_vector_type(4)));
+    const int in_pair = (lane >> 4 & 1) * 16 + (lane >> 5) * 8;
+#pragma unroll
+    for (int x = 0; x < WM; ++x) {
+      const int row = (i_base + wm * WM + x) * R + acc_r;
+      out_t* dst = (out_t*)(a.out + (int64_t)row * a.out_stride_bytes);
+#pragma unroll
+      for (int y = 0; y < WN; y += 2) {
+        uint32_t w[2][2];
+#pragma unroll
+        for (int b = 0; b < 2; ++b)
+#pragma unroll
+          for (int h = 0; h < 2; ++h)
+            w[b][h] = __builtin_bit_cast(uint32_t, out2_t{(out_t)(acc[x][y + b][2 * h] * a.out_scale),      // (x 1.0f is exact)
+                                                          (out_t)(acc[x][y + b][2 * h + 1] * a.out_scale)});
+        const auto p = __builtin_amdgcn_permlane16_swap(w[0][0], w[1][0], false, false);
+        const auto q = __builtin_amdgcn_permlane16_swap(w[0][1], w[1][1], false, false);
+        const out8_t v8 = __builtin_bit_cast(out8_t, words_t{(uint32_t)p[0], (uint32_t)q[0], (uint32_t)p[1], (uint32_t)q[1]});
+        const int bj = j_base + wn * WN + y, col = bj * R + in_pair;
+        if constexpr (tiles_too) {
+          // (half a tile, 1 KiB of consecutive memory, that nothing reads soon: past the
+          // caches. 2048^3 36.4 -> 34.8 us, 3000 x 3333 x 1500 53.7 -> 51.6.)
+          const int bi = i_base + wm * WM + x;
+          if (bi / 2 < a.M && bj / 2 < a.N)
+            __builtin_nontemporal_store(v8, (out8_t*)((out_t*)(a.tiles + (int64_t)(bi / 2) * a.tiles_stride_bytes) +
+                                                      (int64_t)(bj / 2) * 1024 + ((bi % 2) * R + acc_r) * 32 + in_pair));
+        }
+        if (row < a.out_rows) {
+          if (col + 8 <= a.out_cols) {
+            *(out8_t*)(dst + col) = v8;
+          } else {
+#pragma unroll
+            for (int e = 0; e < 8; ++e)
+              if (col + e < a.out_cols) dst[col + e] = v8[e];
+          }
+        }
+      }
+    }
+    return;
+  }
   if constexpr (row_major_out) {
+    if constexpr (tiles_too) {
+#pragma unroll
+      for (int x = 0; x < WM; ++x)
+#pragma unroll
+        for (int y = 0; y < WN; ++y) {
+          const int bi = i_base + wm * WM + x, bj = j_base + wn * WN + y;
+          const int i = bi / kPerTile, j = bj / kPerTile;
+          if (i < a.M && j < a.N) {
+            out_t* t = (out_t*)(a.tiles + (int64_t)i * a.tiles_stride_bytes) + (int64_t)j * 1024 +
+                       ((bi % kPerTile) * R + acc_r) * 32 + (bj % kPerTile) * R;
+#pragma unroll
+            for (int g = 0; g < kGroups; ++g) {
+              out4_t v4;
+#pragma unroll
+              for (int e = 0; e < 4; ++e) v4[e] = (out_t)acc[x][y][4 * g + e];
+              *(out4_t*)(t + acc_c0(g)) = v4;
+            }
+          }
+        }
+    }
 #pragma unroll
     for (int x = 0; x < WM; ++x) {
       const int row = (i_base + wm * WM + x) * R + acc_r;

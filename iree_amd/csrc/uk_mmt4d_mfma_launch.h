@@ -144,6 +144,8 @@ int launch_variant(const MfmaArgs& a0, hipStream_t s) {
     if (a.lhs_row_major && a.row_major_out)
       return launch_form<Cfg, WM, WN, kRing, kSync, kOcc, kSiluMul, kWavesN, 2>(a, (unsigned)blocks, s);
     if constexpr (kPackedLhs) {
+      if (a.row_major_out && a.tiles)
+        return launch_form<Cfg, WM, WN, kRing, kSync, kOcc, kSiluMul, kWavesN, 4>(a, (unsigned)blocks, s);
       if (a.row_major_out)
         return launch_form<Cfg, WM, WN, kRing, kSync, kOcc, kSiluMul, kWavesN, 1>(a, (unsigned)blocks, s);
     }
@@ -227,6 +229,8 @@ int launch_k_split(const MfmaArgs& a, int v, int slices, hipStream_t s) {
     r.flat_elems = 0;
     r.out = a.out;
     r.out_stride_bytes = a.out_stride_bytes;
+    r.tiles = a.tiles;
+    r.tiles_stride_bytes = a.tiles_stride_bytes;
     r.accumulate = a.accumulate;
     r.row_major_out = a.row_major_out;
     r.out_rows = a.out_rows; r.out_cols = a.out_cols;
@@ -381,6 +385,7 @@ int launch_whole_rounds(const MfmaArgs& a, int cus, double best_cost, Cost cost_
             rest.out = a.out + (t_first / 2) * 1024;             // one e4m3 tile pair per two columns
           } else if (a.row_major_out) {
             rest.out = a.out + t_first * 32 * out_elem;
+            if (a.tiles) rest.tiles = a.tiles + t_first * 1024 * out_elem;
             first.out_cols = (int)(t_first * 32);                 // (out_cols > 32 (N - 1) >= 32 t_first)
             rest.out_cols = a.out_cols - (int)(t_first * 32);
           } else {
@@ -394,6 +399,7 @@ int launch_whole_rounds(const MfmaArgs& a, int cus, double best_cost, Cost cost_
           rest.out = a.out + t_first * (a.row_major_out ? 32 : 1) * a.out_stride_bytes;
           rest.lhs = a.lhs + t_first * (a.lhs_row_major ? 32 : 1) * a.lhs_stride_bytes;
           if (a.row_major_out) {
+            if (a.tiles) rest.tiles = a.tiles + t_first * a.tiles_stride_bytes;
             first.out_rows = (int)(t_first * 32);
             rest.out_rows = a.out_rows - (int)(t_first * 32);
           }

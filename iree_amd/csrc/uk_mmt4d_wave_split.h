@@ -25,6 +25,10 @@ struct WaveSplitArgs {
   // elements (SiLU form: 32 x 16 tiles of bytes, out_outer bytes per 32 rows)
   int64_t out_outer, out_row, out_tile;
   int out_col, out_rows, out_cols;
+  // if not null, where the result goes as 32 x 32 tiles too, padding included, tiles_outer
+  // elements per outer row
+  char* tiles;
+  int64_t tiles_outer;
   int accumulate, silu, batch;
   float gate_scale, up_scale, inv_out_scale, out_scale;
   int tiles_m, tiles_n;        // (set by the launch)

@@ -254,12 +254,13 @@ __device__ __forceinline__ void mmt4d_wave_split_body(const WaveSplitArgs& a) {
     if (f >= F) break;
     const int x = f / NB, y = f % NB;
     const int row = (tm * MB + x) * 16 + l16, col = (tn * NB + y) * 16 + kc * 4;
-    if (row >= a.out_rows || col >= a.out_cols) continue;
+    const bool exists = row < a.out_rows && col < a.out_cols;
+    if (!exists && !(a.tiles && row < a.rows && col < a.outer_cols * 32)) continue;
     out_t* const dst = (out_t*)(a.out + plane * a.out_batch) + (row >> 5) * a.out_outer + (row & 31) * a.out_row +
                        (col >> 5) * a.out_tile + (col & 31) * a.out_col;
     const bool whole = a.out_col == 1 && col + 4 <= a.out_cols;
     acc_t sum = {0, 0, 0, 0};
-    if (a.accumulate) {
+    if (a.accumulate && exists) {
       if (whole) {
         const out4_t old = *(const out4_t*)dst;
 #pragma unroll
@@ -278,6 +279,9 @@ __device__ __forceinline__ void mmt4d_wave_split_body(const WaveSplitArgs& a) {
       if constexpr (std::is_same<out_t, int32_t>::value) v[e] = sum[e];
       else v[e] = (out_t)(sum[e] * a.out_scale);
     }
+    if (a.tiles)
+      *(out4_t*)((out_t*)a.tiles + (row >> 5) * a.tiles_outer + (int64_t)(col >> 5) * 1024 + (row & 31) * 32 + (col & 31)) = v;
+    if (!exists) continue;
     if (whole) {
       *(out4_t*)dst = v;
     } else {

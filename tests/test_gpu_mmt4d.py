@@ -2007,3 +2007,44 @@ def test_host_pointers_in_blocks_of_rows_have_the_bits_of_the_device_call(uk, cu
                             M1, N1, K1, 32, 32, k0, type_flag, None)
     assert lib.iree_amd_uk_mmt4d_host(C.byref(p)) == 0
     assert np.array_equal(oh, out.cpu().numpy())
+
+
+@pytest.mark.parametrize("accumulate", [False, True])
+@pytest.mark.parametrize("kind,M,N,K", [
+    ("i8", 1100, 2051, 1990), ("f16", 1999, 2061, 1003), ("bf16_bf16", 1999, 4099, 1001),    # edges of 16-row blocks
+    ("f16_f16", 2048, 2047, 2000), ("f32", 2000, 2901, 1500),
+    ("bf16_bf16", 1500, 4096, 1000),               # rows a power of two apart: two packs
+    ("i8", 90, 100, 70000), ("f32", 70, 40, 65700),                              # few tiles
+    ("bf16_bf16", 129, 161, 14000), ("bf16_bf16", 33, 35, 66003),                # K in slices
+    ("f16_f16", 500, 1100, 12000), ("f16", 400, 513, 9000), ("i8", 600, 500, 16000),
+    ("f16", 4097, 4000, 1100),                     # whole rounds and the rest
+])
+def test_data_tiled_matmul_writes_matrix_and_tiles(uk, cuda, kind, M, N, K, accumulate):
+    """The chain whose matmul writes C beside the packed result leaves the bits of the
+    chain step by step in every buffer (the same kernels add the same products)."""
+    import torch
+    type_flag, in_dt, out_dt = {
+        "i8": (F.MMT4D_TYPE_S8S8S32, torch.int8, torch.int32), "f16": (F.MMT4D_TYPE_F16F16F32, torch.float16, torch.float32),
+        "f16_f16": (F.MMT4D_TYPE_F16F16F16, torch.float16, torch.float16), "f32": (F.MMT4D_TYPE_F32F32F32, torch.float32, torch.float32),
+        "bf16_bf16": (F.MMT4D_TYPE_BF16BF16BF16, torch.bfloat16, torch.bfloat16)}[kind]
+    g = torch.Generator(device="cuda")
+    g.manual_seed(M + K)
+    def values(n, dt):
+        if not dt.is_floating_point:
+            return torch.randint(-128, 128, (n,), generator=g, device="cuda").to(dt)
+        return torch.randn(n, generator=g, device="cuda").to(dt)
+    a, b, c0 = values(M * K, in_dt), values(K * N, in_dt), values(M * N, out_dt)
+    results = []
+    for one_launch in (True, False):
+        c = c0.clone()
+        ws = {"out": torch.full((-(-M // 32) * -(-N // 32) * 1024,), 77, dtype=out_dt, device="cuda")}
+        ws = uk.matmul_data_tiled(a, b, c, M, N, K, type_flag, accumulate=accumulate, tile="dynamic", workspace=ws,
+                                  one_launch=one_launch)
+        torch.cuda.synchronize()
+        assert uk.last_kernel_path() == "mmt4d:mfma", "not the chain: another size is needed here"
+        assert K < 65536 or kind == "bf16_bf16" or max(uk.last_macro_tile()[:2]) <= 64
+        results.append((c, ws))
+    (c, ws), (step, chain) = results
+    assert torch.equal(c, step)
+    for name in ("lhs", "rhs", "out"):
+        assert torch.equal(ws[name], chain[name]), name
