@@ -157,8 +157,8 @@ int launch_dequant_gemv_i4(const i4::I4Args& p, int m_base, int m_eff, hipStream
 // Many rows of activations (uk_quant_gemm.hip): tiled weights, packed uint4 zero
 // points, power-of-two groups of 32 and more, K in whole 128s, 16-byte aligned
 // operands (the caller has checked); NOT_FOUND for sizes that 32-bit offsets
-// cannot address.
-int launch_dequant_gemm_i4(const i4::I4Args& p, hipStream_t s);
+// cannot address, and, with limit_us > 0, where that is the shorter time.
+int launch_dequant_gemm_i4(const i4::I4Args& p, double limit_us, hipStream_t s);
 
 }  // namespace uk
 

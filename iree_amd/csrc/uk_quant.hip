@@ -186,6 +186,23 @@ int launch_fast(I4Args a, int k_rows, hipStream_t s) {
   return launch_ksplit_reduce(r, s);
 }
 
+// Estimated time in microseconds of 33 to 64 rows on this kernel, two launches, the second
+// of 16 rows up to row 48, and for a split K their sum: a workgroup walks its tiles of
+// 32 columns. By slice length and group size (32, 64, 128, 256 and more); fitted to
+// 9700 problems (512 to 14336 columns, K 512 to 14336), 3 % off on average.
+double two_passes_us(const I4Args& a, int slice_kb, int k_rows) {
+  struct Cost { double start, of32[4], of16[4], second16, split, per_mb; };
+  static const Cost costs[2] = {{8.0, {1.87, 1.39, 1.13, 1.05}, {1.44, 0.92, 0.77, 0.75}, -0.7, 3.9, 2.95},
+                                {11.8, {3.48, 2.57, 1.80, 1.83}, {2.69, 2.22, 2.10, 1.80}, -2.2, 3.2, 6.7}};
+  const Cost& c = costs[slice_kb == 8];
+  const int g = a.log2_gs < 6 ? 0 : a.log2_gs < 8 ? a.log2_gs - 5 : 3;
+  int blocks = device_cu_count() / k_rows;
+  blocks = blocks < 1 ? 1 : blocks < a.n_tiles ? blocks : a.n_tiles;
+  const int walked = (int)ceil_div(a.n_tiles, blocks);
+  return c.start + walked * c.of32[g] + (a.M > 48 ? walked * c.of32[g] : walked * c.of16[g] + c.second16) +
+         (k_rows > 1 ? c.split : 0.0) + c.per_mb * 1e-6 * k_rows * (double)a.M * a.N;
+}
+
 }  // namespace
 
 int launch_dequant_matmul_i4(const void* x, const void* w, const void* scale, const void* zp,
@@ -235,11 +252,15 @@ int launch_dequant_matmul_i4(const void* x, const void* w, const void* scale, co
   // K = 4096: 128 rows 46.2 -> 28.5 us, 512 183 -> 66). Both sides on 1900 problems
   // of 33 to 128 rows, times of the kernels below over those of the tiled one: from
   // 65 rows at least 1.08 with groups of 64 and more and 0.94 with groups of 32 (96
-  // x 7424 x 2048: 18.5 and 19.9 us); at 49 to 64 rows down to 0.85 where there are
-  // many columns (64 x 8192 x 2048: 11.9 and 13.4), up to 1.6 where there are few.
-  if (M > 64 && tiled && a.zp_u4 && gs_ok && K % 128 == 0 && size_ok && aligned) {
+  // x 7424 x 2048: 18.5 and 19.9 us). At 33 to 64 rows whichever is estimated to be
+  // the faster: on 9700 problems 0.80 times the time of the kernels below on average,
+  // 0.4 % from the faster of the two and 16 problems over 4 % slower than there (10 %
+  // at most). 59 x 2496 x 13056 with groups of 64 23.2 -> 17.0 us, 40 x 5120 x 2304
+  // 15.0 -> 11.0; 36 x 6528 x 2048 stays below, 9.8 against 11.7.
+  if (M > 32 && tiled && a.zp_u4 && gs_ok && K % 128 == 0 && size_ok && aligned) {
     a.w_bytes = (uint32_t)w_bytes;
-    const int st = launch_dequant_gemm_i4(a, s);
+    const double limit_us = M > 64 || !k_ok ? 0.0 : two_passes_us(a, slice_kb, (int)k_rows);
+    const int st = launch_dequant_gemm_i4(a, limit_us, s);
     if (st != IREE_AMD_UK_STATUS_NOT_FOUND) { note_kernel_path("dequant_i4:gemm"); return st; }
   }
   // (one row against few tiles of columns and a split K: the kernel below, in

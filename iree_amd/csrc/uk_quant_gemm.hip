@@ -723,7 +723,7 @@ double gemm_estimate_us(const I4Args& p, int v, int log2_ge, int64_t tiles, int 
 
 }  // namespace
 
-int launch_dequant_gemm_i4(const I4Args& p, hipStream_t s) {
+int launch_dequant_gemm_i4(const I4Args& p, double limit_us, hipStream_t s) {
   I4GemmArgs a;
   a.x = p.x; a.w = p.w; a.scale = p.scale; a.zp = (const uint8_t*)p.zp; a.out = p.out;
   a.partial = nullptr;
@@ -735,9 +735,9 @@ int launch_dequant_gemm_i4(const I4Args& p, hipStream_t s) {
   if ((int64_t)p.M * p.K * 2 >= (1ll << 31) || (int64_t)p.N * p.G * 2 >= (1ll << 31)) return IREE_AMD_UK_STATUS_NOT_FOUND;
   const int cus = device_cu_count();
   int best = -1, slices = 1;
+  double best_us = 0;
   auto choose = [&](int max_slices) {
     best = -1;
-    double best_us = 0;
     for (int v = 0; v < kShapes; ++v) {
       const int64_t tiles = ceil_div((int64_t)p.M, (int64_t)kGemmShapes[v].rows) *
                             ceil_div((int64_t)p.N, (int64_t)kGemmShapes[v].cols);
@@ -753,14 +753,17 @@ int launch_dequant_gemm_i4(const I4Args& p, hipStream_t s) {
     slices = (int)ceil_div(a.spans, a.slice_spans);
   };
   choose(8);
-  if (best < 0) return IREE_AMD_UK_STATUS_NOT_FOUND;
+  if (best < 0 || (limit_us > 0 && best_us > limit_us)) return IREE_AMD_UK_STATUS_NOT_FOUND;
   // A call being captured takes no scratch memory where the kernels for fewer
   // rows need none (K up to 4096, and what only this kernel serves): it need not
   // have been made before, and the graph may be replayed beside others.
   const bool may_split = slices > 1 && ((p.K > 4096 && p.K % 256 == 0) || !scratch_under_capture(s));
   ScratchLease lease(s, may_split ? (size_t)slices * p.M * p.N * 4 : 0);
   a.partial = (float*)lease.ptr();
-  if (slices > 1 && !a.partial) choose(1);
+  if (slices > 1 && !a.partial) {
+    choose(1);
+    if (limit_us > 0 && best_us > limit_us) return IREE_AMD_UK_STATUS_NOT_FOUND;
+  }
   a.tiles_m = (int)ceil_div(p.M, kGemmShapes[best].rows);
   a.tiles_n = (int)ceil_div(p.N, kGemmShapes[best].cols);
   int st;

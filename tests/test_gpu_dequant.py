@@ -323,6 +323,18 @@ def test_many_rows(uk, cuda, M, N, K, gs):
     assert err <= float(np.spacing(np.float16(max(1.0, mag))))
 
 
+@pytest.mark.parametrize("M,N,K,gs,path", [
+    (33, 32, 128, 128, "gemm"), (49, 96, 384, 32, "gemm"), (64, 5120, 2304, 128, "gemm"),     # K in whole 128s and 256s
+    (59, 2496, 13056, 64, "gemm"),                                                             # K split
+    (36, 6528, 2048, 128, "mfma"), (36, 576, 13824, 32, "mfma"),     # two passes over the weights are faster
+])
+def test_33_to_64_rows(uk, cuda, M, N, K, gs, path):
+    """Up to a tile of rows: the tiled kernel or two passes of the streaming one,
+    whichever is estimated to be the faster. Within one f16 unit of the oracle's."""
+    err, mag = run_case(uk, M, N, K, gs, True, True, seed=M + N + K, want_path="dequant_i4:" + path, repeats=1)
+    assert err <= float(np.spacing(np.float16(max(1.0, mag))))
+
+
 @pytest.mark.parametrize("M,N,K,gs", [
     (257, 13088, 384, 32), (385, 13984, 384, 64), (470, 12320, 384, 128), (257, 13088, 768, 256),   # 128 x 256
     (65, 10816, 3200, 32), (65, 10976, 3200, 64), (512, 4096, 14336, 128),                          # ... K split
