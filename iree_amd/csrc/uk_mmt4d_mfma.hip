@@ -273,6 +273,7 @@ int make_args(const iree_amd_uk_mmt4d_params_t& p, int out_elem_bytes, bool silu
   a.gate_scale = a.up_scale = a.inv_out_scale = a.out_scale = 1.0f;
   a.other_us = a.other_whole_us = 0.0f;
   a.compare_only = false;
+  a.few_rows = false;
   return 0;
 }
 }  // namespace
@@ -485,7 +486,7 @@ struct FewTiles {
 thread_local bool t_macro_tiles_only = false;
 FewTiles consider_few_tiles(const iree_amd_uk_mmt4d_params_t& p, const MfmaArgs& a, bool silu) {
   FewTiles few;
-  few.choice = {-1, 0.0, false};
+  few.choice = {-1, 0.0, false, false, -1, 0.0};
   if (!t_macro_tiles_only && as_few_tiles(p, a, silu, &few.args))
     few.choice = choose_wave_split(few.args, p.flags & IREE_AMD_UK_FLAG_MMT4D_TYPE_MASK);
   // (up to four macro tiles and 8 KB of K, or less than half a KB of K: it was no slower on
@@ -500,7 +501,8 @@ FewTiles consider_few_tiles(const iree_amd_uk_mmt4d_params_t& p, const MfmaArgs&
 // problems, as with 0.95 times; 2.0 instead of 3.6 % from the faster of the two on average:
 // fp8 128x7808x2848 12.1 us on the macro tiles, 9.1 here; with the SiLU epilogue 14.9 and
 // 9.9 at 128 x 2 x 3104 x 4240).
-float whole_us(const WaveSplitChoice& c) { return (float)(c.one_round ? c.us * (0.95 / 1.3) : c.us); }
+// (Up to 64 rows the times of both are from a fit to such problems: few_rows_us.)
+float whole_us(const WaveSplitChoice& c) { return (float)(c.one_round && !c.few_rows ? c.us * (0.95 / 1.3) : c.us); }
 // The time to compare with a K split. 16-bit types on 16 x 32 and 32 x 32 results per workgroup
 // with K from 6144 on, where the estimate is the less certain: a tenth longer (of 934 such
 // problems in 8 slices 32 then take over 5 % longer here, without it 85: f16 32 rows 10688 -> 2112
@@ -509,9 +511,9 @@ float whole_us(const WaveSplitChoice& c) { return (float)(c.one_round ? c.us * (
 float split_us(const iree_amd_uk_mmt4d_params_t& p, const MfmaArgs& a, const FewTiles& few) {
   Mmt4dTypeInfo ti;
   mmt4d_type_info(p.flags, &ti);
-  const bool longer = ti.lhs_bits == 16 && p.K * p.K0 >= 6144 && (few.choice.tile == 1 || few.choice.tile == 2) &&
+  const bool longer = ti.lhs_bits == 16 && p.K * p.K0 >= 6144 && (few.choice.general_tile == 1 || few.choice.general_tile == 2) &&
                       (int64_t)a.M * a.N * 4096 * 8 <= (int64_t)IREE_AMD_UK_NOALLOC_SCRATCH_BYTES;
-  return (float)(longer ? few.choice.us / 0.9 : few.choice.us);
+  return (float)(longer ? few.choice.general_us / 0.9 : few.choice.general_us);
 }
 int launch_few_tiles(const iree_amd_uk_mmt4d_params_t& p, const FewTiles& few, hipStream_t s) {
   return launch_mmt4d_wave_split(few.args, p.flags & IREE_AMD_UK_FLAG_MMT4D_TYPE_MASK, few.choice.tile, s);
@@ -526,6 +528,7 @@ int launch_faster(const iree_amd_uk_mmt4d_params_t& p, const MfmaArgs& a, const 
   if (few.choice.tile >= 0) {
     b.other_us = split_us(p, a, few);
     b.other_whole_us = silu ? (float)few.choice.us : whole_us(few.choice);
+    b.few_rows = few.choice.few_rows;
   }
   const int st = launch(b);
   return st == kSlowerThanOther ? launch_few_tiles(p, few, s) : st;
@@ -580,8 +583,9 @@ int launch_mmt4d_silu_mul_mfma(const iree_amd_uk_mmt4d_params_t& p, float gate_s
     MfmaArgs plain = a;
     plain.compare_only = true;
     const FewTiles of_plain = consider_few_tiles(p, a, false);
-    plain.other_us = (float)of_plain.choice.us;
+    plain.other_us = (float)of_plain.choice.general_us;
     plain.other_whole_us = whole_us(of_plain.choice);
+    plain.few_rows = of_plain.choice.few_rows;
     const int st = launch_mfma_f8f8f32(plain, s);
     if (st == kSlowerThanOther) return launch_few_tiles(p, few, s);
     if (st != kSplitsK) return launch(a);

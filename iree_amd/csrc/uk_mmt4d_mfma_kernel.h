@@ -112,9 +112,10 @@ struct MfmaArgs {
   int panel_rows;
   // launch side: estimated time in us of another kernel that could serve the
   // call (0: there is none), against a K split and against whole K; whether only to
-  // compare with it, launching nothing (fp8 and f32)
+  // compare with it, launching nothing (fp8 and f32), and whether its time is of the fit
+  // for few rows
   float other_us, other_whole_us;
-  bool compare_only;
+  bool compare_only, few_rows;
 };
 
 namespace {

@@ -343,11 +343,23 @@ double costed_us(const MfmaArgs& a, int wm, int wn, int occ, int64_t tiles, doub
   return us + 2.33 + 0.62 * sums_mb - (less ? 0.4 * (sums_mb - 12) : 0.0);
 }
 
+// The time of macro tiles that keep K whole for up to 64 rows of packed fp8: us of the
+// estimate above, corrected by the size of the operands (per MB). Fitted to 3000 problems
+// (the kernel for few tiles has their ranges), 3 % off on average where the estimate is at 10.
+template <typename Cfg, bool kSiluMul>
+double few_rows_us(const MfmaArgs& a, double us) {
+  const double k_mb = (double)a.ksteps * Cfg::kMfmaK * Cfg::kElemBytes * 1e-6;
+  return (kSiluMul ? 0.65 : 1.12) + (kSiluMul ? 0.82 : 0.73) * us + 0.065 * a.N * 32 * k_mb +
+         (kSiluMul ? 9.0 : 7.7) * a.M * 32 * k_mb;
+}
+
 // The other kernel's estimate has to be 5 % below this one's (with no margin 75 of
 // 7333 problems got slower by more than 4 %, with it 32, by 16 % at most).
-inline bool other_wins(const MfmaArgs& a, double us, bool whole) {
+// (Up to 64 rows with whole K: 10 %, with 5 % half as many problems again got slower by as much.)
+template <typename Cfg, bool kSiluMul>
+bool other_wins(const MfmaArgs& a, double us, bool whole) {
   const float other = whole ? a.other_whole_us : a.other_us;
-  return other > 0 && other < 0.95 * us;
+  return other > 0 && other < (whole && a.few_rows ? 0.9 * few_rows_us<Cfg, kSiluMul>(a, us) : 0.95 * us);
 }
 
 // A last round that fills only part of the device costs a whole round. When
@@ -469,12 +481,12 @@ int launch_estimated(const MfmaArgs& a, hipStream_t s) {
     const int64_t whole_tiles = ceil_div((int64_t)a.M, (int64_t)2 * whole.wm) * ceil_div((int64_t)a.N, (int64_t)2 * whole.wn);
     const bool worth = a.ksteps >= 64 && whole_tiles * 2 <= (int64_t)whole.occ * cus;
     if (split.n > 1 && (worth || !scratch_under_capture(s))) {
-      if (other_wins(a, straightened_us(split.us), false)) return kSlowerThanOther;
+      if (other_wins<Cfg, false>(a, straightened_us(split.us), false)) return kSlowerThanOther;
       const int st = launch_k_split<Cfg>(a, split.v, split.n, s);
       if (st != IREE_AMD_UK_STATUS_NOT_FOUND) return st;     // (without scratch memory: whole, or the other kernel)
     }
   }
-  if (other_wins(a, straightened_us(best_us), true)) return kSlowerThanOther;
+  if (other_wins<Cfg, false>(a, straightened_us(best_us), true)) return kSlowerThanOther;
   const int st = launch_whole_rounds<Cfg, false>(a, cus, best_us, us_of, pick, s);
   if (st != IREE_AMD_UK_STATUS_NOT_FOUND) return st;
   return launch_by_index<Cfg, false>(best, a, s);
@@ -560,7 +572,7 @@ int launch_costed(const MfmaArgs& a, hipStream_t s) {
   auto other_is_faster = [&](int v, int n) {
     const Variant& t = variants[v];
     const int64_t tiles = ceil_div((int64_t)a.M, (int64_t)2 * t.wm) * ceil_div((int64_t)a.N, (int64_t)2 * t.wn) * n;
-    return other_wins(a, costed_us<Cfg, kSiluMul>(a, t.wm, t.wn, t.occ, tiles, steps / n, n, cus), n == 1);
+    return other_wins<Cfg, kSiluMul>(a, costed_us<Cfg, kSiluMul>(a, t.wm, t.wn, t.occ, tiles, steps / n, n, cus), n == 1);
   };
   // Few macro tiles and a long K (a few hundred rows against a wide K, as in the
   // down projection of an MLP at small batch) leave most compute units idle:

@@ -36,8 +36,9 @@ struct WaveSplitArgs {
 
 // The best tile for a problem, its estimated time and whether each of its workgroups
 // has a compute unit; tile < 0: not served. The caller compares it with what else
-// serves the call.
-struct WaveSplitChoice { int tile; double us; bool one_round; };
+// serves the call. few_rows: `us` is of the fit for up to 64 rows, and general_tile and
+// general_us are what the fit for any number of rows gives (else the same as tile and us).
+struct WaveSplitChoice { int tile; double us; bool one_round, few_rows; int general_tile; double general_us; };
 WaveSplitChoice choose_wave_split(const WaveSplitArgs& a, uint32_t type);
 int launch_mmt4d_wave_split(const WaveSplitArgs& a, uint32_t type, int tile, hipStream_t s);
 

@@ -365,6 +365,34 @@ def test_gate_up_silu_of_few_tiles_has_the_bits_of_mmt4d(uk, cuda, M1, P, K1, ti
     assert torch.equal(fused, want) and want.unique().numel() > 100
 
 
+@pytest.mark.parametrize("M1,P,K1", [(1, 256, 128), (1, 231, 159), (1, 203, 200), (2, 231, 200), (2, 249, 259)])
+def test_gate_up_silu_on_large_weights(uk, cuda, M1, P, K1):
+    """Up to 64 rows against weights of 32 MB and more, which go past the caches: ragged
+    columns and K, plain mmt4d within the error of the instruction's sums (2e-5 of the sum of
+    the magnitudes of the terms) of float64, the fused form with its bytes."""
+    import torch
+    type_flag, K0 = F.MMT4D_TYPE_F8E4M3F8E4M3F32, 16
+    g = torch.Generator(device="cuda").manual_seed(M1 * 100 + P + K1)
+    lhs, rhs = (torch.randn(n * K1 * 32 * K0, generator=g, device="cuda").to(torch.float8_e4m3fn).view(torch.uint8)
+                for n in (M1, 2 * P))
+    scale, out_scale = (K1 * K0) ** -0.5, 8.0
+    acc = torch.full((M1 * 2 * P * 1024,), float("nan"), dtype=torch.float32, device="cuda")
+    uk.mmt4d(lhs, rhs, acc, M1, 2 * P, K1, 32, 32, K0, type_flag)
+    on = uk.last_macro_tile()
+    if torch.cuda.get_device_properties(0).multi_processor_count == 256:
+        assert max(on[:2]) <= 64
+    a64, b64 = (t.view(torch.float8_e4m3fn).double().view(-1, K1, 32, K0).transpose(1, 2).reshape(-1, K1 * K0) for t in (lhs, rhs))
+    got = acc.view(M1, 2 * P, 32, 32).transpose(1, 2).reshape(M1 * 32, -1).double()
+    assert bool(((got - a64 @ b64.t()).abs() <= 2e-5 * (a64.abs() @ b64.abs().t())).all())
+    fused, want = (torch.zeros(M1 * P * 1024, dtype=torch.uint8, device="cuda") for _ in range(2))
+    uk.mmt4d_silu_mul_f8e4m3(lhs, rhs, fused, M1, 2 * P, K1, K0, type_flag, scale, scale, out_scale)
+    assert (uk.last_macro_tile()[0] < 128) == (on[0] < 128)
+    a4 = acc.view(M1, P, 2, 1024)
+    split = torch.cat([a4[:, :, 0], a4[:, :, 1]], dim=1).contiguous()     # [M1][gate tiles | up tiles]
+    uk.silu_mul_quantize_tiled(split, 2 * P * 1024, 0, P, want, P * 1024, M1, P, scale, scale, out_scale)
+    assert torch.equal(fused, want) and want.unique().numel() > 100
+
+
 def test_fused_gate_up_silu_invalid_arguments(uk, cuda):
     import torch
     t = torch.zeros(4096, dtype=torch.uint8, device="cuda")
