@@ -232,11 +232,13 @@ __device__ __forceinline__ void mmt4d_mfma_body(const MfmaArgs a, const int bid 
   // time; measured 3 % faster at 4096^3 f16 for the row-major result. Tiled
   // results keep the instruction's own layout: there every 32-bit store
   // instruction already writes whole 128-byte lines, which measured 1-2 %
-  // FASTER than 128-bit stores of quarter lines.
-  constexpr bool kSwap = row_major_out || kSiluMul;
+  // FASTER than 128-bit stores of quarter lines; but 16-bit ones of 16-row blocks leave
+  // two blocks at a time, half a tile of 1 KiB an instruction (see the epilogue).
   typedef typename Cfg::frag_t frag_t;
   typedef typename Cfg::acc_t acc_t;
   typedef typename Cfg::out_t out_t;
+  constexpr bool kBlockPairs = Cfg::kRows == 16 && sizeof(out_t) == 2 && WN % 2 == 0 && kForm != 3 && !kSiluMul;
+  constexpr bool kSwap = row_major_out || kSiluMul || kBlockPairs;
   constexpr int kWaves = 2 * kWavesN;                // a 2 x kWavesN grid of waves
   // WM, WN, TM, TN count BLOCKS of R rows (R = 32 or 16: the instruction's
   // block); an outer tile of 32 rows is kPerTile of them.
@@ -430,8 +432,14 @@ __device__ __forceinline__ void mmt4d_mfma_body(const MfmaArgs a, const int bid 
           j = j < a.N ? j : a.N - 1;
           const out_t* t = (const out_t*)(a.out + (int64_t)i * a.out_stride_bytes) + (int64_t)j * 1024 +
                            (bi % kPerTile) * R * 32 + (bj % kPerTile) * R;
+          if constexpr (kSwap) {
+            const out4_t v4 = *(const out4_t*)(t + acc_r * 32 + acc_c0(0));
 #pragma unroll
-          for (int v = 0; v < kAccRegs; ++v) acc[x][y][v] = t[acc_row(v) * 32 + acc_col];
+            for (int e = 0; e < 4; ++e) acc[x][y][e] = v4[e];
+          } else {
+#pragma unroll
+            for (int v = 0; v < kAccRegs; ++v) acc[x][y][v] = t[acc_row(v) * 32 + acc_col];
+          }
         }
     }
   };
@@ -716,12 +724,14 @@ __device__ __forceinline__ void mmt4d_mfma_body(const MfmaArgs a, const int bid 
       }
     return;
   }
-  if constexpr (row_major_out && R == 16 && sizeof(out_t) == 2 && WN % 2 == 0) {
+  if constexpr (kBlockPairs) {
     // 16-bit results of 16-row blocks: a lane has 4 columns, 8 bytes, of one block. Two
     // neighbouring blocks of an outer tile exchange lane rows (v_permlane16_swap: the odd
     // ones of the first register against the even ones of the second), after which lane
     // group g (of 16) has columns 8 (g / 2) .. + 8 of block g % 2: one store of 16 bytes a
-    // lane for both blocks, 64 bytes of a row, instead of two of 8.
+    // lane for both blocks, 64 bytes of a row, instead of two of 8. Tiled results too, which
+    // the instruction's own layout stores as 2 bytes a lane: bf16 4096 x 4096 x 512 23.3 ->
+    // 21.8 us, 3200 x 2560 x 96 8.5 -> 7.8, 6144 x 8192 x 1024 98.2 -> 94.5, 4096^3 within 1 %.
     typedef out_t out2_t __attribute__((ext_vector_type(2)));
     typedef out_t out8_t __attribute__((ext_vector_type(8), aligned(sizeof(out_t))));
     typedef uint32_t words_t __attribute__((ext_vector_type(4)));
@@ -737,21 +747,27 @@ __device__ __forceinline__ void mmt4d_mfma_body(const MfmaArgs a, const int bid 
         for (int b = 0; b < 2; ++b)
 #pragma unroll
           for (int h = 0; h < 2; ++h)
-            w[b][h] = __builtin_bit_cast(uint32_t, out2_t{(out_t)(acc[x][y + b][2 * h] * a.out_scale),      // (x 1.0f is exact)
-                                                          (out_t)(acc[x][y + b][2 * h + 1] * a.out_scale)});
+            // (x 1.0f is exact)
+            w[b][h] = __builtin_bit_cast(uint32_t, out2_t{(out_t)(acc[x][y + b][2 * h] * (row_major_out ? a.out_scale : 1.0f)),
+                                                          (out_t)(acc[x][y + b][2 * h + 1] * (row_major_out ? a.out_scale : 1.0f))});
         const auto p = __builtin_amdgcn_permlane16_swap(w[0][0], w[1][0], false, false);
         const auto q = __builtin_amdgcn_permlane16_swap(w[0][1], w[1][1], false, false);
         const out8_t v8 = __builtin_bit_cast(out8_t, words_t{(uint32_t)p[0], (uint32_t)q[0], (uint32_t)p[1], (uint32_t)q[1]});
         const int bj = j_base + wn * WN + y, col = bj * R + in_pair;
-        if constexpr (tiles_too) {
-          // (half a tile, 1 KiB of consecutive memory, that nothing reads soon: past the
-          // caches. 2048^3 36.4 -> 34.8 us, 3000 x 3333 x 1500 53.7 -> 51.6.)
+        if constexpr (tiles_too || !row_major_out) {
+          // (half a tile, 1 KiB of consecutive memory. Beside the matrix nothing reads it
+          // soon: past the caches, 2048^3 36.4 -> 34.8 us, 3000 x 3333 x 1500 53.7 -> 51.6.)
           const int bi = i_base + wm * WM + x;
-          if (bi / 2 < a.M && bj / 2 < a.N)
-            __builtin_nontemporal_store(v8, (out8_t*)((out_t*)(a.tiles + (int64_t)(bi / 2) * a.tiles_stride_bytes) +
-                                                      (int64_t)(bj / 2) * 1024 + ((bi % 2) * R + acc_r) * 32 + in_pair));
+          if (bi / 2 < a.M && bj / 2 < a.N) {
+            char* const base = row_major_out ? a.tiles : a.out;
+            const int64_t pitch = row_major_out ? a.tiles_stride_bytes : a.out_stride_bytes;
+            out8_t* t = (out8_t*)((out_t*)(base + (int64_t)(bi / 2) * pitch) + (int64_t)(bj / 2) * 1024 +
+                                  ((bi % 2) * R + acc_r) * 32 + in_pair);
+            if (tiles_too || (kStreamOut && a.stream_out)) __builtin_nontemporal_store(v8, t);
+            else *t = v8;
+          }
         }
-        if (row < a.out_rows) {
+        if (row_major_out && row < a.out_rows) {
           if (col + 8 <= a.out_cols) {
             *(out8_t*)(dst + col) = v8;
           } else {

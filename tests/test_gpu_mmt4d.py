@@ -2048,3 +2048,32 @@ def test_data_tiled_matmul_writes_matrix_and_tiles(uk, cuda, kind, M, N, K, accu
     assert torch.equal(c, step)
     for name in ("lhs", "rhs", "out"):
         assert torch.equal(ws[name], chain[name]), name
+
+
+@pytest.mark.parametrize("accumulate", [False, True])
+@pytest.mark.parametrize("M1,N1,K1", [(33, 41, 20), (64, 64, 9), (37, 129, 33)])
+@pytest.mark.parametrize("type_flag,dtype", [(F.MMT4D_TYPE_F16F16F16, "float16"), (F.MMT4D_TYPE_BF16BF16BF16, "bfloat16")])
+def test_tiled_16_bit_results_in_block_pairs(uk, cuda, type_flag, dtype, M1, N1, K1, accumulate):
+    """Edges of macro tiles, partial K steps, a result that starts at an odd element and
+    outer rows with a gap between them: each value is the f32 sum rounded once (half a unit of
+    the type, 2^-11 or 2^-8 of the value, and K 2^-24 of the sum of the terms' sizes), and
+    nothing between the rows is written."""
+    import torch
+    dt = getattr(torch, dtype)
+    g = torch.Generator(device="cuda").manual_seed(M1 + N1 + K1)
+    lhs, rhs = (torch.randn(n, K1, 32, 8, generator=g, device="cuda").to(dt) for n in (M1, N1))
+    pitch = N1 * 1024 + 6
+    out = torch.randn(1 + M1 * pitch, generator=g, device="cuda").to(dt)
+    before = out.clone()
+    flags = type_flag | F.MMT4D_SKIP_INTERMEDIATE_ROUNDINGS | (F.MMT4D_ACCUMULATE if accumulate else 0)
+    uk.mmt4d(lhs.view(-1), rhs.view(-1), out, M1, N1, K1, 32, 32, 8, flags, out_offset=1, out_stride0=pitch)
+    assert min(uk.last_macro_tile()[:2]) >= 128 and uk.last_macro_tile()[2] == 1
+    a, b = (t.double().transpose(1, 2).reshape(-1, K1 * 8) for t in (lhs, rhs))
+    tiles = lambda t: t[1:].view(M1, pitch)[:, :N1 * 1024].reshape(M1, N1, 32, 32).transpose(1, 2).reshape(M1 * 32, -1).double()  # noqa: E731
+    want, size = a @ b.t(), a.abs() @ b.abs().t()
+    if accumulate:
+        want, size = want + tiles(before), size + tiles(before).abs()
+    bound = want.abs() * (2.0 ** -11 if dtype == "float16" else 2.0 ** -8) + size * (K1 * 8 * 2.0 ** -24) + 2.0 ** -24
+    assert bool(((tiles(out) - want).abs() <= bound).all())
+    gaps = lambda t: t[1:].view(M1, pitch)[:, N1 * 1024:]  # noqa: E731
+    assert torch.equal(gaps(out), gaps(before)) and out[0] == before[0]
