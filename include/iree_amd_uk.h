@@ -436,10 +436,11 @@ IREE_AMD_UK_EXPORT int iree_amd_uk_query_matmul_tile_sizes(
  * (two per byte, even group in the low nibble) when ..._ZP_U4 is set. f32
  * accumulation, result rounded to f16 once (RNE). out: f16 [M][N] row-major.
  * Requires K % group_size == 0, group_size % 32 == 0, 1 <= M. A K beyond
- * 4096, and with more than 64 rows a shorter one where that is faster, is
+ * 4096, and with more than 32 rows a shorter one where that is faster, is
  * multiplied in slices whose f32 sums go through the stream's scratch buffer
  * (see iree_amd_uk_mmt4d on that buffer; a call with K <= 4096 and more than 64
- * rows that is being captured into a graph is not split).
+ * rows that is being captured into a graph is not split, one of 33 to 64 rows is where
+ * one of fewer rows would be).
  *===------------------------------------------------------------------------===*/
 #define IREE_AMD_UK_FLAG_DEQUANT_MATMUL_ZP_F16 0x0
 #define IREE_AMD_UK_FLAG_DEQUANT_MATMUL_ZP_U4 0x1
@@ -643,7 +644,8 @@ IREE_AMD_UK_EXPORT int iree_amd_uk_matmul_packed_rhs(
 
 /* The whole data-tiled matmul: what pack(A), pack(B, inner and outer transposed),
  * [pack(C)], mmt4d and unpack do (a small problem as one launch or two, another in full
- * tiles as that chain with both operands packed by one launch)
+ * tiles as that chain with both operands packed by one launch, or 2-byte elements whose
+ * rows of b are whole 8 KiB by two, and c written by the matmul)
  * (REF compiler/src/iree/compiler/Codegen/Common/CPU/CPULowerToUKernels.cpp:339-480).
  *   c[m][n] (+)= sum_k a[m][k] * b[k][n]
  * a is M x K, b K x N, c M x N, all row-major and tight, element types as in
@@ -657,8 +659,7 @@ IREE_AMD_UK_EXPORT int iree_amd_uk_matmul_packed_rhs(
  * third), with an error no larger.
  * Returns IREE_AMD_UK_STATUS_NOT_FOUND, with no error recorded and nothing
  * written, for what it does not serve: run the chain then. That is a null lhs or
- * rhs, or a narrow tile, of a large problem; 2-byte elements whose rows of b are whole
- * 8 KiB, of a large problem; tiles without a matrix-core kernel; buffers that
+ * rhs, or a narrow tile, of a large problem; tiles without a matrix-core kernel; buffers that
  * overlap; operands or results that are not aligned to their elements, lhs and rhs
  * to 16 bytes. A long K
  * of few tiles is split over workgroups, whose partial sums lie in the stream's

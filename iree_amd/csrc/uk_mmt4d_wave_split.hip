@@ -347,8 +347,8 @@ double estimate_us(const WaveSplitArgs& a, bool f32, int out_bytes, const Tile& 
 // -> 18.3, so not for less.) Fitted to the geometric mean of the times with weights beyond
 // the last-level cache and with three layers in turn, 7200 problems (1 to 64 rows, 512 to
 // 28672 columns, K 768 to 14336), 6 to 9 % off on average. The tile that it picks and, against
-// macro tiles that keep K whole (few_rows_us), the kernel: the SiLU form 1.12 times as fast as
-// with the estimate above on 200 other problems, none slower by 3 % (32 rows x 2 x 8192 x 2048
+// macro tiles that keep K whole (few_rows_us), the kernel: the SiLU form 1.09 times as fast as
+// with the estimate above on 78 other problems, in either state, none slower by 2 % (32 rows x 2 x 8192 x 2048
 // 11.7 -> 8.5 us, 2 x 14336 x 4096 23.2 -> 21.9), the plain form 1.01. Below these sizes and
 // for the other types and forms it gave nothing, and costs a call of 4 us a tenth of them.
 struct RowsTile { float first, round, rhs, lhs, memory, store, silu; };
