@@ -257,7 +257,8 @@ int launch_dequant_matmul_i4(const void* x, const void* w, const void* scale, co
   // 0.4 % from the faster of the two and 16 problems over 4 % slower than there (10 %
   // at most). 59 x 2496 x 13056 with groups of 64 23.2 -> 17.0 us, 40 x 5120 x 2304
   // 15.0 -> 11.0; 36 x 6528 x 2048 stays below, 9.8 against 11.7.
-  if (M > 32 && tiled && a.zp_u4 && gs_ok && K % 128 == 0 && size_ok && aligned) {
+  // (an empty K, whose result is zeros, is the element-wise kernel's)
+  if (M > 32 && tiled && a.zp_u4 && gs_ok && K > 0 && K % 128 == 0 && size_ok && aligned) {
     a.w_bytes = (uint32_t)w_bytes;
     const double limit_us = M > 64 || !k_ok ? 0.0 : two_passes_us(a, slice_kb, (int)k_rows);
     const int st = launch_dequant_gemm_i4(a, limit_us, s);

@@ -358,6 +358,33 @@ def test_validation_happens_before_any_device_work():
     assert lib.iree_amd_uk_version() >= 1
 
 
+EMPTY_K = """
+import ctypes as C
+import sys
+import iree_amd
+from iree_amd import flags as F
+lib = iree_amd.load_library()
+memory = C.create_string_buffer(1 << 16)
+at = C.c_void_p((C.addressof(memory) + 255) // 256 * 256)
+for M in (1, 32, 33, 40, 64, 65, 70):
+    for flags in (F.DEQUANT_MATMUL_ZP_U4, F.DEQUANT_MATMUL_ZP_U4 | F.DEQUANT_MATMUL_W_TILED):
+        assert lib.iree_amd_uk_dequant_matmul_i4(at, at, at, at, at, M, 32, 0, 128, flags, None) != 0
+print("ended")
+"""
+
+
+def test_int4_matmul_of_an_empty_k_reaches_its_launch():
+    """Every number of rows with no K at all: the choice of a kernel comes to its end, so that
+    without a device the launch fails with a status (a process of its own: a division by
+    zero would end it). Needs a machine without a device: the buffers are host memory."""
+    import torch
+    if torch.cuda.is_available():
+        pytest.skip("the result on a device: test_an_empty_k_gives_zeros")
+    r = subprocess.run([sys.executable, "-c", EMPTY_K], cwd=ROOT,
+                       capture_output=True, text=True, timeout=300)
+    assert r.returncode == 0 and r.stdout.strip().endswith("ended"), r.stderr[-2000:]
+
+
 @pytest.mark.parametrize("form,calls", [
     ({}, ["pack", "pack", "mmt4d", "unpack"]), ({"accumulate": True}, ["pack", "pack", "pack", "mmt4d", "unpack"]),
     ({"fuse_unpack": True}, ["pack", "pack", "mmt4d_unpack"]), ({"fuse_pack_lhs": True}, ["pack", "matmul_packed_rhs"]),

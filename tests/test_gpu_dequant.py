@@ -335,6 +335,20 @@ def test_33_to_64_rows(uk, cuda, M, N, K, gs, path):
     assert err <= float(np.spacing(np.float16(max(1.0, mag))))
 
 
+@pytest.mark.parametrize("M", [1, 32, 33, 40, 64, 65, 70])
+@pytest.mark.parametrize("tiled", [False, True])
+def test_an_empty_k_gives_zeros(uk, cuda, M, tiled):
+    import torch
+    N, gs = 64, 128
+    x = torch.ones(M, gs, dtype=torch.float16, device="cuda")
+    w = torch.full((N, gs // 2), 0x77, dtype=torch.uint8, device="cuda")
+    scale, zp = torch.ones(N, dtype=torch.float16, device="cuda"), torch.zeros(N, dtype=torch.uint8, device="cuda")
+    out = torch.full((M + 1, N), float("nan"), dtype=torch.float16, device="cuda")
+    uk.dequant_matmul_i4(x, w, scale, zp, out, M, N, 0, gs,
+                         F.DEQUANT_MATMUL_ZP_U4 | (F.DEQUANT_MATMUL_W_TILED if tiled else 0))
+    assert bool((out[:M] == 0).all()) and bool(out[M].isnan().all())
+
+
 @pytest.mark.parametrize("M,N,K,gs", [
     (257, 13088, 384, 32), (385, 13984, 384, 64), (470, 12320, 384, 128), (257, 13088, 768, 256),   # 128 x 256
     (65, 10816, 3200, 32), (65, 10976, 3200, 64), (512, 4096, 14336, 128),                          # ... K split
