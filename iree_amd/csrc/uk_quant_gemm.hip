@@ -314,6 +314,10 @@ __device__ __forceinline__ void dequant_matmul_i4_gemm_body(const I4GemmArgs& a)
   __builtin_amdgcn_sched_barrier(0);
   gemm_wait_vmcnt<2 * kWLoads + (kRing - 1) * kXLoads>();
   params.convert_first(s0);
+  // (the first span's rows come from every wave; and step 0 counts on all of this: its
+  // wait for span 1 allows for a step's loads before it, its wait for a refill, which may
+  // be the last thing requested here, for a step's activations behind it)
+  gemm_wait_vmcnt<0>();
   __syncthreads();
   read_block(0, 0);
 #pragma unroll
@@ -519,6 +523,9 @@ __device__ __forceinline__ void dequant_matmul_i4_gemm_small_body(const I4GemmAr
   __builtin_amdgcn_sched_barrier(0);
   gemm_wait_vmcnt<2 + (kRing - 1) * kXLoads>();
   params.convert_first(s0);
+  // (as above: the first span's rows come from every wave, and the waits of step 0 allow
+  // for loads that only later steps have behind them)
+  gemm_wait_vmcnt<0>();
   __syncthreads();
   auto read_pair = [&](int from, int xp) {
 #pragma unroll

@@ -385,6 +385,19 @@ def test_int4_matmul_of_an_empty_k_reaches_its_launch():
     assert r.returncode == 0 and r.stdout.strip().endswith("ended"), r.stderr[-2000:]
 
 
+def test_int4_tiled_kernels_wait_for_what_the_first_step_reads():
+    """Between the first scales of a workgroup and the barrier that publishes them and the
+    first rows, both bodies wait for every load in flight: other waves read those rows, and the
+    counted waits of the first step allow for loads that only later steps have behind them.
+    (In the source: a barrier that happens to wait as well would hide that it is missing.)"""
+    with open(os.path.join(ROOT, "iree_amd", "csrc", "uk_quant_gemm.hip")) as f:
+        source = f.read()
+    starts = source.split("params.convert_first(s0);")[1:]
+    assert len(starts) == 2
+    for start in starts:
+        assert "gemm_wait_vmcnt<0>();" in start[:start.index("__syncthreads();")]
+
+
 @pytest.mark.parametrize("form,calls", [
     ({}, ["pack", "pack", "mmt4d", "unpack"]), ({"accumulate": True}, ["pack", "pack", "pack", "mmt4d", "unpack"]),
     ({"fuse_unpack": True}, ["pack", "pack", "mmt4d_unpack"]), ({"fuse_pack_lhs": True}, ["pack", "matmul_packed_rhs"]),
