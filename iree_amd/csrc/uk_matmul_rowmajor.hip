@@ -731,15 +731,28 @@ template <typename Cfg>
 int launch(RowMajorArgs p, hipStream_t s) {
   constexpr int kStep = 64 / Cfg::kElemBytes;                     // elements of K per step
   const int64_t rows = (int64_t)p.M1 * p.M0, cols = (int64_t)p.N1 * p.N0;
-  // (the chain as it was fitted packed the operands one after the other; in one launch
-  // they take 2.0 to 3.5 us less: 1500 x 1501 x 1502 int8 26.4 -> 22.9 us in all)
-  const double chain = full_tiles_chain<Cfg>(p) ? full_tiles_chain_us<Cfg>(p) : chain_us<Cfg>(p);
-  const bool together = p.lhs && p.rhs && p.M0 == 32 && p.N0 == 32 && (Cfg::kElemBytes != 2 || p.N % 4096 != 0);
-  // (f32: its chain takes longer than estimated, for results of up to 3 million elements; on
-  // 2343 problems 2.6 % from the best kernel on average and 5 over 20 % longer than as the
-  // chain, with 0.9 of it 3.1 % and 4, and 531x2782x605 42.0 us as the chain, 27.8 in one launch)
+  // The chain on full tiles is taken where its estimate is the shorter. 16-bit types with
+  // rows of b of whole 8 KiB and results of up to 6 million elements: by a quarter and more,
+  // since there the estimate of one launch is the one that is off (420 problems of 4096 to
+  // 16384 columns take 0.56 to 1.0 times it, 0.75 in the middle), and the chain packs each
+  // operand by its own launch. On those 1.8 % from the faster of the two on average and 1.41
+  // times its time at most, at 1.0 instead of 1.35 4.9 % and 1.75 times (bf16 130x8192x523
+  // 11.6 us in one launch, 21.1 as the chain; f16 601x4096x73 10.0 and 16.5); with larger
+  // results among them 2.5 % (bf16 added to C 3874x4096x357 70 us in one launch, 52 as a
+  // chain). Other row lengths lose by such a factor: whole 64s 2.2 -> 2.8 %, odd ones 0.5 -> 2.6 %.
+  // f32 (the chain as it was fitted packed the operands one after the other; in one launch
+  // they take 2.0 to 3.5 us less) takes longer as the chain than estimated, for results of up
+  // to 3 million elements; on 2343 problems 2.6 % from the best kernel on average and 5 over
+  // 20 % longer than as the chain, with 0.9 of it 3.1 % and 4, and 531x2782x605 42.0 us as the
+  // chain, 27.8 in one launch.
+  const bool full = full_tiles_chain<Cfg>(p);
+  const bool whole_rows = Cfg::kElemBytes == 2 && p.N % 4096 == 0 && rows * cols <= 6000000;
+  const double chain = full ? full_tiles_chain_us<Cfg>(p) : chain_us<Cfg>(p);
+  const bool together = p.lhs && p.rhs && p.out && p.M0 == 32 && p.N0 == 32;
   const bool slow_chain = Cfg::kElemBytes == 4 && rows * cols <= 3000000;
-  const double limit = full_tiles_chain<Cfg>(p) ? chain : together && p.out && chain < 24.0 ? chain - 2.4 : (slow_chain ? 1.1 : 0.9) * chain;
+  const double limit = full                       ? (whole_rows ? 1.35 : 1.0) * chain
+                       : together && chain < 24.0 ? chain - 2.4
+                                                  : (slow_chain ? 1.1 : 0.9) * chain;
   int mb = 1, slices = 1;
   double us = limit;
   const bool found = choose<Cfg>(p, 16, &us, &mb, &slices);

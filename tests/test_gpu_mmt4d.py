@@ -1812,6 +1812,28 @@ def test_scaled_rows_on_either_kernel(uk, cuda, type_flag, dt, M, N, K, narrow):
     assert torch.equal(y[:M * N].view(M, N).double(), want) and (y[M * N:] == 7.0).all()
 
 
+@pytest.mark.parametrize("type_flag,dt,out_dt,M,N,K,accumulate,path", [
+    (F.MMT4D_TYPE_BF16BF16F32, "bfloat16", "float32", 130, 8192, 523, False, "mmt4d:mfma-one-launch"),
+    (F.MMT4D_TYPE_F16F16F32, "float16", "float32", 601, 4096, 73, False, "mmt4d:mfma-one-launch"),
+    (F.MMT4D_TYPE_F16F16F16, "float16", "float16", 155, 4096, 1048, True, "mmt4d:mfma-one-launch"),
+    (F.MMT4D_TYPE_BF16BF16BF16, "bfloat16", "bfloat16", 900, 4096, 2000, True, "mmt4d:mfma"),
+])
+def test_b_of_whole_8_kib_rows(uk, cuda, type_flag, dt, out_dt, M, N, K, accumulate, path):
+    """One launch where the chain, which packs such a B by a launch of its own, takes half
+    as long again. Small whole numbers: the same bits as step by step."""
+    import torch
+    g = torch.Generator(device="cuda").manual_seed(M + N + K)
+    a = torch.randint(-1, 2, (M * K,), generator=g, device="cuda").to(getattr(torch, dt))
+    b = torch.randint(-1, 2, (K * N,), generator=g, device="cuda").to(getattr(torch, dt))
+    c = torch.randint(-3, 4, (M * N,), generator=g, device="cuda").to(getattr(torch, out_dt))
+    step = c.clone()
+    uk.matmul_data_tiled(a, b, c, M, N, K, type_flag, accumulate=accumulate)
+    if torch.cuda.get_device_properties(0).multi_processor_count == 256:
+        assert uk.last_kernel_path() == path
+    uk.matmul_data_tiled(a, b, step, M, N, K, type_flag, accumulate=accumulate, one_launch=False)
+    assert torch.equal(c, step)
+
+
 @pytest.mark.parametrize("type_flag,dt,out_dt,M,N,K,path", [
     (F.MMT4D_TYPE_F16F16F32, "float16", "float32", 2945, 3940, 145, "mmt4d:mfma"),
     (F.MMT4D_TYPE_S8S8S32, "int8", "int32", 3357, 3403, 44, "mmt4d:mfma"),
