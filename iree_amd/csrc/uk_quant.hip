@@ -260,7 +260,10 @@ int launch_dequant_matmul_i4(const void* x, const void* w, const void* scale, co
   // (an empty K, whose result is zeros, is the element-wise kernel's)
   if (M > 32 && tiled && a.zp_u4 && gs_ok && K > 0 && K % 128 == 0 && size_ok && aligned) {
     a.w_bytes = (uint32_t)w_bytes;
-    const double limit_us = M > 64 || !k_ok ? 0.0 : two_passes_us(a, slice_kb, (int)k_rows);
+    // (up to 48 rows, whose second pass is the short one, and groups of 32: of 115 problems 8
+    // took 2 to 8 % longer on the tiled kernel, with 3 % less to beat 2, which gives up a
+    // fortieth of its gain; the other rows and groups 1 of 275)
+    const double limit_us = M > 64 || !k_ok ? 0.0 : (M <= 48 && a.log2_gs == 5 ? 0.97 : 1.0) * two_passes_us(a, slice_kb, (int)k_rows);
     const int st = launch_dequant_gemm_i4(a, limit_us, s);
     if (st != IREE_AMD_UK_STATUS_NOT_FOUND) { note_kernel_path("dequant_i4:gemm"); return st; }
   }

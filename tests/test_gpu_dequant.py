@@ -327,6 +327,7 @@ def test_many_rows(uk, cuda, M, N, K, gs):
     (33, 32, 128, 128, "gemm"), (49, 96, 384, 32, "gemm"), (64, 5120, 2304, 128, "gemm"),     # K in whole 128s and 256s
     (59, 2496, 13056, 64, "gemm"),                                                             # K split
     (36, 6528, 2048, 128, "mfma"), (36, 576, 13824, 32, "mfma"),     # two passes over the weights are faster
+    (44, 3136, 11520, 32, "mfma"),                                    # ... groups of 32, estimates 1 % apart
 ])
 def test_33_to_64_rows(uk, cuda, M, N, K, gs, path):
     """Up to a tile of rows: the tiled kernel or two passes of the streaming one,
