@@ -97,8 +97,7 @@ __device__ __forceinline__ void wait_loads() {
 // 64 bytes of one row, and are read from there in operand order. A block lies
 // in LDS row by row, the pieces of row r rotated by r / 4: the reads of 16 rows
 // touch every bank alike.)
-// kStreamed: the right-hand side goes past the caches.
-template <typename T, typename out_t, int MB, int NB, int D, bool kRowMajor, bool kStreamed>
+template <typename T, typename out_t, int MB, int NB, int D, bool kRowMajor>
 __device__ __forceinline__ void mmt4d_wave_split_body(const WaveSplitArgs& a) {
   typedef typename BlockProduct<T>::acc_t acc_t;
   constexpr int F = MB * NB;
@@ -174,8 +173,7 @@ __device__ __forceinline__ void mmt4d_wave_split_body(const WaveSplitArgs& a) {
 #pragma unroll
     for (int y = 0; y < NB; ++y)
       fb[d][y] = __builtin_bit_cast(
-          u32x4, __builtin_amdgcn_raw_buffer_load_b128(rhs_src, rhs_exists ? rhs_at[y] : kNowhere, step * 2048,
-                                                       kStreamed ? 2 /* non-temporal */ : 0));
+          u32x4, __builtin_amdgcn_raw_buffer_load_b128(rhs_src, rhs_exists ? rhs_at[y] : kNowhere, step * 2048, 0));
     if constexpr (kRowMajor) __builtin_amdgcn_sched_barrier(0);
   };
   // (row-major) the blocks of step d from LDS; `behind`: loads issued after theirs
@@ -295,9 +293,9 @@ __device__ __forceinline__ void mmt4d_wave_split_body(const WaveSplitArgs& a) {
 }
 
 // (the body is a function of its own: the host pass has no buffer descriptors)
-template <typename T, typename out_t, int MB, int NB, int D, int kOcc, bool kRowMajor, bool kStreamed = false>
+template <typename T, typename out_t, int MB, int NB, int D, int kOcc, bool kRowMajor>
 __global__ __launch_bounds__(kWaves * 64, kOcc) void mmt4d_wave_split_kernel(WaveSplitArgs a) {
-  mmt4d_wave_split_body<T, out_t, MB, NB, D, kRowMajor, kStreamed>(a);
+  mmt4d_wave_split_body<T, out_t, MB, NB, D, kRowMajor>(a);
 }
 
 // Estimated time in microseconds on a tile of mb x nb blocks. Workgroups run in
@@ -340,27 +338,25 @@ double estimate_us(const WaveSplitArgs& a, bool f32, int out_bytes, const Tile& 
 
 // Up to 64 rows of fp8 in packed tiles (a decode step of the MLP block) with 1.5 KB of K and
 // weights of 16 MB and more: the intake of a compute unit and the time at memory's rate
-// (both operands, `memory` us per MB) add up. The last three are the tiles 2 to 4 with the
-// weights streamed past the caches: of a layer of 32 MB and more, whose next use is far off,
-// and rows that one workgroup has all of, so that nobody else asks for them. (32 rows x 14336
-// x 4096 on 32 x 32 results 14.9 -> 13.8 us; weights that stay in the last-level cache 12.6
-// -> 18.3, so not for less.) Fitted to the geometric mean of the times with weights beyond
-// the last-level cache and with three layers in turn, 7200 problems (1 to 64 rows, 512 to
-// 28672 columns, K 768 to 14336), 6 to 9 % off on average. The tile that it picks and, against
-// macro tiles that keep K whole (few_rows_us), the kernel: the SiLU form 1.09 times as fast as
-// with the estimate above on 78 other problems, in either state, none slower by 2 % (32 rows x 2 x 8192 x 2048
-// 11.7 -> 8.5 us, 2 x 14336 x 4096 23.2 -> 21.9), the plain form 1.01. Below these sizes and
-// for the other types and forms it gave nothing, and costs a call of 4 us a tenth of them.
+// (both operands, `memory` us per MB) add up. Fitted to the geometric mean of the times with
+// weights beyond the last-level cache and with three layers in turn, 7200 problems (1 to 64 rows, 512 to
+// 28672 columns, K 768 to 14336), 6 to 9 % off on average. It decides the tile and, against
+// macro tiles that keep K whole (few_rows_us), the kernel: the SiLU form 1.14 times as fast as with
+// the estimate above on 75 other problems, with weights in the last-level cache and beyond it
+// alike (32 rows x 2 x 8192 x 2048 9.3 -> 7.8 us with three layers in turn, 11.6 -> 8.7 beyond
+// it); the plain form, 29 problems, as fast as before. 2 x 14336 x 4096 stays on macro tiles.
+// Below these sizes and for the other types and forms it gave nothing, and costs a call of
+// 4 us a tenth of them.
+// (Weights past the caches by non-temporal loads, one workgroup having all rows: 5 to 8 %
+// faster on 27 problems of 38 to 128 MB whose weights come from memory, 3 to 15 % slower where
+// three layers stay in the last-level cache. The call cannot know, so not.)
 struct RowsTile { float first, round, rhs, lhs, memory, store, silu; };
-constexpr int kStreamedTiles = 3;
-constexpr RowsTile kRowsTile[kTiles + kStreamedTiles] = {
+constexpr RowsTile kRowsTile[kTiles] = {
     {3.52f, 0.23f, 6.07f, 9.48f, 0.085f, 0.15f, 0.0f},  {3.34f, 0.19f, 7.77f, 9.98f, 0.090f, 0.31f, 0.17f},
     {3.36f, 0.30f, 6.16f, 11.7f, 0.086f, 0.16f, 0.06f}, {3.78f, 1.14f, 5.72f, 12.9f, 0.108f, 0.11f, -0.14f},
-    {4.29f, 1.78f, 2.97f, 9.93f, 0.112f, 0.21f, 0.01f}, {3.01f, 0.16f, 10.4f, 16.4f, 0.064f, 0.22f, 0.46f},
-    {3.92f, 1.40f, 8.14f, 19.9f, 0.080f, 0.12f, -0.32f}, {3.56f, 1.84f, 5.76f, 16.3f, 0.069f, 0.62f, 0.84f}};
-constexpr int base_tile(int v) { return v < kTiles ? v : v - kStreamedTiles; }
+    {4.29f, 1.78f, 2.97f, 9.93f, 0.112f, 0.21f, 0.01f}};
 double few_rows_estimate_us(const WaveSplitArgs& a, int out_bytes, int v, int cus) {
-  const Tile& t = kTile[base_tile(v)];
+  const Tile& t = kTile[v];
   const RowsTile& f = kRowsTile[v];
   const uint32_t groups = (uint32_t)((a.rows + t.mb * 16 - 1) / (t.mb * 16)) * (uint32_t)((a.outer_cols * 2 + t.nb - 1) / t.nb);
   const double rounds = groups <= (uint32_t)cus ? 1.0 : (double)((groups + cus - 1) / cus);
@@ -374,18 +370,14 @@ double few_rows_estimate_us(const WaveSplitArgs& a, int out_bytes, int v, int cu
 template <typename T, typename out_t, bool kRowMajor>
 int launch_tile(WaveSplitArgs a, int v, hipStream_t s) {
   void (*kernel)(WaveSplitArgs) = nullptr;
-  constexpr bool kStreamed = std::is_same<T, F8>::value && !kRowMajor;      // (has streamed tiles)
   switch (v) {
-    case 5: kernel = mmt4d_wave_split_kernel<T, out_t, 2, 2, 4, 4, kRowMajor, kStreamed>; break;
-    case 6: kernel = mmt4d_wave_split_kernel<T, out_t, 2, 4, 4, 2, kRowMajor, kStreamed>; break;
-    case 7: kernel = mmt4d_wave_split_kernel<T, out_t, 4, 4, 2, 2, kRowMajor, kStreamed>; break;
     case 0: kernel = mmt4d_wave_split_kernel<T, out_t, 1, 1, 8, 4, kRowMajor>; break;
     case 1: kernel = mmt4d_wave_split_kernel<T, out_t, 1, 2, 6, 4, kRowMajor>; break;
     case 2: kernel = mmt4d_wave_split_kernel<T, out_t, 2, 2, 4, 4, kRowMajor>; break;
     case 3: kernel = mmt4d_wave_split_kernel<T, out_t, 2, 4, 4, 2, kRowMajor>; break;
     default: kernel = mmt4d_wave_split_kernel<T, out_t, 4, 4, 2, 2, kRowMajor>; break;
   }
-  const Tile& t = kTile[base_tile(v)];
+  const Tile& t = kTile[v];
   a.tiles_m = (int)ceil_div((int64_t)a.rows, (int64_t)(t.mb * 16));
   a.tiles_n = (int)ceil_div((int64_t)a.outer_cols * 2, (int64_t)t.nb);
   const int64_t blocks = (int64_t)a.tiles_m * a.tiles_n * a.batch;
@@ -421,16 +413,14 @@ WaveSplitChoice choose_wave_split(const WaveSplitArgs& a, uint32_t type) {
   }
   const int64_t weights = (int64_t)a.outer_cols * 512 * a.k_chunks;
   if (best.tile >= 0 && f8 && a.rows <= 64 && a.lhs_chunk != 16 && a.batch == 1 && a.k_chunks >= 96 && weights >= 16000000) {
-    const bool large = weights >= (32 << 20);
-    for (int v = 0; v < kTiles + (large ? kStreamedTiles : 0); ++v) {
-      const Tile& t = kTile[base_tile(v)];
-      if ((a.silu && t.nb == 1) || (v >= kTiles && a.rows > t.mb * 16)) continue;
+    for (int v = 0; v < kTiles; ++v) {
+      if (a.silu && kTile[v].nb == 1) continue;
       const double us = few_rows_estimate_us(a, out_bytes, v, cus);
       if (!best.few_rows || us < best.us) { best.tile = v; best.us = us; best.few_rows = true; }
     }
   }
   if (best.tile >= 0) {
-    const Tile& t = kTile[base_tile(best.tile)];
+    const Tile& t = kTile[best.tile];
     best.one_round = ceil_div((int64_t)a.rows, (int64_t)(t.mb * 16)) *
                          ceil_div((int64_t)a.outer_cols * 2, (int64_t)t.nb) * a.batch <= cus;
   }

@@ -367,8 +367,8 @@ def test_gate_up_silu_of_few_tiles_has_the_bits_of_mmt4d(uk, cuda, M1, P, K1, ti
 
 @pytest.mark.parametrize("M1,P,K1", [(1, 256, 128), (1, 231, 159), (1, 203, 200), (2, 231, 200), (2, 249, 259)])
 def test_gate_up_silu_on_large_weights(uk, cuda, M1, P, K1):
-    """Up to 64 rows against weights of 32 MB and more, which go past the caches: ragged
-    columns and K, plain mmt4d within the error of the instruction's sums (2e-5 of the sum of
+    """Up to 64 rows against weights of 32 MB and more, where the tile and the kernel are
+    chosen by a fit of their own: ragged columns and K, plain mmt4d within the error of the instruction's sums (2e-5 of the sum of
     the magnitudes of the terms) of float64, the fused form with its bytes."""
     import torch
     type_flag, K0 = F.MMT4D_TYPE_F8E4M3F8E4M3F32, 16
