@@ -685,7 +685,9 @@ int launch_gemm_instance(const I4GemmArgs& a, int slices, hipStream_t s) {
 template <int WC, int XB>
 int launch_gemm_shape(const I4GemmArgs& a, int log2_ge, int slices, hipStream_t s) {
   switch (log2_ge) {
-    case 5: return launch_gemm_instance<WC, XB, 5>(a, slices, s);
+    case 5:
+      if constexpr (WC == 4) return IREE_AMD_UK_STATUS_NOT_FOUND;     // (serves_groups)
+      else return launch_gemm_instance<WC, XB, 5>(a, slices, s);
     case 6: return launch_gemm_instance<WC, XB, 6>(a, slices, s);
     default: return launch_gemm_instance<WC, XB, 7>(a, slices, s);
   }
@@ -710,9 +712,12 @@ constexpr GemmShape kGemmShapes[kShapes] = {
     {64, 64, {0.84f, 0.63f, 0.54f}, {1.20f, 0.92f, 0.77f}, {1.14f, 0.86f, 0.75f}, 0.23f},
     {128, 256, {2.12f, 1.61f, 1.34f}, {}, {1.85f, 1.45f, 1.18f}, 3.57f},
     {64, 256, {1.50f, 1.11f, 0.93f}, {}, {1.46f, 1.09f, 0.94f}, 1.49f},
-    {64, 128, {1.26f, 0.86f, 0.70f}, {0.0f, 1.25f, 1.05f}, {1.33f, 1.03f, 0.87f}, 1.10f}};
+    {64, 128, {0.0f, 0.86f, 0.70f}, {0.0f, 1.25f, 1.05f}, {0.0f, 1.03f, 0.87f}, 1.10f}};
+// (64 x 128 with groups of 32, of which a compute unit takes one workgroup, took 1.26 us a span
+// alone and 1.33 in the rounds before the last: 64 x 64, of which it takes two, is never slower)
+constexpr bool serves_groups(int v, int log2_ge) { return v != 3 || log2_ge > 5; }
 // Workgroups of shape v on one compute unit: two of the smaller ones.
-constexpr int workgroups_per_cu(int v, int log2_ge) { return v == 0 || (v == 3 && log2_ge > 5) ? 2 : 1; }
+constexpr int workgroups_per_cu(int v) { return v == 0 || v == 3 ? 2 : 1; }
 static_assert(2 * i4_gemm_lds_bytes<2, 2, 5>() <= 160 * 1024 && 2 * i4_gemm_lds_bytes<4, 2, 6>() <= 160 * 1024 &&
               2 * i4_gemm_lds_bytes<4, 2, 5>() > 160 * 1024 && 2 * i4_gemm_lds_bytes<8, 2, 7>() > 160 * 1024,
               "workgroups_per_cu");
@@ -720,7 +725,7 @@ double gemm_estimate_us(const I4Args& p, int v, int log2_ge, int64_t tiles, int 
   const GemmShape& t = kGemmShapes[v];
   const int64_t slice_spans = ceil_div((int64_t)spans, (int64_t)slices);
   slices = (int)ceil_div((int64_t)spans, slice_spans);                     // (as launched)
-  const int64_t blocks = tiles * slices, slots = (int64_t)workgroups_per_cu(v, log2_ge) * cus;
+  const int64_t blocks = tiles * slices, slots = (int64_t)workgroups_per_cu(v) * cus;
   const int64_t before = ceil_div(blocks, slots) - 1, last = blocks - before * slots;
   const int g = log2_ge - 5;
   const double mb = (double)p.M * p.N * 1e-6;
@@ -746,6 +751,7 @@ int launch_dequant_gemm_i4(const I4Args& p, double limit_us, hipStream_t s) {
   auto choose = [&](int max_slices) {
     best = -1;
     for (int v = 0; v < kShapes; ++v) {
+      if (!serves_groups(v, log2_ge)) continue;
       const int64_t tiles = ceil_div((int64_t)p.M, (int64_t)kGemmShapes[v].rows) *
                             ceil_div((int64_t)p.N, (int64_t)kGemmShapes[v].cols);
       if (tiles > 0x7FFFFFFF) continue;
