@@ -731,26 +731,28 @@ template <typename Cfg>
 int launch(RowMajorArgs p, hipStream_t s) {
   constexpr int kStep = 64 / Cfg::kElemBytes;                     // elements of K per step
   const int64_t rows = (int64_t)p.M1 * p.M0, cols = (int64_t)p.N1 * p.N0;
-  // The chain on full tiles is taken where its estimate is the shorter. 16-bit types with
-  // rows of b of whole 8 KiB and results of up to 6 million elements: by a quarter and more,
-  // since there the estimate of one launch is the one that is off (420 problems of 4096 to
-  // 16384 columns take 0.56 to 1.0 times it, 0.75 in the middle), and the chain packs each
-  // operand by its own launch. On those 1.8 % from the faster of the two on average and 1.41
-  // times its time at most, at 1.0 instead of 1.35 4.9 % and 1.75 times (bf16 130x8192x523
-  // 11.6 us in one launch, 21.1 as the chain; f16 601x4096x73 10.0 and 16.5); with larger
-  // results among them 2.5 % (bf16 added to C 3874x4096x357 70 us in one launch, 52 as a
-  // chain). Other row lengths lose by such a factor: whole 64s 2.2 -> 2.8 %, odd ones 0.5 -> 2.6 %.
+  // The chain on full tiles is taken where its estimate is the shorter. 16-bit types with rows
+  // of b of whole 128-byte lines and results of up to 6 million elements: by 1.15 times, since
+  // there the estimate of one launch, fitted mostly to odd sizes, is too long (298 problems
+  // take 0.70 to 1.06 of it, 0.91 in the middle, odd columns 1.02). On 433 of them 1.8 % from
+  // the faster of the two on average and 4 over 10 % longer than as before this chain, without
+  // it 2.2 % and 19 (f16 480x4736x146 11.1 us in one launch, 14.5 as the chain); odd columns
+  // lose by it, 0.6 -> 2.6 %. Whole 8 KiB: 1.35 times; one launch takes 0.56 to 1.0 of its
+  // estimate, 0.75 in the middle, and the chain packs each operand by its own launch. On 420 of
+  // those 1.8 % from the faster and 1.41 times its time at most, without it 4.9 % and 1.75
+  // times (bf16 130x8192x523 11.6 us in one launch, 21.1 as the chain); with larger results
+  // among them 2.5 % (bf16 added to C 3874x4096x357 70 us in one launch, 52 as a chain).
   // f32 (the chain as it was fitted packed the operands one after the other; in one launch
   // they take 2.0 to 3.5 us less) takes longer as the chain than estimated, for results of up
   // to 3 million elements; on 2343 problems 2.6 % from the best kernel on average and 5 over
   // 20 % longer than as the chain, with 0.9 of it 3.1 % and 4, and 531x2782x605 42.0 us as the
   // chain, 27.8 in one launch.
   const bool full = full_tiles_chain<Cfg>(p);
-  const bool whole_rows = Cfg::kElemBytes == 2 && p.N % 4096 == 0 && rows * cols <= 6000000;
+  const bool whole_lines = Cfg::kElemBytes == 2 && p.N % 64 == 0 && rows * cols <= 6000000;
   const double chain = full ? full_tiles_chain_us<Cfg>(p) : chain_us<Cfg>(p);
   const bool together = p.lhs && p.rhs && p.out && p.M0 == 32 && p.N0 == 32;
   const bool slow_chain = Cfg::kElemBytes == 4 && rows * cols <= 3000000;
-  const double limit = full                       ? (whole_rows ? 1.35 : 1.0) * chain
+  const double limit = full                       ? (!whole_lines ? 1.0 : p.N % 4096 ? 1.15 : 1.35) * chain
                        : together && chain < 24.0 ? chain - 2.4
                                                   : (slow_chain ? 1.1 : 0.9) * chain;
   int mb = 1, slices = 1;
