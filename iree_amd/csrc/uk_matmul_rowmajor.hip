@@ -677,6 +677,23 @@ double full_tiles_chain_us(const RowMajorArgs& p) {
          (p.accumulate ? 1.1 + (sizeof(typename Cfg::out_t) == 2 ? 0.8 : 0.43) * out_mb : 0.0);
 }
 
+// By how much the estimate of the chain has to be the shorter: by the bytes of a result and
+// the rows of b (any, whole 128-byte lines, whole 8 KiB, where the chain packs each operand by
+// a launch of its own as well). Time over estimate of one launch, over the same of the chain,
+// where the estimates are within 1.6 of each other, has its middle at 0.86, 0.76 and 0.64 for f32
+// results, 1.09, 1.01 and 0.90 for 16-bit ones, and is larger where C is added; the
+// factors are those that gave the shortest times in all. Not for results of more than 24 MB (f32)
+// or 6 MB, which lose by it (bf16 added to C 3874x4096x357 70 us in one launch, 52 as a chain).
+template <typename Cfg>
+double times_shorter(const RowMajorArgs& p) {
+  constexpr bool kF32Out = sizeof(typename Cfg::out_t) == 4;
+  const int64_t elems = (int64_t)p.M1 * p.M0 * p.N1 * p.N0;
+  if (Cfg::kElemBytes != 2 || elems > (kF32Out ? 6000000 : 3000000)) return 1.0;
+  if (p.N % 4096 == 0) return kF32Out ? 1.4 : 1.2;
+  if (p.N % 64 == 0) return kF32Out && !p.accumulate ? 1.25 : 1.1;
+  return kF32Out ? 1.1 : 1.0;
+}
+
 // The fastest of both shapes and 1 to max_slices slices of K, whose time replaces *us;
 // false when none takes *us or less.
 template <typename Cfg>
@@ -731,28 +748,22 @@ template <typename Cfg>
 int launch(RowMajorArgs p, hipStream_t s) {
   constexpr int kStep = 64 / Cfg::kElemBytes;                     // elements of K per step
   const int64_t rows = (int64_t)p.M1 * p.M0, cols = (int64_t)p.N1 * p.N0;
-  // The chain on full tiles is taken where its estimate is the shorter. 16-bit types with rows
-  // of b of whole 128-byte lines and results of up to 6 million elements: by 1.15 times, since
-  // there the estimate of one launch, fitted mostly to odd sizes, is too long (298 problems
-  // take 0.70 to 1.06 of it, 0.91 in the middle, odd columns 1.02). On 433 of them 1.8 % from
-  // the faster of the two on average and 4 over 10 % longer than as before this chain, without
-  // it 2.2 % and 19 (f16 480x4736x146 11.1 us in one launch, 14.5 as the chain); odd columns
-  // lose by it, 0.6 -> 2.6 %. Whole 8 KiB: 1.35 times; one launch takes 0.56 to 1.0 of its
-  // estimate, 0.75 in the middle, and the chain packs each operand by its own launch. On 420 of
-  // those 1.8 % from the faster and 1.41 times its time at most, without it 4.9 % and 1.75
-  // times (bf16 130x8192x523 11.6 us in one launch, 21.1 as the chain); with larger results
-  // among them 2.5 % (bf16 added to C 3874x4096x357 70 us in one launch, 52 as a chain).
+  // The chain on full tiles is taken where its estimate is the shorter, 16-bit types by
+  // times_shorter: there the estimate of one launch is the longer by as much where the two are
+  // near each other, more with f32 results and with rows of b of whole cache lines. On 1236
+  // problems 1.1 % from the faster of the two on average and 3 over 10 % longer than before
+  // this chain had an estimate of its own, without it 2.7 % and 41; on 400 others none (bf16 130x8192x523 11.6 us in
+  // one launch, 21.1 as the chain; f16 480x4736x146 11.1 and 14.5; 838x2220x468 13.6 and 16.3).
   // f32 (the chain as it was fitted packed the operands one after the other; in one launch
   // they take 2.0 to 3.5 us less) takes longer as the chain than estimated, for results of up
   // to 3 million elements; on 2343 problems 2.6 % from the best kernel on average and 5 over
   // 20 % longer than as the chain, with 0.9 of it 3.1 % and 4, and 531x2782x605 42.0 us as the
   // chain, 27.8 in one launch.
   const bool full = full_tiles_chain<Cfg>(p);
-  const bool whole_lines = Cfg::kElemBytes == 2 && p.N % 64 == 0 && rows * cols <= 6000000;
   const double chain = full ? full_tiles_chain_us<Cfg>(p) : chain_us<Cfg>(p);
   const bool together = p.lhs && p.rhs && p.out && p.M0 == 32 && p.N0 == 32;
   const bool slow_chain = Cfg::kElemBytes == 4 && rows * cols <= 3000000;
-  const double limit = full                       ? (!whole_lines ? 1.0 : p.N % 4096 ? 1.15 : 1.35) * chain
+  const double limit = full                       ? times_shorter<Cfg>(p) * chain
                        : together && chain < 24.0 ? chain - 2.4
                                                   : (slow_chain ? 1.1 : 0.9) * chain;
   int mb = 1, slices = 1;

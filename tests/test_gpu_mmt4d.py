@@ -1819,10 +1819,12 @@ def test_scaled_rows_on_either_kernel(uk, cuda, type_flag, dt, M, N, K, narrow):
     (F.MMT4D_TYPE_BF16BF16BF16, "bfloat16", "bfloat16", 900, 4096, 2000, True, "mmt4d:mfma"),
     (F.MMT4D_TYPE_F16F16F32, "float16", "float32", 480, 4736, 146, False, "mmt4d:mfma-one-launch"),
     (F.MMT4D_TYPE_F16F16F16, "float16", "float16", 1000, 1984, 1500, True, "mmt4d:mfma"),
+    (F.MMT4D_TYPE_BF16BF16F32, "bfloat16", "float32", 1547, 1297, 166, False, "mmt4d:mfma-one-launch"),
+    (F.MMT4D_TYPE_BF16BF16F32, "bfloat16", "float32", 1547, 1297, 1166, False, "mmt4d:mfma"),
 ])
-def test_b_of_whole_lines(uk, cuda, type_flag, dt, out_dt, M, N, K, accumulate, path):
-    """Rows of B of whole lines and of whole 8 KiB: one launch where the chain takes a third to
-    half as long again, and the chain. Small whole numbers: the same bits as step by step."""
+def test_one_launch_near_the_chain(uk, cuda, type_flag, dt, out_dt, M, N, K, accumulate, path):
+    """Rows of B of whole 8 KiB, of whole lines and others: one launch where the chain takes a
+    fifth to half as long again, and the chain. Small whole numbers: the same bits as step by step."""
     import torch
     g = torch.Generator(device="cuda").manual_seed(M + N + K)
     a = torch.randint(-1, 2, (M * K,), generator=g, device="cuda").to(getattr(torch, dt))
