@@ -684,11 +684,15 @@ double full_tiles_chain_us(const RowMajorArgs& p) {
 // results, 1.09, 1.01 and 0.90 for 16-bit ones, and is larger where C is added; the
 // factors are those that gave the shortest times in all. Not for results of more than 24 MB (f32)
 // or 6 MB, which lose by it (bf16 added to C 3874x4096x357 70 us in one launch, 52 as a chain).
+// int8 that is not added to C: 0.93, with rows of whole 64 bytes 0.81 (8 KiB 0.89, where it
+// gave nothing); of 300 other problems 7 instead of 16 over 5 % longer than before the chain's
+// own estimate (715x3648x157 11.7 us in one launch, 14.9 as the chain).
 template <typename Cfg>
 double times_shorter(const RowMajorArgs& p) {
   constexpr bool kF32Out = sizeof(typename Cfg::out_t) == 4;
   const int64_t elems = (int64_t)p.M1 * p.M0 * p.N1 * p.N0;
-  if (Cfg::kElemBytes != 2 || elems > (kF32Out ? 6000000 : 3000000)) return 1.0;
+  if (Cfg::kElemBytes == 1) return p.accumulate || p.N % 4096 == 0 ? 1.0 : p.N % 64 == 0 ? 1.2 : 1.05;
+  if (elems > (kF32Out ? 6000000 : 3000000)) return 1.0;
   if (p.N % 4096 == 0) return kF32Out ? 1.4 : 1.2;
   if (p.N % 64 == 0) return kF32Out && !p.accumulate ? 1.25 : 1.1;
   return kF32Out ? 1.1 : 1.0;
@@ -748,10 +752,9 @@ template <typename Cfg>
 int launch(RowMajorArgs p, hipStream_t s) {
   constexpr int kStep = 64 / Cfg::kElemBytes;                     // elements of K per step
   const int64_t rows = (int64_t)p.M1 * p.M0, cols = (int64_t)p.N1 * p.N0;
-  // The chain on full tiles is taken where its estimate is the shorter, 16-bit types by
-  // times_shorter: there the estimate of one launch is the longer by as much where the two are
-  // near each other, more with f32 results and with rows of b of whole cache lines. On 1236
-  // problems 1.1 % from the faster of the two on average and 3 over 10 % longer than before
+  // The chain on full tiles is taken where its estimate is the shorter by times_shorter: the
+  // estimate of one launch is the longer by as much where the two are near each other, more
+  // with f32 results and with rows of b of whole cache lines. On 1236 problems of 16-bit types 1.1 % from the faster of the two on average and 3 over 10 % longer than before
   // this chain had an estimate of its own, without it 2.7 % and 41; on 400 others none (bf16 130x8192x523 11.6 us in
   // one launch, 21.1 as the chain; f16 480x4736x146 11.1 and 14.5; 838x2220x468 13.6 and 16.3).
   // f32 (the chain as it was fitted packed the operands one after the other; in one launch

@@ -1821,6 +1821,8 @@ def test_scaled_rows_on_either_kernel(uk, cuda, type_flag, dt, M, N, K, narrow):
     (F.MMT4D_TYPE_F16F16F16, "float16", "float16", 1000, 1984, 1500, True, "mmt4d:mfma"),
     (F.MMT4D_TYPE_BF16BF16F32, "bfloat16", "float32", 1547, 1297, 166, False, "mmt4d:mfma-one-launch"),
     (F.MMT4D_TYPE_BF16BF16F32, "bfloat16", "float32", 1547, 1297, 1166, False, "mmt4d:mfma"),
+    (F.MMT4D_TYPE_S8S8S32, "int8", "int32", 715, 3648, 157, False, "mmt4d:mfma-one-launch"),
+    (F.MMT4D_TYPE_S8S8S32, "int8", "int32", 715, 3648, 1570, False, "mmt4d:mfma"),
 ])
 def test_one_launch_near_the_chain(uk, cuda, type_flag, dt, out_dt, M, N, K, accumulate, path):
     """Rows of B of whole 8 KiB, of whole lines and others: one launch where the chain takes a
