@@ -659,10 +659,9 @@ double chain_us(const RowMajorArgs& p) {
 
 // The chain on full tiles whose matmul writes C beside the packed result
 // (launch_matmul_chain): two launches. Fitted to 18000 problems (33 to 4096 rows and
-// columns, K 16 to 4096), 11 to 12 % off on average; on 7000 others the faster of the two
-// is taken but for the noise of their timing (4 %), 1.19 times its time in the 99th
-// percentile, where the fit of three launches above left 1.30. f32, whose matrix
-// instructions weigh more than the launches, keeps that one.
+// columns, K 16 to 4096), 11 to 12 % off on average; see times_shorter for what that leaves.
+// f32 keeps the fit above, which counts an unpack (and a pack of C) that its chain no longer
+// launches; it has not been fitted again.
 template <typename Cfg>
 bool full_tiles_chain(const RowMajorArgs& p) {
   return Cfg::kElemBytes != 4 && p.lhs && p.rhs && p.out && p.M0 == 32 && p.N0 == 32;
@@ -754,9 +753,11 @@ int launch(RowMajorArgs p, hipStream_t s) {
   const int64_t rows = (int64_t)p.M1 * p.M0, cols = (int64_t)p.N1 * p.N0;
   // The chain on full tiles is taken where its estimate is the shorter by times_shorter: the
   // estimate of one launch is the longer by as much where the two are near each other, more
-  // with f32 results and with rows of b of whole cache lines. On 1236 problems of 16-bit types 1.1 % from the faster of the two on average and 3 over 10 % longer than before
-  // this chain had an estimate of its own, without it 2.7 % and 41; on 400 others none (bf16 130x8192x523 11.6 us in
-  // one launch, 21.1 as the chain; f16 480x4736x146 11.1 and 14.5; 838x2220x468 13.6 and 16.3).
+  // with f32 results and with rows of b of whole cache lines. On 1236 problems of 16-bit types
+  // 1.1 % from the faster of the two on average and 3 over 10 % longer than before this chain
+  // had an estimate of its own, without it 2.7 % and 41; on 400 others none (bf16 130x8192x523
+  // 11.6 us in one launch, 21.1 as the chain; f16 480x4736x146 11.1 and 14.5; 838x2220x468
+  // 13.6 and 16.3).
   // f32 (the chain as it was fitted packed the operands one after the other; in one launch
   // they take 2.0 to 3.5 us less) takes longer as the chain than estimated, for results of up
   // to 3 million elements; on 2343 problems 2.6 % from the best kernel on average and 5 over
@@ -857,9 +858,9 @@ int launch_matmul_chain(const void* a, const void* b, void* c, void* lhs, void* 
   if (M0 == 32 && N0 == 32) {
     // The matmul writes the matrix beside the tiles (and adds to the matrix itself), and
     // the launch that would read the tiles back (and the one that packs C) is not needed:
-    // bf16 1999 x 4099 x 3001 72.5 -> 69.7 us, f16 2048^3 with f16 results 38.4 -> 34.8,
-    // 1000 x 4000 x 3000 added to C 56.1 -> 49.5, i8 4096^3 96 -> 89, 2000 x 3000 x 1000
-    // 29.6 -> 27.1. What is left of the unpack is its store, at the rate of memory: all
+    // bf16 1999 x 4099 x 3001 67.1 -> 63.3 us, f16 2048^3 with f16 results 34.6 -> 31.1,
+    // 1000 x 4000 x 3000 added to C 51.0 -> 44.7, i8 4096^3 96.2 -> 85.7, 2000 x 3000 x 1000
+    // 30.5 -> 26.0. What is left of the unpack is its store, at the rate of memory: all
     // workgroups of a round store at once.
     const iree_amd_uk_mmt4d_params_t p = {lhs, 0, K1 * M0 * K0, rhs, 0, K1 * N0 * K0, c, 0, N, M1, N1, K1, M0, N0, K0,
                                           flags, nullptr};

@@ -249,21 +249,22 @@ int launch_dequant_matmul_i4(const void* x, const void* w, const void* scale, co
                        ((uintptr_t)scale % 16) == 0 && ((uintptr_t)zp % 16) == 0;
   // More than 64 rows (a prompt): the tiled kernel of uk_quant_gemm.hip, where
   // the kernels below stream the weights again for every 32 rows (N = 14336,
-  // K = 4096: 128 rows 46.2 -> 28.5 us, 512 183 -> 66). Both sides on 1900 problems
+  // K = 4096: 128 rows 46.2 -> 28.5 us, 512 183 -> 66.9). Both sides on 1900 problems
   // of 33 to 128 rows, times of the kernels below over those of the tiled one: from
   // 65 rows at least 1.08 with groups of 64 and more and 0.94 with groups of 32 (96
   // x 7424 x 2048: 18.5 and 19.9 us). At 33 to 64 rows whichever is estimated to be
   // the faster: on 9700 problems 0.80 times the time of the kernels below on average,
-  // 0.4 % from the faster of the two and 16 problems over 4 % slower than there (10 %
-  // at most). 59 x 2496 x 13056 with groups of 64 23.2 -> 17.0 us, 40 x 5120 x 2304
-  // 15.0 -> 11.0; 36 x 6528 x 2048 stays below, 9.8 against 11.7.
+  // 0.4 % from the faster of the two and 16 problems over 4 % slower than there. 59 x 2496
+  // x 13056 with groups of 64 23.2 -> 17.0 us, 40 x 5120 x 2304 15.0 -> 11.0; 36 x 6528
+  // x 2048 stays below, 9.8 against 11.7.
   // (an empty K, whose result is zeros, is the element-wise kernel's)
   if (M > 32 && tiled && a.zp_u4 && gs_ok && K > 0 && K % 128 == 0 && size_ok && aligned) {
     a.w_bytes = (uint32_t)w_bytes;
     // (up to 48 rows, whose second pass is the short one, and groups of 32: of 115 problems 8
     // took 2 to 8 % longer on the tiled kernel, with 3 % less to beat 2, which gives up a
     // fortieth of its gain; the other rows and groups 1 of 275)
-    const double limit_us = M > 64 || !k_ok ? 0.0 : (M <= 48 && a.log2_gs == 5 ? 0.97 : 1.0) * two_passes_us(a, slice_kb, (int)k_rows);
+    const double less = M <= 48 && a.log2_gs == 5 ? 0.97 : 1.0;
+    const double limit_us = M > 64 || !k_ok ? 0.0 : less * two_passes_us(a, slice_kb, (int)k_rows);
     const int st = launch_dequant_gemm_i4(a, limit_us, s);
     if (st != IREE_AMD_UK_STATUS_NOT_FOUND) { note_kernel_path("dequant_i4:gemm"); return st; }
   }
