@@ -83,6 +83,10 @@ __device__ __forceinline__ void gemm_wait_vmcnt() {
   asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
 }
 
+// Every load and LDS access of the wave (vmcnt and lgkmcnt 0, expcnt not waited for): as the
+// builtin, which becomes one instruction with the wait of the barrier behind it.
+__device__ __forceinline__ void gemm_wait_all() { __builtin_amdgcn_s_waitcnt(0x0070); }
+
 // 8 nibbles of one dword -> 8 f16 integers (nibble - zero point) in k order: a
 // byte permute puts both nibbles of a byte into the two halves, (t & mask) |
 // 0x6400'6400 makes them 1024 + n and 1024 + 16 n', and one packed FMA with
@@ -317,7 +321,7 @@ __device__ __forceinline__ void dequant_matmul_i4_gemm_body(const I4GemmArgs& a)
   // (the first span's rows come from every wave; and step 0 counts on all of this: its
   // wait for span 1 allows for a step's loads before it, its wait for a refill, which may
   // be the last thing requested here, for a step's activations behind it)
-  gemm_wait_vmcnt<0>();
+  gemm_wait_all();
   __syncthreads();
   read_block(0, 0);
 #pragma unroll
@@ -525,7 +529,7 @@ __device__ __forceinline__ void dequant_matmul_i4_gemm_small_body(const I4GemmAr
   params.convert_first(s0);
   // (as above: the first span's rows come from every wave, and the waits of step 0 allow
   // for loads that only later steps have behind them)
-  gemm_wait_vmcnt<0>();
+  gemm_wait_all();
   __syncthreads();
   auto read_pair = [&](int from, int xp) {
 #pragma unroll

@@ -395,7 +395,7 @@ def test_int4_tiled_kernels_wait_for_what_the_first_step_reads():
     starts = source.split("params.convert_first(s0);")[1:]
     assert len(starts) == 2
     for start in starts:
-        assert "gemm_wait_vmcnt<0>();" in start[:start.index("__syncthreads();")]
+        assert "gemm_wait_all();" in start[:start.index("__syncthreads();")]
 
 
 @pytest.mark.parametrize("form,calls", [
